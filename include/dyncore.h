@@ -162,7 +162,10 @@ void *dyn_stream(dyn_ctx *ctx);
 /* ---- launch-shape parameters ------------------------------------------------------------- */
 /* Knobs of the fused kernels (no counterpart in the reference: they set how the work maps onto the
  * GPU, never what is computed).  0 restores the built-in default; a value the kernels do not support
- * returns DYN_E_ARG.  Setting a knob drops the captured step graph. */
+ * returns DYN_E_ARG.  Setting a knob drops the captured step graph.  dyn_tune_get returns a knob's value or
+ * its nominal default.  While the knobs of a stage kernel are unset, grids whose nominal blocks would leave
+ * compute units idle, and level counts far from a wavefront's 64 lanes, are launched in a shape chosen from
+ * the grid's size instead, and DYN_TUNE_STAGE_STREAMS likewise; the values computed never depend on it. */
 enum {
     DYN_TUNE_MOMENTUM_TJ = 0, /* j-rows per block of the momentum stage kernel: 2, 4, 8 or 16 (16, like 8,
                                  only with one wavefront per column) */

@@ -869,7 +869,7 @@ static int fused_step(dyn_ctx *ctx, StageHook hook = nullptr, void *arg = nullpt
     // first pass instead (2.08 -> 1.99 ms per FP64 step at 256x256x64; elsewhere neutral or slower).
     // Value 4 keeps the fork after the momentum kernel but queues (and captures) the scalar launches
     // after the solve's first pass, which measured faster for FP64 on the other grids.
-    const int streams = fused_shape(c, DYN_TUNE_STAGE_STREAMS);
+    const int streams = stage_streams(c);
     const bool two = streams >= 2, late = streams >= 3;
     // With shared roles on two streams, the copy into stage 2's output buffer runs during stage 1, on
     // the second stream after the scalar half: it reads the step's starting state and writes the spare

@@ -1,12 +1,11 @@
 // Fused stage advection for gfx950: advect_uvw_velocity + advect_theta + advect_microphysics_cell
 // (+ the fall speed and the interior part of zero_moisture) in one pass over HBM.
 //
-// Mapping: one 64-lane wavefront per j-row, lane = level k (NZ <= 64; two wavefronts for 66 <= NZ <= 128,
-// which hand the values crossing levels 63/64 over in LDS); a block of TJ rows marches
-// along i over a chunk of TI columns, as the reference's slab loop does (advection.cpp:313-325):
+// Mapping: a block of tj j-rows, one lane per level of a row (RowMap), marches along i over a chunk of ti
+// columns, as the reference's slab loop does (advection.cpp:313-325):
 //   * i-stencils come from per-thread register queues (own j,k; columns i-3..i+3) and the east-face
 //     flux of column i is carried as the west face of column i+1 (fluxes.cpp:891,1322,1504);
-//   * j- and k-stencils read LDS planes of TJ+6 rows; U/UB are kept for planes i and i+1, V/VB/W/WB for
+//   * j- and k-stencils read LDS planes of tj+6 rows; U/UB are kept for planes i and i+1, V/VB/W/WB for
 //     planes i-1 and i (staggered advecting velocities), the scalars for plane i;
 //   * north and top faces are computed once per point and exchanged through LDS as the south and
 //     bottom faces of the neighbours.
@@ -35,8 +34,8 @@ __device__ __forceinline__ T i2(T p0, T p1) { return T(0.5) * (p1 + p0); }
 // Neighbouring levels of a column sit in neighbouring lanes.  Level k+1 and level k-1 come by the
 // wavefront shifts of DPP (wave_shl:1 and wave_shr:1, a modifier of a VALU move: no LDS round trip); a
 // lane whose source lies outside the wavefront keeps its own value.  That is the clamp the callers want at
-// level 0 and at the last lane, and the wavefront boundary of a two-wavefront column is overwritten from
-// LDS by the callers.  Lanes past NZ-1 hold the values loaded at level NZ-1 (clamped loads) or values no
+// level 0 and at the last lane, and where packed rows cross a wavefront's edge the callers overwrite it
+// from LDS.  Lanes past NZ-1 hold the values loaded at level NZ-1 (clamped loads) or values no
 // active lane reads.  A fixed level comes by readlane (lane index uniform).
 __device__ __forceinline__ int dpp_next(int x) { return __builtin_amdgcn_update_dpp(x, x, 0x130, 0xf, 0xf, false); }
 __device__ __forceinline__ int dpp_prev(int x) { return __builtin_amdgcn_update_dpp(x, x, 0x138, 0xf, 0xf, false); }
@@ -82,38 +81,98 @@ struct StageArgs {
     int il, ih, jl, jh;   // advected box
     int ti;               // columns one block marches
     int nbj;              // j-blocks
+    int tj;               // rows per block
 };
+
+// Rows of a block.  Two mappings of levels and rows onto lanes, chosen on the host by the level count:
+//   * one wavefront per row (PACK false, 57 <= NZ <= 64): lane = level, TJ rows per block;
+//   * packed rows (PACK true, every other NZ up to 128): the block's rows lie one after another over its
+//     lanes, lane q holding level q % NZ of row q / NZ.  A 40-level column fills 40 lanes instead of 64 and
+//     an 80-level one 80 instead of 128; what bounds these kernels is the instructions each wavefront
+//     issues, so an idle lane costs as much as a busy one.  A wavefront's edge may fall anywhere in a
+//     column: the values that cross it go through a few LDS words (xch, xw, xb).
+// Measured against a wavefront (two above 64 levels) per row, each at its best launch shape, FP32 moist: the
+// momentum and scalar kernels 34 and 47 -> 26 and 37 us at 192x192x40, 57 and 74 -> 33 and 48 us at
+// 160x120x90; FP64 78 and 159 -> 53 and 107 us at 192x192x40.
+template <int TJ, bool PACK>
+struct RowMap {
+    int tj;     // rows per block
+    int pitch;  // lanes (and LDS words of one field) per row
+    int r, k;   // this lane's row and level; packed lanes past the last row repeat its last level
+    int wave, lane;
+    __device__ __forceinline__ RowMap(int tj_, int NZ) {
+        tj = PACK ? tj_ : TJ;
+        pitch = PACK ? NZ : KP;
+        if (PACK) {
+            const int q = min((int)threadIdx.x, tj * NZ - 1);
+            r = q / NZ;
+            k = q - r * NZ;
+            wave = threadIdx.x / KP;
+            lane = threadIdx.x % KP;
+        } else {
+            r = threadIdx.y;
+            k = threadIdx.x;
+            wave = r;
+            lane = k;
+        }
+    }
+};
+// halo rows (and W rows) a lane loads: a block of tj rows has six halo rows and tj + 1 W rows
+template <int TJ>
+constexpr int halo_loads() { return TJ >= 6 ? 1 : TJ >= 3 ? 2 : 3; }
+
+// Two or four neighbouring LDS words in one access (the addresses are multiples of the access's size)
+template <typename T>
+struct LdsVec;
+template <>
+struct LdsVec<float> {
+    typedef float v2 __attribute__((ext_vector_type(2)));
+};
+template <>
+struct LdsVec<double> {
+    typedef double v2 __attribute__((ext_vector_type(2)));
+};
+template <typename T>
+__device__ __forceinline__ void lds_ld2(const T *p, T &x, T &y) {
+    const typename LdsVec<T>::v2 v = *(const typename LdsVec<T>::v2 *)p;
+    x = v.x;
+    y = v.y;
+}
+template <typename T>
+__device__ __forceinline__ void lds_st2(T *p, T x, T y) {
+    typename LdsVec<T>::v2 v;
+    v.x = x;
+    v.y = y;
+    *(typename LdsVec<T>::v2 *)p = v;
+}
 
 // ---- momentum: advect_uvw_velocity (u, v fluxes and Coriolis; w = buoyancy, advection.cpp:304-339) -------
-// LDS: U UB (planes i, i+1) and V VB (planes i-1, i) on rows j0-3 .. j0+TJ+2, W WB (planes i-1, i) on rows
-// j0-1 .. j0+TJ-1, each in a ring of three slots (plane p in slot p % 3); north faces of rows j0-1 .. j0+TJ-1.
+// LDS: (U, UB) of planes i, i+1 and (V, VB) of planes i-1, i on rows j0-3 .. j0+tj+2, (W, WB) of planes i-1, i
+// on rows j0-1 .. j0+tj-1, each in a ring of three slots (plane p in slot p % 3); north faces of rows
+// j0-1 .. j0+tj-1.  The fields of a pair lie side by side, so one LDS access moves both.
 // Register queues hold U UB V VB of the own row at columns i-2 .. i+3.
-template <typename T, int TJ, int KW = 1>
+template <typename T>
 struct MomLds {
-    static constexpr int KPW = KP * KW;
-    static constexpr int R = TJ + 6;
-    static constexpr int RW = TJ + 1;
-    static constexpr size_t uv = 3 * 4 * (size_t)R * KPW;    // [slot][U UB V VB][row][k]
-    static constexpr size_t w = 3 * 2 * (size_t)RW * KPW;    // [slot][W WB][row][k]
-    static constexpr size_t nf = 2 * (size_t)(TJ + 1) * KPW; // [u v][row + 1][k]
-    static constexpr size_t x = KW == 2 ? 3 * (size_t)TJ : 0;  // [row][bu bv bk] from level 63 to 64
-    static constexpr size_t bytes = (uv + w + nf + x) * sizeof(T);
+    __host__ __device__ static constexpr size_t uv(int tj, int pitch) { return 3 * 4 * (size_t)(tj + 6) * pitch; }  // [slot][u, v][row][k][2]
+    __host__ __device__ static constexpr size_t w(int tj, int pitch) { return 3 * 2 * (size_t)(tj + 1) * pitch; }   // [slot][row][k][2]
+    __host__ __device__ static constexpr size_t nf(int tj, int pitch) { return 2 * (size_t)(tj + 1) * pitch; }      // [row + 1][k][u v]
+    static constexpr size_t x = 3 * 16;  // packed rows: top faces and buoyancy from each wavefront to the next
+    static constexpr size_t bytes(int tj, int pitch) { return (uv(tj, pitch) + w(tj, pitch) + nf(tj, pitch) + x) * sizeof(T); }
 };
 
-// one tile (TJ rows x ti columns x all levels) of the momentum stage; every thread of the block calls it
-template <typename T, int TJ, bool MOIST, int KW = 1>
+// one tile (tj rows x ti columns x all levels) of the momentum stage; every thread of the block calls it
+template <typename T, int TJ, bool MOIST, bool PACK>
 __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, const StageArgs &a, T step, int t, unsigned char *smem_raw) {
-    using L = MomLds<T, TJ, KW>;
-    constexpr int KPW = L::KPW;
-    constexpr int R = L::R, RW = L::RW;
-    constexpr int HH = (6 + TJ - 1) / TJ, HW = (RW + TJ - 1) / TJ;  // halo / W plane rows per wavefront
+    const RowMap<TJ, PACK> map(a.tj, g.NZ);
+    const int tj = map.tj, KPW = map.pitch, k = map.k, r = map.r;
+    const int R = tj + 6, RW = tj + 1;
+    constexpr int HH = halo_loads<TJ>(), HW = 2;  // halo / W plane rows per lane
     T *uvp = (T *)smem_raw;
-    T *wpl = uvp + L::uv;
-    T *nface = wpl + L::w;
-    T *xch = nface + L::nf;
+    T *wpl = uvp + MomLds<T>::uv(tj, KPW);
+    T *nface = wpl + MomLds<T>::w(tj, KPW);
+    T *xch = nface + MomLds<T>::nf(tj, KPW);
 
-    const int k = threadIdx.x, r = threadIdx.y;
-    const int j0 = a.jl + (t % a.nbj) * TJ;
+    const int j0 = a.jl + (t % a.nbj) * tj;
     const int i0 = a.il + (t / a.nbj) * a.ti;
     const int i1 = min(i0 + a.ti, a.ih);
     const int NZ = g.NZ, NY = g.NY;
@@ -125,20 +184,21 @@ __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, c
     const unsigned rowoff = (unsigned)(jc * NZ + kc);
     const int RO = r + 3, WO = r + 1;  // own row in the U/V and W planes
 
-    auto UV = [&](int slot, int f, int row) -> T * { return uvp + ((slot * 4 + f) * R + row) * KPW; };
-    auto WW = [&](int slot, int f, int row) -> T * { return wpl + ((slot * 2 + f) * RW + row) * KPW; };
+    // the pair (U, UB) (p = 0) or (V, VB) (p = 1), and (W, WB), of a plane row at level kk
+    auto UV = [&](int slot, int p, int row, int kk) -> T * { return uvp + (((slot * 2 + p) * R + row) * KPW + kk) * 2; };
+    auto WW = [&](int slot, int row, int kk) -> T * { return wpl + ((slot * RW + row) * KPW + kk) * 2; };
     const void *qsrc[4] = {a.cur[0], a.bar[0], a.cur[1], a.bar[1]};
     T q[4][6], qs[4];  // U UB V VB of the own row at columns i-2 .. i+3 (i-3 .. i+2 in the prologue)
 
     // plane rows: U UB of plane iu, V VB W WB of plane iv.  The own row of U UB V VB comes from the
-    // queues (which hold those columns already); only the six halo rows j0-3..j0-1, j0+TJ..j0+TJ+2 are
+    // queues (which hold those columns already); only the six halo rows j0-3..j0-1, j0+tj..j0+tj+2 are
     // loaded
-    auto halo_row = [&](int hh) { return hh < 3 ? hh : TJ + hh; };
+    auto halo_row = [&](int hh) { return hh < 3 ? hh : tj + hh; };
     T su[HH][4], sw[HW][2];
     auto fetch_planes = [&](int iu, int iv) {
 #pragma unroll
         for (int h = 0; h < HH; h++) {
-            const int hh = r + h * TJ;
+            const int hh = r + h * tj;
             if (hh < 6) {
                 const int rr = halo_row(hh);
                 const int jj = min(max(j0 - 3 + rr, 0), NY - 1);
@@ -151,7 +211,7 @@ __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, c
         }
 #pragma unroll
         for (int h = 0; h < HW; h++) {
-            const int rr = r + h * TJ;
+            const int rr = r + h * tj;
             if (rr < RW) {
                 const int jj = min(max(j0 - 1 + rr, 0), NY - 1);
                 const unsigned pv = (unsigned)iv * NYNZ + (unsigned)(jj * NZ + kc);
@@ -163,28 +223,21 @@ __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, c
     // qu, qv: queue positions of columns iu and iv
     auto store_planes = [&](int iu, int iv, int qu, int qv) {
         const int su_slot = iu % 3, sv_slot = iv % 3;
-        UV(su_slot, 0, RO)[k] = q[0][qu];
-        UV(su_slot, 1, RO)[k] = q[1][qu];
-        UV(sv_slot, 2, RO)[k] = q[2][qv];
-        UV(sv_slot, 3, RO)[k] = q[3][qv];
+        lds_st2(UV(su_slot, 0, RO, k), q[0][qu], q[1][qu]);
+        lds_st2(UV(sv_slot, 1, RO, k), q[2][qv], q[3][qv]);
 #pragma unroll
         for (int h = 0; h < HH; h++) {
-            const int hh = r + h * TJ;
+            const int hh = r + h * tj;
             if (hh < 6) {
                 const int rr = halo_row(hh);
-                UV(su_slot, 0, rr)[k] = su[h][0];
-                UV(su_slot, 1, rr)[k] = su[h][1];
-                UV(sv_slot, 2, rr)[k] = su[h][2];
-                UV(sv_slot, 3, rr)[k] = su[h][3];
+                lds_st2(UV(su_slot, 0, rr, k), su[h][0], su[h][1]);
+                lds_st2(UV(sv_slot, 1, rr, k), su[h][2], su[h][3]);
             }
         }
 #pragma unroll
         for (int h = 0; h < HW; h++) {
-            const int rr = r + h * TJ;
-            if (rr < RW) {
-                WW(sv_slot, 0, rr)[k] = sw[h][0];
-                WW(sv_slot, 1, rr)[k] = sw[h][1];
-            }
+            const int rr = r + h * tj;
+            if (rr < RW) lds_st2(WW(sv_slot, rr, k), sw[h][0], sw[h][1]);
         }
     };
     // own-column inputs of column i: the buoyancy term's theta', qv, qc, qr and the M values of u, v, w
@@ -221,9 +274,11 @@ __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, c
     const T tbvk = T(c.tbv[kc]);
     const bool low = (k == 1 || k == NZ - 2);
 
-    // east faces of the queue's centre column (u_east, v_east; fluxes.cpp:1384-1592); Ujm1/UBjm1: row j-1 of
-    // the U planes at the column east of the centre
-    auto east_faces = [&](const T *Ujm1, const T *UBjm1, T *e) {
+    // east faces of the queue's centre column (u_east, v_east; fluxes.cpp:1384-1592); slot: the U plane of the
+    // column east of the centre, read at row j-1
+    auto east_faces = [&](int slot, T *e) {
+        T Ujm1, UBjm1;
+        lds_ld2(UV(slot, 0, RO - 1, k), Ujm1, UBjm1);
         {
             T ua = T(0.5) * (q[0][3] + q[0][2]);
             T uba = T(0.5) * (q[1][3] + q[1][2]);
@@ -232,8 +287,8 @@ __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, c
             e[0] = ua * ube + (uba + ua) * ue;
         }
         {
-            T ua = T(0.5) * (q[0][3] + Ujm1[k]);
-            T uba = T(0.5) * (q[1][3] + UBjm1[k]);
+            T ua = T(0.5) * (q[0][3] + Ujm1);
+            T uba = T(0.5) * (q[1][3] + UBjm1);
             T ve = i5(q[2][0], q[2][1], q[2][2], q[2][3], q[2][4], q[2][5], sgn(uba + ua));
             T vbe = i5(q[3][0], q[3][1], q[3][2], q[3][3], q[3][4], q[3][5], sgn(ua));
             e[1] = ua * vbe + (uba + ua) * ve;
@@ -241,7 +296,7 @@ __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, c
     };
     __syncthreads();
     T west[2], east[2];
-    east_faces(UV(i0 % 3, 0, RO - 1), UV(i0 % 3, 1, RO - 1), west);  // column i0-1
+    east_faces(i0 % 3, west);  // column i0-1
 #pragma unroll
     for (int f = 0; f < 4; f++) {
 #pragma unroll
@@ -265,69 +320,66 @@ __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, c
         }
         const T um = cb[4], vm = cb[5], wm = cb[6];
 
-        east_faces(UV(cp1, 0, RO - 1), UV(cp1, 1, RO - 1), east);
+        east_faces(cp1, east);
         // north faces (u_north, v_north) of row RR of the U/V planes
         auto north_faces = [&](int RR, T *nf) {
-            const T *U0 = UV(c0, 0, 0), *UB0 = UV(c0, 1, 0), *V0 = UV(c0, 2, 0), *VB0 = UV(c0, 3, 0);
-            const T *Vm = UV(cm1, 2, 0), *VBm = UV(cm1, 3, 0);
-#define PL(ptr, row) ptr[(row) * KPW + k]
+            T v[6], vb[6], vm1, vbm1;
+#pragma unroll
+            for (int d = 0; d < 6; d++) lds_ld2(UV(c0, 1, RR - 2 + d, k), v[d], vb[d]);
+            lds_ld2(UV(cm1, 1, RR + 1, k), vm1, vbm1);
             {
-                T va = T(0.5) * (PL(V0, RR + 1) + PL(Vm, RR + 1));
-                T vba = T(0.5) * (PL(VB0, RR + 1) + PL(VBm, RR + 1));
-                T un = i5(PL(U0, RR - 2), PL(U0, RR - 1), PL(U0, RR), PL(U0, RR + 1), PL(U0, RR + 2), PL(U0, RR + 3), sgn(vba + va));
-                T ubn = i5(PL(UB0, RR - 2), PL(UB0, RR - 1), PL(UB0, RR), PL(UB0, RR + 1), PL(UB0, RR + 2), PL(UB0, RR + 3), sgn(va));
-                nf[0] = va * ubn + (vba + va) * un;
-            }
-            {
-                T va = T(0.5) * (PL(V0, RR + 1) + PL(V0, RR));
-                T vba = T(0.5) * (PL(VB0, RR + 1) + PL(VB0, RR));
-                T vn = i5(PL(V0, RR - 2), PL(V0, RR - 1), PL(V0, RR), PL(V0, RR + 1), PL(V0, RR + 2), PL(V0, RR + 3), sgn(vba + va));
-                T vbn = i5(PL(VB0, RR - 2), PL(VB0, RR - 1), PL(VB0, RR), PL(VB0, RR + 1), PL(VB0, RR + 2), PL(VB0, RR + 3), sgn(va));
+                T va = T(0.5) * (v[3] + v[2]);
+                T vba = T(0.5) * (vb[3] + vb[2]);
+                T vn = i5(v[0], v[1], v[2], v[3], v[4], v[5], sgn(vba + va));
+                T vbn = i5(vb[0], vb[1], vb[2], vb[3], vb[4], vb[5], sgn(va));
                 nf[1] = va * vbn + (vba + va) * vn;
             }
-#undef PL
+            {
+                T va = T(0.5) * (v[3] + vm1);
+                T vba = T(0.5) * (vb[3] + vbm1);
+#pragma unroll
+                for (int d = 0; d < 6; d++) lds_ld2(UV(c0, 0, RR - 2 + d, k), v[d], vb[d]);
+                T un = i5(v[0], v[1], v[2], v[3], v[4], v[5], sgn(vba + va));
+                T ubn = i5(vb[0], vb[1], vb[2], vb[3], vb[4], vb[5], sgn(va));
+                nf[0] = va * ubn + (vba + va) * un;
+            }
         };
         T nf[2];
         north_faces(RO, nf);
-        nface[(0 * (TJ + 1) + r + 1) * KPW + k] = nf[0];
-        nface[(1 * (TJ + 1) + r + 1) * KPW + k] = nf[1];
+        lds_st2(nface + ((r + 1) * KPW + k) * 2, nf[0], nf[1]);
         if (r == 0) {
             T sf[2];
             north_faces(RO - 1, sf);
-            nface[(0 * (TJ + 1)) * KPW + k] = sf[0];
-            nface[(1 * (TJ + 1)) * KPW + k] = sf[1];
+            lds_st2(nface + k * 2, sf[0], sf[1]);
         }
         // top faces (u_top, v_top) of this level; level 0 has none
         T tf[2];
-        {
-            const T *U0 = UV(c0, 0, RO), *UB0 = UV(c0, 1, RO);
-            const T *W0 = WW(c0, 0, WO), *WB0 = WW(c0, 1, WO), *Wm = WW(cm1, 0, WO), *WBm = WW(cm1, 1, WO);
-            T wa = T(0.5) * (W0[kp1] + Wm[kp1]);
-            T wba = T(0.5) * (WB0[kp1] + WBm[kp1]);
-            T ut, ubt;
+        T w1, wb1;  // w, wbar at k+1
+        lds_ld2(WW(c0, WO, kp1), w1, wb1);
+        auto top_face = [&](int pr, T wo, T wbo) -> T {
+            T wa = T(0.5) * (w1 + wo);
+            T wba = T(0.5) * (wb1 + wbo);
+            T s0, s1, b0, b1, st_, bt;
+            lds_ld2(UV(c0, pr, RO, kc), s0, b0);
+            lds_ld2(UV(c0, pr, RO, kp1), s1, b1);
             if (low) {
-                ut = i2(U0[kc], U0[kp1]);
-                ubt = i2(UB0[kc], UB0[kp1]);
+                st_ = i2(s0, s1);
+                bt = i2(b0, b1);
             } else {
-                ut = i3(U0[km1], U0[kc], U0[kp1], U0[kp2], sgn(wba + wa));
-                ubt = i3(UB0[km1], UB0[kc], UB0[kp1], UB0[kp2], sgn(wa));
+                T sm, bm, s2, b2;
+                lds_ld2(UV(c0, pr, RO, km1), sm, bm);
+                lds_ld2(UV(c0, pr, RO, kp2), s2, b2);
+                st_ = i3(sm, s0, s1, s2, sgn(wba + wa));
+                bt = i3(bm, b0, b1, b2, sgn(wa));
             }
-            tf[0] = wa * ubt + (wba + wa) * ut;
-        }
+            return wa * bt + (wba + wa) * st_;
+        };
         {
-            const T *V0 = UV(c0, 2, RO), *VB0 = UV(c0, 3, RO);
-            const T *W0 = WW(c0, 0, WO), *WB0 = WW(c0, 1, WO), *Wj = WW(c0, 0, WO - 1), *WBj = WW(c0, 1, WO - 1);
-            T wa = T(0.5) * (W0[kp1] + Wj[kp1]);
-            T wba = T(0.5) * (WB0[kp1] + WBj[kp1]);
-            T vt, vbt;
-            if (low) {
-                vt = i2(V0[kc], V0[kp1]);
-                vbt = i2(VB0[kc], VB0[kp1]);
-            } else {
-                vt = i3(V0[km1], V0[kc], V0[kp1], V0[kp2], sgn(wba + wa));
-                vbt = i3(VB0[km1], VB0[kc], VB0[kp1], VB0[kp2], sgn(wa));
-            }
-            tf[1] = wa * vbt + (wba + wa) * vt;
+            T wo, wbo;
+            lds_ld2(WW(cm1, WO, kp1), wo, wbo);
+            tf[0] = top_face(0, wo, wbo);
+            lds_ld2(WW(c0, WO - 1, kp1), wo, wbo);
+            tf[1] = top_face(1, wo, wbo);
         }
         if (k == 0) tf[0] = tf[1] = T(0);
         // bottom face of level k = top face of level k-1; buoyancy of level k-1 (advection.cpp:42-58)
@@ -335,30 +387,29 @@ __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, c
         T bk = cb[0] / tbvk;
         if (MOIST) bk = cb[0] / tbvk + T(0.61) * cb[1] - cb[2] - cb[3];
         T bkm = lane_prev(bk);
-        // two wavefronts per column: level 64 (the second one's first lane) takes level 63's values from LDS
-        if (KW == 2 && k == KP - 1) {
-            xch[3 * r] = tf[0];
-            xch[3 * r + 1] = tf[1];
-            xch[3 * r + 2] = bk;
+        // packed rows: a wavefront's first lane takes the last lane's values of the wavefront before it
+        if (PACK && map.lane == KP - 1) {
+            xch[3 * map.wave] = tf[0];
+            xch[3 * map.wave + 1] = tf[1];
+            xch[3 * map.wave + 2] = bk;
         }
         __syncthreads();
-        if (KW == 2 && k == KP) {
-            bu = xch[3 * r];
-            bv = xch[3 * r + 1];
-            bkm = xch[3 * r + 2];
+        if (PACK && map.lane == 0 && map.wave > 0) {
+            bu = xch[3 * map.wave - 3];
+            bv = xch[3 * map.wave - 2];
+            bkm = xch[3 * map.wave - 1];
         }
         T ou = T(0), ov = T(0), ow = T(0);  // this level's new values, stored after the barrier below
         if (active) {
-            const T su0 = nface[(0 * (TJ + 1) + r) * KPW + k], sv0 = nface[(1 * (TJ + 1) + r) * KPW + k];
+            T su0, sv0;
+            lds_ld2(nface + (r * KPW + k) * 2, su0, sv0);
             {  // u (advection.cpp:73-99)
-                const T *V0 = UV(c0, 2, 0), *Vm = UV(cm1, 2, 0);
-                T other = T(0.25) * (V0[RO * KPW + k] + V0[(RO + 1) * KPW + k] + Vm[RO * KPW + k] + Vm[(RO + 1) * KPW + k]);
+                T other = T(0.25) * (UV(c0, 1, RO, k)[0] + UV(c0, 1, RO + 1, k)[0] + UV(cm1, 1, RO, k)[0] + UV(cm1, 1, RO + 1, k)[0]);
                 T tend = -dtx * (east[0] - west[0]) - dty * (nf[0] - su0) - DTZ * (rw1 * tf[0] - rw0 * bu) * odr + dt * fj * other;
                 ou = um + step * tend;
             }
             {  // v (advection.cpp:104-128)
-                const T *U0 = UV(c0, 0, 0), *Up = UV(cp1, 0, 0);
-                T other = T(0.25) * (U0[RO * KPW + k] + Up[RO * KPW + k] + U0[(RO - 1) * KPW + k] + Up[(RO - 1) * KPW + k]);
+                T other = T(0.25) * (UV(c0, 0, RO, k)[0] + UV(cp1, 0, RO, k)[0] + UV(c0, 0, RO - 1, k)[0] + UV(cp1, 0, RO - 1, k)[0]);
                 T tend = -dtx * (east[1] - west[1]) - dty * (nf[1] - sv0) - DTZ * (rw1 * tf[1] - rw0 * bv) * odr - dt * fj * other;
                 ov = vm + step * tend;
             }
@@ -393,35 +444,34 @@ __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, c
 }
 
 // ---- scalars: advect_theta (+ advect_microphysics_cell, the fall speed and the interior zero_moisture) ----
-// LDS: theta' thetabar (qv qbar qc qr) of plane i on rows j0-3 .. j0+TJ+2 in a ring of two slots, north
-// faces of rows j0-1 .. j0+TJ-1.  Register queues: the same fields of the own row at columns i-2 .. i+3.
-// Own-column inputs (u at i+1, v at j+1, w, the M values) are loaded per wavefront.
-template <typename T, int TJ, bool MOIST, int KW = 1>
+// LDS: the pairs (theta', thetabar) ((qv, qbar), (qc, qr)) of plane i on rows j0-3 .. j0+tj+2 in a ring of two
+// slots, north faces of rows j0-1 .. j0+tj-1.  Register queues: the same fields of the own row at columns
+// i-2 .. i+3.  Own-column inputs (u at i+1, v at j+1, w, the M values) are loaded per lane.
+template <typename T, bool MOIST>
 struct ScalLds {
-    static constexpr int KPW = KP * KW;
-    static constexpr int R = TJ + 6;
-    static constexpr int NS = MOIST ? 6 : 2;
-    static constexpr int NFS = MOIST ? 4 : 1;
-    static constexpr size_t s = 2 * NS * (size_t)R * KPW;          // [slot][field][row][k]
-    static constexpr size_t nf = NFS * (size_t)(TJ + 1) * KPW;     // [face][row + 1][k]
-    // two wavefronts per column: [row][w wbar] from level 64 to 63, [row][top faces, rain face] from 63 to 64
-    static constexpr size_t xw = KW == 2 ? 2 * (size_t)TJ : 0;
-    static constexpr size_t xb = KW == 2 ? (NFS + 1) * (size_t)TJ : 0;
-    static constexpr size_t bytes = (s + nf + xw + xb) * sizeof(T);
+    static constexpr int NP = MOIST ? 3 : 1;   // pairs
+    static constexpr int NFS = MOIST ? 4 : 1;  // face kinds
+    __host__ __device__ static constexpr size_t s(int tj, int pitch) { return 2 * 2 * NP * (size_t)(tj + 6) * pitch; }  // [slot][pair][row][k][2]
+    __host__ __device__ static constexpr size_t nf(int tj, int pitch) { return NFS * (size_t)(tj + 1) * pitch; }        // [row + 1][k][face]
+    // packed rows, per wavefront: w, wbar and the fall speed of its first lane for the wavefront before it; top
+    // faces and the rain face of its last lane for the one after it
+    static constexpr size_t xw = 3 * 16, xb = (NFS + 1) * 16;
+    static constexpr size_t bytes(int tj, int pitch) { return (s(tj, pitch) + nf(tj, pitch) + xw + xb) * sizeof(T); }
 };
 
-template <typename T, int TJ, bool MOIST, int KW = 1>
+template <typename T, int TJ, bool MOIST, bool PACK>
 __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, const StageArgs &a, T step, int t, unsigned char *smem_raw) {
-    using L = ScalLds<T, TJ, MOIST, KW>;
-    constexpr int KPW = L::KPW;
-    constexpr int R = L::R, NS = L::NS, NFS = L::NFS;
-    constexpr int HH = (6 + TJ - 1) / TJ;  // halo plane rows per wavefront
+    using L = ScalLds<T, MOIST>;
+    constexpr int NP = L::NP, NS = 2 * NP, NFS = L::NFS;
+    const RowMap<TJ, PACK> map(a.tj, g.NZ);
+    const int tj = map.tj, KPW = map.pitch, k = map.k, r = map.r;
+    const int R = tj + 6;
+    constexpr int HH = halo_loads<TJ>();  // halo plane rows per lane
     T *spl = (T *)smem_raw;
-    T *nface = spl + L::s;
-    T *xw = nface + L::nf, *xb = xw + L::xw;
+    T *nface = spl + L::s(tj, KPW);
+    T *xw = nface + L::nf(tj, KPW), *xb = xw + L::xw;
 
-    const int k = threadIdx.x, r = threadIdx.y;
-    const int j0 = a.jl + (t % a.nbj) * TJ;
+    const int j0 = a.jl + (t % a.nbj) * tj;
     const int i0 = a.il + (t / a.nbj) * a.ti;
     const int i1 = min(i0 + a.ti, a.ih);
     const int NZ = g.NZ, NY = g.NY;
@@ -434,17 +484,18 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
     const unsigned topoff = (unsigned)(jc * NZ + NZ - 1);
     const int RO = r + 3;
 
-    auto SP = [&](int slot, int f) -> T * { return spl + (slot * NS + f) * R * KPW; };
+    // pair pr of a plane row at level kk
+    auto SP = [&](int slot, int pr, int row, int kk) -> T * { return spl + (((slot * NP + pr) * R + row) * KPW + kk) * 2; };
     const void *src[6] = {a.cur[3], a.bar[3], a.cur[4], a.bar[4], a.cur[5], a.cur[6]};
     T q[NS][6], qs[NS];  // the own row at columns i-2 .. i+3 (i-3 .. i+2 in the prologue)
 
-    // plane rows: the own row comes from the queue, the six halo rows j0-3..j0-1, j0+TJ..j0+TJ+2 are loaded
-    auto halo_row = [&](int hh) { return hh < 3 ? hh : TJ + hh; };
+    // plane rows: the own row comes from the queue, the six halo rows j0-3..j0-1, j0+tj..j0+tj+2 are loaded
+    auto halo_row = [&](int hh) { return hh < 3 ? hh : tj + hh; };
     T ss[HH][NS];
     auto fetch_plane = [&](int i) {
 #pragma unroll
         for (int h = 0; h < HH; h++) {
-            const int hh = r + h * TJ;
+            const int hh = r + h * tj;
             if (hh < 6) {
                 const int jj = min(max(j0 - 3 + halo_row(hh), 0), NY - 1);
                 const unsigned pp = (unsigned)i * NYNZ + (unsigned)(jj * NZ + kc);
@@ -457,14 +508,14 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
     auto store_plane = [&](int i, int qd) {
         const int slot = i % 2;
 #pragma unroll
-        for (int f = 0; f < NS; f++) SP(slot, f)[RO * KPW + k] = q[f][qd];
+        for (int f = 0; f < NP; f++) lds_st2(SP(slot, f, RO, k), q[2 * f][qd], q[2 * f + 1][qd]);
 #pragma unroll
         for (int h = 0; h < HH; h++) {
-            const int hh = r + h * TJ;
+            const int hh = r + h * tj;
             if (hh < 6) {
                 const int rr = halo_row(hh);
 #pragma unroll
-                for (int f = 0; f < NS; f++) SP(slot, f)[rr * KPW + k] = ss[h][f];
+                for (int f = 0; f < NP; f++) lds_st2(SP(slot, f, rr, k), ss[h][2 * f], ss[h][2 * f + 1]);
             }
         }
     };
@@ -508,7 +559,7 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
 #pragma unroll
         for (int d = 0; d < 6; d++) q[f][d] = ld<T>(src[f], (unsigned)(i0 - 3 + d) * NYNZ + rowoff);
 
-    const T dtx = T(g.dtx), dty = T(g.dty), dt = T(g.dt);
+    const T dtx = T(g.dtx), dty = T(g.dty);
     const T DTZ = T(g.dtz) * T(c.mu[kc]);
     const T rw1 = T(c.rhow[kp1]), rw0 = T(c.rhow[kc]), odr = T(c.one_d_rhou[kc]);
     const bool low = (k == 1 || k == NZ - 2);
@@ -517,25 +568,34 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
     // so one there would also wait for the next column's prefetch.  Indices are clamped for the lanes
     // outside the active levels, which never use the values.
     const T tbu = T(c.tb[kp1]) - T(c.tb[kc]), tbd = T(c.tb[kc]) - T(c.tb[km1]);
-    T qbu = T(0), qbd = T(0), qbk = T(0), rk = T(1), vtden = T(0), rk64 = T(1), vtden64 = T(0);
+    T qbu = T(0), qbd = T(0), qbk = T(0), rk = T(1), vtden = T(0);
     if (MOIST) {
         qbu = T(c.qb[kp1]) - T(c.qb[kc]);
         qbd = T(c.qb[kc]) - T(c.qb[km1]);
         qbk = T(c.qb[kc]);
         rk = T(c.rhou[kc]);
         vtden = sqrt(T(c.rhou[1]) / rk);
-        if (KW == 2) {  // level 64, whose fall speed level 63 evaluates
-            rk64 = T(c.rhou[KP]);
-            vtden64 = sqrt(T(c.rhou[1]) / rk64);
-        }
     }
+    // fall speed of this level (kessler.cpp:222-252) from its rain; NZ-1 keeps the array's
+    auto fall = [&](T qr, T top) -> T {
+        T v = T(0);
+        if (k >= 1 && k <= NZ - 2) {
+            if (qr > T(1.0e-12)) {
+                T qrr = fmax(qr * T(0.001) * rk, T(0));
+                v = T(36.34) * (pow(qrr, T(0.1364))) * vtden;
+            }
+        } else if (k == NZ - 1) {
+            v = top;
+        }
+        return v;
+    };
 
     // east faces (s_east; fluxes.cpp:797-1032) of the queue's centre column with u, ubar at the column east of it
     auto east_faces = [&](T U1, T UB1, T *e) {
         T se = i5(q[0][0], q[0][1], q[0][2], q[0][3], q[0][4], q[0][5], sgn(UB1 + U1));
         T be = i5(q[1][0], q[1][1], q[1][2], q[1][3], q[1][4], q[1][5], sgn(U1));
         e[0] = U1 * be + (UB1 + U1) * se;
-        if (MOIST) {
+        if constexpr (MOIST) {
             T sv = i5(q[2][0], q[2][1], q[2][2], q[2][3], q[2][4], q[2][5], sgn(UB1 + U1));
             T bv = i5(q[3][0], q[3][1], q[3][2], q[3][3], q[3][4], q[3][5], sgn(U1));
             e[1] = U1 * bv + (UB1 + U1) * sv;
@@ -557,11 +617,18 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
     }
     Col cc{}, cs{};
     fetch_col(i0, cc);
-    // two wavefronts per column: level 63 reads w, wbar of level 64 from LDS
+    // Packed rows: a wavefront's last lane reads w, wbar and the fall speed of the level above it, which
+    // sit in the next wavefront's first lane, from LDS.  The fall speed of a column is therefore formed
+    // before the barrier that ends the column before it.
+    T vtk = T(0);
     auto publish_w = [&]() {
-        if (KW == 2 && k == KP) {
-            xw[2 * r] = cc.w0;
-            xw[2 * r + 1] = cc.wb0;
+        if constexpr (PACK) {
+            if (MOIST) vtk = fall(q[NS - 1][2], cc.vtt);
+            if (map.lane == 0) {
+                xw[3 * map.wave] = cc.w0;
+                xw[3 * map.wave + 1] = cc.wb0;
+                if (MOIST) xw[3 * map.wave + 2] = vtk;
+            }
         }
     };
     publish_w();
@@ -598,90 +665,94 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
         east_faces(cc.u1, cc.ub1, east);
         // north faces (s_north) of row RR with v, vbar at the face
         auto north_faces = [&](int RR, T V1, T VB1, T *nf) {
-#define PL(f, row) SP(c0, f)[(row) * KPW + k]
-            T sn = i5(PL(0, RR - 2), PL(0, RR - 1), PL(0, RR), PL(0, RR + 1), PL(0, RR + 2), PL(0, RR + 3), sgn(VB1 + V1));
-            T bn = i5(PL(1, RR - 2), PL(1, RR - 1), PL(1, RR), PL(1, RR + 1), PL(1, RR + 2), PL(1, RR + 3), sgn(V1));
+            T x[6], y[6];
+            auto rows = [&](int pr) {
+#pragma unroll
+                for (int d = 0; d < 6; d++) lds_ld2(SP(c0, pr, RR - 2 + d, k), x[d], y[d]);
+            };
+            rows(0);
+            T sn = i5(x[0], x[1], x[2], x[3], x[4], x[5], sgn(VB1 + V1));
+            T bn = i5(y[0], y[1], y[2], y[3], y[4], y[5], sgn(V1));
             nf[0] = V1 * bn + (VB1 + V1) * sn;
-            if (MOIST) {
-                T sv = i5(PL(2, RR - 2), PL(2, RR - 1), PL(2, RR), PL(2, RR + 1), PL(2, RR + 2), PL(2, RR + 3), sgn(VB1 + V1));
-                T bv = i5(PL(3, RR - 2), PL(3, RR - 1), PL(3, RR), PL(3, RR + 1), PL(3, RR + 2), PL(3, RR + 3), sgn(V1));
+            if constexpr (MOIST) {
+                rows(1);
+                T sv = i5(x[0], x[1], x[2], x[3], x[4], x[5], sgn(VB1 + V1));
+                T bv = i5(y[0], y[1], y[2], y[3], y[4], y[5], sgn(V1));
                 nf[1] = V1 * bv + (VB1 + V1) * sv;
                 T vb = VB1 + V1;
-                nf[2] = vb * i5(PL(4, RR - 2), PL(4, RR - 1), PL(4, RR), PL(4, RR + 1), PL(4, RR + 2), PL(4, RR + 3), sgn(vb));
-                nf[3] = vb * i5(PL(5, RR - 2), PL(5, RR - 1), PL(5, RR), PL(5, RR + 1), PL(5, RR + 2), PL(5, RR + 3), sgn(vb));
+                rows(2);
+                nf[2] = vb * i5(x[0], x[1], x[2], x[3], x[4], x[5], sgn(vb));
+                nf[3] = vb * i5(y[0], y[1], y[2], y[3], y[4], y[5], sgn(vb));
             }
-#undef PL
+        };
+        auto put_faces = [&](int row, const T *nf) {
+            T *o = nface + (row * KPW + k) * NFS;
+            if constexpr (MOIST) {
+                lds_st2(o, nf[0], nf[1]);
+                lds_st2(o + 2, nf[2], nf[3]);
+            } else {
+                o[0] = nf[0];
+            }
         };
         T nf[NFS];
         north_faces(RO, cc.vn, cc.vbn, nf);
-#pragma unroll
-        for (int f = 0; f < NFS; f++) nface[(f * (TJ + 1) + r + 1) * KPW + k] = nf[f];
+        put_faces(r + 1, nf);
         if (r == 0) {
             T sf[NFS];
             north_faces(RO - 1, cc.vs, cc.vbs, sf);
-#pragma unroll
-            for (int f = 0; f < NFS; f++) nface[(f * (TJ + 1)) * KPW + k] = sf[f];
+            put_faces(0, sf);
         }
-        // top faces (s_top) of this level from the own column of the plane; w, wbar at k+1 by lane exchange
+        // top faces (s_top) of this level from the own column of the plane; w, wbar (and the fall speed) at
+        // k+1 by lane exchange
         T W1 = lane_next(cc.w0), WB1 = lane_next(cc.wb0);
-        if (KW == 2 && k == KP - 1) {
-            W1 = xw[2 * r];
-            WB1 = xw[2 * r + 1];
+        if (MOIST && !PACK) vtk = fall(q[NS - 1][2], cc.vtt);
+        T vk1 = MOIST ? lane_next(vtk) : T(0);
+        if (PACK && map.lane == KP - 1) {  // (past the block's last wavefront: words no lane uses)
+            W1 = xw[3 * map.wave + 3];
+            WB1 = xw[3 * map.wave + 4];
+            if (MOIST) vk1 = xw[3 * map.wave + 5];
         }
-        auto s_top = [&](int fs, int fb) -> T {
-            const T *S = SP(c0, fs) + RO * KPW, *B = SP(c0, fb) + RO * KPW;
+        // the pair's fields at levels k-1 .. k+2 of the own column
+        T x[4], y[4];
+        auto column = [&](int pr) {
+            lds_ld2(SP(c0, pr, RO, km1), x[0], y[0]);
+            lds_ld2(SP(c0, pr, RO, kc), x[1], y[1]);
+            lds_ld2(SP(c0, pr, RO, kp1), x[2], y[2]);
+            lds_ld2(SP(c0, pr, RO, kp2), x[3], y[3]);
+        };
+        auto s_top = [&](int pr) -> T {
+            column(pr);
             T st_, bt;
             if (low) {
-                st_ = i2(S[kc], S[kp1]);
-                bt = i2(B[kc], B[kp1]);
+                st_ = i2(x[1], x[2]);
+                bt = i2(y[1], y[2]);
             } else {
-                st_ = i3(S[km1], S[kc], S[kp1], S[kp2], sgn(WB1 + W1));
-                bt = i3(B[km1], B[kc], B[kp1], B[kp2], sgn(W1));
+                st_ = i3(x[0], x[1], x[2], x[3], sgn(WB1 + W1));
+                bt = i3(y[0], y[1], y[2], y[3], sgn(W1));
             }
             return W1 * bt + (WB1 + W1) * st_;
         };
         T tf[NFS];
-        tf[0] = s_top(0, 1);
-        T vtk = T(0), qrt = T(0);
-        if (MOIST) {
-            tf[1] = s_top(2, 3);
+        tf[0] = s_top(0);
+        T qrt = T(0);
+        if constexpr (MOIST) {
+            tf[1] = s_top(1);
+            column(2);
             {
-                const T *S = SP(c0, 4) + RO * KPW;
                 T wb = WB1 + W1;
-                T tq = low ? i2(S[kc], S[kp1]) : i3(S[km1], S[kc], S[kp1], S[kp2], sgn(wb));
+                T tq = low ? i2(x[1], x[2]) : i3(x[0], x[1], x[2], x[3], sgn(wb));
                 tf[2] = wb * tq;
             }
-            // fall speed of this level (kessler.cpp:222-252); level 0 stores level 1's, NZ-1 keeps the array's
-            auto fall = [&](T qr, T rho, T den) -> T {
-                T v = T(0);
-                if (qr > T(1.0e-12)) {
-                    T qrr = fmax(qr * T(0.001) * rho, T(0));
-                    v = T(36.34) * (pow(qrr, T(0.1364))) * den;
-                }
-                return v;
-            };
-            if (k >= 1 && k <= NZ - 2) {
-                vtk = fall(q[5][2], rk, vtden);
-            } else if (k == NZ - 1) {
-                vtk = cc.vtt;
-            }
-            // rain top face with the fall speed (fluxes.cpp:734, 780; 966-1030)
-            const T *QRr = SP(c0, 5) + RO * KPW;
-            const T v1l = lane_read(vtk, 1);
-            const T vte = k == 0 ? v1l : vtk;
-            T vk1 = lane_next(vte);
-            // two wavefronts per column: level 63 evaluates level 64's fall speed itself (NZ >= 66, so
-            // level 64 is an interior level), from the same plane value the other wavefront uses
-            if (KW == 2 && k == KP - 1) vk1 = fall(QRr[KP], rk64, vtden64);
+            // rain top face with the fall speed (fluxes.cpp:734, 780; 966-1030); level 0 falls as level 1 does
             if (k == 0) {
-                T t0 = T(0.5) * (QRr[0] + QRr[1]);
-                qrt = -T(0.5) * (v1l + v1l) * t0;
+                T t0 = T(0.5) * (y[1] + y[2]);
+                qrt = -T(0.5) * (vk1 + vk1) * t0;
             } else {
                 T wb = WB1 + W1;
                 T tq;
-                if (kc == 1 || kc == NZ - 2) tq = i2(QRr[kc], QRr[kp1]);
-                else tq = i3(QRr[km1], QRr[kc], QRr[kp1], QRr[kp2], sgn(WB1 + W1 - T(0.5) * (vte + vk1)));
-                qrt = (wb - T(0.5) * (vk1 + vte)) * tq;
+                if (kc == 1 || kc == NZ - 2) tq = i2(y[1], y[2]);
+                else tq = i3(y[0], y[1], y[2], y[3], sgn(WB1 + W1 - T(0.5) * (vtk + vk1)));
+                qrt = (wb - T(0.5) * (vk1 + vtk)) * tq;
             }
         }
         if (k == 0) {
@@ -689,25 +760,32 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
             for (int f = 0; f < NFS; f++) tf[f] = T(0);
         }
         T bot[NFS];
+        constexpr int NB = MOIST ? 3 : 1;  // top faces handed up (rain has its own)
 #pragma unroll
-        for (int f = 0; f < NFS; f++) bot[f] = lane_prev(tf[f]);
+        for (int f = 0; f < NB; f++) bot[f] = lane_prev(tf[f]);
         T qrb = MOIST ? lane_prev(qrt) : T(0);
-        if (KW == 2 && k == KP - 1) {
+        if (PACK && map.lane == KP - 1) {
 #pragma unroll
-            for (int f = 0; f < NFS; f++) xb[(NFS + 1) * r + f] = tf[f];
-            xb[(NFS + 1) * r + NFS] = qrt;
+            for (int f = 0; f < NB; f++) xb[(NFS + 1) * map.wave + f] = tf[f];
+            xb[(NFS + 1) * map.wave + NFS] = qrt;
         }
         __syncthreads();
-        if (KW == 2 && k == KP) {
+        if (PACK && map.lane == 0 && map.wave > 0) {
 #pragma unroll
-            for (int f = 0; f < NFS; f++) bot[f] = xb[(NFS + 1) * r + f];
-            if (MOIST) qrb = xb[(NFS + 1) * r + NFS];
+            for (int f = 0; f < NB; f++) bot[f] = xb[(NFS + 1) * (map.wave - 1) + f];
+            if (MOIST) qrb = xb[(NFS + 1) * (map.wave - 1) + NFS];
         }
+        const T vtk0 = vtk;  // this column's fall speed, stored below
         T oth = T(0), oqv = T(0), oqc = T(0), oqr = T(0);  // this level's final values (active levels)
         if (active) {
-            T south[NFS];
-#pragma unroll
-            for (int f = 0; f < NFS; f++) south[f] = nface[(f * (TJ + 1) + r) * KPW + k];
+            T south[4];
+            const T *so = nface + (r * KPW + k) * NFS;
+            if constexpr (MOIST) {
+                lds_ld2(so, south[0], south[1]);
+                lds_ld2(so + 2, south[2], south[3]);
+            } else {
+                south[0] = so[0];
+            }
             // Z_ADVECT_BASE (advection.cpp:16-18) with the base-state differences du = b[k+1] - b[k],
             // dd = b[k] - b[k-1] of this level
             auto zbase = [&](T du, T dd) -> T { return (T(0.50) * (rw1 * W1 * du + rw0 * cc.w0 * dd) * odr); };
@@ -716,7 +794,7 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
                          DTZ * zbase(tbu, tbd);
                 oth = mth + step * tend;
             }
-            if (MOIST) {  // advection.cpp:197-253
+            if constexpr (MOIST) {  // advection.cpp:197-253
                 T tq = -dtx * (east[1] - west[1]) - dty * (nf[1] - south[1]) - DTZ * (rw1 * tf[1] - rw0 * bot[1]) * odr -
                        DTZ * zbase(qbu, qbd);
                 T qv = mqv + step * tq;
@@ -733,47 +811,31 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
                 oqr = qrv;
             }
         }
-        // the lid of upper_lower_boundaries (boundaries.cpp:304-312) for this column: level 0 takes level 1,
-        // NZ-1 takes NZ-2.  These are the final values of an interior column (no sponge or periodic copy
-        // touches it); the boundary epilogue redoes the columns it rewrites whole.  The sources of the
-        // periodic copy are left to it: halo column 0 receives column NX-6's values from before the lid.
-        // A lane writes either its own level (active levels) or a lid level (levels 0 and NZ-1).
-        unsigned ps = p;
-        const bool lid = j < a.jh && i >= 6 && i < g.NX - 6 && (k == 0 || k == NZ - 1);
-        {
-            const int lz = (NZ - 2) & (KP - 1);  // lane of level NZ-2 in its wavefront
-            const int src = k == 0 ? 1 : lz;
-            const T t1 = lane_read(oth, 1), tz = lane_read(oth, lz);
-            T v1 = T(0), vz = T(0), c1 = T(0), cz = T(0), r1 = T(0), rz = T(0);
-            if (MOIST) {
-                v1 = lane_read(oqv, 1);
-                vz = lane_read(oqv, lz);
-                c1 = lane_read(oqc, 1);
-                cz = lane_read(oqc, lz);
-                r1 = lane_read(oqr, 1);
-                rz = lane_read(oqr, lz);
-            }
-            if (lid) {
-                const bool bot_lvl = src == 1;
-                ps = (unsigned)i * NYNZ + (unsigned)(jc * NZ + k);
-                oth = bot_lvl ? t1 : tz;
-                oqv = bot_lvl ? v1 : vz;
-                oqc = bot_lvl ? c1 : cz;
-                oqr = bot_lvl ? r1 : rz;
-            }
-        }
+        // With its own level, the lane of level 1 (NZ-2) writes the lid of upper_lower_boundaries
+        // (boundaries.cpp:304-312): level 0 (NZ-1) takes its value.  These are the final values of an
+        // interior column (no sponge or periodic copy touches it); the boundary epilogue redoes the columns
+        // it rewrites whole.  The sources of the periodic copy are left to it: halo column 0 receives
+        // column NX-6's values from before the lid.
+        const bool lid = active && (k == 1 || k == NZ - 2) && i >= 6 && i < g.NX - 6;
         auto store_column = [&]() {
-            if (active || lid) {
-                st<T>(a.out[3], ps, oth);
+            if (active) {
+                st<T>(a.out[3], p, oth);
                 if (MOIST) {
-                    st<T>(a.out[4], ps, oqv);
-                    st<T>(a.out[5], ps, oqc);
-                    st<T>(a.out[6], ps, oqr);
+                    st<T>(a.out[4], p, oqv);
+                    st<T>(a.out[5], p, oqc);
+                    st<T>(a.out[6], p, oqr);
+                    st<T>(a.vt, p, vtk0);
+                    if (k == 1) st<T>(a.vt, p - 1, vtk0);
                 }
             }
-            if (MOIST && active) {
-                st<T>(a.vt, p, vtk);
-                if (k == 1) st<T>(a.vt, p - 1, vtk);
+            if (lid) {
+                const unsigned pl = k == 1 ? p - 1 : p + 1;
+                st<T>(a.out[3], pl, oth);
+                if (MOIST) {
+                    st<T>(a.out[4], pl, oqv);
+                    st<T>(a.out[5], pl, oqc);
+                    st<T>(a.out[6], pl, oqr);
+                }
             }
         };
         if (kLean) store_column();
@@ -800,16 +862,21 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
     }
 }
 
-template <typename T, int TJ, bool MOIST, int KW>
-__global__ void __launch_bounds__(KP *KW *TJ) k_adv_momentum(Geo g, Cols c, StageArgs a, T step) {
-    extern __shared__ unsigned char smem_raw[];
-    adv_momentum_tile<T, TJ, MOIST, KW>(g, c, a, step, xcd_tile(blockIdx.x, gridDim.x), smem_raw);
+// threads of the largest block: TJ rows of one wavefront each, or kPackThreads lanes of packed rows
+constexpr int kPackThreads = 512;
+template <int TJ, bool PACK>
+constexpr int stage_threads() { return PACK ? kPackThreads : KP * TJ; }
+
+template <typename T, int TJ, bool MOIST, bool PACK>
+__global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_adv_momentum(Geo g, Cols c, StageArgs a, T step) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    adv_momentum_tile<T, TJ, MOIST, PACK>(g, c, a, step, xcd_tile(blockIdx.x, gridDim.x), smem_raw);
 }
 
-template <typename T, int TJ, bool MOIST, int KW>
-__global__ void __launch_bounds__(KP *KW *TJ) k_adv_scalars(Geo g, Cols c, StageArgs a, T step) {
-    extern __shared__ unsigned char smem_raw[];
-    adv_scalars_tile<T, TJ, MOIST, KW>(g, c, a, step, xcd_tile(blockIdx.x, gridDim.x), smem_raw);
+template <typename T, int TJ, bool MOIST, bool PACK>
+__global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_adv_scalars(Geo g, Cols c, StageArgs a, T step) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    adv_scalars_tile<T, TJ, MOIST, PACK>(g, c, a, step, xcd_tile(blockIdx.x, gridDim.x), smem_raw);
 }
 
 // zero_moisture outside the advected box (the fused kernel clips the points it writes)
@@ -831,30 +898,33 @@ __global__ void k_zero_moisture_shell(Geo g, Cols c, T *__restrict__ QVP, T *__r
     }
 }
 
-template <typename T, int TJ, bool MOIST, int KW>
-int momentum_t(Ctx *c, const StageArgs &a0, T step, int ti) {
+// shape: rows per block, march length and lane mapping of one launch
+template <typename T, int TJ, bool MOIST, bool PACK>
+int momentum_t(Ctx *c, const StageArgs &a0, T step, const StageShape &sh) {
     StageArgs a = a0;
-    a.ti = ti;
-    a.nbj = (a.jh - a.jl + TJ - 1) / TJ;
-    const int nbi = (a.ih - a.il + ti - 1) / ti;
-    const size_t sh = MomLds<T, TJ, KW>::bytes;
+    a.ti = sh.ti;
+    a.tj = sh.tj;
+    a.nbj = (a.jh - a.jl + sh.tj - 1) / sh.tj;
+    const int nbi = (a.ih - a.il + sh.ti - 1) / sh.ti;
+    const dim3 blk = PACK ? dim3((sh.tj * c->geo.NZ + KP - 1) / KP * KP) : dim3(KP, TJ);
     Timed _t(c, "adv_momentum", (double)(a.ih - a.il) * (a.jh - a.jl) * (c->geo.NZ - 2));
-    hipLaunchKernelGGL((k_adv_momentum<T, TJ, MOIST, KW>), dim3(a.nbj * nbi), dim3(KP * KW, TJ), sh, c->stream, c->geo, c->cols, a,
-                       step);
+    hipLaunchKernelGGL((k_adv_momentum<T, TJ, MOIST, PACK>), dim3(a.nbj * nbi), blk, MomLds<T>::bytes(sh.tj, PACK ? c->geo.NZ : KP),
+                       c->stream, c->geo, c->cols, a, step);
     DYN_LAUNCH_CHECK();
     return DYN_OK;
 }
 
-template <typename T, int TJ, bool MOIST, int KW>
-int scalars_t(Ctx *c, const StageArgs &a0, T step, int ti) {
+template <typename T, int TJ, bool MOIST, bool PACK>
+int scalars_t(Ctx *c, const StageArgs &a0, T step, const StageShape &sh) {
     StageArgs a = a0;
-    a.ti = ti;
-    a.nbj = (a.jh - a.jl + TJ - 1) / TJ;
-    const int nbi = (a.ih - a.il + ti - 1) / ti;
-    const size_t sh = ScalLds<T, TJ, MOIST, KW>::bytes;
+    a.ti = sh.ti;
+    a.tj = sh.tj;
+    a.nbj = (a.jh - a.jl + sh.tj - 1) / sh.tj;
+    const int nbi = (a.ih - a.il + sh.ti - 1) / sh.ti;
+    const dim3 blk = PACK ? dim3((sh.tj * c->geo.NZ + KP - 1) / KP * KP) : dim3(KP, TJ);
     Timed _t(c, "adv_scalars", (double)(a.ih - a.il) * (a.jh - a.jl) * (c->geo.NZ - 2));
-    hipLaunchKernelGGL((k_adv_scalars<T, TJ, MOIST, KW>), dim3(a.nbj * nbi), dim3(KP * KW, TJ), sh, c->stream, c->geo, c->cols, a,
-                       step);
+    hipLaunchKernelGGL((k_adv_scalars<T, TJ, MOIST, PACK>), dim3(a.nbj * nbi), blk,
+                       (ScalLds<T, MOIST>::bytes(sh.tj, PACK ? c->geo.NZ : KP)), c->stream, c->geo, c->cols, a, step);
     DYN_LAUNCH_CHECK();
     return DYN_OK;
 }
@@ -873,29 +943,29 @@ int stage_t(Ctx *c, double step, int il, int ih, int jl, int jh, int parts) {
     a.ih = ih;
     a.jl = jl;
     a.jh = jh;
-    const int mtj = fused_shape(c, DYN_TUNE_MOMENTUM_TJ), mti = fused_shape(c, DYN_TUNE_MOMENTUM_TI);
-    const int stj = fused_shape(c, DYN_TUNE_SCALAR_TJ), sti = fused_shape(c, DYN_TUNE_SCALAR_TI);
     int rc = DYN_OK;
-    if (fused_waves(c) == 2) {  // two wavefronts per column: 2 or 4 rows per block
-        if (parts & kStageMomentum) {
-            if (mtj == 2) rc = momentum_t<T, 2, MOIST, 2>(c, a, T(step), mti);
-            else rc = momentum_t<T, 4, MOIST, 2>(c, a, T(step), mti);
-        }
-        if (rc || !(parts & kStageScalars)) return rc;
-        if (stj == 2) return scalars_t<T, 2, MOIST, 2>(c, a, T(step), sti);
-        return scalars_t<T, 4, MOIST, 2>(c, a, T(step), sti);
-    }
     if (parts & kStageMomentum) {
-        if (mtj == 2) rc = momentum_t<T, 2, MOIST, 1>(c, a, T(step), mti);
-        else if (mtj == 4) rc = momentum_t<T, 4, MOIST, 1>(c, a, T(step), mti);
-        else if (mtj == 16) rc = momentum_t<T, 16, MOIST, 1>(c, a, T(step), mti);
-        else rc = momentum_t<T, 8, MOIST, 1>(c, a, T(step), mti);
+        const StageShape m = stage_shape(c, true);
+        if (m.pack) {
+            if (m.tj >= 6) rc = momentum_t<T, 8, MOIST, true>(c, a, T(step), m);
+            else if (m.tj >= 3) rc = momentum_t<T, 4, MOIST, true>(c, a, T(step), m);
+            else rc = momentum_t<T, 2, MOIST, true>(c, a, T(step), m);
+        } else if (m.tj == 2) rc = momentum_t<T, 2, MOIST, false>(c, a, T(step), m);
+        else if (m.tj == 4) rc = momentum_t<T, 4, MOIST, false>(c, a, T(step), m);
+        else if (m.tj == 16) rc = momentum_t<T, 16, MOIST, false>(c, a, T(step), m);
+        else rc = momentum_t<T, 8, MOIST, false>(c, a, T(step), m);
     }
     if (rc || !(parts & kStageScalars)) return rc;
-    if (stj == 2) return scalars_t<T, 2, MOIST, 1>(c, a, T(step), sti);
-    if (stj == 4) return scalars_t<T, 4, MOIST, 1>(c, a, T(step), sti);
-    if (stj == 12) return scalars_t<T, 12, MOIST, 1>(c, a, T(step), sti);
-    return scalars_t<T, 8, MOIST, 1>(c, a, T(step), sti);
+    const StageShape m = stage_shape(c, false);
+    if (m.pack) {
+        if (m.tj >= 6) return scalars_t<T, 8, MOIST, true>(c, a, T(step), m);
+        if (m.tj >= 3) return scalars_t<T, 4, MOIST, true>(c, a, T(step), m);
+        return scalars_t<T, 2, MOIST, true>(c, a, T(step), m);
+    }
+    if (m.tj == 2) return scalars_t<T, 2, MOIST, false>(c, a, T(step), m);
+    if (m.tj == 4) return scalars_t<T, 4, MOIST, false>(c, a, T(step), m);
+    if (m.tj == 12) return scalars_t<T, 12, MOIST, false>(c, a, T(step), m);
+    return scalars_t<T, 8, MOIST, false>(c, a, T(step), m);
 }
 
 template <typename T>
@@ -1110,8 +1180,9 @@ __global__ void __launch_bounds__(256) k_post_scalars_shell(Geo g, Cols c, PostA
 }
 
 // ---- batched over the members of an ensemble: one block per work item of the concatenated work list ----
-__device__ __forceinline__ StageArgs ens_stage_args(const EnsMember &e, const EnsRoles &ro, int ti, int nbj) {
+__device__ __forceinline__ StageArgs ens_stage_args(const EnsMember &e, const EnsRoles &ro, int tj, int ti, int nbj) {
     StageArgs a;
+    a.tj = tj;
     for (int f = 0; f < 7; f++) {
         a.cur[f] = e.buf[f][ro.r[f][DYN_ROLE_CUR]];
         a.mprev[f] = e.buf[f][ro.r[f][DYN_ROLE_M]];
@@ -1143,22 +1214,22 @@ __device__ __forceinline__ PostArgs ens_post_args(const EnsMember &e, const EnsR
     return a;
 }
 
-template <typename T, int TJ, bool MOIST>
+template <typename T, int TJ, bool MOIST, bool PACK>
 __global__ void __launch_bounds__(KP *TJ) k_ens_momentum(const EnsMember *mem, int nmem, EnsRoles ro, T step, int ti, int total) {
-    extern __shared__ unsigned char smem_raw[];
+    extern __shared__ __align__(16) unsigned char smem_raw[];
     const int item = blockIdx.x;
     const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::mom0)];
-    const StageArgs a = ens_stage_args(e, ro, ti, e.nbj_mom);
-    adv_momentum_tile<T, TJ, MOIST>(e.g, e.c, a, step, item - e.mom0, smem_raw);
+    const StageArgs a = ens_stage_args(e, ro, TJ, ti, e.nbj_mom);
+    adv_momentum_tile<T, TJ, MOIST, PACK>(e.g, e.c, a, step, item - e.mom0, smem_raw);
 }
 
-template <typename T, int TJ, bool MOIST>
+template <typename T, int TJ, bool MOIST, bool PACK>
 __global__ void __launch_bounds__(KP *TJ) k_ens_scalars(const EnsMember *mem, int nmem, EnsRoles ro, T step, int ti, int total) {
-    extern __shared__ unsigned char smem_raw[];
+    extern __shared__ __align__(16) unsigned char smem_raw[];
     const int item = blockIdx.x;
     const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::scal0)];
-    const StageArgs a = ens_stage_args(e, ro, ti, e.nbj_scal);
-    adv_scalars_tile<T, TJ, MOIST>(e.g, e.c, a, step, item - e.scal0, smem_raw);
+    const StageArgs a = ens_stage_args(e, ro, TJ, ti, e.nbj_scal);
+    adv_scalars_tile<T, TJ, MOIST, PACK>(e.g, e.c, a, step, item - e.scal0, smem_raw);
 }
 
 template <typename T>
@@ -1238,8 +1309,9 @@ int post_t(Ctx *c, double step, bool pgf, bool scalars, bool clip, bool uvw, int
 
 }  // namespace
 
-// Wavefronts per column of the stage kernels: one up to NZ = 64; two for NZ in [66, 128], where the lid's
-// source levels 1 and NZ-2 sit in the wavefronts of the levels they feed (0 and NZ-1); 0 otherwise
+// Wavefronts per column of the boundary kernels: one up to NZ = 64; two for NZ in [66, 128], where the lid's
+// source levels 1 and NZ-2 sit in the wavefronts of the levels they feed (0 and NZ-1); 0 otherwise: the
+// fused step is not offered
 int fused_waves(const Ctx *c) {
     const int nz = c->g.nz;
     return nz <= KP ? 1 : (nz >= KP + 2 && nz <= 2 * KP ? 2 : 0);
@@ -1252,30 +1324,23 @@ bool fused_supported(const Ctx *c) {
 }
 
 namespace {
-template <typename T, int KW>
-size_t stage_lds_t(bool momentum, bool moist, int tj) {
-    if (tj == 2) return momentum ? MomLds<T, 2, KW>::bytes : moist ? ScalLds<T, 2, true, KW>::bytes : ScalLds<T, 2, false, KW>::bytes;
-    if (tj == 4) return momentum ? MomLds<T, 4, KW>::bytes : moist ? ScalLds<T, 4, true, KW>::bytes : ScalLds<T, 4, false, KW>::bytes;
-    if (tj == 12) return moist ? ScalLds<T, 12, true, KW>::bytes : ScalLds<T, 12, false, KW>::bytes;  // scalar kernel only
-    if (tj == 16) return MomLds<T, 16, KW>::bytes;  // momentum kernel only
-    return momentum ? MomLds<T, 8, KW>::bytes : moist ? ScalLds<T, 8, true, KW>::bytes : ScalLds<T, 8, false, KW>::bytes;
-}
-// LDS bytes per block of a stage kernel with tj rows
-size_t stage_lds(const Ctx *c, bool momentum, int tj) {
-    const bool moist = c->g.microphysics != 0, two = fused_waves(c) == 2;
-    if (c->prec == DYN_FP32) return two ? stage_lds_t<float, 2>(momentum, moist, tj) : stage_lds_t<float, 1>(momentum, moist, tj);
-    return two ? stage_lds_t<double, 2>(momentum, moist, tj) : stage_lds_t<double, 1>(momentum, moist, tj);
+// LDS bytes per block of a stage kernel with tj rows of `pitch` lanes
+size_t stage_lds(const Ctx *c, bool momentum, int tj, int pitch) {
+    const bool moist = c->g.microphysics != 0;
+    if (c->prec == DYN_FP32)
+        return momentum ? MomLds<float>::bytes(tj, pitch) : moist ? ScalLds<float, true>::bytes(tj, pitch) : ScalLds<float, false>::bytes(tj, pitch);
+    return momentum ? MomLds<double>::bytes(tj, pitch) : moist ? ScalLds<double, true>::bytes(tj, pitch) : ScalLds<double, false>::bytes(tj, pitch);
 }
 }  // namespace
 
-// launch-shape knobs of the stage kernels: rows per block (instantiated widths: 2, 4, 8 with one wavefront
-// per column, and 16 for the momentum kernel, 12 for the scalar kernel; 2, 4 with two; within the LDS)
-// and march length
+// launch-shape knobs of the stage kernels: rows per block (2, 4 and 8 up to 64 levels, and 16 for the
+// momentum kernel, 12 for the scalar kernel; 2 and 4 above; within the LDS that rows of whole wavefronts
+// take) and march length
 bool fused_shape_ok(const Ctx *c, int param, int value) {
     if (param == DYN_TUNE_MOMENTUM_TJ || param == DYN_TUNE_SCALAR_TJ) {
         const bool one = fused_waves(c) != 2, mom = param == DYN_TUNE_MOMENTUM_TJ;
         const bool inst = value == 2 || value == 4 || (one && (value == 8 || value == (mom ? 16 : 12)));
-        return inst && stage_lds(c, param == DYN_TUNE_MOMENTUM_TJ, value) <= c->pp.lds_max;
+        return inst && stage_lds(c, mom, value, KP * (one ? 1 : 2)) <= c->pp.lds_max;
     }
     if (param == DYN_TUNE_MOMENTUM_TI || param == DYN_TUNE_SCALAR_TI) return value >= 2 && value <= 512;
     if (param == DYN_TUNE_PRESSURE_JPASS) return value == 2 || (value == 1 && c->pp.fused_y) || (value == 3 && c->pp.half_y);
@@ -1340,46 +1405,124 @@ int fused_shape(const Ctx *c, int param) {
     }
 }
 
-// shapes whose LDS exceeds the device's are never launched (fused_shape_ok), so their limit stays unset
-template <typename T, int TJ, int KW>
-int set_lds_limits(const Ctx *c) {
-    const size_t mom = MomLds<T, TJ, KW>::bytes, sm = ScalLds<T, TJ, true, KW>::bytes, sd = ScalLds<T, TJ, false, KW>::bytes;
-    if (mom <= c->pp.lds_max) {
-        DYN_HIP(hipFuncSetAttribute((const void *)k_adv_momentum<T, TJ, true, KW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mom));
-        DYN_HIP(hipFuncSetAttribute((const void *)k_adv_momentum<T, TJ, false, KW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mom));
+namespace {
+// Lanes of packed rows (see RowMap) unless a 64-lane wavefront is nearly full: at 57 levels and more a row
+// per wavefront wastes at most one lane in nine and needs no exchange at wavefront edges
+bool stage_packs(const Ctx *c) { return c->g.nz < 57 || c->g.nz > KP; }
+
+// Modelled microseconds of a stage kernel's launch with tj rows and ti columns per block.  A block marches
+// ti columns after a prologue worth about one more; a column takes `lat` while few wavefronts share a SIMD
+// (the march is a chain of barriers and loads) and `issue` for each wavefront on the fullest SIMD once
+// they are many; blocks beyond what fits on a CU wait for a round of their own, and each block loads six
+// halo rows beside its own.  Blocks whose wavefronts do not fill the four SIMDs evenly run at the pace of
+// the fullest one: at 192x192x40 (FP32 moist) the momentum kernel takes 26.7 us with 6 rows (4 wavefronts),
+// 36.6 with 8 (5 wavefronts) and 27.6 with 12 (8 wavefronts).  The constants are fitted to timings of
+// 32x32x20 to 512x512x80 grids in every form, 2 to 25 rows and 2 to 32 columns (one kernel on the device);
+// the shape the model picks is within 10 % of the fastest of them in all but the smallest launches.
+struct StageCost {
+    double lat, issue;
+    int simd;  // wavefronts per SIMD that the kernel's registers allow
+};
+StageCost stage_cost(const Ctx *c, bool momentum) {
+    const bool f32 = c->prec == DYN_FP32, moist = c->g.microphysics != 0;
+    if (momentum) return f32 ? StageCost{1.65, 0.70, 4} : StageCost{2.15, 1.40, 2};
+    if (moist) return f32 ? StageCost{2.70, 1.00, 3} : StageCost{5.30, 3.00, 2};
+    return f32 ? StageCost{1.00, 0.38, 5} : StageCost{1.40, 0.65, 3};
+}
+double stage_model(const Ctx *c, bool momentum, bool pack, int tj, int ti) {
+    const StageCost k = stage_cost(c, momentum);
+    const int waves = pack ? (tj * c->g.nz + KP - 1) / KP : tj, per_simd = (waves + 3) / 4, cus = std::max(1, c->pp.cus);
+    const int fit = std::max(1, std::min(k.simd / per_simd, (int)(c->pp.lds_max / stage_lds(c, momentum, tj, pack ? c->g.nz : KP))));
+    const long long blocks = (long long)((c->g.ny - 6 + tj - 1) / tj) * ((c->g.nx - 6 + ti - 1) / ti);
+    const int per_cu = (int)((blocks + cus - 1) / cus);
+    auto column = [&](int n) { return n ? std::max(k.lat, k.issue * n * per_simd) : 0.0; };
+    return (ti + 1) * (per_cu / fit * column(fit) + column(per_cu % fit)) * (1.0 + 0.3 / tj);
+}
+}  // namespace
+
+// The launch of a stage kernel.  With a knob of its own set, or on grids of 57 to 64 levels whose nominal
+// blocks (fused_shape) number one per CU or more, the nominal shape; else the one the model above takes to
+// be fastest: small grids get short marches (64x64x40 FP32: momentum 34.3 us in 32 blocks of 16 columns,
+// 10.0 in 256 of 2), and packed rows the row count that fills whole groups of four wavefronts.
+StageShape stage_shape(const Ctx *c, bool momentum) {
+    const int ptj = momentum ? DYN_TUNE_MOMENTUM_TJ : DYN_TUNE_SCALAR_TJ, pti = momentum ? DYN_TUNE_MOMENTUM_TI : DYN_TUNE_SCALAR_TI;
+    if (!c->tune[ptj] && !c->tune[pti] && c->auto_shape[momentum].tj) return c->auto_shape[momentum];
+    StageShape s{fused_shape(c, ptj), fused_shape(c, pti), stage_packs(c)};
+    if (s.pack && s.tj * c->g.nz > kPackThreads) s.pack = false;  // 12 or 16 rows asked for
+    return s;
+}
+
+// How a step's stages use the second stream (the values of DYN_TUNE_STAGE_STREAMS) while the knob is unset.
+// With short marches the scalar kernel no longer delays the divergence pass it is queued behind, so the late
+// queueing (4) is the faster form up to a few million points (FP32 moist, 2 against 4: 361 and 335 us per
+// step at 128x128x64, 692 and 666 at 256x256x40; FP64 moist, 3 against 4: 625 and 563 at 128x128x64), and for
+// every dry FP32 grid; the largest moist grids keep the nominal form (FP32 256x256x64: 834 against 871 us).
+int stage_streams(const Ctx *c) {
+    const int nominal = fused_shape(c, DYN_TUNE_STAGE_STREAMS);
+    if (c->tune[DYN_TUNE_STAGE_STREAMS]) return nominal;
+    const bool few = c->npts < (nominal == 3 ? 2000000u : 3000000u);
+    return few || (nominal == 2 && !c->g.microphysics) ? 4 : nominal;
+}
+
+namespace {
+// auto_shape of both kernels; left empty (tj = 0) where the nominal shape is kept
+void choose_stage_shapes(Ctx *c) {
+    const bool pack = stage_packs(c);
+    const int nx = c->g.nx - 6, ny = c->g.ny - 6;
+    for (int m = 0; m < 2; m++) {
+        const bool momentum = m == 1;
+        c->auto_shape[m] = StageShape{0, 0, pack};
+        if (!pack) {
+            const int tj = fused_shape(c, momentum ? DYN_TUNE_MOMENTUM_TJ : DYN_TUNE_SCALAR_TJ);
+            const int ti = fused_shape(c, momentum ? DYN_TUNE_MOMENTUM_TI : DYN_TUNE_SCALAR_TI);
+            if ((long long)((ny + tj - 1) / tj) * ((nx + ti - 1) / ti) >= c->pp.cus) continue;
+        }
+        double best = 0.0;
+        for (int tj = 2; tj * (pack ? c->g.nz : KP) <= kPackThreads; tj++) {
+            if (!pack && tj != 2 && tj != 4 && tj != 8) continue;
+            if (stage_lds(c, momentum, tj, pack ? c->g.nz : KP) > c->pp.lds_max) continue;
+            for (int ti = 2; ti <= 48; ti++) {
+                const double t = stage_model(c, momentum, pack, tj, ti);
+                if (c->auto_shape[m].tj == 0 || t < best) {
+                    best = t;
+                    c->auto_shape[m] = StageShape{tj, ti, pack};
+                }
+            }
+        }
     }
-    if (sm <= c->pp.lds_max)
-        DYN_HIP(hipFuncSetAttribute((const void *)k_adv_scalars<T, TJ, true, KW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm));
-    if (sd <= c->pp.lds_max)
-        DYN_HIP(hipFuncSetAttribute((const void *)k_adv_scalars<T, TJ, false, KW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sd));
+}
+
+template <typename T, int TJ, bool PACK>
+int set_lds_limits(const Ctx *c) {
+    const int most = (int)c->pp.lds_max;
+    const void *k[] = {(const void *)k_adv_momentum<T, TJ, true, PACK>, (const void *)k_adv_momentum<T, TJ, false, PACK>,
+                       (const void *)k_adv_scalars<T, TJ, true, PACK>, (const void *)k_adv_scalars<T, TJ, false, PACK>};
+    for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, most));
     return DYN_OK;
 }
 
 template <typename T>
 int set_lds_limits_all(const Ctx *c) {
-    if (fused_waves(c) == 2) {
-        int rc = set_lds_limits<T, 2, 2>(c);
-        if (!rc) rc = set_lds_limits<T, 4, 2>(c);
-        return rc;
-    }
-    int rc = set_lds_limits<T, 2, 1>(c);
-    if (!rc) rc = set_lds_limits<T, 4, 1>(c);
-    if (!rc) rc = set_lds_limits<T, 8, 1>(c);
+    int rc = set_lds_limits<T, 2, true>(c);
+    if (!rc) rc = set_lds_limits<T, 4, true>(c);
+    if (!rc) rc = set_lds_limits<T, 8, true>(c);
+    if (!rc) rc = set_lds_limits<T, 2, false>(c);
+    if (!rc) rc = set_lds_limits<T, 4, false>(c);
+    if (!rc) rc = set_lds_limits<T, 8, false>(c);
     if (rc) return rc;
-    const size_t mom = MomLds<T, 16, 1>::bytes, sm = ScalLds<T, 12, true, 1>::bytes, sd = ScalLds<T, 12, false, 1>::bytes;
-    if (mom <= c->pp.lds_max) {
-        DYN_HIP(hipFuncSetAttribute((const void *)k_adv_momentum<T, 16, true, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mom));
-        DYN_HIP(hipFuncSetAttribute((const void *)k_adv_momentum<T, 16, false, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)mom));
-    }
-    if (sm <= c->pp.lds_max)
-        DYN_HIP(hipFuncSetAttribute((const void *)k_adv_scalars<T, 12, true, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm));
-    if (sd <= c->pp.lds_max)
-        DYN_HIP(hipFuncSetAttribute((const void *)k_adv_scalars<T, 12, false, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sd));
+    const int most = (int)c->pp.lds_max;
+    const void *k[] = {(const void *)k_adv_momentum<T, 16, true, false>, (const void *)k_adv_momentum<T, 16, false, false>,
+                       (const void *)k_adv_scalars<T, 12, true, false>, (const void *)k_adv_scalars<T, 12, false, false>};
+    for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, most));
     return DYN_OK;
 }
+}  // namespace
 
 // the stage kernels may use more than 64 KiB of LDS: raise the per-launch limit once, outside any capture
-int fused_prepare(Ctx *c) { return c->prec == DYN_FP32 ? set_lds_limits_all<float>(c) : set_lds_limits_all<double>(c); }
+int fused_prepare(Ctx *c) {
+    choose_stage_shapes(c);
+    return c->prec == DYN_FP32 ? set_lds_limits_all<float>(c) : set_lds_limits_all<double>(c);
+}
 
 // advect_uvw_velocity + advect_theta (+ advect_microphysics_cell and the interior zero_moisture)
 // over the box [il,ih) x [jl,jh)
@@ -1411,34 +1554,35 @@ int launch_zero_moisture_shell(Ctx *c, int il, int ih, int jl, int jh) {
 
 // ---- ensemble launchers ----------------------------------------------------------------------------
 namespace {
-template <typename T, int TJ>
+// packed rows in the ensemble's batches too (every member has the same level count; at most 8 rows of 64)
+template <typename T, int TJ, bool PACK>
 int ens_momentum_t(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, T step, int ti, int total) {
-    const size_t sh = MomLds<T, TJ>::bytes;
-    const int grid = total;
+    const dim3 blk = PACK ? dim3((TJ * c0->geo.NZ + KP - 1) / KP * KP) : dim3(KP, TJ);
     Timed _t(c0, "ens_momentum", 0.0);
-    hipLaunchKernelGGL((k_ens_momentum<T, TJ, false>), dim3(grid), dim3(KP, TJ), sh, c0->stream, d, nmem, ro, step, ti, total);
+    hipLaunchKernelGGL((k_ens_momentum<T, TJ, false, PACK>), dim3(total), blk, MomLds<T>::bytes(TJ, PACK ? c0->geo.NZ : KP), c0->stream,
+                       d, nmem, ro, step, ti, total);
     DYN_LAUNCH_CHECK();
     return DYN_OK;
 }
-template <typename T, int TJ>
+template <typename T, int TJ, bool PACK>
 int ens_scalars_t(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, T step, int ti, int total) {
-    const size_t sh = ScalLds<T, TJ, false>::bytes;
-    const int grid = total;
+    const dim3 blk = PACK ? dim3((TJ * c0->geo.NZ + KP - 1) / KP * KP) : dim3(KP, TJ);
     Timed _t(c0, "ens_scalars", 0.0);
-    hipLaunchKernelGGL((k_ens_scalars<T, TJ, false>), dim3(grid), dim3(KP, TJ), sh, c0->stream, d, nmem, ro, step, ti, total);
+    hipLaunchKernelGGL((k_ens_scalars<T, TJ, false, PACK>), dim3(total), blk, (ScalLds<T, false>::bytes(TJ, PACK ? c0->geo.NZ : KP)),
+                       c0->stream, d, nmem, ro, step, ti, total);
     DYN_LAUNCH_CHECK();
     return DYN_OK;
 }
-template <typename T>
+template <typename T, bool PACK>
 int ens_stage_t(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, const int *shape, int tot_mom, int tot_scal) {
     int rc;
-    if (shape[0] == 2) rc = ens_momentum_t<T, 2>(c0, d, nmem, ro, T(step), shape[1], tot_mom);
-    else if (shape[0] == 4) rc = ens_momentum_t<T, 4>(c0, d, nmem, ro, T(step), shape[1], tot_mom);
-    else rc = ens_momentum_t<T, 8>(c0, d, nmem, ro, T(step), shape[1], tot_mom);
+    if (shape[0] == 2) rc = ens_momentum_t<T, 2, PACK>(c0, d, nmem, ro, T(step), shape[1], tot_mom);
+    else if (shape[0] == 4) rc = ens_momentum_t<T, 4, PACK>(c0, d, nmem, ro, T(step), shape[1], tot_mom);
+    else rc = ens_momentum_t<T, 8, PACK>(c0, d, nmem, ro, T(step), shape[1], tot_mom);
     if (rc) return rc;
-    if (shape[2] == 2) return ens_scalars_t<T, 2>(c0, d, nmem, ro, T(step), shape[3], tot_scal);
-    if (shape[2] == 4) return ens_scalars_t<T, 4>(c0, d, nmem, ro, T(step), shape[3], tot_scal);
-    return ens_scalars_t<T, 8>(c0, d, nmem, ro, T(step), shape[3], tot_scal);
+    if (shape[2] == 2) return ens_scalars_t<T, 2, PACK>(c0, d, nmem, ro, T(step), shape[3], tot_scal);
+    if (shape[2] == 4) return ens_scalars_t<T, 4, PACK>(c0, d, nmem, ro, T(step), shape[3], tot_scal);
+    return ens_scalars_t<T, 8, PACK>(c0, d, nmem, ro, T(step), shape[3], tot_scal);
 }
 template <typename T>
 int ens_post_t(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, bool pgf, int total) {
@@ -1456,26 +1600,34 @@ int ens_copy_t(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, int to
     DYN_LAUNCH_CHECK();
     return DYN_OK;
 }
-template <typename T, int TJ>
+template <typename T, int TJ, bool PACK>
 int ens_lds_limits() {
-    DYN_HIP(hipFuncSetAttribute((const void *)k_ens_momentum<T, TJ, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)MomLds<T, TJ>::bytes));
-    DYN_HIP(hipFuncSetAttribute((const void *)k_ens_scalars<T, TJ, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)ScalLds<T, TJ, false>::bytes));
+    DYN_HIP(hipFuncSetAttribute((const void *)k_ens_momentum<T, TJ, false, PACK>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)MomLds<T>::bytes(TJ, KP)));
+    DYN_HIP(hipFuncSetAttribute((const void *)k_ens_scalars<T, TJ, false, PACK>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)ScalLds<T, false>::bytes(TJ, KP)));
     return DYN_OK;
+}
+template <typename T>
+int ens_lds_limits_all() {
+    int rc = ens_lds_limits<T, 2, true>();
+    if (!rc) rc = ens_lds_limits<T, 4, true>();
+    if (!rc) rc = ens_lds_limits<T, 8, true>();
+    if (!rc) rc = ens_lds_limits<T, 2, false>();
+    if (!rc) rc = ens_lds_limits<T, 4, false>();
+    if (!rc) rc = ens_lds_limits<T, 8, false>();
+    return rc;
 }
 }  // namespace
 
-int ens_prepare(bool fp32) {
-    int rc = fp32 ? ens_lds_limits<float, 2>() : ens_lds_limits<double, 2>();
-    if (!rc) rc = fp32 ? ens_lds_limits<float, 4>() : ens_lds_limits<double, 4>();
-    if (!rc) rc = fp32 ? ens_lds_limits<float, 8>() : ens_lds_limits<double, 8>();
-    return rc;
-}
+int ens_prepare(bool fp32) { return fp32 ? ens_lds_limits_all<float>() : ens_lds_limits_all<double>(); }
 // the stage advection of every member (one momentum and one scalar launch); shape = {mom TJ, mom TI, scal TJ, scal TI}
 int launch_ens_stage(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, const int *shape, int tot_mom, int tot_scal) {
-    return c0->prec == DYN_FP32 ? ens_stage_t<float>(c0, d, nmem, ro, step, shape, tot_mom, tot_scal)
-                                : ens_stage_t<double>(c0, d, nmem, ro, step, shape, tot_mom, tot_scal);
+    if (stage_packs(c0))
+        return c0->prec == DYN_FP32 ? ens_stage_t<float, true>(c0, d, nmem, ro, step, shape, tot_mom, tot_scal)
+                                    : ens_stage_t<double, true>(c0, d, nmem, ro, step, shape, tot_mom, tot_scal);
+    return c0->prec == DYN_FP32 ? ens_stage_t<float, false>(c0, d, nmem, ro, step, shape, tot_mom, tot_scal)
+                                : ens_stage_t<double, false>(c0, d, nmem, ro, step, shape, tot_mom, tot_scal);
 }
 int launch_ens_post(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, bool pgf, int total) {
     return c0->prec == DYN_FP32 ? ens_post_t<float>(c0, d, nmem, ro, step, pgf, total) : ens_post_t<double>(c0, d, nmem, ro, step, pgf, total);

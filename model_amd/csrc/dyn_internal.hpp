@@ -161,6 +161,11 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
     const int q = n / 8, rem = n % 8, x = b % 8;
     return x * q + min(x, rem) + b / 8;
 }
+// rows per block, march length and lane mapping of a stage kernel's launch (dyn_fused.hip)
+struct StageShape {
+    int tj, ti;
+    bool pack;
+};
 // the two halves of a fused stage (launch_fused_advect's `parts`)
 constexpr int kStageMomentum = 1, kStageScalars = 2;
 
@@ -233,6 +238,9 @@ struct Ctx {
     };
     std::vector<StepGraph> graphs;
     AdjState *adj = nullptr;
+    // launches of the scalar [0] and the momentum [1] stage kernel while their knobs are unset (tj = 0: the
+    // nominal shape), chosen from the grid's size at creation
+    StageShape auto_shape[2] = {};
     // launch-shape knobs (DYN_TUNE_*), 0 = default
     int tune[DYN_TUNE_COUNT] = {0};
     // timing
@@ -303,5 +311,7 @@ int launch_pressure_ens(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &r
 // launch shapes of the stage kernels (DYN_TUNE_*): validity and the value in force
 bool fused_shape_ok(const Ctx *c, int param, int value);
 int fused_shape(const Ctx *c, int param);
+StageShape stage_shape(const Ctx *c, bool momentum);
+int stage_streams(const Ctx *c);
 
 }  // namespace dyn
