@@ -7,8 +7,9 @@
 //   P3  1/(ni*nj) scaling + tridiagonal solve in k, FP64      spec -> spec (in place)
 //   P4  backward DFT along j                                 spec -> spec
 //   P5  backward DFT along i + real part -> PI with the k=0/NZ-1 copies and periodic halos fused
-// The DFTs are Stockham auto-sort passes over an LDS tile [n][kc] (radix 4/2/3/5), batched over a
-// chunk of kc consecutive levels so every global access is a contiguous kc-run of a k column.
+// The DFTs of lengths with factors 2, 3 and 5 are Stockham auto-sort passes over an LDS tile [n][kc] (radix
+// 4/2/3/5), batched over a chunk of kc consecutive levels so every global access is a contiguous kc-run of a
+// k column; other lengths are products with their matrices (dyn_dft.hpp).
 #include <cmath>
 #include <cstdlib>
 #include <type_traits>
@@ -94,6 +95,14 @@ __device__ __forceinline__ void st4(T *p, T a, T b, T c, T d) {
         st2(p + 2, c, d);
     }
 }
+
+}  // namespace
+}  // namespace dyn
+
+#include "dyn_dft.hpp"
+
+namespace dyn {
+namespace {
 
 // in-register DFT of length R with exponent sign `sign`
 template <typename T>
@@ -487,7 +496,7 @@ __global__ void __launch_bounds__(kThreads) k_ifft_x_out(Geo g, const T *__restr
 }
 
 
-// ---- half-spectrum path (even ni) ------------------------------------------------------------------
+// ---- half-spectrum path -----------------------------------------------------------------------------
 // The divergence is real, so two levels travel as the real and imaginary parts of one complex DFT along
 // i and only kx = 0..ni/2 is kept (the rest is the conjugate mirror).  After the j-transform and the
 // tridiagonal solve the real part of the inverse is rebuilt from that half, which is what taking the real
@@ -917,7 +926,7 @@ __device__ __forceinline__ void irfft_x_out_block(const Geo &g, const T *__restr
                     bi = x[u][3];
                 }
             }
-            if (ms == 0 || ms == half) {  // self-conjugate wavenumbers: only the real part is kept
+            if (ms == 0 || 2 * ms == n) {  // self-conjugate wavenumbers: only the real part is kept
                 ai = T(0);
                 bi = T(0);
             }
@@ -1313,7 +1322,7 @@ __device__ __forceinline__ void irfft_x_out_pair_block(const Geo &g, const T *__
                 br = e[2] + sg * o[2];
                 bi = e[3] + sg * o[3];
             }
-            if (ms == 0 || ms == half) {  // self-conjugate wavenumbers: only the real part is kept
+            if (ms == 0 || 2 * ms == n) {  // self-conjugate wavenumbers: only the real part is kept
                 ai = T(0);
                 bi = T(0);
             }
@@ -1568,11 +1577,55 @@ void launch_irfft_x_out(Ctx *c, const T *spec, T *out, const Radix &rx, int kc, 
                        pp.nk2, kc, half);
 }
 
-// one j transform of the three-kernel j pass over nrows kx rows: the power-of-two kernel when nj is a
-// power of two and its plan fits, else the mixed-radix one
+// launches of the matrix-product transforms (dyn_dft.hpp) with 4, 2 or 1 column tiles per block
+template <typename T>
+void launch_div_dft_x(Ctx *c, T *spec, double step) {
+    const PressurePlan &pp = c->pp;
+    const Geo &g = c->geo;
+    const int ncol = pp.nj * pp.nk2, nt = dft_tiles(pp.ni, 1, ncol, pp.cus), nc = 16 * nt;
+    const dim3 grid((ncol + nc - 1) / nc), blk(dft_threads(pp.ni));
+    const size_t sh = dft_lds(pp.ni, nc);
+    const T *u = (const T *)c->prog[DYN_U][2], *v = (const T *)c->prog[DYN_V][2], *w = (const T *)c->prog[DYN_W][2];
+    if (nt == 4) hipLaunchKernelGGL((k_div_dft_x<T, 4>), grid, blk, sh, c->stream, g, c->cols, u, v, w, spec, pp.ni, pp.dftx, pp.nk2, step);
+    else if (nt == 2) hipLaunchKernelGGL((k_div_dft_x<T, 2>), grid, blk, sh, c->stream, g, c->cols, u, v, w, spec, pp.ni, pp.dftx, pp.nk2, step);
+    else hipLaunchKernelGGL((k_div_dft_x<T, 1>), grid, blk, sh, c->stream, g, c->cols, u, v, w, spec, pp.ni, pp.dftx, pp.nk2, step);
+}
+template <typename T>
+int dft_lds_limits() {  // their operands may take more than 64 KiB: kDftMax with one column tile, 80 KiB with more
+    const void *k[] = {(const void *)k_div_dft_x<T, 1>, (const void *)k_div_dft_x<T, 2>, (const void *)k_div_dft_x<T, 4>,
+                       (const void *)k_idft_x_out<T, 1>, (const void *)k_idft_x_out<T, 2>, (const void *)k_idft_x_out<T, 4>,
+                       (const void *)k_dft_y<T, 1>, (const void *)k_dft_y<T, 2>, (const void *)k_dft_y<T, 4>};
+    for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024));
+    return DYN_OK;
+}
+template <typename T>
+void launch_idft_x_out(Ctx *c, const T *spec, T *out) {
+    const PressurePlan &pp = c->pp;
+    const int ncol = pp.nj * pp.nk2, nt = dft_tiles(pp.ni, 1, ncol, pp.cus), nc = 16 * nt;
+    const dim3 grid((ncol + nc - 1) / nc), blk(dft_threads(pp.ni));
+    const size_t sh = dft_lds(pp.ni, nc);
+    if (nt == 4) hipLaunchKernelGGL((k_idft_x_out<T, 4>), grid, blk, sh, c->stream, c->geo, spec, out, pp.ni, pp.dftx, pp.nk2);
+    else if (nt == 2) hipLaunchKernelGGL((k_idft_x_out<T, 2>), grid, blk, sh, c->stream, c->geo, spec, out, pp.ni, pp.dftx, pp.nk2);
+    else hipLaunchKernelGGL((k_idft_x_out<T, 1>), grid, blk, sh, c->stream, c->geo, spec, out, pp.ni, pp.dftx, pp.nk2);
+}
+template <typename T>
+void launch_dft_y(Ctx *c, T *spec, int nrows, int sign) {
+    const PressurePlan &pp = c->pp;
+    const int nt = dft_tiles(pp.nj, nrows, 2 * pp.nk2, pp.cus), nc = 16 * nt;
+    const dim3 grid(nrows, (2 * pp.nk2 + nc - 1) / nc), blk(dft_threads(pp.nj));
+    const size_t sh = dft_lds(pp.nj, nc);
+    if (nt == 4) hipLaunchKernelGGL((k_dft_y<T, 4>), grid, blk, sh, c->stream, spec, pp.nj, pp.dfty, pp.nk2, sign);
+    else if (nt == 2) hipLaunchKernelGGL((k_dft_y<T, 2>), grid, blk, sh, c->stream, spec, pp.nj, pp.dfty, pp.nk2, sign);
+    else hipLaunchKernelGGL((k_dft_y<T, 1>), grid, blk, sh, c->stream, spec, pp.nj, pp.dfty, pp.nk2, sign);
+}
+
+// one j transform of the three-kernel j pass over nrows kx rows: the matrix products for lengths with a
+// prime factor above 5, the power-of-two kernel when nj is a power of two and its plan fits, else the
+// mixed-radix one
 template <typename T>
 void launch_fft_y(Ctx *c, T *spec, int nrows, const Radix &ry, int sign) {
     const PressurePlan &pp = c->pp;
+    if (pp.dfty) return launch_dft_y<T>(c, spec, nrows, sign);
     Radix rp{};
     const int kcp = pow2_plan48(pp.nj, rp, true) ? fft_y_pow2_chunk<T>(rp, pp.nk2) : 0;
     if (kcp > 0) {
@@ -1655,13 +1708,17 @@ int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
     const double pts = (double)pp.ni * pp.nj * pp.nk2;
     ThomasArgs ta{pp.coskx, pp.cosly, c->cols.rhou, c->cols.rhow, c->cols.mu, c->cols.mw, pp.acoef, pp.ffac, c->g.dx, c->g.dz,
                   pp.ni, pp.nj, c->g.nz, pp.zpiv};
-    // even ni of factors 2, 3, 5: half-spectrum transforms in place; otherwise the full complex spectrum
-    if (pp.ni % 2 == 0 && pp.smooth_x) {
+    // half-spectrum transforms, except for lengths with a prime factor above 5 that are too long for the
+    // matrix products: those take the full complex spectrum
+    if (pp.smooth_x || pp.dftx) {
         const int nkx = pp.ni / 2 + 1;
         const int kc = x_level_chunk(pp, g, rx, sizeof(T));
         const size_t shx = x_pass_lds(pp.ni, kc, sizeof(T));
         dim3 gx(g.NY, (pp.nk2 + kc - 1) / kc);
-        {
+        if (pp.dftx) {
+            Timed _t(c, "p1_div_dft_x", pts);
+            launch_div_dft_x<T>(c, spec, step);
+        } else {
             Timed _t(c, "p1_div_rfft_x", pts);
             hipLaunchKernelGGL(k_div_rfft_x<T>, gx, dim3(kThreadsX), shx, c->stream, g, c->cols, (const T *)c->prog[DYN_U][2],
                                (const T *)c->prog[DYN_V][2], (const T *)c->prog[DYN_W][2], spec, rx, pp.twx, pp.nk2, kc, step,
@@ -1707,14 +1764,17 @@ int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
             }
             DYN_LAUNCH_CHECK();
         }
-        {
+        if (pp.dftx) {
+            Timed _t(c, "p5_idft_x_out", pts);
+            launch_idft_x_out<T>(c, spec, (T *)c->pi);
+        } else {
             Timed _t(c, "p5_irfft_x_out", pts);
             launch_irfft_x_out<T>(c, half ? (const T *)pp.spec2 : spec, (T *)c->pi, rx, kc, half);
         }
         DYN_LAUNCH_CHECK();
         return DYN_OK;
     }
-    // odd ni, or a prime factor above 5: full complex spectrum, out-of-place transforms
+    // full complex spectrum, out-of-place transforms
     int kcx = level_chunk(pp.ni, sizeof(T), pp.nk2), kcy = level_chunk(pp.nj, sizeof(T), pp.nk2);
     size_t shx = 4 * (size_t)pp.ni * kcx * sizeof(T), shy = 4 * (size_t)pp.nj * kcy * sizeof(T);
     dim3 gx(g.NY, (pp.nk2 + kcx - 1) / kcx), gy(pp.ni, (pp.nk2 + kcy - 1) / kcy);
@@ -1919,6 +1979,17 @@ int pressure_init(Ctx *c) {
         set_error("pressure solver: twiddle upload failed");
         return DYN_E_HIP;
     }
+    auto matrices = [](int n, bool smooth, double **out) -> int {
+        if (smooth || n > kDftMax) return DYN_OK;
+        const std::vector<double> h = dft_matrices(n);
+        DYN_HIP(hipMalloc(out, sizeof(double) * h.size()));
+        DYN_HIP(hipMemcpy(*out, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
+        return DYN_OK;
+    };
+    int rc = matrices(pp.ni, pp.smooth_x, &pp.dftx);
+    if (!rc) rc = matrices(pp.nj, pp.smooth_y, &pp.dfty);
+    if (!rc && (pp.dftx || pp.dfty)) rc = c->prec == DYN_FP32 ? dft_lds_limits<float>() : dft_lds_limits<double>();
+    if (rc) return rc;
     DYN_HIP(hipMalloc(&pp.spec, sizeof(double) * 2 * (size_t)pp.ni * pp.nj * pp.nk2));
     int dev = 0, lds = 0;
     DYN_HIP(hipGetDevice(&dev));
@@ -2009,7 +2080,7 @@ int pressure_coefficients(Ctx *c) {
 
 int pressure_free(Ctx *c) {
     PressurePlan &pp = c->pp;
-    void *ptrs[] = {pp.twx, pp.twy, pp.spec, pp.spec2, pp.ffac, pp.zpiv, pp.coskx, pp.cosly, pp.acoef, pp.ccoef};
+    void *ptrs[] = {pp.twx, pp.twy, pp.dftx, pp.dfty, pp.spec, pp.spec2, pp.ffac, pp.zpiv, pp.coskx, pp.cosly, pp.acoef, pp.ccoef};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     pp = PressurePlan{};
