@@ -1,5 +1,5 @@
-// Transforms of lengths with a prime factor above 5 (up to kDftMax), as products with the matrices of their
-// cosines and sines on the FP64 matrix units.
+// Transforms as products with the matrices of their cosines and sines on the FP64 matrix units: lengths with
+// a prime factor above 5 (up to kDftMax), and the smooth lengths up to dft_x_smooth() (along i) and kDftYSmooth (along j).
 //
 // A length-n transform needs only rows 0 .. n/2 of the cosine matrix C and the sine matrix S once its input
 // is folded into sums and differences of mirrored elements, E(i) = x(i) + x(n-i), D(i) = x(i) - x(n-i):
@@ -8,10 +8,15 @@
 // and the real inverse is the same two products of the half spectrum's real and imaginary parts.  C and S
 // are (n/2+1) x (n/2+1) and symmetric.  The levels (and rows, and real and imaginary parts) of the other
 // dimensions are the columns of the right operand, so the work is a contraction: n^2/2 multiply-adds per
-// real line in 16x16x4 FP64 tiles whatever the factors of n.  Direct sums over each prime factor (the
-// Stockham passes of dyn_pressure.hip) took 194 + 185 us per solve for the two i transforms of a 194x100x40
-// grid (194 = 2 * 97) in FP32, and needed the full complex spectrum; these take 14 + 12 us and hand the
-// half spectrum to the same j passes as the smooth lengths.  Sums run in FP64 in both forms.
+// real line in 16x16x4 FP64 tiles whatever the factors of n, in one pass over LDS instead of one per radix.
+// Sums run in FP64 in both forms.
+//
+// Measured, us of the i transforms (forward with the divergence, then inverse): against direct sums over the
+// prime factors, 194x100x40 FP32 194 + 185 -> 14.5 + 12.6, 251x251x94 FP64 2214 + 2166 -> 73 + 51; against the
+// radix passes of smooth lengths, FP64 64x64x40 20.6 + 18.7 -> 7.3 + 8.3, 192x192x40 42.2 + 33.4 -> 26.5 + 18.8,
+// 384x384x80 238 + 171 -> 211 + 141; FP32 64x64x40 14.9 + 14.2 -> 7.5 + 7.9, 192x192x40 27.3 + 23.7 -> 22.5 +
+// 18.1, but 256x256x64 33.1 + 28.3 -> 52.7 + 38.2: the work grows with n where the passes' grows with log n,
+// and FP32 passes move half the bytes, so FP32 changes over below 256.
 #pragma once
 
 #include <cmath>
@@ -21,6 +26,11 @@
 
 namespace dyn {
 namespace {
+
+// smooth lengths that take the matrix products: measured faster up to these
+template <typename T>
+constexpr int dft_x_smooth() { return sizeof(T) == 4 ? 192 : 384; }
+constexpr int kDftYSmooth = 192, kDftYThree = 112;
 
 constexpr int kDftMax = 511;  // 256 matrix rows: 16 tiles, one per wavefront of the largest block
 typedef double dvec4 __attribute__((ext_vector_type(4)));
@@ -103,22 +113,26 @@ __device__ __forceinline__ void dft_products(const double *__restrict__ tab, int
     }
 }
 
-// Forward along i: the divergence (as div_rfft_x_block forms it) of NC = 16 NT columns (j, level), folded, and
-// its half spectrum.  Threads keep their column, so its coefficients and row offsets are read once.
-template <typename T, int NT>
-__global__ void __launch_bounds__(dft_bound(NT)) k_div_dft_x(Geo g, Cols c, const T *__restrict__ UP, const T *__restrict__ VP,
-                                                    const T *__restrict__ WP, T *__restrict__ spec, int n, const double *__restrict__ tab,
-                                                    int nk2, double step) {
-    extern __shared__ __align__(16) unsigned char smem[];
+// Forward along i: the divergence (as div_rfft_x_block forms it), or with SRC the ready field src(i+3, j, k)
+// (the transposed solve of the adjoint), of NC = 16 NT columns (j, level), folded, and its half spectrum.
+// Threads keep their column, so its coefficients and row offsets are read once.
+template <typename T, int NT, bool SRC>
+__device__ __forceinline__ void div_dft_x_block(const Geo &g, const Cols &c, const T *__restrict__ UP, const T *__restrict__ VP,
+                                                const T *__restrict__ WP, T *__restrict__ spec, int n, const double *__restrict__ tab,
+                                                int nk2, double step, const T *__restrict__ src, int block, unsigned char *smem) {
     constexpr int NC = 16 * NT;
     const int pitch = dft_pitch(NC), h = dft_rows(n), hk = (h + 3) & ~3, ncol = g.NY * nk2;
     double *E = (double *)smem, *D = E + hk * pitch;
-    const int c0 = blockIdx.x * NC, b = threadIdx.x % NC, q = min(c0 + b, ncol - 1), j = q / nk2, k = q - j * nk2 + 1;
+    const int c0 = block * NC, b = threadIdx.x % NC, q = min(c0 + b, ncol - 1), j = q / nk2, k = q - j * nk2 + 1;
     const int jj = j == 0 ? 1 : (j == g.NY - 1 ? g.NY - 2 : j);  // mirrored rows, pressure.cpp:1408-1415
     const T rhou = T(c.rhou[k]), rw1 = T(c.rhow[k + 1]), rw0 = T(c.rhow[k]), odz = T(g.one_d_dz) * T(c.mu[k]);
     const T sdt = T(step * g.dt);
     const T *u = UP + (long long)jj * g.NZ + k, *v = VP + (long long)jj * g.NZ + k, *w = WP + (long long)jj * g.NZ + k;
     auto load = [&](int i, T (&f)[6]) {
+        if (SRC) {
+            f[0] = src[(long long)(i + 3) * g.NYNZ + (long long)j * g.NZ + k];
+            return;
+        }
         const int ia = i + 3, ie = ia + 1 == g.NX - 3 ? 3 : ia + 1;  // the periodic column UP(NX-3) is read as UP(3)
         f[0] = u[(long long)ie * g.NYNZ];
         f[1] = u[(long long)ia * g.NYNZ];
@@ -128,6 +142,7 @@ __global__ void __launch_bounds__(dft_bound(NT)) k_div_dft_x(Geo g, Cols c, cons
         f[5] = w[(long long)ia * g.NYNZ];
     };
     auto value = [&](const T (&f)[6]) -> double {
+        if (SRC) return double(f[0]);
         T d = rhou * (f[0] - f[1]) * T(g.one_d_dx) + rhou * (f[2] - f[3]) * T(g.one_d_dy) + (rw1 * f[4] - rw0 * f[5]) * odz;
         d /= sdt;
         return double(d);
@@ -168,23 +183,49 @@ __global__ void __launch_bounds__(dft_bound(NT)) k_div_dft_x(Geo g, Cols c, cons
         }
     }
 }
+template <typename T, int NT, bool SRC>
+__global__ void __launch_bounds__(dft_bound(NT)) k_div_dft_x(Geo g, Cols c, const T *__restrict__ UP, const T *__restrict__ VP,
+                                                             const T *__restrict__ WP, T *__restrict__ spec, int n,
+                                                             const double *__restrict__ tab, int nk2, double step,
+                                                             const T *__restrict__ src) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    div_dft_x_block<T, NT, SRC>(g, c, UP, VP, WP, spec, n, tab, nk2, step, src, blockIdx.x, smem);
+}
 
 // Backward along i: the half spectrum's rows, weighted for their mirror images (2, and 1 for the
 // self-conjugate wavenumbers, whose imaginary part is dropped), to PI with its ghost levels and periodic
-// halos (pressure.cpp:878-892, boundaries.cpp:533-540)
+// halos (pressure.cpp:878-892, boundaries.cpp:533-540).  With jhalf the half-slab j pass left row j of the full
+// inverse as v0(j') + s v1(j'), j' = j mod jhalf (see irfft_x_out_block).
 template <typename T, int NT>
-__global__ void __launch_bounds__(dft_bound(NT)) k_idft_x_out(Geo g, const T *__restrict__ spec, T *__restrict__ PI, int n,
-                                                     const double *__restrict__ tab, int nk2) {
-    extern __shared__ __align__(16) unsigned char smem[];
+__device__ __forceinline__ void idft_x_out_block(const Geo &g, const T *__restrict__ spec, T *__restrict__ PI, int n,
+                                                 const double *__restrict__ tab, int nk2, int block, unsigned char *smem, int jhalf = 0) {
     constexpr int NC = 16 * NT;
     const int pitch = dft_pitch(NC), h = dft_rows(n), hk = (h + 3) & ~3, ncol = g.NY * nk2;
     double *E = (double *)smem, *D = E + hk * pitch;
-    const int c0 = blockIdx.x * NC, b = threadIdx.x % NC, q = min(c0 + b, ncol - 1);
+    const int c0 = block * NC, b = threadIdx.x % NC, q = min(c0 + b, ncol - 1);
+    const bool second = jhalf && q >= jhalf * nk2;
+    const int q0 = second ? q - jhalf * nk2 : q;
+    const T sg = second ? T(-1) : T(1);
     const int rows = blockDim.x / NC;
     for (int i = threadIdx.x / NC; i < hk; i += 4 * rows) {
         T a[4], m[4];
+        if (jhalf) {
+            T a1[4], m1[4];
 #pragma unroll
-        for (int r = 0; r < 4; r++) ld2(spec + ((long long)min(i + r * rows, h - 1) * ncol + q) * 2, a[r], m[r]);
+            for (int r = 0; r < 4; r++) {
+                const T *o = spec + ((long long)min(i + r * rows, h - 1) * ncol + q0) * 2;
+                ld2(o, a[r], m[r]);
+                ld2(o + 2LL * jhalf * nk2, a1[r], m1[r]);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                a[r] = a[r] + sg * a1[r];
+                m[r] = m[r] + sg * m1[r];
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; r++) ld2(spec + ((long long)min(i + r * rows, h - 1) * ncol + q) * 2, a[r], m[r]);
+        }
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int ir = i + r * rows;
@@ -223,6 +264,13 @@ __global__ void __launch_bounds__(dft_bound(NT)) k_idft_x_out(Geo g, const T *__
             }
         }
     }
+}
+
+template <typename T, int NT>
+__global__ void __launch_bounds__(dft_bound(NT)) k_idft_x_out(Geo g, const T *__restrict__ spec, T *__restrict__ PI, int n,
+                                                              const double *__restrict__ tab, int nk2, int jhalf) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    idft_x_out_block<T, NT>(g, spec, PI, n, tab, nk2, blockIdx.x, smem, jhalf);
 }
 
 // value of the neighbouring lane (lane ^ 1) by a DPP quad permutation

@@ -72,7 +72,7 @@ void offsets(const Ensemble *e, std::vector<EnsMember> &h, int &tmom, int &tscal
         t.post0 = post;
         post += ((t.g.NY + 3) / 4) * (t.g.NX - 6);
         t.px0 = px;
-        if (e->batched_pressure) px += t.g.NY * ((t.nk2 + t.kcx - 1) / t.kcx);
+        if (e->batched_pressure) px += t.pxn;
         t.py0 = py;
         if (e->batched_pressure) py += t.ni / 2 + 1;
         t.cp0 = cp;
@@ -339,6 +339,7 @@ int dyn_ensemble_create(dyn_ctx *const *members, int n, dyn_ensemble **out) {
         e->shape[0] = e->shape[2] = 4;
     }
     int rc = ens_prepare(c0->prec == DYN_FP32);
+    if (!rc && all_batched) rc = pressure_ens_prepare(c0);
     if (!rc && hipMalloc(&e->d, sizeof(EnsMember) * n) != hipSuccess) {
         set_error("dyn_ensemble_create: table allocation failed");
         rc = DYN_E_HIP;

@@ -1454,14 +1454,13 @@ StageShape stage_shape(const Ctx *c, bool momentum) {
 
 // How a step's stages use the second stream (the values of DYN_TUNE_STAGE_STREAMS) while the knob is unset.
 // With short marches the scalar kernel no longer delays the divergence pass it is queued behind, so the late
-// queueing (4) is the faster form up to a few million points (FP32 moist, 2 against 4: 361 and 335 us per
-// step at 128x128x64, 692 and 666 at 256x256x40; FP64 moist, 3 against 4: 625 and 563 at 128x128x64), and for
-// every dry FP32 grid; the largest moist grids keep the nominal form (FP32 256x256x64: 834 against 871 us).
+// queueing (4) is the faster form nearly everywhere (us per step, nominal form against 4: FP32 moist 344 and
+// 319 at 128x128x64, 679 and 655 at 256x256x40; FP64 579 and 522 moist at 128x128x64, 1314 and 1239 dry at
+// 256x256x64); the largest moist FP32 grids keep the nominal form (256x256x64: 833 against 874).
 int stage_streams(const Ctx *c) {
     const int nominal = fused_shape(c, DYN_TUNE_STAGE_STREAMS);
     if (c->tune[DYN_TUNE_STAGE_STREAMS]) return nominal;
-    const bool few = c->npts < (nominal == 3 ? 2000000u : 3000000u);
-    return few || (nominal == 2 && !c->g.microphysics) ? 4 : nominal;
+    return nominal == 2 && c->g.microphysics && c->npts >= 3000000u ? nominal : 4;
 }
 
 namespace {

@@ -101,7 +101,6 @@ struct PressurePlan {
     double *coskx = nullptr, *cosly = nullptr; // cos(kwave[i]), cos(lwave[j]) as init_fft3d evaluates them
     double *acoef = nullptr, *ccoef = nullptr; // pressure.cpp:779-782
     void *spec = nullptr;              // spectral work array [kx][ky][kk] complex (T)
-    double *ffac = nullptr;            // Thomas multipliers F2 [kx][kk][ky] (FP64)
     double *zpiv = nullptr;            // Thomas pivot reciprocals [kx][kk][ky] (FP64)
     // transform lengths whose factors are all 2, 3 and 5 (the in-place LDS transforms' butterflies); a
     // length with a larger prime factor takes the matrix products, or above their largest length the
@@ -110,6 +109,7 @@ struct PressurePlan {
     // cosine and sine matrices of the lengths that are transformed by matrix products (dyn_dft.hpp)
     double *dftx = nullptr, *dfty = nullptr;
     bool fused_y = false;              // j-transforms and the vertical solve in one LDS-resident kernel
+    bool ydft = false;                 // ... its transforms by matrix products
     bool half_y = false;               // ... or in two per kx on half slabs (even nj; one radix-2 split)
     void *spec2 = nullptr;             // output of the half-slab j pass ([kx][j][kk] complex, T)
     size_t lds_max = 0;
@@ -136,10 +136,10 @@ struct EnsMember {
     int js, jn;
     // pressure plan
     void *spec;
-    const double *twx, *twy, *ffac, *zpiv, *coskx, *cosly, *acoef;
+    const double *twx, *twy, *zpiv, *acoef, *ccoef, *dftx, *dfty;
+    int ydft, pxn;  // the j pass by matrix products; work items of its i passes
     Radix rx, ry;
     int ni, nj, nk2, kcx;
-    double dx, dz;
     // first work item of this member in each batched launch
     int mom0, scal0, post0, px0, py0, cp0;
     int nbj_mom, nbj_scal;
@@ -309,6 +309,7 @@ int launch_ens_stage(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, 
 int launch_ens_post(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, bool pgf, int total);
 int launch_ens_copy(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, int total);
 bool pressure_ens_fill(Ctx *c, EnsMember &e, size_t &lds_x, size_t &lds_y);
+int pressure_ens_prepare(const Ctx *c);
 int launch_pressure_ens(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, int tot_px, int tot_py, size_t lds_x,
                         size_t lds_y);
 // launch shapes of the stage kernels (DYN_TUNE_*): validity and the value in force

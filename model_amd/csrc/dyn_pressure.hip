@@ -368,18 +368,18 @@ __global__ void __launch_bounds__(kThreads) k_fft_y(T *__restrict__ spec, int nj
     }
 }
 
-// Tridiagonal multipliers F2 of pressure.cpp:840-855 for every (kx,ky): a pure function of the
-// coefficients, so they are formed once per context instead of once per solve.
+// Pivot reciprocals z of pressure.cpp:840-855 for every (kx,ky): a pure function of the coefficients, so they
+// are formed once per context instead of once per solve.  The multipliers F2 = ccoef z are one product away
+// and are formed where they are used (the same bits).  Layout [kx][kk][ky]: the columns of one kx are
+// adjacent for every level.
 __global__ void k_thomas_factors(int ni, int nj, int nk, const double *__restrict__ coskx, const double *__restrict__ cosly,
                                  const double *__restrict__ rhou, const double *__restrict__ rhow, const double *__restrict__ mu,
                                  const double *__restrict__ mw, const double *__restrict__ acoef, const double *__restrict__ ccoef,
-                                 double dx, double dz, double *__restrict__ ffac, double *__restrict__ zpiv) {
+                                 double dx, double dz, double *__restrict__ zpiv) {
     int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= ni * nj) return;
     int kx = q / nj, ky = q % nj;
     int nk2 = nk - 2;
-    // layout [kx][kk][ky]: the columns of one kx are adjacent for every level
-    double *F = ffac + (long long)kx * nk2 * nj + ky;
     double *Z = zpiv + (long long)kx * nk2 * nj + ky;
     const long long fs = nj;
     double ck = coskx[kx], cl = cosly[ky];
@@ -387,14 +387,12 @@ __global__ void k_thomas_factors(int ni, int nj, int nk, const double *__restric
     double B = rhou[1] * 2.0 * (ck + cl - 2.0) / (dx * dx) - mu[1] * mw[2] * rhow[2] / (dz * dz);
     double z = 1.0 / B;
     double Fp = ccoef[1] * z;
-    F[0] = Fp;
     Z[0] = z;
     for (int k = 2; k < nk - 1; k++) {
         if (k < nk - 2) B = rhou[k] * 2.0 * (ck + cl - 2.0) / (dx * dx) - mu[k] * (mw[k + 1] * rhow[k + 1] + mw[k] * rhow[k]) / (dz * dz);
         else B = rhou[nk - 2] * 2.0 * (ck + cl - 2.0) / (dx * dx) - (mu[nk - 2] * mw[nk - 2] * rhow[nk - 2]) / (dz * dz);
         z = 1.0 / (B - acoef[k] * Fp);
         Fp = ccoef[k] * z;
-        F[(k - 1) * fs] = Fp;
         Z[(k - 1) * fs] = z;
     }
 }
@@ -402,35 +400,27 @@ __global__ void k_thomas_factors(int ni, int nj, int nk, const double *__restric
 // P3: normalisation (pressure.cpp:824-827), forward elimination (837-856), mean-mode gauge (858-859)
 // and back substitution (864-871), in FP64 whatever the storage precision.
 template <typename T>
-__global__ void k_thomas(T *__restrict__ spec, int ni, int nj, int nk, const double *__restrict__ coskx, const double *__restrict__ cosly,
-                         const double *__restrict__ rhou, const double *__restrict__ rhow, const double *__restrict__ mu,
-                         const double *__restrict__ mw, const double *__restrict__ acoef, const double *__restrict__ ffac, double dx,
-                         double dz) {
+__global__ void k_thomas(T *__restrict__ spec, int ni, int nj, int nk, const double *__restrict__ acoef, const double *__restrict__ ccoef,
+                         const double *__restrict__ zpiv) {
     int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= ni * nj) return;
     int kx = q / nj, ky = q % nj;
     const int nk2 = nk - 2;
     T *x = spec + (long long)q * nk2 * 2;
     const long long fs = nj;
-    const double *F = ffac + (long long)kx * nk2 * nj + ky;
+    const double *Z = zpiv + (long long)kx * nk2 * nj + ky;
     const double size2d = (double)(ni * nj);
-    double ck = coskx[kx], cl = cosly[ky];
-    double B = rhou[1] * 2.0 * (ck + cl - 2.0) / (dx * dx) - mu[1] * mw[2] * rhow[2] / (dz * dz);
-    double z = 1.0 / B;
+    double z = Z[0];
     double pr = (double(x[0]) / size2d) * z, pi = (double(x[1]) / size2d) * z;
     x[0] = T(pr);
     x[1] = T(pi);
-    double Fp = F[0];
     for (int k = 2; k < nk - 1; k++) {
-        if (k < nk - 2) B = rhou[k] * 2.0 * (ck + cl - 2.0) / (dx * dx) - mu[k] * (mw[k + 1] * rhow[k + 1] + mw[k] * rhow[k]) / (dz * dz);
-        else B = rhou[nk - 2] * 2.0 * (ck + cl - 2.0) / (dx * dx) - (mu[nk - 2] * mw[nk - 2] * rhow[nk - 2]) / (dz * dz);
-        z = 1.0 / (B - acoef[k] * Fp);
+        z = Z[(k - 1) * fs];
         double xr = double(x[2 * (k - 1)]) / size2d, xi = double(x[2 * (k - 1) + 1]) / size2d;
         pr = (xr - acoef[k] * pr) * z;
         pi = (xi - acoef[k] * pi) * z;
         x[2 * (k - 1)] = T(pr);
         x[2 * (k - 1) + 1] = T(pi);
-        Fp = F[(k - 1) * fs];
     }
     if (kx == 0 && ky == 0) {  // OUT3D(0,0,NZ-2) = 0
         pr = 0.0;
@@ -439,7 +429,7 @@ __global__ void k_thomas(T *__restrict__ spec, int ni, int nj, int nk, const dou
         x[2 * (nk2 - 1) + 1] = T(0);
     }
     for (int k = nk - 3; k >= 1; k--) {
-        double f = F[(k - 1) * fs];
+        double f = ccoef[k] * Z[(k - 1) * fs];
         pr = double(x[2 * (k - 1)]) - f * pr;
         pi = double(x[2 * (k - 1) + 1]) - f * pi;
         x[2 * (k - 1)] = T(pr);
@@ -967,24 +957,34 @@ __device__ __forceinline__ void irfft_x_out_block(const Geo &g, const T *__restr
     }
 }
 
-// B2 of pressure.cpp:787-791 for level k (1..nk-2) of column (ck, cl)
-__device__ __forceinline__ double bcoef(int k, int nk, double ck, double cl, const double *rhou, const double *rhow, const double *mu,
-                                        const double *mw, double dx, double dz) {
-    if (k == 1) return rhou[1] * 2.0 * (ck + cl - 2.0) / (dx * dx) - mu[1] * mw[2] * rhow[2] / (dz * dz);
-    if (k < nk - 2) return rhou[k] * 2.0 * (ck + cl - 2.0) / (dx * dx) - mu[k] * (mw[k + 1] * rhow[k + 1] + mw[k] * rhow[k]) / (dz * dz);
-    return rhou[nk - 2] * 2.0 * (ck + cl - 2.0) / (dx * dx) - (mu[nk - 2] * mw[nk - 2] * rhow[nk - 2]) / (dz * dz);
+// a_k and c_k of levels k = 1 .. nk2 in LDS (ac[kk], cc[kk], kk = k-1): read from global memory they are scalar
+// loads of a cache line per chunk, each waited for in turn
+struct ThomasCoef {
+    const double *ac, *cc;
+};
+struct ThomasArgs {
+    const double *acoef, *ccoef;  // by level k
+    const double *zpiv;           // pivot reciprocals z of every column, [kx][kk][ky]
+    int ni, nj, nk;
+};
+inline ThomasArgs thomas_args(const PressurePlan &pp, int nk) { return ThomasArgs{pp.acoef, pp.ccoef, pp.zpiv, pp.ni, pp.nj, nk}; }
+
+__device__ __forceinline__ ThomasCoef thomas_coef(const ThomasArgs &ta, int nk2, double *lds) {
+    for (int q = (int)threadIdx.x; q < 2 * nk2; q += (int)blockDim.x) lds[q] = q < nk2 ? ta.acoef[q + 1] : ta.ccoef[q - nk2 + 1];
+    return ThomasCoef{lds, lds + nk2};
 }
 
-struct ThomasArgs {
-    const double *coskx, *cosly, *rhou, *rhow, *mu, *mw, *acoef, *ffac;
-    double dx, dz;
-    int ni, nj, nk;
-    const double *zpiv;  // pivot reciprocals z_k of every column, same layout as ffac
-};
+// x / d for the divisor's correctly rounded reciprocal r: x r is within an ulp of the quotient, its remainder
+// is exact in a fused multiply-add, and adding remainder r rounds to the quotient itself (Markstein 1990);
+// a dozen FP64 instructions fewer than a division, and the sweeps are bound by what they issue.
+__device__ __forceinline__ double div_exact(double x, double d, double r) {
+    const double q = x * r;
+    return __builtin_fma(__builtin_fma(-q, d, x), r, q);
+}
 
-// The sweeps below walk the levels in chunks of kTC and load the next chunk's table values (pivots or
-// multipliers, one column of the [kx][kk][ky] tables) while the current chunk is eliminated, so the
-// dependent recurrence does not wait on global-memory latency level by level.
+// The sweeps below walk the levels in chunks of kTC and load the next chunk's pivots (one column of the table,
+// from global memory or from a copy in LDS) while the current chunk is eliminated, so the dependent
+// recurrence does not wait on memory latency level by level.  The multipliers are F_k = c_k z_k.
 constexpr int kThomasChunk = 8;  // levels per chunk of the Thomas sweeps
 
 // Forward elimination and back substitution of one real sequence (the real or the imaginary part) of one
@@ -1010,39 +1010,40 @@ __device__ __forceinline__ void thomas_tab_down(const double *Tab, long long fs,
     for (int t = 0; t < kTC; t++) v[t] = Tab[max(k0 - t, 0) * fs];
 }
 // p_kk = (x_kk / (ni nj) - a_k p_{kk-1}) z_kk for the chunk's levels kk = k0 .. k0+kTC-1 (< N unless FULL)
-template <typename T, bool FULL, int kTC>
-__device__ __forceinline__ void thomas_fwd_chunk(const ThomasArgs &ta, const double (&z)[kTC], int k0, int N, double size2d, T *x,
-                                                 int xs, bool m0, double *mean, double &p) {
+template <typename T, bool FULL, int kTC, typename XT>
+__device__ __forceinline__ void thomas_fwd_chunk(const ThomasCoef &co, const double (&z)[kTC], int k0, int N, double size2d,
+                                                 double rsize, XT *x, int xs, bool m0, double *mean, double &p) {
     double v[kTC], ac[kTC];
 #pragma unroll
     for (int t = 0; t < kTC; t++) {
         const int kk = FULL ? k0 + t : min(k0 + t, N - 1);
         v[t] = double(x[kk * xs]);
-        ac[t] = ta.acoef[kk + 1];
+        ac[t] = co.ac[kk];
     }
 #pragma unroll
     for (int t = 0; t < kTC; t++) {
-        if (FULL || k0 + t < N) p = (v[t] / size2d - ac[t] * p) * z[t];
+        if (FULL || k0 + t < N) p = (div_exact(v[t], size2d, rsize) - ac[t] * p) * z[t];
         v[t] = p;
     }
 #pragma unroll
     for (int t = 0; t < kTC; t++) {
         if (FULL || k0 + t < N) {
             if (m0) mean[2 * (k0 + t)] = v[t];
-            else x[(k0 + t) * xs] = T(v[t]);
+            else x[(k0 + t) * xs] = XT(T(v[t]));
         }
     }
 }
 // x_kk = y_kk - F_kk x_{kk+1} for kk = k0 .. k0-kTC+1 (>= 0 unless FULL)
-template <typename T, bool FULL, int kTC>
-__device__ __forceinline__ void thomas_back_chunk(const double (&f)[kTC], int k0, T *x, int xs, bool m0, const double *mean,
-                                                  double &p) {
-    double v[kTC];
+template <typename T, bool FULL, int kTC, typename XT>
+__device__ __forceinline__ void thomas_back_chunk(const ThomasCoef &co, const double (&z)[kTC], int k0, XT *x, int xs, bool m0,
+                                                  const double *mean, double &p) {
+    double v[kTC], f[kTC];
 #pragma unroll
     for (int t = 0; t < kTC; t++) {
         const int kk = FULL ? k0 - t : max(k0 - t, 0);
         const double vm = mean[2 * kk], vx = double(x[kk * xs]);
         v[t] = m0 ? vm : vx;
+        f[t] = co.cc[kk] * z[t];
     }
 #pragma unroll
     for (int t = 0; t < kTC; t++) {
@@ -1051,14 +1052,14 @@ __device__ __forceinline__ void thomas_back_chunk(const double (&f)[kTC], int k0
     }
 #pragma unroll
     for (int t = 0; t < kTC; t++)
-        if (FULL || k0 - t >= 0) x[(k0 - t) * xs] = T(v[t]);
+        if (FULL || k0 - t >= 0) x[(k0 - t) * xs] = XT(T(v[t]));
 }
-template <typename T, int kTC = kThomasChunk>
-__device__ void thomas_part(const ThomasArgs &ta, int kx, int ky, T *x, int xs, double *mean) {
+// Z: the column's pivots, one every fs.  Values are rounded to T whatever the type XT they are held in.
+template <typename T, int kTC = kThomasChunk, typename XT>
+__device__ __forceinline__ void thomas_part(const ThomasArgs &ta, const ThomasCoef &co, int kx, int ky, const double *Z, long long fs, XT *x, int xs,
+                                            double *mean) {
     const int N = ta.nk - 2;
-    const long long fs = ta.nj, col = (long long)kx * N * ta.nj + ky;
-    const double *F = ta.ffac + col, *Z = ta.zpiv + col;
-    const double size2d = (double)(ta.ni * ta.nj);
+    const double size2d = (double)(ta.ni * ta.nj), rsize = 1.0 / size2d;
     const bool m0 = (kx == 0 && ky == 0);
     double A[kTC], B[kTC], p = 0.0;
     // full chunks two at a time (one path through the loop, so the loads of the set not in use stay in
@@ -1067,42 +1068,46 @@ __device__ void thomas_part(const ThomasArgs &ta, int kx, int ky, T *x, int xs, 
     int k0 = 0;
     for (; k0 + 2 * kTC <= N; k0 += 2 * kTC) {
         thomas_tab_up<kTC>(Z, fs, k0 + kTC, N - 1, B);
-        thomas_fwd_chunk<T, true, kTC>(ta, A, k0, N, size2d, x, xs, m0, mean, p);
+        thomas_fwd_chunk<T, true, kTC>(co, A, k0, N, size2d, rsize, x, xs, m0, mean, p);
         thomas_tab_up<kTC>(Z, fs, k0 + 2 * kTC, N - 1, A);
-        thomas_fwd_chunk<T, true, kTC>(ta, B, k0 + kTC, N, size2d, x, xs, m0, mean, p);
+        thomas_fwd_chunk<T, true, kTC>(co, B, k0 + kTC, N, size2d, rsize, x, xs, m0, mean, p);
     }
     if (k0 < N) {
         thomas_tab_up<kTC>(Z, fs, k0 + kTC, N - 1, B);
-        if (k0 + kTC <= N) thomas_fwd_chunk<T, true, kTC>(ta, A, k0, N, size2d, x, xs, m0, mean, p);
-        else thomas_fwd_chunk<T, false, kTC>(ta, A, k0, N, size2d, x, xs, m0, mean, p);
-        if (k0 + kTC < N) thomas_fwd_chunk<T, false, kTC>(ta, B, k0 + kTC, N, size2d, x, xs, m0, mean, p);
+        if (k0 + kTC <= N) thomas_fwd_chunk<T, true, kTC>(co, A, k0, N, size2d, rsize, x, xs, m0, mean, p);
+        else thomas_fwd_chunk<T, false, kTC>(co, A, k0, N, size2d, rsize, x, xs, m0, mean, p);
+        if (k0 + kTC < N) thomas_fwd_chunk<T, false, kTC>(co, B, k0 + kTC, N, size2d, rsize, x, xs, m0, mean, p);
     }
     if (m0) p = 0.0;  // OUT3D(0,0,NZ-2) = 0
-    x[(N - 1) * xs] = T(p);
+    x[(N - 1) * xs] = XT(T(p));
     if (N < 2) return;
     // back substitution x_kk = y_kk - F_kk x_{kk+1} for kk = N-2 .. 0, walking down in chunks
-    thomas_tab_down<kTC>(F, fs, N - 2, A);
+    thomas_tab_down<kTC>(Z, fs, N - 2, A);
     k0 = N - 2;
     for (; k0 - 2 * kTC + 1 >= 0; k0 -= 2 * kTC) {
-        thomas_tab_down<kTC>(F, fs, k0 - kTC, B);
-        thomas_back_chunk<T, true, kTC>(A, k0, x, xs, m0, mean, p);
-        thomas_tab_down<kTC>(F, fs, k0 - 2 * kTC, A);
-        thomas_back_chunk<T, true, kTC>(B, k0 - kTC, x, xs, m0, mean, p);
+        thomas_tab_down<kTC>(Z, fs, k0 - kTC, B);
+        thomas_back_chunk<T, true, kTC>(co, A, k0, x, xs, m0, mean, p);
+        thomas_tab_down<kTC>(Z, fs, k0 - 2 * kTC, A);
+        thomas_back_chunk<T, true, kTC>(co, B, k0 - kTC, x, xs, m0, mean, p);
     }
     if (k0 >= 0) {
-        thomas_tab_down<kTC>(F, fs, k0 - kTC, B);
-        if (k0 - kTC + 1 >= 0) thomas_back_chunk<T, true, kTC>(A, k0, x, xs, m0, mean, p);
-        else thomas_back_chunk<T, false, kTC>(A, k0, x, xs, m0, mean, p);
-        if (k0 - kTC >= 0) thomas_back_chunk<T, false, kTC>(B, k0 - kTC, x, xs, m0, mean, p);
+        thomas_tab_down<kTC>(Z, fs, k0 - kTC, B);
+        if (k0 - kTC + 1 >= 0) thomas_back_chunk<T, true, kTC>(co, A, k0, x, xs, m0, mean, p);
+        else thomas_back_chunk<T, false, kTC>(co, A, k0, x, xs, m0, mean, p);
+        if (k0 - kTC >= 0) thomas_back_chunk<T, false, kTC>(co, B, k0 - kTC, x, xs, m0, mean, p);
     }
 }
 
-// q_kk = x_kk - F_{kk-1} q_{kk-1} for the chunk's levels kk = k0 .. k0+kTC-1 (< N unless FULL), f[t] = F_{k0+t-1}
-template <typename T, bool FULL, int kTC>
-__device__ __forceinline__ void thomas_t_fwd_chunk(const double (&f)[kTC], int k0, int N, T *x, int xs, double &q) {
-    double v[kTC];
+// q_kk = x_kk - F_{kk-1} q_{kk-1} for the chunk's levels kk = k0 .. k0+kTC-1 (< N unless FULL), z[t] = z_{k0+t-1}
+template <typename T, bool FULL, int kTC, typename XT>
+__device__ __forceinline__ void thomas_t_fwd_chunk(const ThomasCoef &co, const double (&z)[kTC], int k0, int N, XT *x, int xs, double &q) {
+    double v[kTC], f[kTC];
 #pragma unroll
-    for (int t = 0; t < kTC; t++) v[t] = double(x[(FULL ? k0 + t : min(k0 + t, N - 1)) * xs]);
+    for (int t = 0; t < kTC; t++) {
+        const int kk = FULL ? k0 + t : min(k0 + t, N - 1);
+        v[t] = double(x[kk * xs]);
+        f[t] = co.cc[kk - 1] * z[t];
+    }
 #pragma unroll
     for (int t = 0; t < kTC; t++) {
         if (FULL || k0 + t < N) q = v[t] - f[t] * q;
@@ -1110,27 +1115,27 @@ __device__ __forceinline__ void thomas_t_fwd_chunk(const double (&f)[kTC], int k
     }
 #pragma unroll
     for (int t = 0; t < kTC; t++)
-        if (FULL || k0 + t < N) x[(k0 + t) * xs] = T(v[t]);
+        if (FULL || k0 + t < N) x[(k0 + t) * xs] = XT(T(v[t]));
 }
 // b_kk = z_kk (q_kk - a_{kk+2} b_{kk+1}), stored as b / (ni nj), for kk = k0 .. k0-kTC+1 (>= 0 unless FULL)
-template <typename T, bool FULL, int kTC>
-__device__ __forceinline__ void thomas_t_back_chunk(const ThomasArgs &ta, const double (&z)[kTC], int k0, double size2d, T *x, int xs,
-                                                    double &b) {
+template <typename T, bool FULL, int kTC, typename XT>
+__device__ __forceinline__ void thomas_t_back_chunk(const ThomasCoef &co, const double (&z)[kTC], int k0, double size2d, double rsize,
+                                                    XT *x, int xs, double &b) {
     double v[kTC], ac[kTC];
 #pragma unroll
     for (int t = 0; t < kTC; t++) {
         const int kk = FULL ? k0 - t : max(k0 - t, 0);
         v[t] = double(x[kk * xs]);
-        ac[t] = ta.acoef[kk + 2];
+        ac[t] = co.ac[kk + 1];
     }
 #pragma unroll
     for (int t = 0; t < kTC; t++) {
         if (FULL || k0 - t >= 0) b = (v[t] - ac[t] * b) * z[t];
-        v[t] = b / size2d;
+        v[t] = div_exact(b, size2d, rsize);
     }
 #pragma unroll
     for (int t = 0; t < kTC; t++)
-        if (FULL || k0 - t >= 0) x[(k0 - t) * xs] = T(v[t]);
+        if (FULL || k0 - t >= 0) x[(k0 - t) * xs] = XT(T(v[t]));
 }
 // Transpose of thomas_part (the adjoint's vertical solve), in place.  The forward map is p = L'^{-1} x / S
 // (L' lower bidiagonal: 1/z_k on the diagonal, a_k below) followed by x_k = p_k - F_k x_{k+1}; for the
@@ -1138,47 +1143,45 @@ __device__ __forceinline__ void thomas_t_back_chunk(const ThomasArgs &ta, const 
 // reverse order: q_1 = x_1, q_k = x_k - F_{k-1} q_{k-1} (q_N = 0 for (0,0)), then b_N = z_N q_N,
 // b_k = z_k (q_k - a_{k+1} b_{k+1}), result b / S.  The singular last pivot of (0,0) is never used.
 // The table entries come in chunks through two register sets that take turns, as in thomas_part.
-template <typename T, int kTC = kThomasChunk>
-__device__ void thomas_part_t(const ThomasArgs &ta, int kx, int ky, T *x, int xs) {
+template <typename T, int kTC = kThomasChunk, typename XT>
+__device__ __forceinline__ void thomas_part_t(const ThomasArgs &ta, const ThomasCoef &co, int kx, int ky, const double *Z, long long fs, XT *x, int xs) {
     const int N = ta.nk - 2;
-    const long long fs = ta.nj, col = (long long)kx * N * ta.nj + ky;
-    const double *F = ta.ffac + col, *Z = ta.zpiv + col;
-    const double size2d = (double)(ta.ni * ta.nj);
+    const double size2d = (double)(ta.ni * ta.nj), rsize = 1.0 / size2d;
     const bool m0 = (kx == 0 && ky == 0);
     double A[kTC], B[kTC];
     // q_kk = x_kk - F_{kk-1} q_{kk-1}, kk = 1 .. N-1 (q_0 = x_0)
     double q = double(x[0]);
-    thomas_tab_up<kTC>(F, fs, 0, N - 2, A);
+    thomas_tab_up<kTC>(Z, fs, 0, N - 2, A);
     int k0 = 1;
     for (; k0 + 2 * kTC <= N; k0 += 2 * kTC) {
-        thomas_tab_up<kTC>(F, fs, k0 + kTC - 1, N - 2, B);
-        thomas_t_fwd_chunk<T, true, kTC>(A, k0, N, x, xs, q);
-        thomas_tab_up<kTC>(F, fs, k0 + 2 * kTC - 1, N - 2, A);
-        thomas_t_fwd_chunk<T, true, kTC>(B, k0 + kTC, N, x, xs, q);
+        thomas_tab_up<kTC>(Z, fs, k0 + kTC - 1, N - 2, B);
+        thomas_t_fwd_chunk<T, true, kTC>(co, A, k0, N, x, xs, q);
+        thomas_tab_up<kTC>(Z, fs, k0 + 2 * kTC - 1, N - 2, A);
+        thomas_t_fwd_chunk<T, true, kTC>(co, B, k0 + kTC, N, x, xs, q);
     }
     if (k0 < N) {
-        thomas_tab_up<kTC>(F, fs, k0 + kTC - 1, N - 2, B);
-        if (k0 + kTC <= N) thomas_t_fwd_chunk<T, true, kTC>(A, k0, N, x, xs, q);
-        else thomas_t_fwd_chunk<T, false, kTC>(A, k0, N, x, xs, q);
-        if (k0 + kTC < N) thomas_t_fwd_chunk<T, false, kTC>(B, k0 + kTC, N, x, xs, q);
+        thomas_tab_up<kTC>(Z, fs, k0 + kTC - 1, N - 2, B);
+        if (k0 + kTC <= N) thomas_t_fwd_chunk<T, true, kTC>(co, A, k0, N, x, xs, q);
+        else thomas_t_fwd_chunk<T, false, kTC>(co, A, k0, N, x, xs, q);
+        if (k0 + kTC < N) thomas_t_fwd_chunk<T, false, kTC>(co, B, k0 + kTC, N, x, xs, q);
     }
     // b_{N-1} = z_{N-1} q_{N-1} (0 for (0,0)); b_kk = z_kk (q_kk - a_{kk+2} b_{kk+1}), kk = N-2 .. 0
     double b = m0 ? 0.0 : double(x[(N - 1) * xs]) * Z[(N - 1) * fs];
-    x[(N - 1) * xs] = T(b / size2d);
+    x[(N - 1) * xs] = XT(T(div_exact(b, size2d, rsize)));
     if (N < 2) return;
     thomas_tab_down<kTC>(Z, fs, N - 2, A);
     k0 = N - 2;
     for (; k0 - 2 * kTC + 1 >= 0; k0 -= 2 * kTC) {
         thomas_tab_down<kTC>(Z, fs, k0 - kTC, B);
-        thomas_t_back_chunk<T, true, kTC>(ta, A, k0, size2d, x, xs, b);
+        thomas_t_back_chunk<T, true, kTC>(co, A, k0, size2d, rsize, x, xs, b);
         thomas_tab_down<kTC>(Z, fs, k0 - 2 * kTC, A);
-        thomas_t_back_chunk<T, true, kTC>(ta, B, k0 - kTC, size2d, x, xs, b);
+        thomas_t_back_chunk<T, true, kTC>(co, B, k0 - kTC, size2d, rsize, x, xs, b);
     }
     if (k0 >= 0) {
         thomas_tab_down<kTC>(Z, fs, k0 - kTC, B);
-        if (k0 - kTC + 1 >= 0) thomas_t_back_chunk<T, true, kTC>(ta, A, k0, size2d, x, xs, b);
-        else thomas_t_back_chunk<T, false, kTC>(ta, A, k0, size2d, x, xs, b);
-        if (k0 - kTC >= 0) thomas_t_back_chunk<T, false, kTC>(ta, B, k0 - kTC, size2d, x, xs, b);
+        if (k0 - kTC + 1 >= 0) thomas_t_back_chunk<T, true, kTC>(co, A, k0, size2d, rsize, x, xs, b);
+        else thomas_t_back_chunk<T, false, kTC>(co, A, k0, size2d, rsize, x, xs, b);
+        if (k0 - kTC >= 0) thomas_t_back_chunk<T, false, kTC>(co, B, k0 - kTC, size2d, rsize, x, xs, b);
     }
 }
 
@@ -1246,7 +1249,8 @@ __device__ __forceinline__ void ypass_block(T *__restrict__ spec, int nk2, const
     const int nj = rady.n, P2 = nk2 + pad;
     T *re = (T *)smem, *im = re + nj * P2;
     double *mean = (double *)(re + 2 * nj * P2);  // 2*nj*P2 elements of T: 8-byte aligned
-    T *twl = (T *)(mean + 2 * nk2 + 1);
+    T *twl = (T *)(mean + 4 * nk2 + 1);
+    const ThomasCoef co = thomas_coef(ta, nk2, mean + 2 * nk2);
     load_twiddles(twl, twy, nj);
     const long long base = (long long)kx * nj * nk2 * 2;
     slab_to_lds(spec, base, nj * nk2, nk2, P2, re, im);
@@ -1256,8 +1260,9 @@ __device__ __forceinline__ void ypass_block(T *__restrict__ spec, int nk2, const
         // one thread per real sequence: threads [0, nj) take the real parts, [nj, 2 nj) the imaginary parts
         const int part = (int)threadIdx.x >= nj, ky = (int)threadIdx.x - part * nj;
         T *x = (part ? im : re) + ky * P2;
-        if (TR) thomas_part_t<T>(ta, kx, ky, x, 1);
-        else thomas_part<T>(ta, kx, ky, x, 1, mean + part);
+        const double *Z = ta.zpiv + (long long)kx * nj * nk2 + ky;
+        if (TR) thomas_part_t<T>(ta, co, kx, ky, Z, nj, x, 1);
+        else thomas_part<T>(ta, co, kx, ky, Z, nj, x, 1, mean + part);
     }
     __syncthreads();
     lds_fft_ip<T, ypass_maxb<T>(), POW2>(re, im, rady, nk2, P2, 1, twl, +1);
@@ -1377,7 +1382,8 @@ __device__ __forceinline__ void ypass_half_block(const T *__restrict__ in, T *__
     const int L = rh.n, nj = 2 * L, P2 = nk2 + pad;
     T *re = (T *)smem, *im = re + L * P2;
     double *mean = (double *)(re + 2 * L * P2);
-    T *twl = (T *)(mean + 2 * nk2 + 1);
+    T *twl = (T *)(mean + 4 * nk2 + 1);
+    const ThomasCoef co = thomas_coef(ta, nk2, mean + 2 * nk2);
     // the length-L table is every other entry of the length-nj one
     for (int e = threadIdx.x; e < L; e += blockDim.x) {
         twl[2 * e] = T(twy[4 * e]);
@@ -1426,8 +1432,9 @@ __device__ __forceinline__ void ypass_half_block(const T *__restrict__ in, T *__
     if ((int)threadIdx.x < 2 * L) {
         const int part = (int)threadIdx.x >= L, m = (int)threadIdx.x - part * L;
         T *x = (part ? im : re) + m * P2;
-        if (TR) thomas_part_t<T>(ta, kx, 2 * m + h, x, 1);
-        else thomas_part<T>(ta, kx, 2 * m + h, x, 1, mean + part);
+        const double *Z = ta.zpiv + (long long)kx * nj * nk2 + 2 * m + h;
+        if (TR) thomas_part_t<T>(ta, co, kx, 2 * m + h, Z, nj, x, 1);
+        else thomas_part<T>(ta, co, kx, 2 * m + h, Z, nj, x, 1, mean + part);
     }
     __syncthreads();
     lds_fft_pow2<T, half_maxb<T>()>(re, im, rh, nk2, P2, 1, twl, +1);
@@ -1462,22 +1469,183 @@ __global__ void __launch_bounds__(half_threads<T>()) k_ypass_half(const T *__res
     ypass_half_block<T, TR>(in, out, nk2, rh, twy, ta, pad, blockIdx.x >> 1, blockIdx.x & 1, smem);
 }
 
-template <typename T, bool TR = false>
+template <typename T, bool TR>
 __global__ void __launch_bounds__(ypass_threads<T>()) k_ypass(T *__restrict__ spec, int nk2, Radix rady, const double *twy, ThomasArgs ta,
                                                               int pad) {
     extern __shared__ unsigned char smem[];
     ypass_block<T, TR>(spec, nk2, rady, twy, ta, pad, blockIdx.x, smem);
 }
 
+// Q2 by matrix products (dyn_dft.hpp): the whole (j, k) slab of one kx in LDS as rows of 2 nk2 doubles (real
+// and imaginary parts side by side), in place throughout: rows i and n-i hold E(i) and D(i) while the
+// products run, X(i) and X(n-i) afterwards.  A wavefront keeps up to PT tiles' results in registers across
+// the barrier before they replace the operands; the last columns of a tile past 2 nk2 hold the next row's
+// values and their results are dropped.  The bits are those of k_dft_y, k_thomas_staged and k_dft_y in turn
+// (values are rounded to the storage type where those store them).
+// One launch serves slabs of few tiles (a pair of products per wavefront, PT = 1: 48x48x40 FP32 a step of 138 us
+// against 143 with three launches, and the radix passes, a chain of two barriers per radix, take 19 us
+// instead of 14); with more, the matrix units of nkx CUs are outrun by three launches spread over all of them
+// (96x96x40 206 against 181 us), except in an ensemble's batch.
+inline int dft_y_tiles(int nk2) { return (2 * nk2 + 15) / 16; }
+inline int dft_y_pairs(int n, int nk2) { return dft_pad(n) / 16 * dft_y_tiles(nk2); }  // (row tile, column tile)
+// doubles per row: 14 or 18 modulo 32, so that the two rows a half-wavefront of the products reads overlap in
+// few banks and the sweeps' columns (one row apart) in none
+__host__ __device__ __forceinline__ int ypass_dft_pitch(int nk2) {
+    int p = 2 * nk2;
+    while (p % 32 != 14 && p % 32 != 18) p += 2;
+    return p;
+}
+inline size_t ypass_dft_lds(int n, int nk2) { return 8 * ((size_t)n * ypass_dft_pitch(nk2) + 16 + 4 * (size_t)nk2); }
+constexpr int kYDftWaves = 16, kEnsYDftPairs = 3;
+
+// whether a slab fits the LDS and `pt` pairs of products per wavefront, with a thread per sequence of the sweeps
+inline bool ypass_dft_fits(const PressurePlan &pp, int pt) {
+    return ypass_dft_lds(pp.nj, pp.nk2) <= pp.lds_max && dft_y_pairs(pp.nj, pp.nk2) <= kYDftWaves * pt && 2 * pp.nj <= 64 * kYDftWaves;
+}
+
+template <typename T, bool TR, int PT>
+__device__ __forceinline__ void ypass_dft_block(T *__restrict__ spec, int n, const double *__restrict__ tab, int nk2, const ThomasArgs &ta,
+                                                int kx, unsigned char *smem) {
+    const int pitch = ypass_dft_pitch(nk2), h = dft_rows(n), p = dft_pad(n), steps = (h + 3) / 4, ncol = 2 * nk2, nct = (ncol + 15) / 16;
+    double *X = (double *)smem, *mean = X + n * pitch + 16;
+    const ThomasCoef co = thomas_coef(ta, nk2, mean + 2 * nk2);
+    T *x = spec + (long long)kx * n * ncol;
+    const int nt = (int)blockDim.x;
+    // load and fold row pairs (i, n-i); kU pairs per thread per round, their loads issued together
+    constexpr int kU = 4;
+    for (int i0 = (int)threadIdx.x; i0 < h * nk2; i0 += kU * nt) {
+        T a[kU][2], m[kU][2];
+#pragma unroll
+        for (int u = 0; u < kU; u++) {
+            const int idx = min(i0 + u * nt, h * nk2 - 1), i = idx / nk2, kk = idx - i * nk2, im = i == 0 ? 0 : n - i;
+            ld2(x + (long long)i * ncol + 2 * kk, a[u][0], a[u][1]);
+            ld2(x + (long long)im * ncol + 2 * kk, m[u][0], m[u][1]);
+        }
+#pragma unroll
+        for (int u = 0; u < kU; u++) {
+            const int idx = i0 + u * nt, i = idx / nk2, kk = idx - i * nk2;
+            if (idx >= h * nk2) break;
+            const bool self = i == 0 || 2 * i == n;
+            double *e = X + i * pitch + 2 * kk;
+            if (self) {
+                e[0] = double(a[u][0]);
+                e[1] = double(a[u][1]);
+            } else {
+                double *d = X + (n - i) * pitch + 2 * kk;
+                e[0] = double(a[u][0]) + double(m[u][0]);
+                e[1] = double(a[u][1]) + double(m[u][1]);
+                d[0] = double(a[u][0]) - double(m[u][0]);
+                d[1] = double(a[u][1]) - double(m[u][1]);
+            }
+        }
+    }
+    if ((int)threadIdx.x < 16) X[n * pitch + threadIdx.x] = 0.0;
+    __syncthreads();
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, row = lane >> 4, col = lane & 15;
+    const int pairs = p / 16 * nct, per = (pairs + kYDftWaves - 1) / kYDftWaves;  // a wavefront's pairs are consecutive
+    dvec4 pc[PT], ps[PT];
+    auto products = [&]() {
+#pragma unroll
+        for (int t = 0; t < PT; t++) {
+            const int pr = wave * per + t;
+            pc[t] = dvec4{0.0, 0.0, 0.0, 0.0};
+            ps[t] = dvec4{0.0, 0.0, 0.0, 0.0};
+            if (t >= per || pr >= pairs) continue;
+            const int m0 = pr / nct * 16, c0 = pr % nct * 16;
+            const double *ca = tab + (size_t)row * p + m0 + col, *sa = ca + (size_t)p * p;
+            double ac[2][4], as[2][4];
+            auto fetch = [&](int k, double (&fc)[4], double (&fs)[4]) {
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const size_t o = (size_t)min(k + u, steps - 1) * 4 * p;
+                    fc[u] = ca[o];
+                    fs[u] = sa[o];
+                }
+            };
+            auto use = [&](int k, const double (&fc)[4], const double (&fs)[4]) {
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    if (k + u >= steps) break;
+                    const int i = (k + u) * 4 + row;  // rows past h-1 meet zeros of the matrices
+                    pc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(fc[u], X[i * pitch + c0 + col], pc[t], 0, 0, 0);
+                    ps[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(fs[u], X[(i == 0 ? 0 : n - i) * pitch + c0 + col], ps[t], 0, 0, 0);
+                }
+            };
+            fetch(0, ac[0], as[0]);
+            for (int k = 0; k < steps; k += 8) {
+                fetch(k + 4, ac[1], as[1]);
+                use(k, ac[0], as[0]);
+                fetch(k + 8, ac[0], as[0]);
+                use(k + 4, ac[1], as[1]);
+            }
+        }
+    };
+    // put(row, column, value) for every result: X(m) = P + s i Q and X(n-m) = P - s i Q (see k_dft_y)
+    auto results = [&](int sign, auto put) {
+        const double sg = (lane & 1) != (sign < 0) ? 1.0 : -1.0;
+#pragma unroll
+        for (int t = 0; t < PT; t++) {
+            const int pr = wave * per + t;
+            if (t >= per || pr >= pairs) continue;
+            const int m0 = pr / nct * 16, q = pr % nct * 16 + col;
+#pragma unroll
+            for (int v4 = 0; v4 < 4; v4++) {
+                const int m = m0 + row + 4 * v4;
+                const double o = sg * lane_pair(ps[t][v4]);
+                if (m < h && q < ncol) {
+                    put(m, q, pc[t][v4] + o);
+                    if (m > 0 && 2 * m != n) put(n - m, q, pc[t][v4] - o);
+                }
+            }
+        }
+    };
+    products();
+    __syncthreads();
+    results(-1, [&](int r, int q, double v) { X[r * pitch + q] = double(T(v)); });
+    __syncthreads();
+    if ((int)threadIdx.x < 2 * n) {  // neighbouring lanes take the real and the imaginary part of a column
+        const int ky = (int)threadIdx.x >> 1, part = (int)threadIdx.x & 1;
+        const double *Z = ta.zpiv + (long long)kx * n * nk2 + ky;
+        double *xc = X + ky * pitch + part;
+        if (TR) thomas_part_t<T>(ta, co, kx, ky, Z, n, xc, 2);
+        else thomas_part<T>(ta, co, kx, ky, Z, n, xc, 2, mean + part);
+    }
+    __syncthreads();
+    for (int idx = (int)threadIdx.x; idx < (n - 1) / 2 * ncol; idx += nt) {
+        const int i = idx / ncol + 1, q = idx - (i - 1) * ncol;
+        double *e = X + i * pitch + q, *d = X + (n - i) * pitch + q;
+        const double a = *e, m = *d;
+        *e = a + m;
+        *d = a - m;
+    }
+    __syncthreads();
+    products();
+    results(+1, [&](int r, int q, double v) { x[(long long)r * ncol + q] = T(v); });
+}
+template <typename T, bool TR>
+__global__ void __launch_bounds__(64 * kYDftWaves) k_ypass_dft(T *__restrict__ spec, int n, const double *__restrict__ tab, int nk2,
+                                                              ThomasArgs ta) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    ypass_dft_block<T, TR, 1>(spec, n, tab, nk2, ta, blockIdx.x, smem);
+}
+
 // ---- batched over the members of an ensemble: one launch per pass, blocks walk a work list that
 // concatenates the members' (row, level chunk) or (kx) items -------------------------------------------
 
+constexpr int kEnsTiles = 2;  // column tiles per block of a member's matrix products
 template <typename T>
 __global__ void __launch_bounds__(kThreadsX) k_ens_div_rfft_x(const EnsMember *mem, int nmem, EnsRoles roles, int total, double step) {
-    extern __shared__ unsigned char smem[];
+    extern __shared__ __align__(16) unsigned char smem[];
     {
         const int item = blockIdx.x;
         const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::px0)];
+        if (e.dftx) {
+            div_dft_x_block<T, kEnsTiles, false>(e.g, e.c, (const T *)e.buf[DYN_U][roles.r[DYN_U][DYN_ROLE_P]],
+                                                 (const T *)e.buf[DYN_V][roles.r[DYN_V][DYN_ROLE_P]],
+                                                 (const T *)e.buf[DYN_W][roles.r[DYN_W][DYN_ROLE_P]], (T *)e.spec, e.ni, e.dftx, e.nk2, step,
+                                                 (const T *)nullptr, item - e.px0, smem);
+            return;
+        }
         const int local = item - e.px0, nch = (e.nk2 + e.kcx - 1) / e.kcx;
         div_rfft_x_block<T>(e.g, e.c, (const T *)e.buf[DYN_U][roles.r[DYN_U][DYN_ROLE_P]], (const T *)e.buf[DYN_V][roles.r[DYN_V][DYN_ROLE_P]],
                             (const T *)e.buf[DYN_W][roles.r[DYN_W][DYN_ROLE_P]], (T *)e.spec, e.rx, e.twx, e.nk2, e.kcx, step,
@@ -1487,10 +1655,14 @@ __global__ void __launch_bounds__(kThreadsX) k_ens_div_rfft_x(const EnsMember *m
 
 template <typename T>
 __global__ void __launch_bounds__(kThreadsX) k_ens_irfft_x_out(const EnsMember *mem, int nmem, int total) {
-    extern __shared__ unsigned char smem[];
+    extern __shared__ __align__(16) unsigned char smem[];
     {
         const int item = blockIdx.x;
         const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::px0)];
+        if (e.dftx) {
+            idft_x_out_block<T, kEnsTiles>(e.g, (const T *)e.spec, (T *)e.pi, e.ni, e.dftx, e.nk2, item - e.px0, smem);
+            return;
+        }
         const int local = item - e.px0, nch = (e.nk2 + e.kcx - 1) / e.kcx;
         irfft_x_out_block<T>(e.g, (const T *)e.spec, (T *)e.pi, e.rx, e.twx, e.nk2, e.kcx, local / nch, local % nch, smem);
     }
@@ -1498,43 +1670,67 @@ __global__ void __launch_bounds__(kThreadsX) k_ens_irfft_x_out(const EnsMember *
 
 template <typename T>
 __global__ void __launch_bounds__(1024) k_ens_ypass(const EnsMember *mem, int nmem, int total) {
-    extern __shared__ unsigned char smem[];
+    extern __shared__ __align__(16) unsigned char smem[];
     {
         const int item = blockIdx.x;
         const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::py0)];
-        ThomasArgs ta{e.coskx, e.cosly, e.c.rhou, e.c.rhow, e.c.mu, e.c.mw, e.acoef, e.ffac, e.dx, e.dz, e.ni, e.nj, e.g.NZ, e.zpiv};
+        ThomasArgs ta{e.acoef, e.ccoef, e.zpiv, e.ni, e.nj, e.g.NZ};
+        if (e.ydft) {
+            ypass_dft_block<T, false, kEnsYDftPairs>((T *)e.spec, e.nj, e.dfty, e.nk2, ta, item - e.py0, smem);
+            return;
+        }
         // the generic transform passes (the straight-line power-of-two ones measured no faster here)
         ypass_block<T, false, false>((T *)e.spec, e.nk2, e.ry, e.twy, ta, 1, item - e.py0, smem);
     }
 }
 
-// Q2 (staged): tridiagonal solve of tg columns of one kx staged through LDS (coalesced in and out)
+// Q2 (staged): tridiagonal solve of tg columns of one kx with their values and pivots in LDS (coalesced in and
+// out): the whole block loads and stores, 2 tg of its threads run the sweeps
+constexpr int kThomasThreads = 256;
 template <typename T, bool TR = false>
-__global__ void __launch_bounds__(128) k_thomas_staged(T *__restrict__ spec, int nk2, ThomasArgs ta) {
-    extern __shared__ unsigned char smem[];
-    const int tg = blockDim.x / 2, P2 = 2 * nk2 + 1;
-    T *x = (T *)smem;
-    double *mean = (double *)(smem + ((tg * P2 * sizeof(T) + 7) / 8) * 8);
+__global__ void __launch_bounds__(kThomasThreads) k_thomas_staged(T *__restrict__ spec, int nk2, ThomasArgs ta, int tg) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int P2 = 2 * nk2 + 1;
+    double *zl = (double *)smem, *mean = zl + tg * nk2;
+    T *x = (T *)(mean + 4 * nk2);
+    const ThomasCoef co = thomas_coef(ta, nk2, mean + 2 * nk2);
     const int kx = blockIdx.x, ky0 = blockIdx.y * tg;
     const int ncol = min(tg, ta.nj - ky0);
     const long long base = ((long long)kx * ta.nj + ky0) * nk2 * 2;
-    for (int idx = threadIdx.x; idx < ncol * nk2 * 2; idx += blockDim.x) {
-        int col = idx / (2 * nk2), rem = idx % (2 * nk2);
-        x[col * P2 + rem] = spec[base + idx];
+    const double *zg = ta.zpiv + (long long)kx * ta.nj * nk2 + ky0;
+    // kU elements per thread per round, every load of a round issued (clamped indices) before any is used
+    constexpr int kU = 5;
+    const int ne = ncol * nk2, nt = (int)blockDim.x;
+    for (int i0 = (int)threadIdx.x; i0 < ne; i0 += kU * nt) {
+        double z[kU];
+        T vr[kU], vi[kU];
+#pragma unroll
+        for (int u = 0; u < kU; u++) {
+            const int idx = min(i0 + u * nt, ne - 1), kk = idx / ncol;
+            z[u] = zg[(long long)kk * ta.nj + idx - kk * ncol];
+            ld2(spec + base + 2LL * idx, vr[u], vi[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kU; u++) {
+            const int idx = min(i0 + u * nt, ne - 1), kk = idx / ncol, col = idx / nk2, k2 = idx - col * nk2;
+            zl[kk * tg + idx - kk * ncol] = z[u];
+            x[col * P2 + 2 * k2] = vr[u];
+            x[col * P2 + 2 * k2 + 1] = vi[u];
+        }
     }
     __syncthreads();
     {
         // two threads per column: even lanes the real part, odd lanes the imaginary part (interleaved)
         const int colx = (int)threadIdx.x >> 1, part = threadIdx.x & 1;
         if (colx < ncol) {
-            if (TR) thomas_part_t<T>(ta, kx, ky0 + colx, x + colx * P2 + part, 2);
-            else thomas_part<T>(ta, kx, ky0 + colx, x + colx * P2 + part, 2, mean + part);
+            if (TR) thomas_part_t<T>(ta, co, kx, ky0 + colx, zl + colx, tg, x + colx * P2 + part, 2);
+            else thomas_part<T>(ta, co, kx, ky0 + colx, zl + colx, tg, x + colx * P2 + part, 2, mean + part);
         }
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < ncol * nk2 * 2; idx += blockDim.x) {
-        int col = idx / (2 * nk2), rem = idx % (2 * nk2);
-        spec[base + idx] = x[col * P2 + rem];
+    for (int idx = threadIdx.x; idx < ncol * nk2; idx += blockDim.x) {
+        const int col = idx / nk2, kk = idx - col * nk2;
+        st2(spec + base + 2LL * idx, x[col * P2 + 2 * kk], x[col * P2 + 2 * kk + 1]);
     }
 }
 
@@ -1577,36 +1773,47 @@ void launch_irfft_x_out(Ctx *c, const T *spec, T *out, const Radix &rx, int kc, 
                        pp.nk2, kc, half);
 }
 
-// launches of the matrix-product transforms (dyn_dft.hpp) with 4, 2 or 1 column tiles per block
-template <typename T>
-void launch_div_dft_x(Ctx *c, T *spec, double step) {
+// launches of the matrix-product transforms (dyn_dft.hpp) with 4, 2 or 1 column tiles per block; src: transform
+// that field instead of the divergence
+template <typename T, int NT>
+void launch_div_dft_x_t(Ctx *c, T *spec, double step, const T *src) {
     const PressurePlan &pp = c->pp;
-    const Geo &g = c->geo;
-    const int ncol = pp.nj * pp.nk2, nt = dft_tiles(pp.ni, 1, ncol, pp.cus), nc = 16 * nt;
+    const int ncol = pp.nj * pp.nk2, nc = 16 * NT;
     const dim3 grid((ncol + nc - 1) / nc), blk(dft_threads(pp.ni));
     const size_t sh = dft_lds(pp.ni, nc);
-    const T *u = (const T *)c->prog[DYN_U][2], *v = (const T *)c->prog[DYN_V][2], *w = (const T *)c->prog[DYN_W][2];
-    if (nt == 4) hipLaunchKernelGGL((k_div_dft_x<T, 4>), grid, blk, sh, c->stream, g, c->cols, u, v, w, spec, pp.ni, pp.dftx, pp.nk2, step);
-    else if (nt == 2) hipLaunchKernelGGL((k_div_dft_x<T, 2>), grid, blk, sh, c->stream, g, c->cols, u, v, w, spec, pp.ni, pp.dftx, pp.nk2, step);
-    else hipLaunchKernelGGL((k_div_dft_x<T, 1>), grid, blk, sh, c->stream, g, c->cols, u, v, w, spec, pp.ni, pp.dftx, pp.nk2, step);
+    if (src) {
+        hipLaunchKernelGGL((k_div_dft_x<T, NT, true>), grid, blk, sh, c->stream, c->geo, c->cols, src, src, src, spec, pp.ni, pp.dftx, pp.nk2,
+                           step, src);
+        return;
+    }
+    hipLaunchKernelGGL((k_div_dft_x<T, NT, false>), grid, blk, sh, c->stream, c->geo, c->cols, (const T *)c->prog[DYN_U][2],
+                       (const T *)c->prog[DYN_V][2], (const T *)c->prog[DYN_W][2], spec, pp.ni, pp.dftx, pp.nk2, step, src);
+}
+template <typename T>
+void launch_div_dft_x(Ctx *c, T *spec, double step, const T *src = nullptr) {
+    const int nt = dft_tiles(c->pp.ni, 1, c->pp.nj * c->pp.nk2, c->pp.cus);
+    if (nt == 4) launch_div_dft_x_t<T, 4>(c, spec, step, src);
+    else if (nt == 2) launch_div_dft_x_t<T, 2>(c, spec, step, src);
+    else launch_div_dft_x_t<T, 1>(c, spec, step, src);
 }
 template <typename T>
 int dft_lds_limits() {  // their operands may take more than 64 KiB: kDftMax with one column tile, 80 KiB with more
-    const void *k[] = {(const void *)k_div_dft_x<T, 1>, (const void *)k_div_dft_x<T, 2>, (const void *)k_div_dft_x<T, 4>,
+    const void *k[] = {(const void *)k_div_dft_x<T, 1, false>, (const void *)k_div_dft_x<T, 2, false>, (const void *)k_div_dft_x<T, 4, false>,
+                       (const void *)k_div_dft_x<T, 1, true>, (const void *)k_div_dft_x<T, 2, true>, (const void *)k_div_dft_x<T, 4, true>,
                        (const void *)k_idft_x_out<T, 1>, (const void *)k_idft_x_out<T, 2>, (const void *)k_idft_x_out<T, 4>,
                        (const void *)k_dft_y<T, 1>, (const void *)k_dft_y<T, 2>, (const void *)k_dft_y<T, 4>};
     for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024));
     return DYN_OK;
 }
 template <typename T>
-void launch_idft_x_out(Ctx *c, const T *spec, T *out) {
+void launch_idft_x_out(Ctx *c, const T *spec, T *out, int half) {
     const PressurePlan &pp = c->pp;
     const int ncol = pp.nj * pp.nk2, nt = dft_tiles(pp.ni, 1, ncol, pp.cus), nc = 16 * nt;
     const dim3 grid((ncol + nc - 1) / nc), blk(dft_threads(pp.ni));
     const size_t sh = dft_lds(pp.ni, nc);
-    if (nt == 4) hipLaunchKernelGGL((k_idft_x_out<T, 4>), grid, blk, sh, c->stream, c->geo, spec, out, pp.ni, pp.dftx, pp.nk2);
-    else if (nt == 2) hipLaunchKernelGGL((k_idft_x_out<T, 2>), grid, blk, sh, c->stream, c->geo, spec, out, pp.ni, pp.dftx, pp.nk2);
-    else hipLaunchKernelGGL((k_idft_x_out<T, 1>), grid, blk, sh, c->stream, c->geo, spec, out, pp.ni, pp.dftx, pp.nk2);
+    if (nt == 4) hipLaunchKernelGGL((k_idft_x_out<T, 4>), grid, blk, sh, c->stream, c->geo, spec, out, pp.ni, pp.dftx, pp.nk2, half);
+    else if (nt == 2) hipLaunchKernelGGL((k_idft_x_out<T, 2>), grid, blk, sh, c->stream, c->geo, spec, out, pp.ni, pp.dftx, pp.nk2, half);
+    else hipLaunchKernelGGL((k_idft_x_out<T, 1>), grid, blk, sh, c->stream, c->geo, spec, out, pp.ni, pp.dftx, pp.nk2, half);
 }
 template <typename T>
 void launch_dft_y(Ctx *c, T *spec, int nrows, int sign) {
@@ -1674,7 +1881,7 @@ int max_butterflies(const Radix &r, int nbatch, int nthr) {
 // LDS of the i passes for kc levels (kc/2 packed pairs) and of the fused j pass, twiddle tables included
 size_t x_pass_lds(int ni, int kc, size_t elt) { return (2 * (size_t)ni * (kc / 2) + 2 * (size_t)ni) * elt + 32 * (size_t)kc; }
 size_t y_pass_lds(int nj, int nk2, size_t elt) {
-    return 2 * (size_t)nj * (nk2 + 1) * elt + 8 * (2 * (size_t)nk2 + 1) + 2 * (size_t)nj * elt + 8;
+    return 2 * (size_t)nj * (nk2 + 1) * elt + 8 * (4 * (size_t)nk2 + 1) + 2 * (size_t)nj * elt + 8;
 }
 // levels per block of the i passes (even: two levels per complex transform), within the LDS budget and
 // the butterflies a thread holds.  One grid alone wants enough blocks to fill the chip (about 512 rows x
@@ -1692,6 +1899,44 @@ int x_level_chunk(const PressurePlan &pp, const Geo &g, const Radix &rx, size_t 
     return kc;
 }
 
+// The j pass of a solve while no form is asked for: the one-slab form by matrix products where a slab has few
+// tiles, three launches with them up to kDftYThree (96x96x40 FP32: 181 us per step against 189 with the radix
+// passes' slab, FP64 210 against 235), the nominal forms beyond (128x128x64 FP32: the slab takes 26 us, three
+// launches 38).
+int jpass_in_use(const Ctx *c) {
+    if (c->tune[DYN_TUNE_PRESSURE_JPASS]) return fused_shape(c, DYN_TUNE_PRESSURE_JPASS);
+    if (c->pp.ydft) return 1;
+    return c->pp.dfty && c->pp.nj <= kDftYThree ? 2 : fused_shape(c, DYN_TUNE_PRESSURE_JPASS);
+}
+// LDS of k_thomas_staged for tg columns; columns per block: 32 (64 running threads, one wavefront), fewer
+// where their values and pivots exceed half the LDS of a CU
+size_t thomas_lds(int tg, int nk2, size_t elt) { return 8 * ((size_t)tg * nk2 + 4 * (size_t)nk2) + (size_t)tg * (2 * (size_t)nk2 + 1) * elt; }
+int thomas_group(int nk2, size_t elt) {
+    int tg = 32;
+    while (tg > 1 && thomas_lds(tg, nk2, elt) > 80 * 1024) tg /= 2;
+    return tg;
+}
+template <typename T, bool TR>
+void launch_thomas(Ctx *c, T *spec, int nkx) {
+    const PressurePlan &pp = c->pp;
+    const int tg = thomas_group(pp.nk2, sizeof(T));
+    hipLaunchKernelGGL((k_thomas_staged<T, TR>), dim3(nkx, (pp.nj + tg - 1) / tg), dim3(kThomasThreads), thomas_lds(tg, pp.nk2, sizeof(T)),
+                       c->stream, spec, pp.nk2, thomas_args(pp, c->g.nz), tg);
+}
+// the LDS-resident j pass: by matrix products where the plan has them, else by radix passes
+template <typename T, bool TR>
+void launch_ypass(Ctx *c, T *spec, int nkx, const Radix &ry) {
+    const PressurePlan &pp = c->pp;
+    const ThomasArgs ta = thomas_args(pp, c->g.nz);
+    if (pp.ydft) {
+        hipLaunchKernelGGL((k_ypass_dft<T, TR>), dim3(nkx), dim3(64 * kYDftWaves), ypass_dft_lds(pp.nj, pp.nk2), c->stream, spec, pp.nj,
+                           pp.dfty, pp.nk2, ta);
+        return;
+    }
+    hipLaunchKernelGGL((k_ypass<T, TR>), dim3(nkx), dim3(ypass_threads<T>()), y_pass_lds(pp.nj, pp.nk2, sizeof(T)), c->stream, spec, pp.nk2,
+                       ry, pp.twy, ta, 1);
+}
+
 template <typename T>
 int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
     PressurePlan &pp = c->pp;
@@ -1706,8 +1951,7 @@ int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
     }
     T *spec = (T *)pp.spec;
     const double pts = (double)pp.ni * pp.nj * pp.nk2;
-    ThomasArgs ta{pp.coskx, pp.cosly, c->cols.rhou, c->cols.rhow, c->cols.mu, c->cols.mw, pp.acoef, pp.ffac, c->g.dx, c->g.dz,
-                  pp.ni, pp.nj, c->g.nz, pp.zpiv};
+    const ThomasArgs ta = thomas_args(pp, c->g.nz);
     // half-spectrum transforms, except for lengths with a prime factor above 5 that are too long for the
     // matrix products: those take the full complex spectrum
     if (pp.smooth_x || pp.dftx) {
@@ -1730,12 +1974,11 @@ int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
             if (rc) return rc;
         }
         const int pad = 1;
-        const size_t shy = y_pass_lds(pp.nj, pp.nk2, sizeof(T));
-        const int jpass = fused_shape(c, DYN_TUNE_PRESSURE_JPASS);
+        const int jpass = jpass_in_use(c);
         int half = 0;
         if (jpass == 1) {
             Timed _t(c, "p2_ypass", pts);
-            hipLaunchKernelGGL(k_ypass<T>, dim3(nkx), dim3(ypass_threads<T>()), shy, c->stream, spec, pp.nk2, ry, pp.twy, ta, pad);
+            launch_ypass<T, false>(c, spec, nkx, ry);
             DYN_LAUNCH_CHECK();
         } else if (jpass == 3) {
             Radix rh{};
@@ -1751,11 +1994,9 @@ int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
                 launch_fft_y<T>(c, spec, nkx, ry, -1);
             }
             DYN_LAUNCH_CHECK();
-            const int tg = 64;
-            size_t sht = ((tg * (2 * (size_t)pp.nk2 + 1) * sizeof(T) + 7) / 8) * 8 + 16 * (size_t)pp.nk2;
             {
                 Timed _t(c, "p3_thomas", pts);
-                hipLaunchKernelGGL(k_thomas_staged<T>, dim3(nkx, (pp.nj + tg - 1) / tg), dim3(2 * tg), sht, c->stream, spec, pp.nk2, ta);
+                launch_thomas<T, false>(c, spec, nkx);
             }
             DYN_LAUNCH_CHECK();
             {
@@ -1766,7 +2007,7 @@ int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
         }
         if (pp.dftx) {
             Timed _t(c, "p5_idft_x_out", pts);
-            launch_idft_x_out<T>(c, spec, (T *)c->pi);
+            launch_idft_x_out<T>(c, half ? (const T *)pp.spec2 : spec, (T *)c->pi, half);
         } else {
             Timed _t(c, "p5_irfft_x_out", pts);
             launch_irfft_x_out<T>(c, half ? (const T *)pp.spec2 : spec, (T *)c->pi, rx, kc, half);
@@ -1796,8 +2037,8 @@ int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
     int nq = pp.ni * pp.nj;
     {
         Timed _t(c, "p3_thomas", pts);
-        hipLaunchKernelGGL(k_thomas<T>, dim3((nq + 127) / 128), dim3(128), 0, c->stream, spec, pp.ni, pp.nj, g.NZ, pp.coskx, pp.cosly,
-                           c->cols.rhou, c->cols.rhow, c->cols.mu, c->cols.mw, pp.acoef, pp.ffac, c->g.dx, c->g.dz);
+        hipLaunchKernelGGL(k_thomas<T>, dim3((nq + 127) / 128), dim3(128), 0, c->stream, spec, pp.ni, pp.nj, g.NZ, pp.acoef, pp.ccoef,
+                           pp.zpiv);
     }
     DYN_LAUNCH_CHECK();
     {
@@ -1899,25 +2140,26 @@ int solve_adjoint_t(Ctx *c, double step, T *pihat, T *uh, T *vh, T *wh, T *r1, T
         DYN_LAUNCH_CHECK();
     }
     T *spec = (T *)pp.spec;
-    ThomasArgs ta{pp.coskx, pp.cosly, c->cols.rhou, c->cols.rhow, c->cols.mu, c->cols.mw, pp.acoef, pp.ffac, c->g.dx, c->g.dz,
-                  pp.ni, pp.nj, c->g.nz, pp.zpiv};
+    const ThomasArgs ta = thomas_args(pp, c->g.nz);
     const int nkx = pp.ni / 2 + 1;
     const int kc = x_level_chunk(pp, g, rx, sizeof(T));
     const size_t shx = x_pass_lds(pp.ni, kc, sizeof(T));
     dim3 gx(g.NY, (pp.nk2 + kc - 1) / kc);
-    {
+    if (pp.dftx) {
+        Timed _t(c, "adj_dft_x", pts);
+        launch_div_dft_x<T>(c, spec, step, (const T *)r1);
+    } else {
         Timed _t(c, "adj_rfft_x", pts);
         hipLaunchKernelGGL(k_div_rfft_x<T>, gx, dim3(kThreadsX), shx, c->stream, g, c->cols, (const T *)nullptr, (const T *)nullptr,
                            (const T *)nullptr, spec, rx, pp.twx, pp.nk2, kc, step, (const T *)r1);
     }
     DYN_LAUNCH_CHECK();
     const int pad = 1;
-    const size_t shy = y_pass_lds(pp.nj, pp.nk2, sizeof(T));
-    const int jpass = fused_shape(c, DYN_TUNE_PRESSURE_JPASS);
+    const int jpass = jpass_in_use(c);
     int half = 0;
     if (jpass == 1) {
         Timed _t(c, "adj_ypass", pts);
-        hipLaunchKernelGGL((k_ypass<T, true>), dim3(nkx), dim3(ypass_threads<T>()), shy, c->stream, spec, pp.nk2, ry, pp.twy, ta, pad);
+        launch_ypass<T, true>(c, spec, nkx, ry);
         DYN_LAUNCH_CHECK();
     } else if (jpass == 3) {
         Radix rh{};
@@ -1931,16 +2173,15 @@ int solve_adjoint_t(Ctx *c, double step, T *pihat, T *uh, T *vh, T *wh, T *r1, T
         Timed _t(c, "adj_ypass", pts);
         launch_fft_y<T>(c, spec, nkx, ry, -1);
         DYN_LAUNCH_CHECK();
-        const int tg = 64;
-        size_t sht = ((tg * (2 * (size_t)pp.nk2 + 1) * sizeof(T) + 7) / 8) * 8 + 16 * (size_t)pp.nk2;
-        hipLaunchKernelGGL((k_thomas_staged<T, true>), dim3(nkx, (pp.nj + tg - 1) / tg), dim3(2 * tg), sht, c->stream, spec, pp.nk2, ta);
+        launch_thomas<T, true>(c, spec, nkx);
         DYN_LAUNCH_CHECK();
         launch_fft_y<T>(c, spec, nkx, ry, +1);
         DYN_LAUNCH_CHECK();
     }
     {
         Timed _t(c, "adj_irfft_x", pts);
-        launch_irfft_x_out<T>(c, half ? (const T *)pp.spec2 : spec, r2, rx, kc, half);
+        if (pp.dftx) launch_idft_x_out<T>(c, half ? (const T *)pp.spec2 : spec, r2, half);
+        else launch_irfft_x_out<T>(c, half ? (const T *)pp.spec2 : spec, r2, rx, kc, half);
     }
     DYN_LAUNCH_CHECK();
     {
@@ -1949,6 +2190,14 @@ int solve_adjoint_t(Ctx *c, double step, T *pihat, T *uh, T *vh, T *wh, T *r1, T
                            (const T *)r2, uh, vh, wh, step);
     }
     DYN_LAUNCH_CHECK();
+    return DYN_OK;
+}
+
+template <typename T>
+int y_lds_limits(int most) {
+    const void *k[] = {(const void *)k_ypass<T, false>, (const void *)k_ypass<T, true>, (const void *)k_thomas_staged<T, false>,
+                       (const void *)k_thomas_staged<T, true>, (const void *)k_ypass_dft<T, false>, (const void *)k_ypass_dft<T, true>};
+    for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, most));
     return DYN_OK;
 }
 
@@ -1979,15 +2228,15 @@ int pressure_init(Ctx *c) {
         set_error("pressure solver: twiddle upload failed");
         return DYN_E_HIP;
     }
-    auto matrices = [](int n, bool smooth, double **out) -> int {
-        if (smooth || n > kDftMax) return DYN_OK;
+    auto matrices = [](int n, bool smooth, int smooth_max, double **out) -> int {
+        if (n > (smooth ? smooth_max : kDftMax)) return DYN_OK;
         const std::vector<double> h = dft_matrices(n);
         DYN_HIP(hipMalloc(out, sizeof(double) * h.size()));
         DYN_HIP(hipMemcpy(*out, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
         return DYN_OK;
     };
-    int rc = matrices(pp.ni, pp.smooth_x, &pp.dftx);
-    if (!rc) rc = matrices(pp.nj, pp.smooth_y, &pp.dfty);
+    int rc = matrices(pp.ni, pp.smooth_x, c->prec == DYN_FP32 ? dft_x_smooth<float>() : dft_x_smooth<double>(), &pp.dftx);
+    if (!rc) rc = matrices(pp.nj, pp.smooth_y, kDftYSmooth, &pp.dfty);
     if (!rc && (pp.dftx || pp.dfty)) rc = c->prec == DYN_FP32 ? dft_lds_limits<float>() : dft_lds_limits<double>();
     if (rc) return rc;
     DYN_HIP(hipMalloc(&pp.spec, sizeof(double) * 2 * (size_t)pp.ni * pp.nj * pp.nk2));
@@ -2004,13 +2253,9 @@ int pressure_init(Ctx *c) {
     const int nthr = f32 ? ypass_threads<float>() : ypass_threads<double>();
     const int maxb = f32 ? ypass_maxb<float>() : ypass_maxb<double>();
     pp.fused_y = pp.smooth_y && need <= pp.lds_max && 2 * pp.nj <= nthr && max_butterflies(ry, pp.nk2, nthr) <= maxb;
-    if (pp.fused_y && f32) {
-        DYN_HIP(hipFuncSetAttribute((const void *)k_ypass<float>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)need));
-        DYN_HIP(hipFuncSetAttribute((const void *)k_ypass<float, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)need));
-    } else if (pp.fused_y) {
-        DYN_HIP(hipFuncSetAttribute((const void *)k_ypass<double>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)need));
-        DYN_HIP(hipFuncSetAttribute((const void *)k_ypass<double, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)need));
-    }
+    pp.ydft = pp.dfty && ypass_dft_fits(pp, 1);
+    rc = f32 ? y_lds_limits<float>(lds) : y_lds_limits<double>(lds);
+    if (rc) return rc;
     // half slabs (power-of-two nj/2): what a slab of nj/2 rows needs, with one thread per real sequence
     // of the solve
     if (pp.nj % 2 == 0 && pp.nj >= 4 && ((pp.nj / 2) & (pp.nj / 2 - 1)) == 0) {
@@ -2024,7 +2269,7 @@ int pressure_init(Ctx *c) {
             const int items = rh.n / rh.r[st] * pp.nk2, per = (items + hthr - 1) / hthr;
             fits = per <= (rh.r[st] == 8 ? pow2_maxb8(hmaxb) : hmaxb);
         }
-        pp.half_y = fits && pp.smooth_x;  // its inverse i pass (the row pairs) is an in-place transform
+        pp.half_y = fits && pp.smooth_x;
         if (pp.half_y) {
             DYN_HIP(hipMalloc(&pp.spec2, sizeof(double) * 2 * (size_t)pp.ni * pp.nj * pp.nk2));
             if (f32) {
@@ -2039,7 +2284,6 @@ int pressure_init(Ctx *c) {
     // the power-of-two j transforms of the three-kernel j pass may take more than 64 KiB of LDS
     if (f32) DYN_HIP(hipFuncSetAttribute((const void *)k_fft_y_pow2<float, kFftYMaxB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFftYLds));
     else DYN_HIP(hipFuncSetAttribute((const void *)k_fft_y_pow2<double, kFftYMaxB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFftYLds));
-    DYN_HIP(hipMalloc(&pp.ffac, sizeof(double) * (size_t)pp.ni * pp.nj * pp.nk2));
     DYN_HIP(hipMalloc(&pp.zpiv, sizeof(double) * (size_t)pp.ni * pp.nj * pp.nk2));
     DYN_HIP(hipMalloc(&pp.coskx, sizeof(double) * pp.ni));
     DYN_HIP(hipMalloc(&pp.cosly, sizeof(double) * pp.nj));
@@ -2072,7 +2316,7 @@ int pressure_coefficients(Ctx *c) {
     DYN_HIP(hipMemcpy(pp.ccoef, cc.data(), sizeof(double) * nk, hipMemcpyHostToDevice));
     int nq = pp.ni * pp.nj;
     hipLaunchKernelGGL(k_thomas_factors, dim3((nq + 127) / 128), dim3(128), 0, c->stream, pp.ni, pp.nj, nk, pp.coskx, pp.cosly,
-                       c->cols.rhou, c->cols.rhow, c->cols.mu, c->cols.mw, pp.acoef, pp.ccoef, c->g.dx, dz, pp.ffac, pp.zpiv);
+                       c->cols.rhou, c->cols.rhow, c->cols.mu, c->cols.mw, pp.acoef, pp.ccoef, c->g.dx, dz, pp.zpiv);
     DYN_LAUNCH_CHECK();
     DYN_HIP(hipStreamSynchronize(c->stream));
     return DYN_OK;
@@ -2080,7 +2324,7 @@ int pressure_coefficients(Ctx *c) {
 
 int pressure_free(Ctx *c) {
     PressurePlan &pp = c->pp;
-    void *ptrs[] = {pp.twx, pp.twy, pp.dftx, pp.dfty, pp.spec, pp.spec2, pp.ffac, pp.zpiv, pp.coskx, pp.cosly, pp.acoef, pp.ccoef};
+    void *ptrs[] = {pp.twx, pp.twy, pp.dftx, pp.dfty, pp.spec, pp.spec2, pp.zpiv, pp.coskx, pp.cosly, pp.acoef, pp.ccoef};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     pp = PressurePlan{};
@@ -2097,7 +2341,9 @@ int launch_solve_pressure(Ctx *c, double step, bool halos, PressureHook after_i,
 // solve (odd ni, or a (j, k) slab too large for the LDS-resident j pass)
 bool pressure_ens_fill(Ctx *c, EnsMember &e, size_t &lds_x, size_t &lds_y) {
     PressurePlan &pp = c->pp;
-    if (pp.ni % 2 != 0 || !pp.smooth_x || !pp.fused_y || c->prec != DYN_FP32) return false;
+    const int jpass = jpass_in_use(c);
+    const bool by_products = (jpass == 1 && pp.ydft) || (jpass == 2 && pp.dfty);
+    if (c->prec != DYN_FP32 || (!pp.smooth_x && !pp.dftx) || (by_products ? !ypass_dft_fits(pp, kEnsYDftPairs) : jpass != 1)) return false;
     if (!factorize(pp.ni, e.rx) || !factorize(pp.nj, e.ry)) return false;
     e.kcx = x_level_chunk(pp, c->geo, e.rx, sizeof(float), false);
     e.ni = pp.ni;
@@ -2106,26 +2352,34 @@ bool pressure_ens_fill(Ctx *c, EnsMember &e, size_t &lds_x, size_t &lds_y) {
     e.spec = pp.spec;
     e.twx = pp.twx;
     e.twy = pp.twy;
-    e.ffac = pp.ffac;
     e.zpiv = pp.zpiv;
-    e.coskx = pp.coskx;
-    e.cosly = pp.cosly;
     e.acoef = pp.acoef;
-    e.dx = c->g.dx;
-    e.dz = c->g.dz;
-    lds_x = x_pass_lds(pp.ni, e.kcx, sizeof(float));
+    e.ccoef = pp.ccoef;
+    // by matrix products where the member's own solve takes them, so its bits are those of a step on its own
+    e.dftx = pp.dftx;
+    e.dfty = pp.dfty;
+    e.ydft = by_products;
+    e.pxn = pp.dftx ? (pp.nj * pp.nk2 + 16 * kEnsTiles - 1) / (16 * kEnsTiles) : c->g.ny * ((pp.nk2 + e.kcx - 1) / e.kcx);
+    lds_x = pp.dftx ? dft_lds(pp.ni, 16 * kEnsTiles) : x_pass_lds(pp.ni, e.kcx, sizeof(float));
+    if (pp.dftx && lds_x > pp.lds_max) return false;
+    if (e.ydft) {
+        lds_y = ypass_dft_lds(pp.nj, pp.nk2);
+        return true;
+    }
     lds_y = y_pass_lds(pp.nj, pp.nk2, sizeof(float));
     return lds_y <= pp.lds_max && 2 * pp.nj <= 1024 && max_butterflies(e.ry, pp.nk2, 1024) <= kMaxBY;
+}
+
+// the batched passes may take more than 64 KiB of LDS
+int pressure_ens_prepare(const Ctx *c) {
+    const void *k[] = {(const void *)k_ens_div_rfft_x<float>, (const void *)k_ens_irfft_x_out<float>, (const void *)k_ens_ypass<float>};
+    for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->pp.lds_max));
+    return DYN_OK;
 }
 
 // solve_pressure(step) of every member without the uvw halo copy (as in the fused step): three launches
 int launch_pressure_ens(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, int tot_px, int tot_py, size_t lds_x,
                         size_t lds_y) {
-    static size_t lds_y_set = 0;
-    if (lds_y > lds_y_set) {
-        DYN_HIP(hipFuncSetAttribute((const void *)k_ens_ypass<float>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_y));
-        lds_y_set = lds_y;
-    }
     {
         const int grid = tot_px;
         Timed _t(c0, "ens_p1_div_rfft_x", 0.0);
