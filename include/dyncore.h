@@ -115,9 +115,9 @@ int dyn_micro_advance_outer(dyn_ctx *ctx);
 /* Switch the Smagorinsky-Lilly closure on or off (initialize_landsea + init_kmix, turbulence.cpp:85-147,
  * 370-375, with the vertical mixing length from the zsu column).  landsea holds NX*NY values (< 0.5:
  * land, fixed drag 3e-3; otherwise ocean, 1.1e-3 + 4e-5 |V|) or is NULL for all ocean.  With it on, a
- * step computes the coefficients and tendencies at its start and adds them in every stage; steps take
- * the per-operator sequence (the fused stage kernels carry no turbulence), and the adjoint and
- * ensembles refuse the context.  Drops the captured step graphs. */
+ * step computes the coefficients and tendencies at its start and adds them in every stage (dyn_step in the
+ * fused stage kernels, dyn_step_reference operator by operator, with equal results); dyn_step_fused, the
+ * adjoint and ensembles refuse the context.  Drops the captured step graphs. */
 int dyn_set_turbulence(dyn_ctx *ctx, int on, const double *landsea, size_t count);
 /* calculate_diff_tend(il,ih,jl,jh), turbulence.cpp:153-226 (the serial driver calls it over
  * [1,NX-1) x [1,NY-1), driver_serial.cpp:194): mixing coefficients from the M buffers, then the

@@ -875,6 +875,8 @@ static int fused_step(dyn_ctx *ctx, StageHook hook = nullptr, void *arg = nullpt
     // the second stream after the scalar half: it reads the step's starting state and writes the spare
     // buffer, neither of which stage 1 writes or reads, and the second stream's chain is the shorter one.
     const bool copy_beside = shared && two;
+    // calculate_diff_tend(1,NX-1,1,NY-1), driver_serial.cpp:194; the stage kernels add its tendencies
+    if (c->turb.on) RC(turb_step_begin(c));
     for (int s = 0; s < 3; s++) {
         double step = steps[s];
         if (hook) RC(hook(c, s, arg));
@@ -963,9 +965,12 @@ int dyn_step_fused(dyn_ctx *ctx, int nsteps) {
     Ctx *c = as_ctx(ctx);
     CHECK_CTX(c);
     CHECK_COLS(c);
+    if (c->turb.on) {
+        set_error("dyn_step_fused: not offered with turbulence on (dyn_step runs the closure)");
+        return DYN_E_UNSUPPORTED;
+    }
     if (!fused_supported(c)) {
-        set_error(c->turb.on ? "dyn_step_fused: the fused stage kernels carry no turbulence (dyn_step runs the closure)"
-                             : "dyn_step_fused: the fused stage kernels need NZ <= 64 or 66 <= NZ <= 128, and fields below 4 GiB");
+        set_error("dyn_step_fused: the fused stage kernels need NZ <= 64 or 66 <= NZ <= 128, and fields below 4 GiB");
         return DYN_E_UNSUPPORTED;
     }
     if (c->g.rayleigh_level < c->g.nz) {
@@ -1069,7 +1074,7 @@ int dyn_step(dyn_ctx *ctx, int nsteps) {
         int rc = ensure_rayleigh_table(c, c->g.rayleigh_level);
         if (rc) return rc;
     }
-    if (fused_supported(c)) {
+    if (fused_supported(c) && !c->turb.on) {
         if (nsteps == 1) return fused_step(ctx);
         // n = 6 q + (0 | 2 | 3 | 2+2 | 3+2), with 7 = 3+2+2 for r = 1
         int q = nsteps / 6, r = nsteps % 6, n3 = 0, n2 = 0;

@@ -113,6 +113,23 @@ __device__ __forceinline__ void dft_products(const double *__restrict__ tab, int
     }
 }
 
+// The mass divergence over step * dt of one cell from the winds on its six faces (pressure.cpp:1390-1406), in T.
+// The fluxes through a face cancel between its two cells only if they are rounded alike, and what FP32 leaves over,
+// the solve amplifies most in the longest waves: with a matrix product in either horizontal pass the arithmetic is
+// therefore in 64 bits (T = double) for FP32 fields too (pi of 194x100x40 moist after 4 steps, against a 64-bit run:
+// 2e-6 to 1e-5 off by the seed with FP32 arithmetic here).  Factored FP32 transforms of both sides round
+// by more of their own and keep FP32.
+template <typename T>
+struct DivStep {
+    T odx, ody, odz, sdt;
+    __device__ __forceinline__ DivStep(const Geo &g, double step)
+        : odx(T(g.one_d_dx)), ody(T(g.one_d_dy)), odz(T(g.one_d_dz)), sdt(T(step * g.dt)) {}
+    __device__ __forceinline__ T operator()(double rhou, double rw1, double rw0, double mu, T ue, T uw, T vn, T vs, T wt, T wb) const {
+        T d = T(rhou) * (ue - uw) * odx + T(rhou) * (vn - vs) * ody + (T(rw1) * wt - T(rw0) * wb) * (odz * T(mu));
+        return d / sdt;
+    }
+};
+
 // Forward along i: the divergence (as div_rfft_x_block forms it), or with SRC the ready field src(i+3, j, k)
 // (the transposed solve of the adjoint), of NC = 16 NT columns (j, level), folded, and its half spectrum.
 // Threads keep their column, so its coefficients and row offsets are read once.
@@ -125,8 +142,8 @@ __device__ __forceinline__ void div_dft_x_block(const Geo &g, const Cols &c, con
     double *E = (double *)smem, *D = E + hk * pitch;
     const int c0 = block * NC, b = threadIdx.x % NC, q = min(c0 + b, ncol - 1), j = q / nk2, k = q - j * nk2 + 1;
     const int jj = j == 0 ? 1 : (j == g.NY - 1 ? g.NY - 2 : j);  // mirrored rows, pressure.cpp:1408-1415
-    const T rhou = T(c.rhou[k]), rw1 = T(c.rhow[k + 1]), rw0 = T(c.rhow[k]), odz = T(g.one_d_dz) * T(c.mu[k]);
-    const T sdt = T(step * g.dt);
+    const double rhou = c.rhou[k], rw1 = c.rhow[k + 1], rw0 = c.rhow[k], mu = c.mu[k];
+    const DivStep<double> ds(g, step);
     const T *u = UP + (long long)jj * g.NZ + k, *v = VP + (long long)jj * g.NZ + k, *w = WP + (long long)jj * g.NZ + k;
     auto load = [&](int i, T (&f)[6]) {
         if (SRC) {
@@ -143,9 +160,7 @@ __device__ __forceinline__ void div_dft_x_block(const Geo &g, const Cols &c, con
     };
     auto value = [&](const T (&f)[6]) -> double {
         if (SRC) return double(f[0]);
-        T d = rhou * (f[0] - f[1]) * T(g.one_d_dx) + rhou * (f[2] - f[3]) * T(g.one_d_dy) + (rw1 * f[4] - rw0 * f[5]) * odz;
-        d /= sdt;
-        return double(d);
+        return ds(rhou, rw1, rw0, mu, f[0], f[1], f[2], f[3], f[4], f[5]);
     };
     const int rows = blockDim.x / NC;
     for (int i = threadIdx.x / NC; i < hk; i += 2 * rows) {

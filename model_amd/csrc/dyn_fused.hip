@@ -82,6 +82,9 @@ struct StageArgs {
     int ti;               // columns one block marches
     int nbj;              // j-blocks
     int tj;               // rows per block
+    // TURB: the step's turbulence tendencies of U V W TH QV QC QR, added to the new values
+    const void *tend[7];
+    double tdt;           // step * dt, in 64 bits
 };
 
 // Rows of a block.  Two mappings of levels and rows onto lanes, chosen on the host by the level count:
@@ -161,7 +164,9 @@ struct MomLds {
 };
 
 // one tile (tj rows x ti columns x all levels) of the momentum stage; every thread of the block calls it
-template <typename T, int TJ, bool MOIST, bool PACK>
+// TURB: apply_velocity_diffusion (turbulence.cpp:233-258) in the same pass; its box is the advected one.  The
+// tendencies of a column are loaded ahead of the next column's prefetch, so the wait for them is not one for it.
+template <typename T, int TJ, bool MOIST, bool PACK, bool TURB = false>
 __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, const StageArgs &a, T step, int t, unsigned char *smem_raw) {
     const RowMap<TJ, PACK> map(a.tj, g.NZ);
     const int tj = map.tj, KPW = map.pitch, k = map.k, r = map.r;
@@ -272,6 +277,7 @@ __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, c
     const T fj = T(c.f[jc]);
     // read once: a load inside the march would be waited for together with the next column's prefetch
     const T tbvk = T(c.tbv[kc]);
+    const T tdt = T(a.tdt);
     const bool low = (k == 1 || k == NZ - 2);
 
     // east faces of the queue's centre column (u_east, v_east; fluxes.cpp:1384-1592); slot: the U plane of the
@@ -311,6 +317,12 @@ __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, c
         const bool more = i + 1 < i1;
         const int c0 = i % 3, cm1 = (i + 2) % 3, cp1 = (i + 1) % 3;
         const unsigned p = (unsigned)i * NYNZ + rowoff;
+        T du = T(0), dv = T(0), dw = T(0);
+        if (TURB) {
+            du = ld<T>(a.tend[0], p);
+            dv = ld<T>(a.tend[1], p);
+            dw = ld<T>(a.tend[2], p);
+        }
         // loads for the next column go out first, its M values included
         if (more) {
 #pragma unroll
@@ -414,6 +426,11 @@ __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, c
                 ov = vm + step * tend;
             }
             ow = wm + step * dt * T(kGrav) * T(0.5) * (bk + bkm);  // advection.cpp:329-337
+            if (TURB) {
+                ou += du * tdt;
+                ov += dv * tdt;
+                ow += dw * tdt;  // (stored from level 2)
+            }
         }
         west[0] = east[0];
         west[1] = east[1];
@@ -459,7 +476,9 @@ struct ScalLds {
     static constexpr size_t bytes(int tj, int pitch) { return (s(tj, pitch) + nf(tj, pitch) + xw + xb) * sizeof(T); }
 };
 
-template <typename T, int TJ, bool MOIST, bool PACK>
+// TURB: apply_scalar_diffusion and apply_moisture_diffusion (turbulence.cpp:263-292) of the advected points,
+// before zero_moisture as in the reference; the boundary epilogue adds them on the rows beside the box
+template <typename T, int TJ, bool MOIST, bool PACK, bool TURB = false>
 __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, const StageArgs &a, T step, int t, unsigned char *smem_raw) {
     using L = ScalLds<T, MOIST>;
     constexpr int NP = L::NP, NS = 2 * NP, NFS = L::NFS;
@@ -645,6 +664,11 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
         const bool more = i + 1 < i1;
         const int c0 = i % 2;
         const unsigned p = (unsigned)i * NYNZ + rowoff;
+        T td[NFS] = {};
+        if (TURB) {
+#pragma unroll
+            for (int f = 0; f < NFS; f++) td[f] = ld<T>(a.tend[3 + f], p);
+        }
         if (more) {
 #pragma unroll
             for (int f = 0; f < NS; f++) qs[f] = ld<T>(src[f], (unsigned)(i + 4) * NYNZ + rowoff);
@@ -793,6 +817,7 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
                 T tend = -dtx * (east[0] - west[0]) - dty * (nf[0] - south[0]) - DTZ * (rw1 * tf[0] - rw0 * bot[0]) * odr -
                          DTZ * zbase(tbu, tbd);
                 oth = mth + step * tend;
+                if (TURB) oth += td[0] * step * T(g.dt);
             }
             if constexpr (MOIST) {  // advection.cpp:197-253
                 T tq = -dtx * (east[1] - west[1]) - dty * (nf[1] - south[1]) - DTZ * (rw1 * tf[1] - rw0 * bot[1]) * odr -
@@ -802,6 +827,12 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
                 T qc = mqc + step * tc;
                 T tr = -dtx * (east[3] - west[3]) - dty * (nf[3] - south[3]) - DTZ * (rw1 * qrt - rw0 * qrb) * odr;
                 T qrv = mqr + step * tr;
+                if (TURB) {
+                    const T tdt = step * T(g.dt);
+                    qv += td[1] * tdt;
+                    qc += td[2] * tdt;
+                    qrv += td[3] * tdt;
+                }
                 // zero_moisture for the advected points (microphysics.cpp:677-698)
                 if (qc < T(0)) qc = T(0);
                 if (qrv < T(0)) qrv = T(0);
@@ -867,16 +898,16 @@ constexpr int kPackThreads = 512;
 template <int TJ, bool PACK>
 constexpr int stage_threads() { return PACK ? kPackThreads : KP * TJ; }
 
-template <typename T, int TJ, bool MOIST, bool PACK>
+template <typename T, int TJ, bool MOIST, bool PACK, bool TURB>
 __global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_adv_momentum(Geo g, Cols c, StageArgs a, T step) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    adv_momentum_tile<T, TJ, MOIST, PACK>(g, c, a, step, xcd_tile(blockIdx.x, gridDim.x), smem_raw);
+    adv_momentum_tile<T, TJ, MOIST, PACK, TURB>(g, c, a, step, xcd_tile(blockIdx.x, gridDim.x), smem_raw);
 }
 
-template <typename T, int TJ, bool MOIST, bool PACK>
+template <typename T, int TJ, bool MOIST, bool PACK, bool TURB>
 __global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_adv_scalars(Geo g, Cols c, StageArgs a, T step) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    adv_scalars_tile<T, TJ, MOIST, PACK>(g, c, a, step, xcd_tile(blockIdx.x, gridDim.x), smem_raw);
+    adv_scalars_tile<T, TJ, MOIST, PACK, TURB>(g, c, a, step, xcd_tile(blockIdx.x, gridDim.x), smem_raw);
 }
 
 // zero_moisture outside the advected box (the fused kernel clips the points it writes)
@@ -899,7 +930,7 @@ __global__ void k_zero_moisture_shell(Geo g, Cols c, T *__restrict__ QVP, T *__r
 }
 
 // shape: rows per block, march length and lane mapping of one launch
-template <typename T, int TJ, bool MOIST, bool PACK>
+template <typename T, int TJ, bool MOIST, bool PACK, bool TURB>
 int momentum_t(Ctx *c, const StageArgs &a0, T step, const StageShape &sh) {
     StageArgs a = a0;
     a.ti = sh.ti;
@@ -908,13 +939,13 @@ int momentum_t(Ctx *c, const StageArgs &a0, T step, const StageShape &sh) {
     const int nbi = (a.ih - a.il + sh.ti - 1) / sh.ti;
     const dim3 blk = PACK ? dim3((sh.tj * c->geo.NZ + KP - 1) / KP * KP) : dim3(KP, TJ);
     Timed _t(c, "adv_momentum", (double)(a.ih - a.il) * (a.jh - a.jl) * (c->geo.NZ - 2));
-    hipLaunchKernelGGL((k_adv_momentum<T, TJ, MOIST, PACK>), dim3(a.nbj * nbi), blk, MomLds<T>::bytes(sh.tj, PACK ? c->geo.NZ : KP),
+    hipLaunchKernelGGL((k_adv_momentum<T, TJ, MOIST, PACK, TURB>), dim3(a.nbj * nbi), blk, MomLds<T>::bytes(sh.tj, PACK ? c->geo.NZ : KP),
                        c->stream, c->geo, c->cols, a, step);
     DYN_LAUNCH_CHECK();
     return DYN_OK;
 }
 
-template <typename T, int TJ, bool MOIST, bool PACK>
+template <typename T, int TJ, bool MOIST, bool PACK, bool TURB>
 int scalars_t(Ctx *c, const StageArgs &a0, T step, const StageShape &sh) {
     StageArgs a = a0;
     a.ti = sh.ti;
@@ -923,13 +954,13 @@ int scalars_t(Ctx *c, const StageArgs &a0, T step, const StageShape &sh) {
     const int nbi = (a.ih - a.il + sh.ti - 1) / sh.ti;
     const dim3 blk = PACK ? dim3((sh.tj * c->geo.NZ + KP - 1) / KP * KP) : dim3(KP, TJ);
     Timed _t(c, "adv_scalars", (double)(a.ih - a.il) * (a.jh - a.jl) * (c->geo.NZ - 2));
-    hipLaunchKernelGGL((k_adv_scalars<T, TJ, MOIST, PACK>), dim3(a.nbj * nbi), blk,
+    hipLaunchKernelGGL((k_adv_scalars<T, TJ, MOIST, PACK, TURB>), dim3(a.nbj * nbi), blk,
                        (ScalLds<T, MOIST>::bytes(sh.tj, PACK ? c->geo.NZ : KP)), c->stream, c->geo, c->cols, a, step);
     DYN_LAUNCH_CHECK();
     return DYN_OK;
 }
 
-template <typename T, bool MOIST>
+template <typename T, bool MOIST, bool TURB>
 int stage_t(Ctx *c, double step, int il, int ih, int jl, int jh, int parts) {
     StageArgs a{};
     for (int f = 0; f < 7; f++) {
@@ -939,6 +970,10 @@ int stage_t(Ctx *c, double step, int il, int ih, int jl, int jh, int parts) {
     }
     for (int f = 0; f < 5; f++) a.bar[f] = c->bar[f];
     a.vt = c->vt;
+    if (TURB) {
+        for (int f = 0; f < 7; f++) a.tend[f] = turb_tendency(c, f);
+        a.tdt = step * c->g.dt;
+    }
     a.il = il;
     a.ih = ih;
     a.jl = jl;
@@ -947,25 +982,25 @@ int stage_t(Ctx *c, double step, int il, int ih, int jl, int jh, int parts) {
     if (parts & kStageMomentum) {
         const StageShape m = stage_shape(c, true);
         if (m.pack) {
-            if (m.tj >= 6) rc = momentum_t<T, 8, MOIST, true>(c, a, T(step), m);
-            else if (m.tj >= 3) rc = momentum_t<T, 4, MOIST, true>(c, a, T(step), m);
-            else rc = momentum_t<T, 2, MOIST, true>(c, a, T(step), m);
-        } else if (m.tj == 2) rc = momentum_t<T, 2, MOIST, false>(c, a, T(step), m);
-        else if (m.tj == 4) rc = momentum_t<T, 4, MOIST, false>(c, a, T(step), m);
-        else if (m.tj == 16) rc = momentum_t<T, 16, MOIST, false>(c, a, T(step), m);
-        else rc = momentum_t<T, 8, MOIST, false>(c, a, T(step), m);
+            if (m.tj >= 6) rc = momentum_t<T, 8, MOIST, true, TURB>(c, a, T(step), m);
+            else if (m.tj >= 3) rc = momentum_t<T, 4, MOIST, true, TURB>(c, a, T(step), m);
+            else rc = momentum_t<T, 2, MOIST, true, TURB>(c, a, T(step), m);
+        } else if (m.tj == 2) rc = momentum_t<T, 2, MOIST, false, TURB>(c, a, T(step), m);
+        else if (m.tj == 4) rc = momentum_t<T, 4, MOIST, false, TURB>(c, a, T(step), m);
+        else if (m.tj == 16) rc = momentum_t<T, 16, MOIST, false, TURB>(c, a, T(step), m);
+        else rc = momentum_t<T, 8, MOIST, false, TURB>(c, a, T(step), m);
     }
     if (rc || !(parts & kStageScalars)) return rc;
     const StageShape m = stage_shape(c, false);
     if (m.pack) {
-        if (m.tj >= 6) return scalars_t<T, 8, MOIST, true>(c, a, T(step), m);
-        if (m.tj >= 3) return scalars_t<T, 4, MOIST, true>(c, a, T(step), m);
-        return scalars_t<T, 2, MOIST, true>(c, a, T(step), m);
+        if (m.tj >= 6) return scalars_t<T, 8, MOIST, true, TURB>(c, a, T(step), m);
+        if (m.tj >= 3) return scalars_t<T, 4, MOIST, true, TURB>(c, a, T(step), m);
+        return scalars_t<T, 2, MOIST, true, TURB>(c, a, T(step), m);
     }
-    if (m.tj == 2) return scalars_t<T, 2, MOIST, false>(c, a, T(step), m);
-    if (m.tj == 4) return scalars_t<T, 4, MOIST, false>(c, a, T(step), m);
-    if (m.tj == 12) return scalars_t<T, 12, MOIST, false>(c, a, T(step), m);
-    return scalars_t<T, 8, MOIST, false>(c, a, T(step), m);
+    if (m.tj == 2) return scalars_t<T, 2, MOIST, false, TURB>(c, a, T(step), m);
+    if (m.tj == 4) return scalars_t<T, 4, MOIST, false, TURB>(c, a, T(step), m);
+    if (m.tj == 12) return scalars_t<T, 12, MOIST, false, TURB>(c, a, T(step), m);
+    return scalars_t<T, 8, MOIST, false, TURB>(c, a, T(step), m);
 }
 
 template <typename T>
@@ -996,6 +1031,10 @@ struct PostArgs {
     // [u v theta][k] then [w][k]; ray_level >= NZ: none
     const double *ray = nullptr;
     int ray_level = 1 << 30;
+    // turbulence tendencies of TH QV QC QR (nullptr: none) for the rows beside the advected box that the
+    // diffusion's box [1, NY-1) still holds, in a stage (step, dt)
+    const void *tend[4] = {};
+    double step = 0.0;
 };
 
 template <typename T>
@@ -1108,10 +1147,16 @@ __device__ __forceinline__ void post_scalars_col(const Geo &g, const Cols &c, co
         }
         return;
     }
+    const bool edge = a.tend[0] && j >= 1 && j < g.NY - 1 && (j < 3 || j >= g.NY - 3);
 #pragma unroll
     for (int f = 0; f < NFLD; f++) {
         T *A = (T *)a.f[3 + f];
         T x = A[col + kc];
+        if (edge && kc >= 1 && kc <= NZ - 2) {
+            const T d = ((const T *)a.tend[f])[col + kc];
+            if (f == 0) x += d * T(a.step) * T(g.dt);
+            else x += d * (T(a.step) * T(g.dt));
+        }
         if (MOIST && clip && f == 2 && x < T(0)) x = T(0);  // qc
         if (MOIST && clip && f == 3 && x < T(0)) x = T(0);  // qr
         if (MOIST && clip && f == 1 && isrc >= a.zl && isrc < a.zh && j >= a.zjl && j < a.zjh && kc >= 1 && kc <= NZ - 2) {
@@ -1278,6 +1323,10 @@ int post_t(Ctx *c, double step, bool pgf, bool scalars, bool clip, bool uvw, int
     a.zh = c->g.nx - 1;
     a.zjl = 1;
     a.zjh = c->g.ny - 1;
+    if (c->turb.on && pgf) {
+        for (int f = 0; f < 4; f++) a.tend[f] = turb_tendency(c, DYN_TH + f);
+        a.step = step;
+    }
     // one wavefront per column, two when NZ > 64; 256 threads per block
     const int kw = c->g.nz > KP ? 2 : 1, rows = 4 / kw;
     dim3 blk(KP * kw, rows), grd((c->g.ny + rows - 1) / rows, c->g.nx - 6);
@@ -1318,9 +1367,8 @@ int fused_waves(const Ctx *c) {
 }
 
 // ... and 32-bit byte offsets into every field
-// the fused stage kernels carry no turbulence: with it on, steps take the per-operator sequence
 bool fused_supported(const Ctx *c) {
-    return !c->turb.on && fused_waves(c) > 0 && (double)c->npts * (double)c->elt < 4294967296.0;
+    return fused_waves(c) > 0 && (double)c->npts * (double)c->elt < 4294967296.0;
 }
 
 namespace {
@@ -1491,27 +1539,27 @@ void choose_stage_shapes(Ctx *c) {
     }
 }
 
-template <typename T, int TJ, bool PACK>
+template <typename T, int TJ, bool PACK, bool TURB>
 int set_lds_limits(const Ctx *c) {
     const int most = (int)c->pp.lds_max;
-    const void *k[] = {(const void *)k_adv_momentum<T, TJ, true, PACK>, (const void *)k_adv_momentum<T, TJ, false, PACK>,
-                       (const void *)k_adv_scalars<T, TJ, true, PACK>, (const void *)k_adv_scalars<T, TJ, false, PACK>};
+    const void *k[] = {(const void *)k_adv_momentum<T, TJ, true, PACK, TURB>, (const void *)k_adv_momentum<T, TJ, false, PACK, TURB>,
+                       (const void *)k_adv_scalars<T, TJ, true, PACK, TURB>, (const void *)k_adv_scalars<T, TJ, false, PACK, TURB>};
     for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, most));
     return DYN_OK;
 }
 
-template <typename T>
+template <typename T, bool TURB>
 int set_lds_limits_all(const Ctx *c) {
-    int rc = set_lds_limits<T, 2, true>(c);
-    if (!rc) rc = set_lds_limits<T, 4, true>(c);
-    if (!rc) rc = set_lds_limits<T, 8, true>(c);
-    if (!rc) rc = set_lds_limits<T, 2, false>(c);
-    if (!rc) rc = set_lds_limits<T, 4, false>(c);
-    if (!rc) rc = set_lds_limits<T, 8, false>(c);
+    int rc = set_lds_limits<T, 2, true, TURB>(c);
+    if (!rc) rc = set_lds_limits<T, 4, true, TURB>(c);
+    if (!rc) rc = set_lds_limits<T, 8, true, TURB>(c);
+    if (!rc) rc = set_lds_limits<T, 2, false, TURB>(c);
+    if (!rc) rc = set_lds_limits<T, 4, false, TURB>(c);
+    if (!rc) rc = set_lds_limits<T, 8, false, TURB>(c);
     if (rc) return rc;
     const int most = (int)c->pp.lds_max;
-    const void *k[] = {(const void *)k_adv_momentum<T, 16, true, false>, (const void *)k_adv_momentum<T, 16, false, false>,
-                       (const void *)k_adv_scalars<T, 12, true, false>, (const void *)k_adv_scalars<T, 12, false, false>};
+    const void *k[] = {(const void *)k_adv_momentum<T, 16, true, false, TURB>, (const void *)k_adv_momentum<T, 16, false, false, TURB>,
+                       (const void *)k_adv_scalars<T, 12, true, false, TURB>, (const void *)k_adv_scalars<T, 12, false, false, TURB>};
     for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, most));
     return DYN_OK;
 }
@@ -1520,7 +1568,9 @@ int set_lds_limits_all(const Ctx *c) {
 // the stage kernels may use more than 64 KiB of LDS: raise the per-launch limit once, outside any capture
 int fused_prepare(Ctx *c) {
     choose_stage_shapes(c);
-    return c->prec == DYN_FP32 ? set_lds_limits_all<float>(c) : set_lds_limits_all<double>(c);
+    int rc = c->prec == DYN_FP32 ? set_lds_limits_all<float, false>(c) : set_lds_limits_all<double, false>(c);
+    if (!rc) rc = c->prec == DYN_FP32 ? set_lds_limits_all<float, true>(c) : set_lds_limits_all<double, true>(c);
+    return rc;
 }
 
 // advect_uvw_velocity + advect_theta (+ advect_microphysics_cell and the interior zero_moisture)
@@ -1532,9 +1582,13 @@ int launch_fused_advect(Ctx *c, double step, int il, int ih, int jl, int jh, int
         return DYN_E_ARG;
     }
     const bool moist = c->g.microphysics != 0;
-    if (c->prec == DYN_FP32)
-        return moist ? stage_t<float, true>(c, step, il, ih, jl, jh, parts) : stage_t<float, false>(c, step, il, ih, jl, jh, parts);
-    return moist ? stage_t<double, true>(c, step, il, ih, jl, jh, parts) : stage_t<double, false>(c, step, il, ih, jl, jh, parts);
+    auto run = [&](auto turb) {
+        constexpr bool TURB = decltype(turb)::value;
+        if (c->prec == DYN_FP32)
+            return moist ? stage_t<float, true, TURB>(c, step, il, ih, jl, jh, parts) : stage_t<float, false, TURB>(c, step, il, ih, jl, jh, parts);
+        return moist ? stage_t<double, true, TURB>(c, step, il, ih, jl, jh, parts) : stage_t<double, false, TURB>(c, step, il, ih, jl, jh, parts);
+    };
+    return c->turb.on ? run(std::true_type{}) : run(std::false_type{});
 }
 
 // PGF (optional) and the boundary update of every prognostic after launch_fused_advect; stands for

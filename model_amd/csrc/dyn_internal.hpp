@@ -281,6 +281,7 @@ int launch_kessler_step_end(Ctx *c, int ray_level);
 // turbulence: tendencies at the start of a step, and their addition to the forecasts in a stage
 void turb_release(Ctx *c);
 int turb_step_begin(Ctx *c);
+const void *turb_tendency(const Ctx *c, int field);  // of DYN_U .. DYN_QR
 int turb_apply_velocity(Ctx *c, double step);
 int turb_apply_scalars(Ctx *c, double step, bool theta);
 void drop_graph(Ctx *c);

@@ -299,7 +299,7 @@ __global__ void __launch_bounds__(kThreads) k_div_fft_x(Geo g, Cols c, const T *
     const int j = blockIdx.x;
     const int kk0 = blockIdx.y * kc;
     const int jj = j == 0 ? 1 : (j == g.NY - 1 ? g.NY - 2 : j);  // mirrored rows, pressure.cpp:1408-1415
-    const double sdt = step * g.dt;
+    const DivStep<T> ds(g, step);
     // element idx = i*kc + b; when kc divides the block size each thread keeps its level b
     const bool fixed_b = (blockDim.x % kc) == 0;
     const int di = blockDim.x / kc;
@@ -315,11 +315,8 @@ __global__ void __launch_bounds__(kThreads) k_div_fft_x(Geo g, Cols c, const T *
             // the periodic column UP(NX-3) is read as UP(3), the value periodic_uvw_boundaries puts there
             int k = kk + 1, ia = i + 3;
             int ie = ia + 1 == g.NX - 3 ? 3 : ia + 1;
-            T rhou = T(c.rhou[k]);
-            d = rhou * (UP[IX(ie, jj, k)] - UP[IX(ia, jj, k)]) * T(g.one_d_dx) +
-                rhou * (VP[IX(ia, jj + 1, k)] - VP[IX(ia, jj, k)]) * T(g.one_d_dy) +
-                (T(c.rhow[k + 1]) * WP[IX(ia, jj, k + 1)] - T(c.rhow[k]) * WP[IX(ia, jj, k)]) * (T(g.one_d_dz) * T(c.mu[k]));
-            d /= T(sdt);
+            d = T(ds(c.rhou[k], c.rhow[k + 1], c.rhow[k], c.mu[k], UP[IX(ie, jj, k)], UP[IX(ia, jj, k)], VP[IX(ia, jj + 1, k)],
+                     VP[IX(ia, jj, k)], WP[IX(ia, jj, k + 1)], WP[IX(ia, jj, k)]));
         }
         re[0][idx] = d;
         im[0][idx] = T(0);
@@ -756,13 +753,12 @@ template <typename T>
 __device__ __forceinline__ void div_rfft_x_block(const Geo &g, const Cols &c, const T *__restrict__ UP, const T *__restrict__ VP,
                                                  const T *__restrict__ WP, T *__restrict__ spec, const Radix &rad, const double *tw,
                                                  int nk2, int kc, double step, const T *__restrict__ src, int j, int chunk,
-                                                 unsigned char *smem) {
+                                                 unsigned char *smem, bool wide) {
     const int n = rad.n, P = kc / 2, nkx = n / 2 + 1;
     T *re = (T *)smem, *im = re + n * P, *twl = im + n * P;
     const int kk0 = chunk * kc;
     load_twiddles(twl, tw, n);
     const int jj = j == 0 ? 1 : (j == g.NY - 1 ? g.NY - 2 : j);  // mirrored rows, pressure.cpp:1408-1415
-    const double sdt = step * g.dt;
     // the column coefficients of the block's kc levels (rhou(k), rhow(k+1), rhow(k), mu(k)), read once
     // into LDS instead of once per element
     double *colc = (double *)(twl + 2 * n);
@@ -781,8 +777,9 @@ __device__ __forceinline__ void div_rfft_x_block(const Geo &g, const Cols &c, co
     // and the divergence form are separate loops for the same reason.
     constexpr int kU = 4;
     const int ne = n * kc, nt = (int)blockDim.x;
-    auto gather = [&](auto from_src) {
+    auto gather = [&](auto from_src, auto arithmetic) {
         constexpr bool kSrc = decltype(from_src)::value;
+        const DivStep<decltype(arithmetic)> ds(g, step);
         for (int idx0 = (int)threadIdx.x; idx0 < ne; idx0 += kU * nt) {
             T f0[kU], f1[kU], f2[kU], f3[kU], f4[kU], f5[kU];
             double ru[kU], rw1[kU], rw0[kU], mk[kU];
@@ -814,10 +811,7 @@ __device__ __forceinline__ void div_rfft_x_block(const Geo &g, const Cols &c, co
                 if (kk < nk2 && kSrc) {
                     d = f0[u];
                 } else if (kk < nk2) {
-                    T rhou = T(ru[u]);
-                    d = rhou * (f0[u] - f1[u]) * T(g.one_d_dx) + rhou * (f2[u] - f3[u]) * T(g.one_d_dy) +
-                        (T(rw1[u]) * f4[u] - T(rw0[u]) * f5[u]) * (T(g.one_d_dz) * T(mk[u]));
-                    d /= T(sdt);
+                    d = T(ds(ru[u], rw1[u], rw0[u], mk[u], f0[u], f1[u], f2[u], f3[u], f4[u], f5[u]));
                 }
                 if (idx < ne) {
                     if (b & 1) im[i * P + (b >> 1)] = d;
@@ -826,8 +820,9 @@ __device__ __forceinline__ void div_rfft_x_block(const Geo &g, const Cols &c, co
             }
         }
     };
-    if (src) gather(std::true_type{});
-    else gather(std::false_type{});
+    if (src) gather(std::true_type{}, T(0));
+    else if (sizeof(T) == 4 && wide) gather(std::false_type{}, double(0));
+    else gather(std::false_type{}, T(0));
     __syncthreads();
     lds_fft_ip<T, kMaxBX>(re, im, rad, P, P, 1, twl, -1);
     // split the packed pair: A = (Z[m] + conj Z[-m]) / 2, B = (Z[m] - conj Z[-m]) / 2i
@@ -1010,9 +1005,9 @@ __device__ __forceinline__ void thomas_tab_down(const double *Tab, long long fs,
     for (int t = 0; t < kTC; t++) v[t] = Tab[max(k0 - t, 0) * fs];
 }
 // p_kk = (x_kk / (ni nj) - a_k p_{kk-1}) z_kk for the chunk's levels kk = k0 .. k0+kTC-1 (< N unless FULL)
-template <typename T, bool FULL, int kTC, typename XT>
+template <bool FULL, int kTC, typename T>
 __device__ __forceinline__ void thomas_fwd_chunk(const ThomasCoef &co, const double (&z)[kTC], int k0, int N, double size2d,
-                                                 double rsize, XT *x, int xs, bool m0, double *mean, double &p) {
+                                                 double rsize, T *x, int xs, bool m0, double *mean, double &p) {
     double v[kTC], ac[kTC];
 #pragma unroll
     for (int t = 0; t < kTC; t++) {
@@ -1029,13 +1024,13 @@ __device__ __forceinline__ void thomas_fwd_chunk(const ThomasCoef &co, const dou
     for (int t = 0; t < kTC; t++) {
         if (FULL || k0 + t < N) {
             if (m0) mean[2 * (k0 + t)] = v[t];
-            else x[(k0 + t) * xs] = XT(T(v[t]));
+            else x[(k0 + t) * xs] = T(v[t]);
         }
     }
 }
 // x_kk = y_kk - F_kk x_{kk+1} for kk = k0 .. k0-kTC+1 (>= 0 unless FULL)
-template <typename T, bool FULL, int kTC, typename XT>
-__device__ __forceinline__ void thomas_back_chunk(const ThomasCoef &co, const double (&z)[kTC], int k0, XT *x, int xs, bool m0,
+template <bool FULL, int kTC, typename T>
+__device__ __forceinline__ void thomas_back_chunk(const ThomasCoef &co, const double (&z)[kTC], int k0, T *x, int xs, bool m0,
                                                   const double *mean, double &p) {
     double v[kTC], f[kTC];
 #pragma unroll
@@ -1052,11 +1047,11 @@ __device__ __forceinline__ void thomas_back_chunk(const ThomasCoef &co, const do
     }
 #pragma unroll
     for (int t = 0; t < kTC; t++)
-        if (FULL || k0 - t >= 0) x[(k0 - t) * xs] = XT(T(v[t]));
+        if (FULL || k0 - t >= 0) x[(k0 - t) * xs] = T(v[t]);
 }
-// Z: the column's pivots, one every fs.  Values are rounded to T whatever the type XT they are held in.
-template <typename T, int kTC = kThomasChunk, typename XT>
-__device__ __forceinline__ void thomas_part(const ThomasArgs &ta, const ThomasCoef &co, int kx, int ky, const double *Z, long long fs, XT *x, int xs,
+// Z: the column's pivots, one every fs
+template <int kTC = kThomasChunk, typename T>
+__device__ __forceinline__ void thomas_part(const ThomasArgs &ta, const ThomasCoef &co, int kx, int ky, const double *Z, long long fs, T *x, int xs,
                                             double *mean) {
     const int N = ta.nk - 2;
     const double size2d = (double)(ta.ni * ta.nj), rsize = 1.0 / size2d;
@@ -1068,39 +1063,39 @@ __device__ __forceinline__ void thomas_part(const ThomasArgs &ta, const ThomasCo
     int k0 = 0;
     for (; k0 + 2 * kTC <= N; k0 += 2 * kTC) {
         thomas_tab_up<kTC>(Z, fs, k0 + kTC, N - 1, B);
-        thomas_fwd_chunk<T, true, kTC>(co, A, k0, N, size2d, rsize, x, xs, m0, mean, p);
+        thomas_fwd_chunk<true, kTC>(co, A, k0, N, size2d, rsize, x, xs, m0, mean, p);
         thomas_tab_up<kTC>(Z, fs, k0 + 2 * kTC, N - 1, A);
-        thomas_fwd_chunk<T, true, kTC>(co, B, k0 + kTC, N, size2d, rsize, x, xs, m0, mean, p);
+        thomas_fwd_chunk<true, kTC>(co, B, k0 + kTC, N, size2d, rsize, x, xs, m0, mean, p);
     }
     if (k0 < N) {
         thomas_tab_up<kTC>(Z, fs, k0 + kTC, N - 1, B);
-        if (k0 + kTC <= N) thomas_fwd_chunk<T, true, kTC>(co, A, k0, N, size2d, rsize, x, xs, m0, mean, p);
-        else thomas_fwd_chunk<T, false, kTC>(co, A, k0, N, size2d, rsize, x, xs, m0, mean, p);
-        if (k0 + kTC < N) thomas_fwd_chunk<T, false, kTC>(co, B, k0 + kTC, N, size2d, rsize, x, xs, m0, mean, p);
+        if (k0 + kTC <= N) thomas_fwd_chunk<true, kTC>(co, A, k0, N, size2d, rsize, x, xs, m0, mean, p);
+        else thomas_fwd_chunk<false, kTC>(co, A, k0, N, size2d, rsize, x, xs, m0, mean, p);
+        if (k0 + kTC < N) thomas_fwd_chunk<false, kTC>(co, B, k0 + kTC, N, size2d, rsize, x, xs, m0, mean, p);
     }
     if (m0) p = 0.0;  // OUT3D(0,0,NZ-2) = 0
-    x[(N - 1) * xs] = XT(T(p));
+    x[(N - 1) * xs] = T(p);
     if (N < 2) return;
     // back substitution x_kk = y_kk - F_kk x_{kk+1} for kk = N-2 .. 0, walking down in chunks
     thomas_tab_down<kTC>(Z, fs, N - 2, A);
     k0 = N - 2;
     for (; k0 - 2 * kTC + 1 >= 0; k0 -= 2 * kTC) {
         thomas_tab_down<kTC>(Z, fs, k0 - kTC, B);
-        thomas_back_chunk<T, true, kTC>(co, A, k0, x, xs, m0, mean, p);
+        thomas_back_chunk<true, kTC>(co, A, k0, x, xs, m0, mean, p);
         thomas_tab_down<kTC>(Z, fs, k0 - 2 * kTC, A);
-        thomas_back_chunk<T, true, kTC>(co, B, k0 - kTC, x, xs, m0, mean, p);
+        thomas_back_chunk<true, kTC>(co, B, k0 - kTC, x, xs, m0, mean, p);
     }
     if (k0 >= 0) {
         thomas_tab_down<kTC>(Z, fs, k0 - kTC, B);
-        if (k0 - kTC + 1 >= 0) thomas_back_chunk<T, true, kTC>(co, A, k0, x, xs, m0, mean, p);
-        else thomas_back_chunk<T, false, kTC>(co, A, k0, x, xs, m0, mean, p);
-        if (k0 - kTC >= 0) thomas_back_chunk<T, false, kTC>(co, B, k0 - kTC, x, xs, m0, mean, p);
+        if (k0 - kTC + 1 >= 0) thomas_back_chunk<true, kTC>(co, A, k0, x, xs, m0, mean, p);
+        else thomas_back_chunk<false, kTC>(co, A, k0, x, xs, m0, mean, p);
+        if (k0 - kTC >= 0) thomas_back_chunk<false, kTC>(co, B, k0 - kTC, x, xs, m0, mean, p);
     }
 }
 
 // q_kk = x_kk - F_{kk-1} q_{kk-1} for the chunk's levels kk = k0 .. k0+kTC-1 (< N unless FULL), z[t] = z_{k0+t-1}
-template <typename T, bool FULL, int kTC, typename XT>
-__device__ __forceinline__ void thomas_t_fwd_chunk(const ThomasCoef &co, const double (&z)[kTC], int k0, int N, XT *x, int xs, double &q) {
+template <bool FULL, int kTC, typename T>
+__device__ __forceinline__ void thomas_t_fwd_chunk(const ThomasCoef &co, const double (&z)[kTC], int k0, int N, T *x, int xs, double &q) {
     double v[kTC], f[kTC];
 #pragma unroll
     for (int t = 0; t < kTC; t++) {
@@ -1115,12 +1110,12 @@ __device__ __forceinline__ void thomas_t_fwd_chunk(const ThomasCoef &co, const d
     }
 #pragma unroll
     for (int t = 0; t < kTC; t++)
-        if (FULL || k0 + t < N) x[(k0 + t) * xs] = XT(T(v[t]));
+        if (FULL || k0 + t < N) x[(k0 + t) * xs] = T(v[t]);
 }
 // b_kk = z_kk (q_kk - a_{kk+2} b_{kk+1}), stored as b / (ni nj), for kk = k0 .. k0-kTC+1 (>= 0 unless FULL)
-template <typename T, bool FULL, int kTC, typename XT>
+template <bool FULL, int kTC, typename T>
 __device__ __forceinline__ void thomas_t_back_chunk(const ThomasCoef &co, const double (&z)[kTC], int k0, double size2d, double rsize,
-                                                    XT *x, int xs, double &b) {
+                                                    T *x, int xs, double &b) {
     double v[kTC], ac[kTC];
 #pragma unroll
     for (int t = 0; t < kTC; t++) {
@@ -1135,7 +1130,7 @@ __device__ __forceinline__ void thomas_t_back_chunk(const ThomasCoef &co, const 
     }
 #pragma unroll
     for (int t = 0; t < kTC; t++)
-        if (FULL || k0 - t >= 0) x[(k0 - t) * xs] = XT(T(v[t]));
+        if (FULL || k0 - t >= 0) x[(k0 - t) * xs] = T(v[t]);
 }
 // Transpose of thomas_part (the adjoint's vertical solve), in place.  The forward map is p = L'^{-1} x / S
 // (L' lower bidiagonal: 1/z_k on the diagonal, a_k below) followed by x_k = p_k - F_k x_{k+1}; for the
@@ -1143,8 +1138,8 @@ __device__ __forceinline__ void thomas_t_back_chunk(const ThomasCoef &co, const 
 // reverse order: q_1 = x_1, q_k = x_k - F_{k-1} q_{k-1} (q_N = 0 for (0,0)), then b_N = z_N q_N,
 // b_k = z_k (q_k - a_{k+1} b_{k+1}), result b / S.  The singular last pivot of (0,0) is never used.
 // The table entries come in chunks through two register sets that take turns, as in thomas_part.
-template <typename T, int kTC = kThomasChunk, typename XT>
-__device__ __forceinline__ void thomas_part_t(const ThomasArgs &ta, const ThomasCoef &co, int kx, int ky, const double *Z, long long fs, XT *x, int xs) {
+template <int kTC = kThomasChunk, typename T>
+__device__ __forceinline__ void thomas_part_t(const ThomasArgs &ta, const ThomasCoef &co, int kx, int ky, const double *Z, long long fs, T *x, int xs) {
     const int N = ta.nk - 2;
     const double size2d = (double)(ta.ni * ta.nj), rsize = 1.0 / size2d;
     const bool m0 = (kx == 0 && ky == 0);
@@ -1155,33 +1150,33 @@ __device__ __forceinline__ void thomas_part_t(const ThomasArgs &ta, const Thomas
     int k0 = 1;
     for (; k0 + 2 * kTC <= N; k0 += 2 * kTC) {
         thomas_tab_up<kTC>(Z, fs, k0 + kTC - 1, N - 2, B);
-        thomas_t_fwd_chunk<T, true, kTC>(co, A, k0, N, x, xs, q);
+        thomas_t_fwd_chunk<true, kTC>(co, A, k0, N, x, xs, q);
         thomas_tab_up<kTC>(Z, fs, k0 + 2 * kTC - 1, N - 2, A);
-        thomas_t_fwd_chunk<T, true, kTC>(co, B, k0 + kTC, N, x, xs, q);
+        thomas_t_fwd_chunk<true, kTC>(co, B, k0 + kTC, N, x, xs, q);
     }
     if (k0 < N) {
         thomas_tab_up<kTC>(Z, fs, k0 + kTC - 1, N - 2, B);
-        if (k0 + kTC <= N) thomas_t_fwd_chunk<T, true, kTC>(co, A, k0, N, x, xs, q);
-        else thomas_t_fwd_chunk<T, false, kTC>(co, A, k0, N, x, xs, q);
-        if (k0 + kTC < N) thomas_t_fwd_chunk<T, false, kTC>(co, B, k0 + kTC, N, x, xs, q);
+        if (k0 + kTC <= N) thomas_t_fwd_chunk<true, kTC>(co, A, k0, N, x, xs, q);
+        else thomas_t_fwd_chunk<false, kTC>(co, A, k0, N, x, xs, q);
+        if (k0 + kTC < N) thomas_t_fwd_chunk<false, kTC>(co, B, k0 + kTC, N, x, xs, q);
     }
     // b_{N-1} = z_{N-1} q_{N-1} (0 for (0,0)); b_kk = z_kk (q_kk - a_{kk+2} b_{kk+1}), kk = N-2 .. 0
     double b = m0 ? 0.0 : double(x[(N - 1) * xs]) * Z[(N - 1) * fs];
-    x[(N - 1) * xs] = XT(T(div_exact(b, size2d, rsize)));
+    x[(N - 1) * xs] = T(div_exact(b, size2d, rsize));
     if (N < 2) return;
     thomas_tab_down<kTC>(Z, fs, N - 2, A);
     k0 = N - 2;
     for (; k0 - 2 * kTC + 1 >= 0; k0 -= 2 * kTC) {
         thomas_tab_down<kTC>(Z, fs, k0 - kTC, B);
-        thomas_t_back_chunk<T, true, kTC>(co, A, k0, size2d, rsize, x, xs, b);
+        thomas_t_back_chunk<true, kTC>(co, A, k0, size2d, rsize, x, xs, b);
         thomas_tab_down<kTC>(Z, fs, k0 - 2 * kTC, A);
-        thomas_t_back_chunk<T, true, kTC>(co, B, k0 - kTC, size2d, rsize, x, xs, b);
+        thomas_t_back_chunk<true, kTC>(co, B, k0 - kTC, size2d, rsize, x, xs, b);
     }
     if (k0 >= 0) {
         thomas_tab_down<kTC>(Z, fs, k0 - kTC, B);
-        if (k0 - kTC + 1 >= 0) thomas_t_back_chunk<T, true, kTC>(co, A, k0, size2d, rsize, x, xs, b);
-        else thomas_t_back_chunk<T, false, kTC>(co, A, k0, size2d, rsize, x, xs, b);
-        if (k0 - kTC >= 0) thomas_t_back_chunk<T, false, kTC>(co, B, k0 - kTC, size2d, rsize, x, xs, b);
+        if (k0 - kTC + 1 >= 0) thomas_t_back_chunk<true, kTC>(co, A, k0, size2d, rsize, x, xs, b);
+        else thomas_t_back_chunk<false, kTC>(co, A, k0, size2d, rsize, x, xs, b);
+        if (k0 - kTC >= 0) thomas_t_back_chunk<false, kTC>(co, B, k0 - kTC, size2d, rsize, x, xs, b);
     }
 }
 
@@ -1261,8 +1256,8 @@ __device__ __forceinline__ void ypass_block(T *__restrict__ spec, int nk2, const
         const int part = (int)threadIdx.x >= nj, ky = (int)threadIdx.x - part * nj;
         T *x = (part ? im : re) + ky * P2;
         const double *Z = ta.zpiv + (long long)kx * nj * nk2 + ky;
-        if (TR) thomas_part_t<T>(ta, co, kx, ky, Z, nj, x, 1);
-        else thomas_part<T>(ta, co, kx, ky, Z, nj, x, 1, mean + part);
+        if (TR) thomas_part_t(ta, co, kx, ky, Z, nj, x, 1);
+        else thomas_part(ta, co, kx, ky, Z, nj, x, 1, mean + part);
     }
     __syncthreads();
     lds_fft_ip<T, ypass_maxb<T>(), POW2>(re, im, rady, nk2, P2, 1, twl, +1);
@@ -1272,9 +1267,9 @@ __device__ __forceinline__ void ypass_block(T *__restrict__ spec, int nk2, const
 template <typename T>
 __global__ void __launch_bounds__(kThreadsX) k_div_rfft_x(Geo g, Cols c, const T *__restrict__ UP, const T *__restrict__ VP,
                                                          const T *__restrict__ WP, T *__restrict__ spec, Radix rad, const double *tw,
-                                                         int nk2, int kc, double step, const T *__restrict__ src) {
+                                                         int nk2, int kc, double step, const T *__restrict__ src, bool wide) {
     extern __shared__ unsigned char smem[];
-    div_rfft_x_block<T>(g, c, UP, VP, WP, spec, rad, tw, nk2, kc, step, src, blockIdx.x, blockIdx.y, smem);
+    div_rfft_x_block<T>(g, c, UP, VP, WP, spec, rad, tw, nk2, kc, step, src, blockIdx.x, blockIdx.y, smem, wide);
 }
 
 template <typename T>
@@ -1433,8 +1428,8 @@ __device__ __forceinline__ void ypass_half_block(const T *__restrict__ in, T *__
         const int part = (int)threadIdx.x >= L, m = (int)threadIdx.x - part * L;
         T *x = (part ? im : re) + m * P2;
         const double *Z = ta.zpiv + (long long)kx * nj * nk2 + 2 * m + h;
-        if (TR) thomas_part_t<T>(ta, co, kx, 2 * m + h, Z, nj, x, 1);
-        else thomas_part<T>(ta, co, kx, 2 * m + h, Z, nj, x, 1, mean + part);
+        if (TR) thomas_part_t(ta, co, kx, 2 * m + h, Z, nj, x, 1);
+        else thomas_part(ta, co, kx, 2 * m + h, Z, nj, x, 1, mean + part);
     }
     __syncthreads();
     lds_fft_pow2<T, half_maxb<T>()>(re, im, rh, nk2, P2, 1, twl, +1);
@@ -1601,14 +1596,14 @@ __device__ __forceinline__ void ypass_dft_block(T *__restrict__ spec, int n, con
     };
     products();
     __syncthreads();
-    results(-1, [&](int r, int q, double v) { X[r * pitch + q] = double(T(v)); });
+    results(-1, [&](int r, int q, double v) { X[r * pitch + q] = v; });
     __syncthreads();
     if ((int)threadIdx.x < 2 * n) {  // neighbouring lanes take the real and the imaginary part of a column
         const int ky = (int)threadIdx.x >> 1, part = (int)threadIdx.x & 1;
         const double *Z = ta.zpiv + (long long)kx * n * nk2 + ky;
         double *xc = X + ky * pitch + part;
-        if (TR) thomas_part_t<T>(ta, co, kx, ky, Z, n, xc, 2);
-        else thomas_part<T>(ta, co, kx, ky, Z, n, xc, 2, mean + part);
+        if (TR) thomas_part_t(ta, co, kx, ky, Z, n, xc, 2);
+        else thomas_part(ta, co, kx, ky, Z, n, xc, 2, mean + part);
     }
     __syncthreads();
     for (int idx = (int)threadIdx.x; idx < (n - 1) / 2 * ncol; idx += nt) {
@@ -1649,7 +1644,7 @@ __global__ void __launch_bounds__(kThreadsX) k_ens_div_rfft_x(const EnsMember *m
         const int local = item - e.px0, nch = (e.nk2 + e.kcx - 1) / e.kcx;
         div_rfft_x_block<T>(e.g, e.c, (const T *)e.buf[DYN_U][roles.r[DYN_U][DYN_ROLE_P]], (const T *)e.buf[DYN_V][roles.r[DYN_V][DYN_ROLE_P]],
                             (const T *)e.buf[DYN_W][roles.r[DYN_W][DYN_ROLE_P]], (T *)e.spec, e.rx, e.twx, e.nk2, e.kcx, step,
-                            (const T *)nullptr, local / nch, local % nch, smem);
+                            (const T *)nullptr, local / nch, local % nch, smem, e.dfty != nullptr);
     }
 }
 
@@ -1723,8 +1718,8 @@ __global__ void __launch_bounds__(kThomasThreads) k_thomas_staged(T *__restrict_
         // two threads per column: even lanes the real part, odd lanes the imaginary part (interleaved)
         const int colx = (int)threadIdx.x >> 1, part = threadIdx.x & 1;
         if (colx < ncol) {
-            if (TR) thomas_part_t<T>(ta, co, kx, ky0 + colx, zl + colx, tg, x + colx * P2 + part, 2);
-            else thomas_part<T>(ta, co, kx, ky0 + colx, zl + colx, tg, x + colx * P2 + part, 2, mean + part);
+            if (TR) thomas_part_t(ta, co, kx, ky0 + colx, zl + colx, tg, x + colx * P2 + part, 2);
+            else thomas_part(ta, co, kx, ky0 + colx, zl + colx, tg, x + colx * P2 + part, 2, mean + part);
         }
     }
     __syncthreads();
@@ -1966,7 +1961,7 @@ int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
             Timed _t(c, "p1_div_rfft_x", pts);
             hipLaunchKernelGGL(k_div_rfft_x<T>, gx, dim3(kThreadsX), shx, c->stream, g, c->cols, (const T *)c->prog[DYN_U][2],
                                (const T *)c->prog[DYN_V][2], (const T *)c->prog[DYN_W][2], spec, rx, pp.twx, pp.nk2, kc, step,
-                               (const T *)nullptr);
+                               (const T *)nullptr, pp.dfty != nullptr);
         }
         DYN_LAUNCH_CHECK();
         if (after_i) {
@@ -2151,7 +2146,7 @@ int solve_adjoint_t(Ctx *c, double step, T *pihat, T *uh, T *vh, T *wh, T *r1, T
     } else {
         Timed _t(c, "adj_rfft_x", pts);
         hipLaunchKernelGGL(k_div_rfft_x<T>, gx, dim3(kThreadsX), shx, c->stream, g, c->cols, (const T *)nullptr, (const T *)nullptr,
-                           (const T *)nullptr, spec, rx, pp.twx, pp.nk2, kc, step, (const T *)r1);
+                           (const T *)nullptr, spec, rx, pp.twx, pp.nk2, kc, step, (const T *)r1, false);
     }
     DYN_LAUNCH_CHECK();
     const int pad = 1;

@@ -2,7 +2,8 @@
 // without terrain or surface heat flux: mixing coefficients and stored tendencies at the start of each
 // step (calculate_diff_tend, driver_serial.cpp:194), added to the forecasts in every stage
 // (apply_velocity_diffusion, solver.cpp:104; apply_scalar_diffusion / apply_moisture_diffusion,
-// driver_serial.cpp:218, 231).
+// driver_serial.cpp:218, 231).  The fused step adds them inside its stage kernels; the per-operator one
+// through the kernels at the end of this file.
 //
 // The reference walks i-slabs and carries the stress tensor of slab i-1 over as the west stress of slab
 // i, and the flux through the top of a level over as the bottom flux of the level above.  Every such
@@ -19,6 +20,7 @@ namespace {
 constexpr double kCmixV = 0.15, kCmixH = 0.05;   // turbulence.cpp:48-49
 constexpr double kPrInv = 3.0, kLvMax = 200.0, kCs = 0.25;  // turbulence.cpp:56-58
 
+// (the tendencies in the order of DYN_U .. DYN_QR)
 enum { TK = 0, TKH, TUF, TVF, TWF, TTD, TQV, TQC, TQR, TCOUNT };
 
 struct TurbArgs {
@@ -425,6 +427,7 @@ int turb_step_begin(Ctx *c) {
     const int NX = c->g.nx, NY = c->g.ny;
     return c->prec == DYN_FP32 ? launch_diff_tend<float>(c, 1, NX - 1, 1, NY - 1) : launch_diff_tend<double>(c, 1, NX - 1, 1, NY - 1);
 }
+const void *turb_tendency(const Ctx *c, int field) { return c->turb.buf[TUF + field]; }
 int turb_apply_velocity(Ctx *c, double step) {
     const int NX = c->g.nx, NY = c->g.ny;
     return c->prec == DYN_FP32 ? launch_apply_velocity<float>(c, step, 3, NX - 3, 3, NY - 3)
