@@ -296,20 +296,23 @@ __device__ __forceinline__ double lane_pair(double x) {
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// Along j, complex, in place, for one kx and NC real columns (level, part): real and imaginary parts sit in
-// neighbouring columns, so the products' cross terms come from the neighbouring lane.  Every element a
-// block reads is in LDS before it writes any, and no other block touches its columns.
-template <typename T, int NT>
-__global__ void __launch_bounds__(dft_bound(NT)) k_dft_y(T *__restrict__ spec, int n, const double *__restrict__ tab, int nk2, int sign) {
+// Along j, complex, for one kx and NC real columns (level, part): real and imaginary parts sit in
+// neighbouring columns, so the products' cross terms come from the neighbouring lane.  In place (in == out) every
+// element a block reads is in LDS before it writes any, and no other block touches its columns.  FP32 spectra are
+// handed to the vertical sweeps in 64 bits (TO = double): rounded there, the longest waves' columns, whose systems
+// are nearly singular, lose most of what a single-precision solve loses in its transforms.
+template <typename TI, typename TO, int NT>
+__global__ void __launch_bounds__(dft_bound(NT)) k_dft_y(const TI *in, TO *out, int n, const double *__restrict__ tab, int nk2, int sign) {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int NC = 16 * NT;
     const int pitch = dft_pitch(NC), h = dft_rows(n), hk = (h + 3) & ~3, ncol = 2 * nk2;
     double *E = (double *)smem, *D = E + hk * pitch;
-    T *x = spec + (long long)blockIdx.x * n * ncol;
+    const TI *x = in + (long long)blockIdx.x * n * ncol;
+    TO *o = out + (long long)blockIdx.x * n * ncol;
     const int c0 = blockIdx.y * NC, b = threadIdx.x % NC, q = min(c0 + b, ncol - 1);
     const int rows = blockDim.x / NC;
     for (int i = threadIdx.x / NC; i < hk; i += 4 * rows) {
-        T a[4], m[4];
+        TI a[4], m[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int ir = min(i + r * rows, h - 1);
@@ -338,10 +341,10 @@ __global__ void __launch_bounds__(dft_bound(NT)) k_dft_y(T *__restrict__ spec, i
 #pragma unroll
             for (int v4 = 0; v4 < 4; v4++) {
                 const int m = m0 + (lane >> 4) + 4 * v4;
-                const double o = sg * lane_pair(ps[t][v4]);
+                const double d = sg * lane_pair(ps[t][v4]);
                 if (m < h && qc < ncol) {
-                    x[(long long)m * ncol + qc] = T(pc[t][v4] + o);
-                    if (m > 0 && 2 * m != n) x[(long long)(n - m) * ncol + qc] = T(pc[t][v4] - o);
+                    o[(long long)m * ncol + qc] = TO(pc[t][v4] + d);
+                    if (m > 0 && 2 * m != n) o[(long long)(n - m) * ncol + qc] = TO(pc[t][v4] - d);
                 }
             }
         }

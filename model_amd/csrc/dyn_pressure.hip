@@ -1029,7 +1029,7 @@ __device__ __forceinline__ void thomas_fwd_chunk(const ThomasCoef &co, const dou
     }
 }
 // x_kk = y_kk - F_kk x_{kk+1} for kk = k0 .. k0-kTC+1 (>= 0 unless FULL)
-template <bool FULL, int kTC, typename T>
+template <typename R, bool FULL, int kTC, typename T>
 __device__ __forceinline__ void thomas_back_chunk(const ThomasCoef &co, const double (&z)[kTC], int k0, T *x, int xs, bool m0,
                                                   const double *mean, double &p) {
     double v[kTC], f[kTC];
@@ -1047,10 +1047,10 @@ __device__ __forceinline__ void thomas_back_chunk(const ThomasCoef &co, const do
     }
 #pragma unroll
     for (int t = 0; t < kTC; t++)
-        if (FULL || k0 - t >= 0) x[(k0 - t) * xs] = T(v[t]);
+        if (FULL || k0 - t >= 0) x[(k0 - t) * xs] = T(R(v[t]));
 }
-// Z: the column's pivots, one every fs
-template <int kTC = kThomasChunk, typename T>
+// Z: the column's pivots, one every fs; R: the type the results are rounded to, whatever type T holds them
+template <typename R, int kTC = kThomasChunk, typename T>
 __device__ __forceinline__ void thomas_part(const ThomasArgs &ta, const ThomasCoef &co, int kx, int ky, const double *Z, long long fs, T *x, int xs,
                                             double *mean) {
     const int N = ta.nk - 2;
@@ -1074,22 +1074,22 @@ __device__ __forceinline__ void thomas_part(const ThomasArgs &ta, const ThomasCo
         if (k0 + kTC < N) thomas_fwd_chunk<false, kTC>(co, B, k0 + kTC, N, size2d, rsize, x, xs, m0, mean, p);
     }
     if (m0) p = 0.0;  // OUT3D(0,0,NZ-2) = 0
-    x[(N - 1) * xs] = T(p);
+    x[(N - 1) * xs] = T(R(p));
     if (N < 2) return;
     // back substitution x_kk = y_kk - F_kk x_{kk+1} for kk = N-2 .. 0, walking down in chunks
     thomas_tab_down<kTC>(Z, fs, N - 2, A);
     k0 = N - 2;
     for (; k0 - 2 * kTC + 1 >= 0; k0 -= 2 * kTC) {
         thomas_tab_down<kTC>(Z, fs, k0 - kTC, B);
-        thomas_back_chunk<true, kTC>(co, A, k0, x, xs, m0, mean, p);
+        thomas_back_chunk<R, true, kTC>(co, A, k0, x, xs, m0, mean, p);
         thomas_tab_down<kTC>(Z, fs, k0 - 2 * kTC, A);
-        thomas_back_chunk<true, kTC>(co, B, k0 - kTC, x, xs, m0, mean, p);
+        thomas_back_chunk<R, true, kTC>(co, B, k0 - kTC, x, xs, m0, mean, p);
     }
     if (k0 >= 0) {
         thomas_tab_down<kTC>(Z, fs, k0 - kTC, B);
-        if (k0 - kTC + 1 >= 0) thomas_back_chunk<true, kTC>(co, A, k0, x, xs, m0, mean, p);
-        else thomas_back_chunk<false, kTC>(co, A, k0, x, xs, m0, mean, p);
-        if (k0 - kTC >= 0) thomas_back_chunk<false, kTC>(co, B, k0 - kTC, x, xs, m0, mean, p);
+        if (k0 - kTC + 1 >= 0) thomas_back_chunk<R, true, kTC>(co, A, k0, x, xs, m0, mean, p);
+        else thomas_back_chunk<R, false, kTC>(co, A, k0, x, xs, m0, mean, p);
+        if (k0 - kTC >= 0) thomas_back_chunk<R, false, kTC>(co, B, k0 - kTC, x, xs, m0, mean, p);
     }
 }
 
@@ -1113,7 +1113,7 @@ __device__ __forceinline__ void thomas_t_fwd_chunk(const ThomasCoef &co, const d
         if (FULL || k0 + t < N) x[(k0 + t) * xs] = T(v[t]);
 }
 // b_kk = z_kk (q_kk - a_{kk+2} b_{kk+1}), stored as b / (ni nj), for kk = k0 .. k0-kTC+1 (>= 0 unless FULL)
-template <bool FULL, int kTC, typename T>
+template <typename R, bool FULL, int kTC, typename T>
 __device__ __forceinline__ void thomas_t_back_chunk(const ThomasCoef &co, const double (&z)[kTC], int k0, double size2d, double rsize,
                                                     T *x, int xs, double &b) {
     double v[kTC], ac[kTC];
@@ -1130,7 +1130,7 @@ __device__ __forceinline__ void thomas_t_back_chunk(const ThomasCoef &co, const 
     }
 #pragma unroll
     for (int t = 0; t < kTC; t++)
-        if (FULL || k0 - t >= 0) x[(k0 - t) * xs] = T(v[t]);
+        if (FULL || k0 - t >= 0) x[(k0 - t) * xs] = T(R(v[t]));
 }
 // Transpose of thomas_part (the adjoint's vertical solve), in place.  The forward map is p = L'^{-1} x / S
 // (L' lower bidiagonal: 1/z_k on the diagonal, a_k below) followed by x_k = p_k - F_k x_{k+1}; for the
@@ -1138,7 +1138,7 @@ __device__ __forceinline__ void thomas_t_back_chunk(const ThomasCoef &co, const 
 // reverse order: q_1 = x_1, q_k = x_k - F_{k-1} q_{k-1} (q_N = 0 for (0,0)), then b_N = z_N q_N,
 // b_k = z_k (q_k - a_{k+1} b_{k+1}), result b / S.  The singular last pivot of (0,0) is never used.
 // The table entries come in chunks through two register sets that take turns, as in thomas_part.
-template <int kTC = kThomasChunk, typename T>
+template <typename R, int kTC = kThomasChunk, typename T>
 __device__ __forceinline__ void thomas_part_t(const ThomasArgs &ta, const ThomasCoef &co, int kx, int ky, const double *Z, long long fs, T *x, int xs) {
     const int N = ta.nk - 2;
     const double size2d = (double)(ta.ni * ta.nj), rsize = 1.0 / size2d;
@@ -1162,21 +1162,21 @@ __device__ __forceinline__ void thomas_part_t(const ThomasArgs &ta, const Thomas
     }
     // b_{N-1} = z_{N-1} q_{N-1} (0 for (0,0)); b_kk = z_kk (q_kk - a_{kk+2} b_{kk+1}), kk = N-2 .. 0
     double b = m0 ? 0.0 : double(x[(N - 1) * xs]) * Z[(N - 1) * fs];
-    x[(N - 1) * xs] = T(div_exact(b, size2d, rsize));
+    x[(N - 1) * xs] = T(R(div_exact(b, size2d, rsize)));
     if (N < 2) return;
     thomas_tab_down<kTC>(Z, fs, N - 2, A);
     k0 = N - 2;
     for (; k0 - 2 * kTC + 1 >= 0; k0 -= 2 * kTC) {
         thomas_tab_down<kTC>(Z, fs, k0 - kTC, B);
-        thomas_t_back_chunk<true, kTC>(co, A, k0, size2d, rsize, x, xs, b);
+        thomas_t_back_chunk<R, true, kTC>(co, A, k0, size2d, rsize, x, xs, b);
         thomas_tab_down<kTC>(Z, fs, k0 - 2 * kTC, A);
-        thomas_t_back_chunk<true, kTC>(co, B, k0 - kTC, size2d, rsize, x, xs, b);
+        thomas_t_back_chunk<R, true, kTC>(co, B, k0 - kTC, size2d, rsize, x, xs, b);
     }
     if (k0 >= 0) {
         thomas_tab_down<kTC>(Z, fs, k0 - kTC, B);
-        if (k0 - kTC + 1 >= 0) thomas_t_back_chunk<true, kTC>(co, A, k0, size2d, rsize, x, xs, b);
-        else thomas_t_back_chunk<false, kTC>(co, A, k0, size2d, rsize, x, xs, b);
-        if (k0 - kTC >= 0) thomas_t_back_chunk<false, kTC>(co, B, k0 - kTC, size2d, rsize, x, xs, b);
+        if (k0 - kTC + 1 >= 0) thomas_t_back_chunk<R, true, kTC>(co, A, k0, size2d, rsize, x, xs, b);
+        else thomas_t_back_chunk<R, false, kTC>(co, A, k0, size2d, rsize, x, xs, b);
+        if (k0 - kTC >= 0) thomas_t_back_chunk<R, false, kTC>(co, B, k0 - kTC, size2d, rsize, x, xs, b);
     }
 }
 
@@ -1256,8 +1256,8 @@ __device__ __forceinline__ void ypass_block(T *__restrict__ spec, int nk2, const
         const int part = (int)threadIdx.x >= nj, ky = (int)threadIdx.x - part * nj;
         T *x = (part ? im : re) + ky * P2;
         const double *Z = ta.zpiv + (long long)kx * nj * nk2 + ky;
-        if (TR) thomas_part_t(ta, co, kx, ky, Z, nj, x, 1);
-        else thomas_part(ta, co, kx, ky, Z, nj, x, 1, mean + part);
+        if (TR) thomas_part_t<T>(ta, co, kx, ky, Z, nj, x, 1);
+        else thomas_part<T>(ta, co, kx, ky, Z, nj, x, 1, mean + part);
     }
     __syncthreads();
     lds_fft_ip<T, ypass_maxb<T>(), POW2>(re, im, rady, nk2, P2, 1, twl, +1);
@@ -1428,8 +1428,8 @@ __device__ __forceinline__ void ypass_half_block(const T *__restrict__ in, T *__
         const int part = (int)threadIdx.x >= L, m = (int)threadIdx.x - part * L;
         T *x = (part ? im : re) + m * P2;
         const double *Z = ta.zpiv + (long long)kx * nj * nk2 + 2 * m + h;
-        if (TR) thomas_part_t(ta, co, kx, 2 * m + h, Z, nj, x, 1);
-        else thomas_part(ta, co, kx, 2 * m + h, Z, nj, x, 1, mean + part);
+        if (TR) thomas_part_t<T>(ta, co, kx, 2 * m + h, Z, nj, x, 1);
+        else thomas_part<T>(ta, co, kx, 2 * m + h, Z, nj, x, 1, mean + part);
     }
     __syncthreads();
     lds_fft_pow2<T, half_maxb<T>()>(re, im, rh, nk2, P2, 1, twl, +1);
@@ -1476,7 +1476,7 @@ __global__ void __launch_bounds__(ypass_threads<T>()) k_ypass(T *__restrict__ sp
 // products run, X(i) and X(n-i) afterwards.  A wavefront keeps up to PT tiles' results in registers across
 // the barrier before they replace the operands; the last columns of a tile past 2 nk2 hold the next row's
 // values and their results are dropped.  The bits are those of k_dft_y, k_thomas_staged and k_dft_y in turn
-// (values are rounded to the storage type where those store them).
+// (64 bits from the first products to the sweeps' results, which are rounded to the storage type).
 // One launch serves slabs of few tiles (a pair of products per wavefront, PT = 1: 48x48x40 FP32 a step of 138 us
 // against 143 with three launches, and the radix passes, a chain of two barriers per radix, take 19 us
 // instead of 14); with more, the matrix units of nkx CUs are outrun by three launches spread over all of them
@@ -1602,8 +1602,8 @@ __device__ __forceinline__ void ypass_dft_block(T *__restrict__ spec, int n, con
         const int ky = (int)threadIdx.x >> 1, part = (int)threadIdx.x & 1;
         const double *Z = ta.zpiv + (long long)kx * n * nk2 + ky;
         double *xc = X + ky * pitch + part;
-        if (TR) thomas_part_t(ta, co, kx, ky, Z, n, xc, 2);
-        else thomas_part(ta, co, kx, ky, Z, n, xc, 2, mean + part);
+        if (TR) thomas_part_t<T>(ta, co, kx, ky, Z, n, xc, 2);
+        else thomas_part<T>(ta, co, kx, ky, Z, n, xc, 2, mean + part);
     }
     __syncthreads();
     for (int idx = (int)threadIdx.x; idx < (n - 1) / 2 * ncol; idx += nt) {
@@ -1682,12 +1682,12 @@ __global__ void __launch_bounds__(1024) k_ens_ypass(const EnsMember *mem, int nm
 // Q2 (staged): tridiagonal solve of tg columns of one kx with their values and pivots in LDS (coalesced in and
 // out): the whole block loads and stores, 2 tg of its threads run the sweeps
 constexpr int kThomasThreads = 256;
-template <typename T, bool TR = false>
-__global__ void __launch_bounds__(kThomasThreads) k_thomas_staged(T *__restrict__ spec, int nk2, ThomasArgs ta, int tg) {
+template <typename T, bool TR, typename TI>
+__global__ void __launch_bounds__(kThomasThreads) k_thomas_staged(const TI *in, T *spec, int nk2, ThomasArgs ta, int tg) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int P2 = 2 * nk2 + 1;
     double *zl = (double *)smem, *mean = zl + tg * nk2;
-    T *x = (T *)(mean + 4 * nk2);
+    TI *x = (TI *)(mean + 4 * nk2);
     const ThomasCoef co = thomas_coef(ta, nk2, mean + 2 * nk2);
     const int kx = blockIdx.x, ky0 = blockIdx.y * tg;
     const int ncol = min(tg, ta.nj - ky0);
@@ -1698,12 +1698,12 @@ __global__ void __launch_bounds__(kThomasThreads) k_thomas_staged(T *__restrict_
     const int ne = ncol * nk2, nt = (int)blockDim.x;
     for (int i0 = (int)threadIdx.x; i0 < ne; i0 += kU * nt) {
         double z[kU];
-        T vr[kU], vi[kU];
+        TI vr[kU], vi[kU];
 #pragma unroll
         for (int u = 0; u < kU; u++) {
             const int idx = min(i0 + u * nt, ne - 1), kk = idx / ncol;
             z[u] = zg[(long long)kk * ta.nj + idx - kk * ncol];
-            ld2(spec + base + 2LL * idx, vr[u], vi[u]);
+            ld2(in + base + 2LL * idx, vr[u], vi[u]);
         }
 #pragma unroll
         for (int u = 0; u < kU; u++) {
@@ -1718,14 +1718,14 @@ __global__ void __launch_bounds__(kThomasThreads) k_thomas_staged(T *__restrict_
         // two threads per column: even lanes the real part, odd lanes the imaginary part (interleaved)
         const int colx = (int)threadIdx.x >> 1, part = threadIdx.x & 1;
         if (colx < ncol) {
-            if (TR) thomas_part_t(ta, co, kx, ky0 + colx, zl + colx, tg, x + colx * P2 + part, 2);
-            else thomas_part(ta, co, kx, ky0 + colx, zl + colx, tg, x + colx * P2 + part, 2, mean + part);
+            if (TR) thomas_part_t<T>(ta, co, kx, ky0 + colx, zl + colx, tg, x + colx * P2 + part, 2);
+            else thomas_part<T>(ta, co, kx, ky0 + colx, zl + colx, tg, x + colx * P2 + part, 2, mean + part);
         }
     }
     __syncthreads();
     for (int idx = threadIdx.x; idx < ncol * nk2; idx += blockDim.x) {
         const int col = idx / nk2, kk = idx - col * nk2;
-        st2(spec + base + 2LL * idx, x[col * P2 + 2 * kk], x[col * P2 + 2 * kk + 1]);
+        st2(spec + base + 2LL * idx, T(x[col * P2 + 2 * kk]), T(x[col * P2 + 2 * kk + 1]));
     }
 }
 
@@ -1796,7 +1796,8 @@ int dft_lds_limits() {  // their operands may take more than 64 KiB: kDftMax wit
     const void *k[] = {(const void *)k_div_dft_x<T, 1, false>, (const void *)k_div_dft_x<T, 2, false>, (const void *)k_div_dft_x<T, 4, false>,
                        (const void *)k_div_dft_x<T, 1, true>, (const void *)k_div_dft_x<T, 2, true>, (const void *)k_div_dft_x<T, 4, true>,
                        (const void *)k_idft_x_out<T, 1>, (const void *)k_idft_x_out<T, 2>, (const void *)k_idft_x_out<T, 4>,
-                       (const void *)k_dft_y<T, 1>, (const void *)k_dft_y<T, 2>, (const void *)k_dft_y<T, 4>};
+                       (const void *)k_dft_y<T, T, 1>, (const void *)k_dft_y<T, T, 2>, (const void *)k_dft_y<T, T, 4>,
+                       (const void *)k_dft_y<T, double, 1>, (const void *)k_dft_y<T, double, 2>, (const void *)k_dft_y<T, double, 4>};
     for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024));
     return DYN_OK;
 }
@@ -1810,16 +1811,19 @@ void launch_idft_x_out(Ctx *c, const T *spec, T *out, int half) {
     else if (nt == 2) hipLaunchKernelGGL((k_idft_x_out<T, 2>), grid, blk, sh, c->stream, c->geo, spec, out, pp.ni, pp.dftx, pp.nk2, half);
     else hipLaunchKernelGGL((k_idft_x_out<T, 1>), grid, blk, sh, c->stream, c->geo, spec, out, pp.ni, pp.dftx, pp.nk2, half);
 }
-template <typename T>
-void launch_dft_y(Ctx *c, T *spec, int nrows, int sign) {
+template <typename T, typename TO>
+void launch_dft_y(Ctx *c, const T *in, TO *out, int nrows, int sign) {
     const PressurePlan &pp = c->pp;
     const int nt = dft_tiles(pp.nj, nrows, 2 * pp.nk2, pp.cus), nc = 16 * nt;
     const dim3 grid(nrows, (2 * pp.nk2 + nc - 1) / nc), blk(dft_threads(pp.nj));
     const size_t sh = dft_lds(pp.nj, nc);
-    if (nt == 4) hipLaunchKernelGGL((k_dft_y<T, 4>), grid, blk, sh, c->stream, spec, pp.nj, pp.dfty, pp.nk2, sign);
-    else if (nt == 2) hipLaunchKernelGGL((k_dft_y<T, 2>), grid, blk, sh, c->stream, spec, pp.nj, pp.dfty, pp.nk2, sign);
-    else hipLaunchKernelGGL((k_dft_y<T, 1>), grid, blk, sh, c->stream, spec, pp.nj, pp.dfty, pp.nk2, sign);
+    if (nt == 4) hipLaunchKernelGGL((k_dft_y<T, TO, 4>), grid, blk, sh, c->stream, in, out, pp.nj, pp.dfty, pp.nk2, sign);
+    else if (nt == 2) hipLaunchKernelGGL((k_dft_y<T, TO, 2>), grid, blk, sh, c->stream, in, out, pp.nj, pp.dfty, pp.nk2, sign);
+    else hipLaunchKernelGGL((k_dft_y<T, TO, 1>), grid, blk, sh, c->stream, in, out, pp.nj, pp.dfty, pp.nk2, sign);
 }
+// the 64-bit half spectrum between k_dft_y and the sweeps: behind the FP32 one in the plan's buffer
+inline size_t wide_spec_at(const PressurePlan &pp) { return ((size_t)(pp.ni / 2 + 1) * pp.nj * pp.nk2 * 8 + 15) & ~(size_t)15; }
+inline double *wide_spec(const PressurePlan &pp) { return (double *)((char *)pp.spec + wide_spec_at(pp)); }
 
 // one j transform of the three-kernel j pass over nrows kx rows: the matrix products for lengths with a
 // prime factor above 5, the power-of-two kernel when nj is a power of two and its plan fits, else the
@@ -1827,7 +1831,10 @@ void launch_dft_y(Ctx *c, T *spec, int nrows, int sign) {
 template <typename T>
 void launch_fft_y(Ctx *c, T *spec, int nrows, const Radix &ry, int sign) {
     const PressurePlan &pp = c->pp;
-    if (pp.dfty) return launch_dft_y<T>(c, spec, nrows, sign);
+    if (pp.dfty) {
+        if (sizeof(T) == 4 && sign < 0) return launch_dft_y(c, (const T *)spec, wide_spec(pp), nrows, sign);
+        return launch_dft_y(c, (const T *)spec, spec, nrows, sign);
+    }
     Radix rp{};
     const int kcp = pow2_plan48(pp.nj, rp, true) ? fft_y_pow2_chunk<T>(rp, pp.nk2) : 0;
     if (kcp > 0) {
@@ -1901,7 +1908,9 @@ int x_level_chunk(const PressurePlan &pp, const Geo &g, const Radix &rx, size_t 
 int jpass_in_use(const Ctx *c) {
     if (c->tune[DYN_TUNE_PRESSURE_JPASS]) return fused_shape(c, DYN_TUNE_PRESSURE_JPASS);
     if (c->pp.ydft) return 1;
-    return c->pp.dfty && c->pp.nj <= kDftYThree ? 2 : fused_shape(c, DYN_TUNE_PRESSURE_JPASS);
+    // (in FP32 a product along i goes with one along j, see pressure_init)
+    const bool three = c->pp.nj <= kDftYThree || (c->prec == DYN_FP32 && c->pp.dftx);
+    return c->pp.dfty && three ? 2 : fused_shape(c, DYN_TUNE_PRESSURE_JPASS);
 }
 // LDS of k_thomas_staged for tg columns; columns per block: 32 (64 running threads, one wavefront), fewer
 // where their values and pivots exceed half the LDS of a CU
@@ -1914,9 +1923,17 @@ int thomas_group(int nk2, size_t elt) {
 template <typename T, bool TR>
 void launch_thomas(Ctx *c, T *spec, int nkx) {
     const PressurePlan &pp = c->pp;
-    const int tg = thomas_group(pp.nk2, sizeof(T));
-    hipLaunchKernelGGL((k_thomas_staged<T, TR>), dim3(nkx, (pp.nj + tg - 1) / tg), dim3(kThomasThreads), thomas_lds(tg, pp.nk2, sizeof(T)),
-                       c->stream, spec, pp.nk2, thomas_args(pp, c->g.nz), tg);
+    const bool wide = sizeof(T) == 4 && pp.dfty;  // the products left the spectrum in 64 bits
+    const size_t elt = wide ? 8 : sizeof(T);
+    const int tg = thomas_group(pp.nk2, elt);
+    const dim3 grid(nkx, (pp.nj + tg - 1) / tg);
+    const size_t sh = thomas_lds(tg, pp.nk2, elt);
+    if (wide)
+        hipLaunchKernelGGL((k_thomas_staged<T, TR, double>), grid, dim3(kThomasThreads), sh, c->stream, (const double *)wide_spec(pp), spec,
+                           pp.nk2, thomas_args(pp, c->g.nz), tg);
+    else
+        hipLaunchKernelGGL((k_thomas_staged<T, TR, T>), grid, dim3(kThomasThreads), sh, c->stream, (const T *)spec, spec, pp.nk2,
+                           thomas_args(pp, c->g.nz), tg);
 }
 // the LDS-resident j pass: by matrix products where the plan has them, else by radix passes
 template <typename T, bool TR>
@@ -2190,8 +2207,9 @@ int solve_adjoint_t(Ctx *c, double step, T *pihat, T *uh, T *vh, T *wh, T *r1, T
 
 template <typename T>
 int y_lds_limits(int most) {
-    const void *k[] = {(const void *)k_ypass<T, false>, (const void *)k_ypass<T, true>, (const void *)k_thomas_staged<T, false>,
-                       (const void *)k_thomas_staged<T, true>, (const void *)k_ypass_dft<T, false>, (const void *)k_ypass_dft<T, true>};
+    const void *k[] = {(const void *)k_ypass<T, false>, (const void *)k_ypass<T, true>, (const void *)k_thomas_staged<T, false, T>,
+                       (const void *)k_thomas_staged<T, true, T>, (const void *)k_thomas_staged<T, false, double>,
+                       (const void *)k_thomas_staged<T, true, double>, (const void *)k_ypass_dft<T, false>, (const void *)k_ypass_dft<T, true>};
     for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, most));
     return DYN_OK;
 }
@@ -2223,18 +2241,9 @@ int pressure_init(Ctx *c) {
         set_error("pressure solver: twiddle upload failed");
         return DYN_E_HIP;
     }
-    auto matrices = [](int n, bool smooth, int smooth_max, double **out) -> int {
-        if (n > (smooth ? smooth_max : kDftMax)) return DYN_OK;
-        const std::vector<double> h = dft_matrices(n);
-        DYN_HIP(hipMalloc(out, sizeof(double) * h.size()));
-        DYN_HIP(hipMemcpy(*out, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
-        return DYN_OK;
-    };
-    int rc = matrices(pp.ni, pp.smooth_x, c->prec == DYN_FP32 ? dft_x_smooth<float>() : dft_x_smooth<double>(), &pp.dftx);
-    if (!rc) rc = matrices(pp.nj, pp.smooth_y, kDftYSmooth, &pp.dfty);
-    if (!rc && (pp.dftx || pp.dfty)) rc = c->prec == DYN_FP32 ? dft_lds_limits<float>() : dft_lds_limits<double>();
-    if (rc) return rc;
-    DYN_HIP(hipMalloc(&pp.spec, sizeof(double) * 2 * (size_t)pp.ni * pp.nj * pp.nk2));
+    // (on the narrowest grids the two half spectra of an FP32 context take more than the full one in 64 bits)
+    DYN_HIP(hipMalloc(&pp.spec, std::max(sizeof(double) * 2 * (size_t)pp.ni * pp.nj * pp.nk2,
+                                         wide_spec_at(pp) + sizeof(double) * 2 * (size_t)(pp.ni / 2 + 1) * pp.nj * pp.nk2)));
     int dev = 0, lds = 0;
     DYN_HIP(hipGetDevice(&dev));
     DYN_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
@@ -2248,6 +2257,30 @@ int pressure_init(Ctx *c) {
     const int nthr = f32 ? ypass_threads<float>() : ypass_threads<double>();
     const int maxb = f32 ? ypass_maxb<float>() : ypass_maxb<double>();
     pp.fused_y = pp.smooth_y && need <= pp.lds_max && 2 * pp.nj <= nthr && max_butterflies(ry, pp.nk2, nthr) <= maxb;
+    // Which sides go by matrix products: lengths with a prime factor above 5, and short smooth ones.  FP32 grids
+    // whose sides are both smooth (and even along i) take them on both sides or on neither: what a factored FP32
+    // transform loses on one side the products' 64 bits on the other don't give back (pi of 160x128x40, 6 steps,
+    // is 2 to 6e-6 off either way, 313 us a step against 314), while both together lose an order less.  Dry ones
+    // that an ensemble can hold, past 64 points a side, keep the factored passes: a member's bits are those of
+    // its run alone, and the batch, which fills the chip without them, is no faster with products (32 members
+    // of 96 to 192 points a side: 4.87 ms a step against 4.82).
+    bool prod_x = pp.ni <= (!pp.smooth_x ? kDftMax : f32 ? dft_x_smooth<float>() : dft_x_smooth<double>());
+    bool prod_y = pp.nj <= (!pp.smooth_y ? kDftMax : kDftYSmooth);
+    if (f32 && pp.smooth_x && pp.smooth_y && pp.ni % 2 == 0) {
+        const bool y_taken = prod_y && (pp.nj <= kDftYThree || !pp.fused_y);
+        const bool batched = !c->g.microphysics && fused_waves(c) == 1 && std::max(pp.ni, pp.nj) > 64;
+        prod_x = prod_y = prod_x && y_taken && !batched;
+    }
+    auto matrices = [](int n, double **out) -> int {
+        const std::vector<double> h = dft_matrices(n);
+        DYN_HIP(hipMalloc(out, sizeof(double) * h.size()));
+        DYN_HIP(hipMemcpy(*out, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
+        return DYN_OK;
+    };
+    int rc = prod_x ? matrices(pp.ni, &pp.dftx) : DYN_OK;
+    if (!rc && prod_y) rc = matrices(pp.nj, &pp.dfty);
+    if (!rc && (pp.dftx || pp.dfty)) rc = f32 ? dft_lds_limits<float>() : dft_lds_limits<double>();
+    if (rc) return rc;
     pp.ydft = pp.dfty && ypass_dft_fits(pp, 1);
     rc = f32 ? y_lds_limits<float>(lds) : y_lds_limits<double>(lds);
     if (rc) return rc;

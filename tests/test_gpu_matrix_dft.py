@@ -30,3 +30,35 @@ def test_solve_against_oracle(nx, ny, nz, precision):
     g.sync()
     a, b = g.get_field(ids.PI, 0), o.get_field(ids.PI)
     assert np.abs(a - b).max() <= (2e-4 if precision else 1e-12) * np.abs(b).max()
+
+
+# the longest smooth lengths that take the products and the next ones that don't, along i and along j, one and
+# both sides by products, and j lengths on either side of the fused j pass
+SMOOTH = [(192, 12, 9), (200, 12, 9), (384, 12, 6), (400, 12, 6), (16, 192, 9), (16, 200, 9), (18, 112, 7), (18, 120, 7), (200, 100, 8)]
+
+
+@pytest.mark.parametrize("nx,ny,nz", SMOOTH)
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "fp32"])
+def test_smooth_lengths_against_oracle(nx, ny, nz, precision):
+    test_solve_against_oracle(nx, ny, nz, precision)
+
+
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "fp32"])
+def test_ensemble_members_match_solo_runs_bitwise(precision):
+    """A batch keeps slabs in one launch that a solo run takes through three: the same bits."""
+    from model_amd.core import DynCore, Ensemble
+    sizes = [(96, 104), (112, 96), (48, 48), (31, 29), (200, 100)]
+    cases = [configs.small_case(nx=nx, ny=ny, nz=20, microphysics=0, amplitude=0.3, seed=n) for n, (nx, ny) in enumerate(sizes)]
+    solo = [DynCore(c, precision=precision) for c in cases]
+    members = [DynCore(c, precision=precision) for c in cases]
+    e = Ensemble(members)
+    e.step(2)
+    e.sync()
+    for s, m in zip(solo, members):
+        s.step(2)
+        s.sync()
+        m.sync()
+        for f in (ids.U, ids.V, ids.W, ids.TH):
+            assert np.array_equal(s.get_field(f), m.get_field(f)), ids.FIELD_NAMES[f]
+        assert np.array_equal(s.get_field(ids.PI, 0), m.get_field(ids.PI, 0))
+    e.close()
