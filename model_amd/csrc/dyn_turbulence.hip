@@ -40,6 +40,24 @@ struct TurbIn {
 
 #define IX3(i, j, k) ((long long)(i) * g.NYNZ + (long long)(j) * g.NZ + (k))
 
+// Threads take the levels of neighbouring columns one after another (kTurbThreads of them, whole columns while a
+// column fits), so that a 40-level column leaves no lanes idle, and a block stays in one i-slab: the slabs' bases
+// are scalars and one 32-bit offset per thread reaches every neighbour.  Consecutive blocks sit behind one L2.
+constexpr int kTurbThreads = 256;
+
+// a point's neighbours: at(F, di, dj, dk)
+template <typename T>
+struct Near {
+    long long slab;  // i * NYNZ
+    long long nynz;
+    int nz;
+    unsigned o;      // j * NZ + k
+    __device__ __forceinline__ T operator()(const T *F, int di, int dj, int dk) const {
+        const T *b = F + (slab + di * nynz);
+        return *(const T *)((const char *)b + (size_t)((o + (unsigned)(dj * nz + dk)) * (unsigned)sizeof(T)));
+    }
+};
+
 template <typename T>
 __device__ __forceinline__ T odz(const Geo &g, const Cols &c, int k) { return T(g.one_d_dz) * T(c.mu[k]); }
 template <typename T>
@@ -47,95 +65,124 @@ __device__ __forceinline__ T odzw(const Geo &g, const Cols &c, int k) { return T
 
 // S^2 = D11^2 + ... + D23^2, turbulence.cpp:596-624
 template <typename T>
-__device__ T deformation2(const Geo &g, const Cols &c, const TurbIn<T> &f, int i, int j, int k) {
+__device__ __forceinline__ T deformation2(const Geo &g, const Cols &c, const TurbIn<T> &f, const Near<T> &A, int k) {
     const T *UM = f.um, *VM = f.vm, *WM = f.wm, *UB = f.ub, *VB = f.vb, *WB = f.wb;
     const T odx = T(g.one_d_dx), ody = T(g.one_d_dy), dzw = odzw<T>(g, c, k);
-#define A(F, a, b, cc) F[IX3(a, b, cc)]
-    T D11 = T(0.50) * (A(UM, i + 1, j, k) + A(UM, i + 1, j, k - 1) - A(UM, i - 1, j, k) - A(UM, i - 1, j, k - 1) +
-                       A(UB, i + 1, j, k) + A(UB, i + 1, j, k - 1) - A(UB, i - 1, j, k) - A(UB, i - 1, j, k - 1)) * odx;
-    T D22 = T(0.50) * (A(VM, i, j + 1, k) + A(VM, i, j + 1, k - 1) - A(VM, i, j - 1, k) - A(VM, i, j - 1, k - 1) +
-                       A(VB, i, j + 1, k) + A(VB, i, j + 1, k - 1) - A(VB, i, j - 1, k) - A(VB, i, j - 1, k - 1)) * ody;
-    T D33 = T(1.0) * (A(WM, i, j, k + 1) - A(WM, i, j, k - 1) + A(WB, i, j, k + 1) - A(WB, i, j, k - 1)) * dzw;
-    T D12 = T(0.5) * ((A(UM, i, j + 1, k) + A(UM, i, j + 1, k - 1) - A(UM, i, j - 1, k) - A(UM, i, j - 1, k - 1) +
-                       A(UB, i, j + 1, k) + A(UB, i, j + 1, k - 1) - A(UB, i, j - 1, k) - A(UB, i, j - 1, k - 1)) * ody +
-                      (A(VM, i + 1, j, k) + A(VM, i + 1, j, k - 1) - A(VM, i - 1, j, k) - A(VM, i - 1, j, k - 1) +
-                       A(VB, i + 1, j, k) + A(VB, i + 1, j, k - 1) - A(VB, i - 1, j, k) - A(VB, i - 1, j, k - 1)) * odx);
-    T D13 = T(0.5) * ((A(UM, i, j, k) + A(UM, i + 1, j, k) - A(UM, i, j, k - 1) - A(UM, i + 1, j, k - 1) +
-                       A(UB, i, j, k) + A(UB, i + 1, j, k) - A(UB, i, j, k - 1) - A(UB, i + 1, j, k - 1)) * dzw +
-                      (A(WM, i + 1, j, k) - A(WM, i - 1, j, k) + A(WB, i + 1, j, k) - A(WB, i - 1, j, k)) * odx);
-    T D23 = T(0.5) * ((A(VM, i, j, k) + A(VM, i, j + 1, k) - A(VM, i, j, k - 1) - A(VM, i, j + 1, k - 1) +
-                       A(VB, i, j, k) + A(VB, i, j + 1, k) - A(VB, i, j, k - 1) - A(VB, i, j + 1, k - 1)) * dzw +
-                      (A(WM, i, j + 1, k) - A(WM, i, j - 1, k) + A(WB, i, j + 1, k) - A(WB, i, j - 1, k)) * ody);
-#undef A
+    T D11 = T(0.50) * (A(UM, 1, 0, 0) + A(UM, 1, 0, -1) - A(UM, -1, 0, 0) - A(UM, -1, 0, -1) +
+                       A(UB, 1, 0, 0) + A(UB, 1, 0, -1) - A(UB, -1, 0, 0) - A(UB, -1, 0, -1)) * odx;
+    T D22 = T(0.50) * (A(VM, 0, 1, 0) + A(VM, 0, 1, -1) - A(VM, 0, -1, 0) - A(VM, 0, -1, -1) +
+                       A(VB, 0, 1, 0) + A(VB, 0, 1, -1) - A(VB, 0, -1, 0) - A(VB, 0, -1, -1)) * ody;
+    T D33 = T(1.0) * (A(WM, 0, 0, 1) - A(WM, 0, 0, -1) + A(WB, 0, 0, 1) - A(WB, 0, 0, -1)) * dzw;
+    T D12 = T(0.5) * ((A(UM, 0, 1, 0) + A(UM, 0, 1, -1) - A(UM, 0, -1, 0) - A(UM, 0, -1, -1) +
+                       A(UB, 0, 1, 0) + A(UB, 0, 1, -1) - A(UB, 0, -1, 0) - A(UB, 0, -1, -1)) * ody +
+                      (A(VM, 1, 0, 0) + A(VM, 1, 0, -1) - A(VM, -1, 0, 0) - A(VM, -1, 0, -1) +
+                       A(VB, 1, 0, 0) + A(VB, 1, 0, -1) - A(VB, -1, 0, 0) - A(VB, -1, 0, -1)) * odx);
+    T D13 = T(0.5) * ((A(UM, 0, 0, 0) + A(UM, 1, 0, 0) - A(UM, 0, 0, -1) - A(UM, 1, 0, -1) +
+                       A(UB, 0, 0, 0) + A(UB, 1, 0, 0) - A(UB, 0, 0, -1) - A(UB, 1, 0, -1)) * dzw +
+                      (A(WM, 1, 0, 0) - A(WM, -1, 0, 0) + A(WB, 1, 0, 0) - A(WB, -1, 0, 0)) * odx);
+    T D23 = T(0.5) * ((A(VM, 0, 0, 0) + A(VM, 0, 1, 0) - A(VM, 0, 0, -1) - A(VM, 0, 1, -1) +
+                       A(VB, 0, 0, 0) + A(VB, 0, 1, 0) - A(VB, 0, 0, -1) - A(VB, 0, 1, -1)) * dzw +
+                      (A(WM, 0, 1, 0) - A(WM, 0, -1, 0) + A(WB, 0, 1, 0) - A(WB, 0, -1, 0)) * ody);
     return D11 * D11 + D22 * D22 + D33 * D33 + D12 * D12 + D13 * D13 + D23 * D23;
 }
 
-// Brunt-Vaisala frequency: get_Kmix_dry (turbulence.cpp:781-791), get_Kmix (:627-690)
+// What the stability of a level needs of each of the two it lies between: the virtual potential temperature,
+// and where the air is saturated the temperature and the potential temperature of the moist form (with its
+// pow and exp, so they are worth forming once a level)
 template <typename T>
-__device__ T brunt_vaisala(const Geo &g, const Cols &c, const TurbIn<T> &f, int i, int j, int k) {
-    const long long h = IX3(i, j, k), l = IX3(i, j, k - 1);
-    if (!f.moist || !f.sat[h] || !f.sat[l]) {
-        T qh = f.moist ? f.qvm[h] + f.qb[h] + T(c.qb[k]) : T(c.qb[k]);
-        T ql = f.moist ? f.qvm[l] + f.qb[l] + T(c.qb[k - 1]) : T(c.qb[k - 1]);
-        T thetaVH = (f.thm[h] + f.thb[h] + T(c.tb[k])) * (T(1) + T(0.61) * qh);
-        T thetaVL = (f.thm[l] + f.thb[l] + T(c.tb[k - 1])) * (T(1) + T(0.61) * ql);
-        T dTheta = thetaVH - thetaVL;
+struct StabilityLevel {
+    T thetav, temp, thetam;
+    int sat;
+};
+template <typename T>
+__device__ __forceinline__ StabilityLevel<T> stability_level(const Geo &g, const Cols &c, const TurbIn<T> &f, const Near<T> &A,
+                                                             long long h, int k) {
+    StabilityLevel<T> s;
+    s.sat = f.moist ? f.sat[h] : 0;
+    T qh = f.moist ? A(f.qvm, 0, 0, 0) + A(f.qb, 0, 0, 0) + T(c.qb[k]) : T(c.qb[k]);
+    T th = A(f.thm, 0, 0, 0) + A(f.thb, 0, 0, 0) + T(c.tb[k]);
+    s.thetav = th * (T(1) + T(0.61) * qh);
+    s.temp = T(0);
+    s.thetam = T(0);
+    if (s.sat) {
+        const T cp = T(kCp), Lv = T(kLv);
+        const T cpRd = T(kCp / kRd);
+        const T pbh = A(f.pb, 0, 0, 0), pih = A(f.pi, 0, 0, 0);
+        s.temp = th * (pbh + pih / (cp * T(c.tbv[k])));
+        T pd = T(kP0) * pow(pbh, cpRd) + pih * T(c.rhou[k]);
+        T esl = T(611.2) * exp(T(17.67) * (s.temp - T(273.15)) / (s.temp - T(29.65)));
+        T qvsat = T(0.62197) * esl / (pd - esl);
+        s.thetam = th * (T(1) + Lv * qvsat / (cp * s.temp));
+    }
+    return s;
+}
+
+// Brunt-Vaisala frequency: get_Kmix_dry (turbulence.cpp:781-791), get_Kmix (:627-690), from the levels k (H) and
+// k-1 (L)
+template <typename T>
+__device__ __forceinline__ T brunt_vaisala(const Geo &g, const Cols &c, const TurbIn<T> &f, const Near<T> &A, const StabilityLevel<T> &H,
+                                           const StabilityLevel<T> &L, int k) {
+    if (!H.sat || !L.sat) {
+        T dTheta = H.thetav - L.thetav;
         return T(2.0) * T(kGrav) / (T(c.tbv[k]) + T(c.tbv[k - 1])) * dTheta * odzw<T>(g, c, k);
     }
     const T cp = T(kCp), Lv = T(kLv), Rd = T(kRd), grav = T(kGrav);
-    const T cpRd = T(kCp / kRd);
-    T thetaVH = f.thm[h] + f.thb[h] + T(c.tb[k]);
-    T thetaVL = f.thm[l] + f.thb[l] + T(c.tb[k - 1]);
-    T tempH = thetaVH * (f.pb[h] + f.pi[h] / (cp * T(c.tbv[k])));
-    T tempL = thetaVL * (f.pb[l] + f.pi[l] / (cp * T(c.tbv[k - 1])));
-    T temp = T(0.5) * (tempH + tempL);
-    T dQL = f.qcm[h] + f.qrm[h] - f.qcm[l] - f.qrm[l] + f.qvm[h] - f.qvm[l] + f.qb[h] - f.qb[l] + T(c.qb[k]) - T(c.qb[k - 1]);
-    T qv = T(0.5) * (f.qvm[h] + f.qvm[l] + f.qb[h] + f.qb[l] + T(c.qb[k]) + T(c.qb[k - 1]));
-    T pdH = T(kP0) * pow(f.pb[h], cpRd) + f.pi[h] * T(c.rhou[k]);
-    T pdL = T(kP0) * pow(f.pb[l], cpRd) + f.pi[l] * T(c.rhou[k - 1]);
-    T eslH = T(611.2) * exp(T(17.67) * (tempH - T(273.15)) / (tempH - T(29.65)));
-    T eslL = T(611.2) * exp(T(17.67) * (tempL - T(273.15)) / (tempL - T(29.65)));
-    T qvsatH = T(0.62197) * eslH / (pdH - eslH);
-    T qvsatL = T(0.62197) * eslL / (pdL - eslL);
-    thetaVH = thetaVH * (T(1) + Lv * qvsatH / (cp * tempH));
-    thetaVL = thetaVL * (T(1) + Lv * qvsatL / (cp * tempL));
-    T dTheta = thetaVH - thetaVL;
+    T temp = T(0.5) * (H.temp + L.temp);
+    T dQL = A(f.qcm, 0, 0, 0) + A(f.qrm, 0, 0, 0) - A(f.qcm, 0, 0, -1) - A(f.qrm, 0, 0, -1) + A(f.qvm, 0, 0, 0) - A(f.qvm, 0, 0, -1) +
+            A(f.qb, 0, 0, 0) - A(f.qb, 0, 0, -1) + T(c.qb[k]) - T(c.qb[k - 1]);
+    T qv = T(0.5) * (A(f.qvm, 0, 0, 0) + A(f.qvm, 0, 0, -1) + A(f.qb, 0, 0, 0) + A(f.qb, 0, 0, -1) + T(c.qb[k]) + T(c.qb[k - 1]));
+    T dTheta = H.thetam - L.thetam;
     T Acoef = (grav / T(c.tbw[k])) * (T(1.0) + Lv * qv / (Rd * temp)) / (T(1.0) + T(0.622) * Lv * Lv * qv / (cp * Rd * temp * temp));
     return (Acoef * dTheta - grav * dQL) * odzw<T>(g, c, k);
 }
 
-// the vertical coefficient of level k before (raw) and after (final) its bound; levels 1 and NZ-1 are 0
+// get_Kmix / get_Kmix_dry, turbulence.cpp:563-831: one thread per level; the horizontal coefficient of level
+// k-1 is set with level k, from level k-1's final and level k's raw value (levels 1 and NZ-1 are 0).  What a
+// level hands the one above goes through LDS, so the deformation and the moist thermodynamics of a level are
+// formed once (194x100x40 FP32 38 -> 16 us, 150x126x50 FP64 95 -> 44; the rest is the 60 neighbour
+// loads of the deformation, from L1 and L2).  Columns longer than the block take several, which overlap by one level.
 template <typename T>
-__device__ void kmix_level(const Geo &g, const Cols &c, const TurbIn<T> &f, const TurbArgs &ta, int i, int j, int k, T *raw,
-                           T *final_) {
-    *raw = T(0);
-    *final_ = T(0);
-    if (k < 2 || k > g.NZ - 2) return;
-    T S2 = deformation2<T>(g, c, f, i, j, k);
-    T bruntv = brunt_vaisala<T>(g, c, f, i, j, k);
-    if (S2 - T(kPrInv) * bruntv > T(0)) {
-        T cc = T(ta.vml2[k]) * T(kCs) * T(kCs);
-        *raw = cc * sqrt(S2 - T(kPrInv) * bruntv);
-        *final_ = *raw > T(ta.vkmax[k]) ? T(ta.vkmax[k]) : *raw;
+__global__ void __launch_bounds__(kTurbThreads) k_turb_kmix(Geo g, Cols c, TurbIn<T> f, TurbArgs ta, T *__restrict__ K, T *__restrict__ KH,
+                                                            int il, int jl, int jh, int rows, int nbj, int nbk) {
+    __shared__ StabilityLevel<T> lev[kTurbThreads];
+    __shared__ T lfin[kTurbThreads];
+    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    const int kb = t % nbk, jb = t / nbk % nbj, i = t / (nbk * nbj) + il;
+    const int q = threadIdx.x, per = min(g.NZ, kTurbThreads), k0 = kb * (kTurbThreads - 1);
+    const int r = q / per, k = k0 + q - r * per, j = jl + jb * rows + r;
+    const bool in = r < rows && j < jh && k < g.NZ;
+    const Near<T> A{(long long)i * g.NYNZ, g.NYNZ, g.NZ, in ? (unsigned)(j * g.NZ + k) : 0u};
+    const long long p = A.slab + A.o;
+    StabilityLevel<T> H{};
+    if (in && k >= 1 && k <= g.NZ - 2) H = stability_level<T>(g, c, f, A, p, k);
+    lev[q] = H;
+    __syncthreads();
+    // raw and final (bounded) coefficient of level k; a block's first level has no level below in LDS: 1 has
+    // the value 0, and further up it is the overlap, whose final value is formed from memory
+    T raw = T(0), fin = T(0);
+    if (in && k >= 2 && k <= g.NZ - 2) {
+        StabilityLevel<T> L;
+        if (q > 0) {
+            L = lev[q - 1];
+        } else {
+            Near<T> B = A;
+            B.o -= 1;
+            L = stability_level<T>(g, c, f, B, p - 1, k - 1);
+        }
+        T S2 = deformation2<T>(g, c, f, A, k);
+        T bruntv = brunt_vaisala<T>(g, c, f, A, H, L, k);
+        if (S2 - T(kPrInv) * bruntv > T(0)) {
+            T cc = T(ta.vml2[k]) * T(kCs) * T(kCs);
+            raw = cc * sqrt(S2 - T(kPrInv) * bruntv);
+            fin = raw > T(ta.vkmax[k]) ? T(ta.vkmax[k]) : raw;
+        }
     }
-}
-
-// get_Kmix / get_Kmix_dry, turbulence.cpp:563-831: one thread per (i, j, k), k in [1, NZ); the
-// horizontal coefficient of level k-1 is set with level k, from level k-1's final and level k's raw value
-template <typename T>
-__global__ void __launch_bounds__(256) k_turb_kmix(Geo g, Cols c, TurbIn<T> f, TurbArgs ta, T *__restrict__ K, T *__restrict__ KH,
-                                                   int il, int jl, int jh) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int j = blockIdx.y + jl, i = blockIdx.z + il;
-    if (k >= g.NZ || j >= jh) return;
-    const long long p = IX3(i, j, k);
-    if (k == 1 || k == g.NZ - 1) {
-        K[p] = T(0);
-        return;
-    }
-    T raw, fin, rawl, finl;
-    kmix_level<T>(g, c, f, ta, i, j, k, &raw, &fin);
-    kmix_level<T>(g, c, f, ta, i, j, k - 1, &rawl, &finl);
+    lfin[q] = fin;
+    __syncthreads();
+    if (!in || k < 1 || (kb > 0 && q == 0)) return;
+    K[p] = fin;
+    if (k == 1 || k == g.NZ - 1) return;
+    const T finl = lfin[q - 1];
     const T lH = T(ta.lH);
     T kh;
     if (raw > T(0)) {
@@ -144,139 +191,138 @@ __global__ void __launch_bounds__(256) k_turb_kmix(Geo g, Cols c, TurbIn<T> f, T
     } else {
         kh = T(0) + T(0.5) * finl / T(ta.vml2[k - 1]) * lH * lH;
     }
-    K[p] = fin;
     KH[p - 1] = kh;
 }
 
-// stress components of slab i (turbulence.cpp:913-933); level 0 of tau_33, tau_13, tau_23 is zero
+// Stress components at (i + di, j + dj, k + dk) (turbulence.cpp:913-933); k is the level of the point `A` stands on,
+// level 0 of tau_33, tau_13, tau_23 is zero
 template <typename T>
-__device__ __forceinline__ T tau11(const Geo &g, const TurbIn<T> &f, int i, int j, int k) {
-    return T(2.0) * (f.um[IX3(i + 1, j, k)] - f.um[IX3(i, j, k)]) * T(g.one_d_dx);
-}
-template <typename T>
-__device__ __forceinline__ T tau22(const Geo &g, const TurbIn<T> &f, int i, int j, int k) {
-    return T(2.0) * (f.vm[IX3(i, j + 1, k)] - f.vm[IX3(i, j, k)]) * T(g.one_d_dy);
-}
-template <typename T>
-__device__ __forceinline__ T tau33(const Geo &g, const Cols &c, const TurbIn<T> &f, int i, int j, int k) {
-    return k < 1 ? T(0) : T(2.0) * (f.wm[IX3(i, j, k + 1)] - f.wm[IX3(i, j, k)]) * odz<T>(g, c, k);
-}
-template <typename T>
-__device__ __forceinline__ T tau13(const Geo &g, const Cols &c, const TurbIn<T> &f, int i, int j, int k) {
-    if (k < 1) return T(0);
-    return (f.wm[IX3(i + 1, j, k + 1)] - f.wm[IX3(i, j, k + 1)]) * T(g.one_d_dx) +
-           (f.um[IX3(i + 1, j, k + 1)] - f.um[IX3(i + 1, j, k)]) * odzw<T>(g, c, k + 1);
-}
-template <typename T>
-__device__ __forceinline__ T tau23(const Geo &g, const Cols &c, const TurbIn<T> &f, int i, int j, int k) {
-    if (k < 1) return T(0);
-    return (f.wm[IX3(i, j + 1, k + 1)] - f.wm[IX3(i, j, k + 1)]) * T(g.one_d_dy) +
-           (f.vm[IX3(i, j + 1, k + 1)] - f.vm[IX3(i, j + 1, k)]) * odzw<T>(g, c, k + 1);
-}
-template <typename T>
-__device__ __forceinline__ T tau12(const Geo &g, const TurbIn<T> &f, int i, int j, int k) {
-    return (f.um[IX3(i + 1, j + 1, k)] - f.um[IX3(i + 1, j, k)]) * T(g.one_d_dy) +
-           (f.vm[IX3(i + 1, j + 1, k)] - f.vm[IX3(i, j + 1, k)]) * T(g.one_d_dx);
-}
+struct Stress {
+    const Geo &g;
+    const Cols &c;
+    const TurbIn<T> &f;
+    const Near<T> &A;
+    int k;
+    __device__ __forceinline__ T t11(int di, int dj, int dk) const {
+        return T(2.0) * (A(f.um, di + 1, dj, dk) - A(f.um, di, dj, dk)) * T(g.one_d_dx);
+    }
+    __device__ __forceinline__ T t22(int di, int dj, int dk) const {
+        return T(2.0) * (A(f.vm, di, dj + 1, dk) - A(f.vm, di, dj, dk)) * T(g.one_d_dy);
+    }
+    __device__ __forceinline__ T t33(int dk) const {
+        return k + dk < 1 ? T(0) : T(2.0) * (A(f.wm, 0, 0, dk + 1) - A(f.wm, 0, 0, dk)) * odz<T>(g, c, k + dk);
+    }
+    __device__ __forceinline__ T t13(int di, int dj, int dk) const {
+        if (k + dk < 1) return T(0);
+        return (A(f.wm, di + 1, dj, dk + 1) - A(f.wm, di, dj, dk + 1)) * T(g.one_d_dx) +
+               (A(f.um, di + 1, dj, dk + 1) - A(f.um, di + 1, dj, dk)) * odzw<T>(g, c, k + dk + 1);
+    }
+    __device__ __forceinline__ T t23(int di, int dj, int dk) const {
+        if (k + dk < 1) return T(0);
+        return (A(f.wm, di, dj + 1, dk + 1) - A(f.wm, di, dj, dk + 1)) * T(g.one_d_dy) +
+               (A(f.vm, di, dj + 1, dk + 1) - A(f.vm, di, dj + 1, dk)) * odzw<T>(g, c, k + dk + 1);
+    }
+    __device__ __forceinline__ T t12(int di, int dj, int dk) const {
+        return (A(f.um, di + 1, dj + 1, dk) - A(f.um, di + 1, dj, dk)) * T(g.one_d_dy) +
+               (A(f.vm, di + 1, dj + 1, dk) - A(f.vm, di, dj + 1, dk)) * T(g.one_d_dx);
+    }
+};
 
-// turbulent_diffusion_velocity, turbulence.cpp:839-1020: friction tendencies of u, v, w at (i, j, k),
-// k in [1, NZ-1); the bottom flux of level 1 is the bulk surface stress (turbulence.cpp:885-907)
+// The tendencies at (i, j, k), k in [1, NZ-1), in one pass (they share the coefficients):
+//   turbulent_diffusion_velocity, turbulence.cpp:839-1020: friction of u, v, w; the bottom flux of level 1 is the
+//   bulk surface stress (turbulence.cpp:885-907);
+//   turbulent_diffusion_theta / turbulent_diffusion_scalars, turbulence.cpp:1027-1276: theta (and qv, qc, qr); no
+//   flux through the ground.
+// Bound by the neighbour loads (40 of the winds and coefficients, 7 a scalar); measured with the packed
+// lanes and the one pass against a kernel each and a wavefront a column: 194x100x40 FP32 40 -> 25 us,
+// 150x126x50 FP64 88 -> 58.
 template <typename T>
-__global__ void __launch_bounds__(256) k_turb_velocity(Geo g, Cols c, TurbIn<T> f, TurbArgs ta, const T *__restrict__ K,
-                                                       const T *__restrict__ KH, T *__restrict__ UF, T *__restrict__ VF,
-                                                       T *__restrict__ WF, int il, int jl, int jh) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int j = blockIdx.y + jl, i = blockIdx.z + il;
-    if (k >= g.NZ - 1 || j >= jh) return;
+__global__ void __launch_bounds__(kTurbThreads) k_turb_tendencies(Geo g, Cols c, TurbIn<T> f, TurbArgs ta, const T *__restrict__ K,
+                                                                  const T *__restrict__ KH, T *__restrict__ UF, T *__restrict__ VF,
+                                                                  T *__restrict__ WF, T *__restrict__ TD, T *__restrict__ QVD,
+                                                                  T *__restrict__ QCD, T *__restrict__ QRD, int il, int jl, int jh, int nbq) {
+    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    const int i = t / nbq + il;
+    const int n = g.NZ - 2, q = t % nbq * kTurbThreads + threadIdx.x;  // (row, active level) of the slab
+    const int r = q / n, j = jl + r, k = q - r * n + 1;
+    if (j >= jh) return;
+    const Near<T> A{(long long)i * g.NYNZ, g.NYNZ, g.NZ, (unsigned)(j * g.NZ + k)};
+    const Stress<T> tau{g, c, f, A, k};
+    const long long p = A.slab + A.o;
     const T odx = T(g.one_d_dx), ody = T(g.one_d_dy);
-#define KM(a, b, cc) K[IX3(a, b, cc)]
-#define KHM(a, b, cc) KH[IX3(a, b, cc)]
+    auto KM = [&](int di, int dj, int dk) -> T { return A(K, di, dj, dk); };
+    auto KHM = [&](int di, int dj, int dk) -> T { return A(KH, di, dj, dk); };
     T tau_u_zl, tau_v_zl;
     if (k == 1) {
-        const long long n = IX3(i, j, 1);
-        T wind_speed = sqrt((f.um[n] + f.ub[n]) * (f.um[n] + f.ub[n]) + (f.vm[n] + f.vb[n]) * (f.vm[n] + f.vb[n]));
-        T wind_speed_base = sqrt(f.ub[n] * f.ub[n] + f.vb[n] * f.vb[n]);
+        const T um = A(f.um, 0, 0, 0), ub = A(f.ub, 0, 0, 0), vm = A(f.vm, 0, 0, 0), vb = A(f.vb, 0, 0, 0);
+        T wind_speed = sqrt((um + ub) * (um + ub) + (vm + vb) * (vm + vb));
+        T wind_speed_base = sqrt(ub * ub + vb * vb);
         if (ta.landsea[(long long)i * g.NY + j] < 0.5) {
-            tau_u_zl = T(0.003) * (wind_speed * f.um[n] + (wind_speed - wind_speed_base) * f.ub[n]);
-            tau_v_zl = T(0.003) * (wind_speed * f.vm[n] + (wind_speed - wind_speed_base) * f.vb[n]);
+            tau_u_zl = T(0.003) * (wind_speed * um + (wind_speed - wind_speed_base) * ub);
+            tau_v_zl = T(0.003) * (wind_speed * vm + (wind_speed - wind_speed_base) * vb);
         } else {
             T drag_coef = (T(1.1e-3) + T(4.0e-5) * wind_speed);
-            tau_u_zl = drag_coef * (wind_speed * f.um[n] + (wind_speed - wind_speed_base) * f.ub[n]);
-            tau_v_zl = drag_coef * (wind_speed * f.vm[n] + (wind_speed - wind_speed_base) * f.vb[n]);
+            tau_u_zl = drag_coef * (wind_speed * um + (wind_speed - wind_speed_base) * ub);
+            tau_v_zl = drag_coef * (wind_speed * vm + (wind_speed - wind_speed_base) * vb);
         }
     } else {  // the top flux of level k-1
-        T uK13V_l = T(0.50) * (KM(i, j, k) + KM(i - 1, j, k));
-        T vK23V_l = T(0.5) * (KM(i, j, k) + KM(i, j - 1, k));
-        tau_u_zl = uK13V_l * tau13<T>(g, c, f, i - 1, j, k - 1);
-        tau_v_zl = vK23V_l * tau23<T>(g, c, f, i, j - 1, k - 1);
+        T uK13V_l = T(0.50) * (KM(0, 0, 0) + KM(-1, 0, 0));
+        T vK23V_l = T(0.5) * (KM(0, 0, 0) + KM(0, -1, 0));
+        tau_u_zl = uK13V_l * tau.t13(-1, 0, -1);
+        tau_v_zl = vK23V_l * tau.t23(0, -1, -1);
     }
-    T uK11H_h = KHM(i, j, k);
-    T uK11H_l = KHM(i - 1, j, k);
-    T uK12H_h = T(0.25) * (KHM(i, j, k) + KHM(i - 1, j, k) + KHM(i - 1, j + 1, k) + KHM(i, j + 1, k));
-    T uK12H_l = T(0.25) * (KHM(i, j - 1, k) + KHM(i - 1, j - 1, k) + KHM(i - 1, j, k) + KHM(i, j, k));
-    T uK13V_h = T(0.50) * (KM(i, j, k + 1) + KM(i - 1, j, k + 1));
-    T vK12H_h = T(0.25) * (KHM(i, j - 1, k) + KHM(i, j, k) + KHM(i + 1, j - 1, k) + KHM(i + 1, j, k));
+    T uK11H_h = KHM(0, 0, 0);
+    T uK11H_l = KHM(-1, 0, 0);
+    T uK12H_h = T(0.25) * (KHM(0, 0, 0) + KHM(-1, 0, 0) + KHM(-1, 1, 0) + KHM(0, 1, 0));
+    T uK12H_l = T(0.25) * (KHM(0, -1, 0) + KHM(-1, -1, 0) + KHM(-1, 0, 0) + KHM(0, 0, 0));
+    T uK13V_h = T(0.50) * (KM(0, 0, 1) + KM(-1, 0, 1));
+    T vK12H_h = T(0.25) * (KHM(0, -1, 0) + KHM(0, 0, 0) + KHM(1, -1, 0) + KHM(1, 0, 0));
     T vK12H_l = uK12H_l;
-    T vK22H_h = KHM(i, j, k);
-    T vK22H_l = KHM(i, j - 1, k);
-    T vK23V_h = T(0.5) * (KM(i, j, k + 1) + KM(i, j - 1, k + 1));
-    T wK13H_h = T(0.25) * (KHM(i, j, k) + KHM(i, j, k - 1) + KHM(i + 1, j, k) + KHM(i + 1, j, k - 1));
-    T wK13H_l = T(0.25) * (KHM(i, j, k) + KHM(i, j, k - 1) + KHM(i - 1, j, k) + KHM(i - 1, j, k - 1));
-    T wK23H_h = T(0.25) * (KHM(i, j, k) + KHM(i, j, k - 1) + KHM(i, j + 1, k) + KHM(i, j + 1, k - 1));
-    T wK23H_l = T(0.25) * (KHM(i, j, k) + KHM(i, j, k - 1) + KHM(i, j - 1, k) + KHM(i, j - 1, k - 1));
-    T wK33V_h = T(0.50) * (KM(i, j, k) + KM(i, j, k + 1));
-    T wK33V_l = T(0.50) * (KM(i, j, k) + KM(i, j, k - 1));
-#undef KM
-#undef KHM
-    T ufric = (uK11H_h * tau11<T>(g, f, i, j, k) - uK11H_l * tau11<T>(g, f, i - 1, j, k)) * odx +
-              (uK12H_h * tau12<T>(g, f, i - 1, j, k) - uK12H_l * tau12<T>(g, f, i - 1, j - 1, k)) * ody +
-              (uK13V_h * tau13<T>(g, c, f, i - 1, j, k) - tau_u_zl) * odz<T>(g, c, k);
-    T vfric = (vK12H_h * tau12<T>(g, f, i, j - 1, k) - vK12H_l * tau12<T>(g, f, i - 1, j - 1, k)) * odx +
-              (vK22H_h * tau22<T>(g, f, i, j, k) - vK22H_l * tau22<T>(g, f, i, j - 1, k)) * ody +
-              (vK23V_h * tau23<T>(g, c, f, i, j - 1, k) - tau_v_zl) * odz<T>(g, c, k);
-    T wfric = (wK13H_h * tau13<T>(g, c, f, i, j, k - 1) - wK13H_l * tau13<T>(g, c, f, i - 1, j, k - 1)) * odx +
-              (wK23H_h * tau23<T>(g, c, f, i, j, k - 1) - wK23H_l * tau23<T>(g, c, f, i, j - 1, k - 1)) * ody +
-              (wK33V_h * tau33<T>(g, c, f, i, j, k) - wK33V_l * tau33<T>(g, c, f, i, j, k - 1)) * odzw<T>(g, c, k);
-    const long long p = IX3(i, j, k);
+    T vK22H_h = KHM(0, 0, 0);
+    T vK22H_l = KHM(0, -1, 0);
+    T vK23V_h = T(0.5) * (KM(0, 0, 1) + KM(0, -1, 1));
+    T wK13H_h = T(0.25) * (KHM(0, 0, 0) + KHM(0, 0, -1) + KHM(1, 0, 0) + KHM(1, 0, -1));
+    T wK13H_l = T(0.25) * (KHM(0, 0, 0) + KHM(0, 0, -1) + KHM(-1, 0, 0) + KHM(-1, 0, -1));
+    T wK23H_h = T(0.25) * (KHM(0, 0, 0) + KHM(0, 0, -1) + KHM(0, 1, 0) + KHM(0, 1, -1));
+    T wK23H_l = T(0.25) * (KHM(0, 0, 0) + KHM(0, 0, -1) + KHM(0, -1, 0) + KHM(0, -1, -1));
+    T wK33V_h = T(0.50) * (KM(0, 0, 0) + KM(0, 0, 1));
+    T wK33V_l = T(0.50) * (KM(0, 0, 0) + KM(0, 0, -1));
+    T ufric = (uK11H_h * tau.t11(0, 0, 0) - uK11H_l * tau.t11(-1, 0, 0)) * odx +
+              (uK12H_h * tau.t12(-1, 0, 0) - uK12H_l * tau.t12(-1, -1, 0)) * ody +
+              (uK13V_h * tau.t13(-1, 0, 0) - tau_u_zl) * odz<T>(g, c, k);
+    T vfric = (vK12H_h * tau.t12(0, -1, 0) - vK12H_l * tau.t12(-1, -1, 0)) * odx +
+              (vK22H_h * tau.t22(0, 0, 0) - vK22H_l * tau.t22(0, -1, 0)) * ody +
+              (vK23V_h * tau.t23(0, -1, 0) - tau_v_zl) * odz<T>(g, c, k);
+    T wfric = (wK13H_h * tau.t13(0, 0, -1) - wK13H_l * tau.t13(-1, 0, -1)) * odx +
+              (wK23H_h * tau.t23(0, 0, -1) - wK23H_l * tau.t23(0, -1, -1)) * ody +
+              (wK33V_h * tau.t33(0) - wK33V_l * tau.t33(-1)) * odzw<T>(g, c, k);
     UF[p] = ufric;
     VF[p] = vfric;
     WF[p] = wfric;
-}
-
-// the top diffusive flux of level k of scalar S, turbulence.cpp:1128-1131, 1226
-template <typename T>
-__device__ __forceinline__ T scalar_top_flux(const Geo &g, const Cols &c, const T *K, const T *S, int i, int j, int k) {
-    return -T(kPrInv) * K[IX3(i, j, k + 1)] * (S[IX3(i, j, k + 1)] - S[IX3(i, j, k)]) * odzw<T>(g, c, k + 1);
-}
-
-// turbulent_diffusion_theta / turbulent_diffusion_scalars, turbulence.cpp:1027-1276: theta (and qv, qc,
-// qr) at (i, j, k), k in [1, NZ-1); no flux through the ground
-template <typename T>
-__global__ void __launch_bounds__(256) k_turb_scalars(Geo g, Cols c, TurbIn<T> f, const T *__restrict__ K, const T *__restrict__ KH,
-                                                      T *__restrict__ TD, T *__restrict__ QVD, T *__restrict__ QCD, T *__restrict__ QRD,
-                                                      int il, int jl, int jh) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int j = blockIdx.y + jl, i = blockIdx.z + il;
-    if (k >= g.NZ - 1 || j >= jh) return;
-    const T Pr = T(kPrInv), odx = T(g.one_d_dx), ody = T(g.one_d_dy);
-    const T *src[4] = {f.thm, f.qvm, f.qcm, f.qrm};
-    T *dst[4] = {TD, QVD, QCD, QRD};
-    const int nf = f.moist ? 4 : 1;
-    const long long p = IX3(i, j, k);
-    // the horizontal coefficients, shared by every scalar
-    const T KHn = T(0.5) * (Pr * KH[IX3(i, j + 1, k)] + Pr * KH[p]);
-    const T KHs = T(0.5) * (Pr * KH[p] + Pr * KH[IX3(i, j - 1, k)]);
-    const T KHe = T(0.5) * (Pr * KH[IX3(i + 1, j, k)] + Pr * KH[p]);
-    const T KHw = T(0.5) * (Pr * KH[p] + Pr * KH[IX3(i - 1, j, k)]);
-    for (int q = 0; q < nf; q++) {
-        const T *S = src[q];
-        T tau_h = scalar_top_flux<T>(g, c, K, S, i, j, k);
-        T tau_l = k == 1 ? T(0) : scalar_top_flux<T>(g, c, K, S, i, j, k - 1);
-        T t22h = -KHn * (S[IX3(i, j + 1, k)] - S[p]) * ody;
-        T t22l = -KHs * (S[p] - S[IX3(i, j - 1, k)]) * ody;
-        T t11h = -KHe * (S[IX3(i + 1, j, k)] - S[p]) * odx;
-        T t11l = -KHw * (S[p] - S[IX3(i - 1, j, k)]) * odx;
-        dst[q][p] = -((t11h - t11l) * odx + (t22h - t22l) * ody + (tau_h - tau_l) * odz<T>(g, c, k));
+    // the scalars: shared coefficients of the faces, then a flux difference each
+    const T Pr = T(kPrInv);
+    const T KHn = T(0.5) * (Pr * KHM(0, 1, 0) + Pr * KHM(0, 0, 0));
+    const T KHs = T(0.5) * (Pr * KHM(0, 0, 0) + Pr * KHM(0, -1, 0));
+    const T KHe = T(0.5) * (Pr * KHM(1, 0, 0) + Pr * KHM(0, 0, 0));
+    const T KHw = T(0.5) * (Pr * KHM(0, 0, 0) + Pr * KHM(-1, 0, 0));
+    const T KVh = -Pr * KM(0, 0, 1), KVl = -Pr * KM(0, 0, 0);
+    const T dzh = odzw<T>(g, c, k + 1), dzl = odzw<T>(g, c, k), dz = odz<T>(g, c, k);
+    auto diffuse = [&](const T *S) -> T {
+        const T s0 = A(S, 0, 0, 0);
+        // the diffusive fluxes through the top and the bottom, turbulence.cpp:1128-1131, 1226
+        T tau_h = KVh * (A(S, 0, 0, 1) - s0) * dzh;
+        T tau_l = k == 1 ? T(0) : KVl * (s0 - A(S, 0, 0, -1)) * dzl;
+        T t22h = -KHn * (A(S, 0, 1, 0) - s0) * ody;
+        T t22l = -KHs * (s0 - A(S, 0, -1, 0)) * ody;
+        T t11h = -KHe * (A(S, 1, 0, 0) - s0) * odx;
+        T t11l = -KHw * (s0 - A(S, -1, 0, 0)) * odx;
+        return -((t11h - t11l) * odx + (t22h - t22l) * ody + (tau_h - tau_l) * dz);
+    };
+    TD[p] = diffuse(f.thm);
+    if (f.moist) {
+        QVD[p] = diffuse(f.qvm);
+        QCD[p] = diffuse(f.qcm);
+        QRD[p] = diffuse(f.qrm);
     }
 }
 
@@ -353,15 +399,17 @@ int launch_diff_tend(Ctx *c, int il, int ih, int jl, int jh) {
     TurbIn<T> f = turb_inputs<T>(c);
     TurbArgs ta = turb_args(c);
     T **b = (T **)c->turb.buf;
-    const int kb = 64;
-    hipLaunchKernelGGL(k_turb_kmix<T>, grid3(c, il, ih, jl, jh, kb), dim3(kb), 0, c->stream, c->geo, c->cols, f, ta, b[TK], b[TKH], il, jl,
-                       jh);
-    DYN_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_turb_velocity<T>, grid3(c, il, ih, jl, jh, kb), dim3(kb), 0, c->stream, c->geo, c->cols, f, ta, (const T *)b[TK],
-                       (const T *)b[TKH], b[TUF], b[TVF], b[TWF], il, jl, jh);
-    DYN_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_turb_scalars<T>, grid3(c, il, ih, jl, jh, kb), dim3(kb), 0, c->stream, c->geo, c->cols, f, (const T *)b[TK],
-                       (const T *)b[TKH], b[TTD], b[TQV], b[TQC], b[TQR], il, jl, jh);
+    const int ni = ih - il, nj = jh - jl, NZ = c->g.nz;
+    {
+        const int rows = std::max(1, kTurbThreads / NZ), nbj = (nj + rows - 1) / rows;
+        const int nbk = NZ <= kTurbThreads ? 1 : (NZ - 2) / (kTurbThreads - 1) + 1;
+        hipLaunchKernelGGL(k_turb_kmix<T>, dim3((unsigned)ni * nbj * nbk), dim3(kTurbThreads), 0, c->stream, c->geo, c->cols, f, ta, b[TK],
+                           b[TKH], il, jl, jh, rows, nbj, nbk);
+        DYN_LAUNCH_CHECK();
+    }
+    const int nbq = (nj * (NZ - 2) + kTurbThreads - 1) / kTurbThreads;
+    hipLaunchKernelGGL(k_turb_tendencies<T>, dim3((unsigned)ni * nbq), dim3(kTurbThreads), 0, c->stream, c->geo, c->cols, f, ta,
+                       (const T *)b[TK], (const T *)b[TKH], b[TUF], b[TVF], b[TWF], b[TTD], b[TQV], b[TQC], b[TQR], il, jl, jh, nbq);
     DYN_LAUNCH_CHECK();
     return DYN_OK;
 }
