@@ -869,7 +869,8 @@ static int fused_step(dyn_ctx *ctx, StageHook hook = nullptr, void *arg = nullpt
     // first pass instead (2.08 -> 1.99 ms per FP64 step at 256x256x64; elsewhere neutral or slower).
     // Value 4 keeps the fork after the momentum kernel but queues (and captures) the scalar launches
     // after the solve's first pass, which measured faster for FP64 on the other grids.
-    const int streams = stage_streams(c);
+    const bool one = stage_in_one(c);
+    const int streams = one ? 1 : stage_streams(c);
     const bool two = streams >= 2, late = streams >= 3;
     // With shared roles on two streams, the copy into stage 2's output buffer runs during stage 1, on
     // the second stream after the scalar half: it reads the step's starting state and writes the spare
@@ -877,10 +878,30 @@ static int fused_step(dyn_ctx *ctx, StageHook hook = nullptr, void *arg = nullpt
     const bool copy_beside = shared && two;
     // calculate_diff_tend(1,NX-1,1,NY-1), driver_serial.cpp:194; the stage kernels add its tendencies
     if (c->turb.on) RC(turb_step_begin(c));
+    // advance_inner / microphysics_advance_inner; from shared roles the forecast role moves to the spare buffer
+    auto rotate = [&](int s) {
+        if (s == 2) return;
+        for (int f = DYN_U; f <= flast; f++) {
+            if (c->prog[f][DYN_ROLE_M] == c->prog[f][DYN_ROLE_CUR]) {
+                c->prog[f][DYN_ROLE_CUR] = c->prog[f][DYN_ROLE_P];
+                c->prog[f][DYN_ROLE_P] = c->spare[f];
+                c->spare[f] = nullptr;
+            } else {
+                std::swap(c->prog[f][DYN_ROLE_CUR], c->prog[f][DYN_ROLE_P]);
+            }
+        }
+    };
     for (int s = 0; s < 3; s++) {
         double step = steps[s];
         if (hook) RC(hook(c, s, arg));
         if (s == 1 && shared && !copy_beside) RC(device_copy_shell(c, DYN_U, flast));
+        if (one) {
+            RC(launch_fused_advect(c, step, 3, NX - 3, 3, NY - 3, kStageMomentum | kStageScalars));
+            RC(launch_solve_pressure(c, step, false));
+            RC(launch_post_stage(c, step, true, true, true, true));
+            rotate(s);
+            continue;
+        }
         RC(launch_fused_advect(c, step, 3, NX - 3, 3, NY - 3, kStageMomentum));
         ScalarHalf half{step, two, streams == 4, DYN_OK};
         if (half.recorded && hipEventRecord(c->ev_fork, c->stream) != hipSuccess) {
@@ -906,18 +927,7 @@ static int fused_step(dyn_ctx *ctx, StageHook hook = nullptr, void *arg = nullpt
         }
         RC(half.rc);
         RC(rm);
-        // advance_inner / microphysics_advance_inner; from shared roles the forecast role moves to the
-        // spare buffer
-        if (s < 2)
-            for (int f = DYN_U; f <= flast; f++) {
-                if (c->prog[f][DYN_ROLE_M] == c->prog[f][DYN_ROLE_CUR]) {
-                    c->prog[f][DYN_ROLE_CUR] = c->prog[f][DYN_ROLE_P];
-                    c->prog[f][DYN_ROLE_P] = c->spare[f];
-                    c->spare[f] = nullptr;
-                } else {
-                    std::swap(c->prog[f][DYN_ROLE_CUR], c->prog[f][DYN_ROLE_P]);
-                }
-            }
+        rotate(s);
     }
     // run_microphysics(1, NX-1, 1, NY-1); apply_boundary_condition_microphysics then
     // apply_boundary_condition (different fields, so one kernel serves both; the moisture pointers swap
@@ -1004,7 +1014,8 @@ int dyn_step_reference(dyn_ctx *ctx, int nsteps) {
 // with the M <- P copy, maps the buffers (M, current, forecast) = (a, b, c) to (b, a, c) (a shared step
 // maps (M = current, forecast, spare) = (X, Y, Z) to (Y, Z, X)); M and current then hold the same
 // values, so naming them back (a, b, c) changes nothing.  Two steps with the roles apart also restore
-// (a, b, c).  Every call of n >= 2 steps is made of runs of 6, 3 and 2 steps, each one graph of the
+// (a, b, c); an even run of steps whose stages are one launch keeps them apart, since on one stream the M <- P copy
+// costs less than the two launches of the stage-2 copy that sharing takes.  Every call of n >= 2 steps is made of runs of 6, 3 and 2 steps, each one graph of the
 // current assignment; a context keeps its assignment from call to call, and single steps (which move
 // it) run eagerly.  The three graphs of an assignment are captured together when it is first met.
 static Ctx::StepGraph *find_step_graph(Ctx *c, int steps) {
@@ -1022,11 +1033,12 @@ static int capture_step_graph(Ctx *c, int steps) {
     DYN_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     c->capturing = true;
     int rc = DYN_OK;
-    for (int n = 0; n < steps && !rc; n++) rc = fused_step(ctx, nullptr, nullptr, steps > 2 && n < steps - 1);
+    const bool share = steps > 2 && !(steps % 2 == 0 && stage_in_one(c));
+    for (int n = 0; n < steps && !rc; n++) rc = fused_step(ctx, nullptr, nullptr, share && n < steps - 1);
     c->capturing = false;
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(c->stream, &graph);
-    if (!rc && steps > 2)
+    if (!rc && share)
         for (int f = DYN_U; f <= flast; f++) std::swap(c->prog[f][DYN_ROLE_M], c->prog[f][DYN_ROLE_CUR]);
     const bool back = !memcmp(ng.key, c->prog, sizeof(ng.key));
     memcpy(c->prog, ng.key, sizeof(ng.key));

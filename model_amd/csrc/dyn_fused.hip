@@ -464,10 +464,12 @@ __device__ __forceinline__ void adv_momentum_tile(const Geo &g, const Cols &c, c
 // LDS: the pairs (theta', thetabar) ((qv, qbar), (qc, qr)) of plane i on rows j0-3 .. j0+tj+2 in a ring of two
 // slots, north faces of rows j0-1 .. j0+tj-1.  Register queues: the same fields of the own row at columns
 // i-2 .. i+3.  Own-column inputs (u at i+1, v at j+1, w, the M values) are loaded per lane.
-template <typename T, bool MOIST>
+enum { kTheta = 1, kVapour = 2, kRain = 4, kMoist = 7 };  // the fields a tile takes (kRain: qc and qr)
+template <typename T, int PARTS>
 struct ScalLds {
-    static constexpr int NP = MOIST ? 3 : 1;   // pairs
-    static constexpr int NFS = MOIST ? 4 : 1;  // face kinds
+    static constexpr int TH = PARTS & kTheta ? 1 : 0, QV = PARTS & kVapour ? 1 : 0, QC = PARTS & kRain ? 1 : 0;
+    static constexpr int NP = TH + QV + QC;       // pairs
+    static constexpr int NFS = TH + QV + 2 * QC;  // face kinds
     __host__ __device__ static constexpr size_t s(int tj, int pitch) { return 2 * 2 * NP * (size_t)(tj + 6) * pitch; }  // [slot][pair][row][k][2]
     __host__ __device__ static constexpr size_t nf(int tj, int pitch) { return NFS * (size_t)(tj + 1) * pitch; }        // [row + 1][k][face]
     // packed rows, per wavefront: w, wbar and the fall speed of its first lane for the wavefront before it; top
@@ -478,10 +480,12 @@ struct ScalLds {
 
 // TURB: apply_scalar_diffusion and apply_moisture_diffusion (turbulence.cpp:263-292) of the advected points,
 // before zero_moisture as in the reference; the boundary epilogue adds them on the rows beside the box
-template <typename T, int TJ, bool MOIST, bool PACK, bool TURB = false>
+template <typename T, int TJ, int PARTS, bool PACK, bool TURB = false>
 __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, const StageArgs &a, T step, int t, unsigned char *smem_raw) {
-    using L = ScalLds<T, MOIST>;
+    using L = ScalLds<T, PARTS>;
     constexpr int NP = L::NP, NS = 2 * NP, NFS = L::NFS;
+    constexpr bool TH = L::TH, QV = L::QV, QC = L::QC;
+    constexpr int PV = L::TH, PC = L::TH + L::QV;  // pair (and face) of qv, pair of qc and qr, face of qc
     const RowMap<TJ, PACK> map(a.tj, g.NZ);
     const int tj = map.tj, KPW = map.pitch, k = map.k, r = map.r;
     const int R = tj + 6;
@@ -505,7 +509,19 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
 
     // pair pr of a plane row at level kk
     auto SP = [&](int slot, int pr, int row, int kk) -> T * { return spl + (((slot * NP + pr) * R + row) * KPW + kk) * 2; };
-    const void *src[6] = {a.cur[3], a.bar[3], a.cur[4], a.bar[4], a.cur[5], a.cur[6]};
+    const void *src[NS];
+    if constexpr (TH) {
+        src[0] = a.cur[3];
+        src[1] = a.bar[3];
+    }
+    if constexpr (QV) {
+        src[2 * PV] = a.cur[4];
+        src[2 * PV + 1] = a.bar[4];
+    }
+    if constexpr (QC) {
+        src[2 * PC] = a.cur[5];
+        src[2 * PC + 1] = a.cur[6];
+    }
     T q[NS][6], qs[NS];  // the own row at columns i-2 .. i+3 (i-3 .. i+2 in the prologue)
 
     // plane rows: the own row comes from the queue, the six halo rows j0-3..j0-1, j0+tj..j0+tj+2 are loaded
@@ -561,14 +577,16 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
         }
         o.w0 = ld<T>(a.cur[2], p);
         o.wb0 = ld<T>(a.bar[2], p);
-        if (MOIST) o.vtt = ld<T>(a.vt, (unsigned)i * NYNZ + topoff);
+        if (QC) o.vtt = ld<T>(a.vt, (unsigned)i * NYNZ + topoff);
         if (!kLean) {
-            o.mth = ld<T>(a.mprev[3], p);
-            if (MOIST) {
+            if (TH) o.mth = ld<T>(a.mprev[3], p);
+            if (QV) {
                 o.mqv = ld<T>(a.mprev[4], p);
+                o.qbp = ld<T>(a.bar[4], p);
+            }
+            if (QC) {
                 o.mqc = ld<T>(a.mprev[5], p);
                 o.mqr = ld<T>(a.mprev[6], p);
-                o.qbp = ld<T>(a.bar[4], p);
             }
         }
     };
@@ -588,10 +606,12 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
     // outside the active levels, which never use the values.
     const T tbu = T(c.tb[kp1]) - T(c.tb[kc]), tbd = T(c.tb[kc]) - T(c.tb[km1]);
     T qbu = T(0), qbd = T(0), qbk = T(0), rk = T(1), vtden = T(0);
-    if (MOIST) {
+    if (QV) {
         qbu = T(c.qb[kp1]) - T(c.qb[kc]);
         qbd = T(c.qb[kc]) - T(c.qb[km1]);
         qbk = T(c.qb[kc]);
+    }
+    if (QC) {
         rk = T(c.rhou[kc]);
         vtden = sqrt(T(c.rhou[1]) / rk);
     }
@@ -611,16 +631,22 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
 
     // east faces (s_east; fluxes.cpp:797-1032) of the queue's centre column with u, ubar at the column east of it
     auto east_faces = [&](T U1, T UB1, T *e) {
-        T se = i5(q[0][0], q[0][1], q[0][2], q[0][3], q[0][4], q[0][5], sgn(UB1 + U1));
-        T be = i5(q[1][0], q[1][1], q[1][2], q[1][3], q[1][4], q[1][5], sgn(U1));
-        e[0] = U1 * be + (UB1 + U1) * se;
-        if constexpr (MOIST) {
-            T sv = i5(q[2][0], q[2][1], q[2][2], q[2][3], q[2][4], q[2][5], sgn(UB1 + U1));
-            T bv = i5(q[3][0], q[3][1], q[3][2], q[3][3], q[3][4], q[3][5], sgn(U1));
-            e[1] = U1 * bv + (UB1 + U1) * sv;
-            T ub = UB1 + U1;
-            e[2] = ub * i5(q[4][0], q[4][1], q[4][2], q[4][3], q[4][4], q[4][5], sgn(ub));
-            e[3] = ub * i5(q[5][0], q[5][1], q[5][2], q[5][3], q[5][4], q[5][5], sgn(ub));
+        const T ub = UB1 + U1;
+        if constexpr (TH) {
+            T se = i5(q[0][0], q[0][1], q[0][2], q[0][3], q[0][4], q[0][5], sgn(ub));
+            T be = i5(q[1][0], q[1][1], q[1][2], q[1][3], q[1][4], q[1][5], sgn(U1));
+            e[0] = U1 * be + ub * se;
+        }
+        if constexpr (QV) {
+            constexpr int f = 2 * PV;
+            T sv = i5(q[f][0], q[f][1], q[f][2], q[f][3], q[f][4], q[f][5], sgn(ub));
+            T bv = i5(q[f + 1][0], q[f + 1][1], q[f + 1][2], q[f + 1][3], q[f + 1][4], q[f + 1][5], sgn(U1));
+            e[PV] = U1 * bv + ub * sv;
+        }
+        if constexpr (QC) {
+            constexpr int f = 2 * PC;
+            e[PC] = ub * i5(q[f][0], q[f][1], q[f][2], q[f][3], q[f][4], q[f][5], sgn(ub));
+            e[PC + 1] = ub * i5(q[f + 1][0], q[f + 1][1], q[f + 1][2], q[f + 1][3], q[f + 1][4], q[f + 1][5], sgn(ub));
         }
     };
     T west[NFS], east[NFS];
@@ -642,11 +668,11 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
     T vtk = T(0);
     auto publish_w = [&]() {
         if constexpr (PACK) {
-            if (MOIST) vtk = fall(q[NS - 1][2], cc.vtt);
+            if (QC) vtk = fall(q[NS - 1][2], cc.vtt);
             if (map.lane == 0) {
                 xw[3 * map.wave] = cc.w0;
                 xw[3 * map.wave + 1] = cc.wb0;
-                if (MOIST) xw[3 * map.wave + 2] = vtk;
+                if (QC) xw[3 * map.wave + 2] = vtk;
             }
         }
     };
@@ -667,7 +693,7 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
         T td[NFS] = {};
         if (TURB) {
 #pragma unroll
-            for (int f = 0; f < NFS; f++) td[f] = ld<T>(a.tend[3 + f], p);
+            for (int f = 0; f < NFS; f++) td[f] = ld<T>(a.tend[(TH ? 3 : QV ? 4 : 5) + f], p);
         }
         if (more) {
 #pragma unroll
@@ -677,12 +703,14 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
         }
         T mth = cc.mth, mqv = cc.mqv, mqc = cc.mqc, mqr = cc.mqr, qbp = cc.qbp;
         if (kLean) {
-            mth = ld<T>(a.mprev[3], p);
-            if (MOIST) {
+            if (TH) mth = ld<T>(a.mprev[3], p);
+            if (QV) {
                 mqv = ld<T>(a.mprev[4], p);
+                qbp = ld<T>(a.bar[4], p);
+            }
+            if (QC) {
                 mqc = ld<T>(a.mprev[5], p);
                 mqr = ld<T>(a.mprev[6], p);
-                qbp = ld<T>(a.bar[4], p);
             }
         }
 
@@ -694,28 +722,32 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
 #pragma unroll
                 for (int d = 0; d < 6; d++) lds_ld2(SP(c0, pr, RR - 2 + d, k), x[d], y[d]);
             };
-            rows(0);
-            T sn = i5(x[0], x[1], x[2], x[3], x[4], x[5], sgn(VB1 + V1));
-            T bn = i5(y[0], y[1], y[2], y[3], y[4], y[5], sgn(V1));
-            nf[0] = V1 * bn + (VB1 + V1) * sn;
-            if constexpr (MOIST) {
-                rows(1);
-                T sv = i5(x[0], x[1], x[2], x[3], x[4], x[5], sgn(VB1 + V1));
+            const T vb = VB1 + V1;
+            if constexpr (TH) {
+                rows(0);
+                T sn = i5(x[0], x[1], x[2], x[3], x[4], x[5], sgn(vb));
+                T bn = i5(y[0], y[1], y[2], y[3], y[4], y[5], sgn(V1));
+                nf[0] = V1 * bn + vb * sn;
+            }
+            if constexpr (QV) {
+                rows(PV);
+                T sv = i5(x[0], x[1], x[2], x[3], x[4], x[5], sgn(vb));
                 T bv = i5(y[0], y[1], y[2], y[3], y[4], y[5], sgn(V1));
-                nf[1] = V1 * bv + (VB1 + V1) * sv;
-                T vb = VB1 + V1;
-                rows(2);
-                nf[2] = vb * i5(x[0], x[1], x[2], x[3], x[4], x[5], sgn(vb));
-                nf[3] = vb * i5(y[0], y[1], y[2], y[3], y[4], y[5], sgn(vb));
+                nf[PV] = V1 * bv + vb * sv;
+            }
+            if constexpr (QC) {
+                rows(PC);
+                nf[PC] = vb * i5(x[0], x[1], x[2], x[3], x[4], x[5], sgn(vb));
+                nf[PC + 1] = vb * i5(y[0], y[1], y[2], y[3], y[4], y[5], sgn(vb));
             }
         };
         auto put_faces = [&](int row, const T *nf) {
             T *o = nface + (row * KPW + k) * NFS;
-            if constexpr (MOIST) {
-                lds_st2(o, nf[0], nf[1]);
-                lds_st2(o + 2, nf[2], nf[3]);
-            } else {
+            if constexpr (NFS == 1) {
                 o[0] = nf[0];
+            } else {
+                lds_st2(o, nf[0], nf[1]);
+                if constexpr (NFS == 4) lds_st2(o + 2, nf[2], nf[3]);
             }
         };
         T nf[NFS];
@@ -729,12 +761,12 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
         // top faces (s_top) of this level from the own column of the plane; w, wbar (and the fall speed) at
         // k+1 by lane exchange
         T W1 = lane_next(cc.w0), WB1 = lane_next(cc.wb0);
-        if (MOIST && !PACK) vtk = fall(q[NS - 1][2], cc.vtt);
-        T vk1 = MOIST ? lane_next(vtk) : T(0);
+        if (QC && !PACK) vtk = fall(q[NS - 1][2], cc.vtt);
+        T vk1 = QC ? lane_next(vtk) : T(0);
         if (PACK && map.lane == KP - 1) {  // (past the block's last wavefront: words no lane uses)
             W1 = xw[3 * map.wave + 3];
             WB1 = xw[3 * map.wave + 4];
-            if (MOIST) vk1 = xw[3 * map.wave + 5];
+            if (QC) vk1 = xw[3 * map.wave + 5];
         }
         // the pair's fields at levels k-1 .. k+2 of the own column
         T x[4], y[4];
@@ -757,15 +789,15 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
             return W1 * bt + (WB1 + W1) * st_;
         };
         T tf[NFS];
-        tf[0] = s_top(0);
+        if constexpr (TH) tf[0] = s_top(0);
+        if constexpr (QV) tf[PV] = s_top(PV);
         T qrt = T(0);
-        if constexpr (MOIST) {
-            tf[1] = s_top(1);
-            column(2);
+        if constexpr (QC) {
+            column(PC);
             {
                 T wb = WB1 + W1;
                 T tq = low ? i2(x[1], x[2]) : i3(x[0], x[1], x[2], x[3], sgn(wb));
-                tf[2] = wb * tq;
+                tf[PC] = wb * tq;
             }
             // rain top face with the fall speed (fluxes.cpp:734, 780; 966-1030); level 0 falls as level 1 does
             if (k == 0) {
@@ -784,10 +816,10 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
             for (int f = 0; f < NFS; f++) tf[f] = T(0);
         }
         T bot[NFS];
-        constexpr int NB = MOIST ? 3 : 1;  // top faces handed up (rain has its own)
+        constexpr int NB = NP;  // top faces handed up (rain has its own)
 #pragma unroll
         for (int f = 0; f < NB; f++) bot[f] = lane_prev(tf[f]);
-        T qrb = MOIST ? lane_prev(qrt) : T(0);
+        T qrb = QC ? lane_prev(qrt) : T(0);
         if (PACK && map.lane == KP - 1) {
 #pragma unroll
             for (int f = 0; f < NB; f++) xb[(NFS + 1) * map.wave + f] = tf[f];
@@ -797,49 +829,47 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
         if (PACK && map.lane == 0 && map.wave > 0) {
 #pragma unroll
             for (int f = 0; f < NB; f++) bot[f] = xb[(NFS + 1) * (map.wave - 1) + f];
-            if (MOIST) qrb = xb[(NFS + 1) * (map.wave - 1) + NFS];
+            if (QC) qrb = xb[(NFS + 1) * (map.wave - 1) + NFS];
         }
         const T vtk0 = vtk;  // this column's fall speed, stored below
         T oth = T(0), oqv = T(0), oqc = T(0), oqr = T(0);  // this level's final values (active levels)
         if (active) {
             T south[4];
             const T *so = nface + (r * KPW + k) * NFS;
-            if constexpr (MOIST) {
-                lds_ld2(so, south[0], south[1]);
-                lds_ld2(so + 2, south[2], south[3]);
-            } else {
+            if constexpr (NFS == 1) {
                 south[0] = so[0];
+            } else {
+                lds_ld2(so, south[0], south[1]);
+                if constexpr (NFS == 4) lds_ld2(so + 2, south[2], south[3]);
             }
             // Z_ADVECT_BASE (advection.cpp:16-18) with the base-state differences du = b[k+1] - b[k],
             // dd = b[k] - b[k-1] of this level
             auto zbase = [&](T du, T dd) -> T { return (T(0.50) * (rw1 * W1 * du + rw0 * cc.w0 * dd) * odr); };
-            {  // theta (advection.cpp:152-168)
+            if constexpr (TH) {  // theta (advection.cpp:152-168)
                 T tend = -dtx * (east[0] - west[0]) - dty * (nf[0] - south[0]) - DTZ * (rw1 * tf[0] - rw0 * bot[0]) * odr -
                          DTZ * zbase(tbu, tbd);
                 oth = mth + step * tend;
                 if (TURB) oth += td[0] * step * T(g.dt);
             }
-            if constexpr (MOIST) {  // advection.cpp:197-253
-                T tq = -dtx * (east[1] - west[1]) - dty * (nf[1] - south[1]) - DTZ * (rw1 * tf[1] - rw0 * bot[1]) * odr -
+            const T tdt = step * T(g.dt);
+            if constexpr (QV) {  // advection.cpp:197-253, then zero_moisture for the advected points (microphysics.cpp:677-698)
+                T tq = -dtx * (east[PV] - west[PV]) - dty * (nf[PV] - south[PV]) - DTZ * (rw1 * tf[PV] - rw0 * bot[PV]) * odr -
                        DTZ * zbase(qbu, qbd);
-                T qv = mqv + step * tq;
-                T tc = -dtx * (east[2] - west[2]) - dty * (nf[2] - south[2]) - DTZ * (rw1 * tf[2] - rw0 * bot[2]) * odr;
-                T qc = mqc + step * tc;
-                T tr = -dtx * (east[3] - west[3]) - dty * (nf[3] - south[3]) - DTZ * (rw1 * qrt - rw0 * qrb) * odr;
-                T qrv = mqr + step * tr;
+                oqv = mqv + step * tq;
+                if (TURB) oqv += td[PV] * tdt;
+                if (oqv + qbp + qbk < T(0)) oqv = -(qbp + qbk);
+            }
+            if constexpr (QC) {
+                T tc = -dtx * (east[PC] - west[PC]) - dty * (nf[PC] - south[PC]) - DTZ * (rw1 * tf[PC] - rw0 * bot[PC]) * odr;
+                oqc = mqc + step * tc;
+                T tr = -dtx * (east[PC + 1] - west[PC + 1]) - dty * (nf[PC + 1] - south[PC + 1]) - DTZ * (rw1 * qrt - rw0 * qrb) * odr;
+                oqr = mqr + step * tr;
                 if (TURB) {
-                    const T tdt = step * T(g.dt);
-                    qv += td[1] * tdt;
-                    qc += td[2] * tdt;
-                    qrv += td[3] * tdt;
+                    oqc += td[PC] * tdt;
+                    oqr += td[PC + 1] * tdt;
                 }
-                // zero_moisture for the advected points (microphysics.cpp:677-698)
-                if (qc < T(0)) qc = T(0);
-                if (qrv < T(0)) qrv = T(0);
-                if (qv + qbp + qbk < T(0)) qv = -(qbp + qbk);
-                oqv = qv;
-                oqc = qc;
-                oqr = qrv;
+                if (oqc < T(0)) oqc = T(0);
+                if (oqr < T(0)) oqr = T(0);
             }
         }
         // With its own level, the lane of level 1 (NZ-2) writes the lid of upper_lower_boundaries
@@ -850,9 +880,9 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
         const bool lid = active && (k == 1 || k == NZ - 2) && i >= 6 && i < g.NX - 6;
         auto store_column = [&]() {
             if (active) {
-                st<T>(a.out[3], p, oth);
-                if (MOIST) {
-                    st<T>(a.out[4], p, oqv);
+                if (TH) st<T>(a.out[3], p, oth);
+                if (QV) st<T>(a.out[4], p, oqv);
+                if (QC) {
                     st<T>(a.out[5], p, oqc);
                     st<T>(a.out[6], p, oqr);
                     st<T>(a.vt, p, vtk0);
@@ -861,9 +891,9 @@ __device__ __forceinline__ void adv_scalars_tile(const Geo &g, const Cols &c, co
             }
             if (lid) {
                 const unsigned pl = k == 1 ? p - 1 : p + 1;
-                st<T>(a.out[3], pl, oth);
-                if (MOIST) {
-                    st<T>(a.out[4], pl, oqv);
+                if (TH) st<T>(a.out[3], pl, oth);
+                if (QV) st<T>(a.out[4], pl, oqv);
+                if (QC) {
                     st<T>(a.out[5], pl, oqc);
                     st<T>(a.out[6], pl, oqr);
                 }
@@ -904,10 +934,49 @@ __global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_adv_momentum(Ge
     adv_momentum_tile<T, TJ, MOIST, PACK, TURB>(g, c, a, step, xcd_tile(blockIdx.x, gridDim.x), smem_raw);
 }
 
+// Blocks per tile of the scalar kernel.  Moist FP64 tiles go in two: theta and qv, qc and qr.  All four fields
+// at once take more than the 256 registers that two wavefronts per SIMD leave each, and their scratch reloads wait
+// behind the prefetch; halves need 199 and half the LDS, and read the winds twice (neighbouring blocks, so mostly
+// from L2).  One block, two, three (theta, qv, qc with qr) at 256x256x64: 292, 222, 246 us; 150x126x50: 74, 58, 70;
+// 160x120x90: 169, 116, 135.  FP32 keeps one: it fits, with three wavefronts per SIMD.
+template <typename T, bool MOIST>
+constexpr int scalar_parts() { return MOIST && sizeof(T) == 8 ? 2 : 1; }
+template <typename T, bool MOIST>
+constexpr size_t scalar_lds(int tj, int pitch) {
+    if (!MOIST) return ScalLds<T, kTheta>::bytes(tj, pitch);
+    return scalar_parts<T, MOIST>() == 1 ? ScalLds<T, kMoist>::bytes(tj, pitch) : ScalLds<T, (kTheta | kVapour)>::bytes(tj, pitch);
+}
+// tile t of the scalar half, counted over the parts
+template <typename T, int TJ, bool MOIST, bool PACK, bool TURB>
+__device__ __forceinline__ void adv_scalars_any(const Geo &g, const Cols &c, const StageArgs &a, T step, int t, unsigned char *smem_raw) {
+    if constexpr (!MOIST) {
+        adv_scalars_tile<T, TJ, kTheta, PACK, TURB>(g, c, a, step, t, smem_raw);
+    } else if constexpr (scalar_parts<T, MOIST>() == 1) {
+        adv_scalars_tile<T, TJ, kMoist, PACK, TURB>(g, c, a, step, t, smem_raw);
+    } else {
+        if (t % 2) adv_scalars_tile<T, TJ, kTheta | kVapour, PACK, TURB>(g, c, a, step, t / 2, smem_raw);
+        else adv_scalars_tile<T, TJ, kRain, PACK, TURB>(g, c, a, step, t / 2, smem_raw);
+    }
+}
 template <typename T, int TJ, bool MOIST, bool PACK, bool TURB>
 __global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_adv_scalars(Geo g, Cols c, StageArgs a, T step) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    adv_scalars_tile<T, TJ, MOIST, PACK, TURB>(g, c, a, step, xcd_tile(blockIdx.x, gridDim.x), smem_raw);
+    adv_scalars_any<T, TJ, MOIST, PACK, TURB>(g, c, a, step, xcd_tile(blockIdx.x, gridDim.x), smem_raw);
+}
+
+// Both halves of a stage in one launch, for grids whose blocks are all on the device at once: the momentum tiles
+// (nm of them), then the scalar tiles with their march length.  Small grids' steps are a chain of launches of 5 to
+// 20 us; a second stream beside it costs a fork and a join of about 8 us each.
+template <typename T, int TJ, bool MOIST, bool PACK, bool TURB>
+__global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_adv_stage(Geo g, Cols c, StageArgs a, T step, int nm, int ti_scal) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int b = blockIdx.x;
+    if (b < nm) {
+        adv_momentum_tile<T, TJ, MOIST, PACK, TURB>(g, c, a, step, xcd_tile(b, nm), smem_raw);
+    } else {
+        a.ti = ti_scal;
+        adv_scalars_any<T, TJ, MOIST, PACK, TURB>(g, c, a, step, xcd_tile(b - nm, gridDim.x - nm), smem_raw);
+    }
 }
 
 // zero_moisture outside the advected box (the fused kernel clips the points it writes)
@@ -928,6 +997,10 @@ __global__ void k_zero_moisture_shell(Geo g, Cols c, T *__restrict__ QVP, T *__r
         if (QVP[p] + QB[p] + T(c.qb[k]) < T(0)) QVP[p] = -(QB[p] + T(c.qb[k]));
     }
 }
+
+// Lanes of packed rows (see RowMap) unless a 64-lane wavefront is nearly full: at 57 levels and more a row
+// per wavefront wastes at most one lane in nine and needs no exchange at wavefront edges
+bool stage_packs(const Ctx *c) { return c->g.nz < 57 || c->g.nz > KP; }
 
 // shape: rows per block, march length and lane mapping of one launch
 template <typename T, int TJ, bool MOIST, bool PACK, bool TURB>
@@ -954,8 +1027,26 @@ int scalars_t(Ctx *c, const StageArgs &a0, T step, const StageShape &sh) {
     const int nbi = (a.ih - a.il + sh.ti - 1) / sh.ti;
     const dim3 blk = PACK ? dim3((sh.tj * c->geo.NZ + KP - 1) / KP * KP) : dim3(KP, TJ);
     Timed _t(c, "adv_scalars", (double)(a.ih - a.il) * (a.jh - a.jl) * (c->geo.NZ - 2));
-    hipLaunchKernelGGL((k_adv_scalars<T, TJ, MOIST, PACK, TURB>), dim3(a.nbj * nbi), blk,
-                       (ScalLds<T, MOIST>::bytes(sh.tj, PACK ? c->geo.NZ : KP)), c->stream, c->geo, c->cols, a, step);
+    hipLaunchKernelGGL((k_adv_scalars<T, TJ, MOIST, PACK, TURB>), dim3(a.nbj * nbi * scalar_parts<T, MOIST>()), blk,
+                       (scalar_lds<T, MOIST>(sh.tj, PACK ? c->geo.NZ : KP)), c->stream, c->geo, c->cols, a, step);
+    DYN_LAUNCH_CHECK();
+    return DYN_OK;
+}
+
+template <typename T, int TJ, bool MOIST, bool PACK, bool TURB>
+int stage_one_t(Ctx *c, const StageArgs &a0, T step, const StageOne &sh) {
+    StageArgs a = a0;
+    a.ti = sh.ti_mom;
+    a.tj = sh.tj;
+    a.nbj = (a.jh - a.jl + sh.tj - 1) / sh.tj;
+    const int nm = a.nbj * ((a.ih - a.il + sh.ti_mom - 1) / sh.ti_mom);
+    const int ns = a.nbj * ((a.ih - a.il + sh.ti_scal - 1) / sh.ti_scal) * scalar_parts<T, MOIST>();
+    const int pitch = PACK ? c->geo.NZ : KP;
+    const dim3 blk = PACK ? dim3((sh.tj * c->geo.NZ + KP - 1) / KP * KP) : dim3(KP, TJ);
+    Timed _t(c, "adv_stage", (double)(a.ih - a.il) * (a.jh - a.jl) * (c->geo.NZ - 2));
+    hipLaunchKernelGGL((k_adv_stage<T, TJ, MOIST, PACK, TURB>), dim3(nm + ns), blk,
+                       (std::max(MomLds<T>::bytes(sh.tj, pitch), scalar_lds<T, MOIST>(sh.tj, pitch))), c->stream, c->geo, c->cols, a, step,
+                       nm, sh.ti_scal);
     DYN_LAUNCH_CHECK();
     return DYN_OK;
 }
@@ -978,6 +1069,17 @@ int stage_t(Ctx *c, double step, int il, int ih, int jl, int jh, int parts) {
     a.ih = ih;
     a.jl = jl;
     a.jh = jh;
+    if (parts == (kStageMomentum | kStageScalars) && stage_in_one(c)) {
+        const StageOne &m = c->auto_one;
+        if (stage_packs(c)) {
+            if (m.tj >= 6) return stage_one_t<T, 8, MOIST, true, TURB>(c, a, T(step), m);
+            if (m.tj >= 3) return stage_one_t<T, 4, MOIST, true, TURB>(c, a, T(step), m);
+            return stage_one_t<T, 2, MOIST, true, TURB>(c, a, T(step), m);
+        }
+        if (m.tj == 2) return stage_one_t<T, 2, MOIST, false, TURB>(c, a, T(step), m);
+        if (m.tj == 4) return stage_one_t<T, 4, MOIST, false, TURB>(c, a, T(step), m);
+        return stage_one_t<T, 8, MOIST, false, TURB>(c, a, T(step), m);
+    }
     int rc = DYN_OK;
     if (parts & kStageMomentum) {
         const StageShape m = stage_shape(c, true);
@@ -1206,12 +1308,9 @@ inline ShellCols shell_cols(const Ctx *c) {
     s.total = (s.rl + s.rh) * ni + s.ncb * s.nb;
     return s;
 }
-template <typename T, bool MOIST>
-__global__ void __launch_bounds__(256) k_post_scalars_shell(Geo g, Cols c, PostArgs a, bool clip, ShellCols s) {
-    const int item = blockIdx.x * blockDim.y + threadIdx.y;
-    if (item >= s.total) return;
+__device__ __forceinline__ bool shell_item(const Geo &g, const ShellCols &s, int item, int &j, int &isrc) {
+    if (item >= s.total) return false;
     const int na = (s.rl + s.rh) * s.ni;
-    int j, isrc;
     if (item < na) {
         const int r = item / s.ni;
         isrc = 3 + item % s.ni;
@@ -1221,7 +1320,27 @@ __global__ void __launch_bounds__(256) k_post_scalars_shell(Geo g, Cols c, PostA
         j = s.rl + q % s.nb;
         isrc = s.ni <= 6 ? 3 + cb : (cb < 3 ? 3 + cb : g.NX - 6 + (cb - 3));
     }
-    post_scalars_col<T, MOIST>(g, c, a, clip, false, j, isrc);
+    return true;
+}
+template <typename T, bool MOIST>
+__global__ void __launch_bounds__(256) k_post_scalars_shell(Geo g, Cols c, PostArgs a, bool clip, ShellCols s) {
+    int j, isrc;
+    if (shell_item(g, s, blockIdx.x * blockDim.y + threadIdx.y, j, isrc)) post_scalars_col<T, MOIST>(g, c, a, clip, false, j, isrc);
+}
+
+// Both in one launch: nu blocks of u, v, w, then the scalars' shell (shell: the items of s) or every column
+template <typename T, bool MOIST>
+__global__ void __launch_bounds__(256) k_post_all(Geo g, Cols c, PostArgs a, T step, bool pgf, int nu, bool clip, bool shell, ShellCols s) {
+    const int nbj = (g.NY + blockDim.y - 1) / blockDim.y;
+    int b = blockIdx.x;
+    if (b < nu) {
+        post_uvw_col<T>(g, c, a, step, pgf, b % nbj, b / nbj + 3);
+        return;
+    }
+    b -= nu;
+    int j, isrc;
+    if (!shell) post_scalars_col<T, MOIST>(g, c, a, clip, true, b % nbj * blockDim.y + threadIdx.y, b / nbj + 3);
+    else if (shell_item(g, s, b * blockDim.y + threadIdx.y, j, isrc)) post_scalars_col<T, MOIST>(g, c, a, clip, false, j, isrc);
 }
 
 // ---- batched over the members of an ensemble: one block per work item of the concatenated work list ----
@@ -1274,7 +1393,7 @@ __global__ void __launch_bounds__(KP *TJ) k_ens_scalars(const EnsMember *mem, in
     const int item = blockIdx.x;
     const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::scal0)];
     const StageArgs a = ens_stage_args(e, ro, TJ, ti, e.nbj_scal);
-    adv_scalars_tile<T, TJ, MOIST, PACK>(e.g, e.c, a, step, item - e.scal0, smem_raw);
+    adv_scalars_tile<T, TJ, kTheta, PACK>(e.g, e.c, a, step, item - e.scal0, smem_raw);
 }
 
 template <typename T>
@@ -1330,6 +1449,18 @@ int post_t(Ctx *c, double step, bool pgf, bool scalars, bool clip, bool uvw, int
     // one wavefront per column, two when NZ > 64; 256 threads per block
     const int kw = c->g.nz > KP ? 2 : 1, rows = 4 / kw;
     dim3 blk(KP * kw, rows), grd((c->g.ny + rows - 1) / rows, c->g.nx - 6);
+    if (uvw && scalars && stage_in_one(c)) {
+        Timed _t(c, "post_all", (double)c->npts);
+        const bool shell = pgf || interior_done;
+        const ShellCols sc = shell_cols(c);
+        const int nu = grd.x * grd.y, ns = shell ? (sc.total + rows - 1) / rows : nu;
+        if (c->g.microphysics)
+            hipLaunchKernelGGL((k_post_all<T, true>), dim3(nu + ns), blk, 0, c->stream, c->geo, c->cols, a, T(step), pgf, nu, clip, shell, sc);
+        else
+            hipLaunchKernelGGL((k_post_all<T, false>), dim3(nu + ns), blk, 0, c->stream, c->geo, c->cols, a, T(step), pgf, nu, clip, shell, sc);
+        DYN_LAUNCH_CHECK();
+        return DYN_OK;
+    }
     if (uvw) {
         Timed _t(c, "post_uvw", (double)c->npts);
         hipLaunchKernelGGL(k_post_uvw<T>, grd, blk, 0, c->stream, c->geo, c->cols, a, T(step), pgf);
@@ -1376,8 +1507,8 @@ namespace {
 size_t stage_lds(const Ctx *c, bool momentum, int tj, int pitch) {
     const bool moist = c->g.microphysics != 0;
     if (c->prec == DYN_FP32)
-        return momentum ? MomLds<float>::bytes(tj, pitch) : moist ? ScalLds<float, true>::bytes(tj, pitch) : ScalLds<float, false>::bytes(tj, pitch);
-    return momentum ? MomLds<double>::bytes(tj, pitch) : moist ? ScalLds<double, true>::bytes(tj, pitch) : ScalLds<double, false>::bytes(tj, pitch);
+        return momentum ? MomLds<float>::bytes(tj, pitch) : moist ? scalar_lds<float, true>(tj, pitch) : scalar_lds<float, false>(tj, pitch);
+    return momentum ? MomLds<double>::bytes(tj, pitch) : moist ? scalar_lds<double, true>(tj, pitch) : scalar_lds<double, false>(tj, pitch);
 }
 }  // namespace
 
@@ -1454,10 +1585,6 @@ int fused_shape(const Ctx *c, int param) {
 }
 
 namespace {
-// Lanes of packed rows (see RowMap) unless a 64-lane wavefront is nearly full: at 57 levels and more a row
-// per wavefront wastes at most one lane in nine and needs no exchange at wavefront edges
-bool stage_packs(const Ctx *c) { return c->g.nz < 57 || c->g.nz > KP; }
-
 // Modelled microseconds of a stage kernel's launch with tj rows and ti columns per block.  A block marches
 // ti columns after a prologue worth about one more; a column takes `lat` while few wavefronts share a SIMD
 // (the march is a chain of barriers and loads) and `issue` for each wavefront on the fullest SIMD once
@@ -1474,14 +1601,14 @@ struct StageCost {
 StageCost stage_cost(const Ctx *c, bool momentum) {
     const bool f32 = c->prec == DYN_FP32, moist = c->g.microphysics != 0;
     if (momentum) return f32 ? StageCost{1.65, 0.70, 4} : StageCost{2.15, 1.40, 2};
-    if (moist) return f32 ? StageCost{2.70, 1.00, 3} : StageCost{5.30, 3.00, 2};
+    if (moist) return f32 ? StageCost{2.70, 1.00, 3} : StageCost{1.60, 1.20, 2};
     return f32 ? StageCost{1.00, 0.38, 5} : StageCost{1.40, 0.65, 3};
 }
 double stage_model(const Ctx *c, bool momentum, bool pack, int tj, int ti) {
     const StageCost k = stage_cost(c, momentum);
     const int waves = pack ? (tj * c->g.nz + KP - 1) / KP : tj, per_simd = (waves + 3) / 4, cus = std::max(1, c->pp.cus);
     const int fit = std::max(1, std::min(k.simd / per_simd, (int)(c->pp.lds_max / stage_lds(c, momentum, tj, pack ? c->g.nz : KP))));
-    const long long blocks = (long long)((c->g.ny - 6 + tj - 1) / tj) * ((c->g.nx - 6 + ti - 1) / ti);
+    const long long blocks = (long long)((c->g.ny - 6 + tj - 1) / tj) * ((c->g.nx - 6 + ti - 1) / ti) * (!momentum && c->g.microphysics && c->prec == DYN_FP64 ? 2 : 1);
     const int per_cu = (int)((blocks + cus - 1) / cus);
     auto column = [&](int n) { return n ? std::max(k.lat, k.issue * n * per_simd) : 0.0; };
     return (ti + 1) * (per_cu / fit * column(fit) + column(per_cu % fit)) * (1.0 + 0.3 / tj);
@@ -1498,6 +1625,12 @@ StageShape stage_shape(const Ctx *c, bool momentum) {
     StageShape s{fused_shape(c, ptj), fused_shape(c, pti), stage_packs(c)};
     if (s.pack && s.tj * c->g.nz > kPackThreads) s.pack = false;  // 12 or 16 rows asked for
     return s;
+}
+
+bool stage_in_one(const Ctx *c) {
+    for (int p : {DYN_TUNE_MOMENTUM_TJ, DYN_TUNE_MOMENTUM_TI, DYN_TUNE_SCALAR_TJ, DYN_TUNE_SCALAR_TI, DYN_TUNE_STAGE_STREAMS})
+        if (c->tune[p]) return false;
+    return c->auto_one.tj > 0;
 }
 
 // How a step's stages use the second stream (the values of DYN_TUNE_STAGE_STREAMS) while the knob is unset.
@@ -1539,10 +1672,46 @@ void choose_stage_shapes(Ctx *c) {
     }
 }
 
+// One launch for both halves of a stage: the shape with the shortest longest march among those whose blocks all run
+// at once (the registers and LDS of the heavier half count for every block), where the model gives it 12 us or
+// less, 15 with the scalar half in two parts.  Past that the halves are worth two streams (us per step, two streams
+// against one launch, with the model's figure: dry FP32 159 and 142 at 64x64x40 (5.1), 230 and 221 at 128x96x40
+// (11.0), 268 and 277 at 150x126x50 (19.3); dry FP64 122 and 96 at 32x32x20 (6.6), 195 and 191 at 64x64x64 (11.6),
+// 247 and 257 at 128x96x40 (20.1); moist FP32 194 and 184 at 64x64x64 (11.3), 218 and 225 at 64x64x80 (13.2);
+// moist FP64 213 and 201 at 64x64x40 (14.3), 225 and 241 at 64x64x64 (20.3)).
+void choose_stage_one(Ctx *c) {
+    c->auto_one = StageOne{};
+    const bool pack = stage_packs(c);
+    const int nx = c->g.nx - 6, ny = c->g.ny - 6, pitch = pack ? c->g.nz : KP, cus = std::max(1, c->pp.cus);
+    const StageCost km = stage_cost(c, true), ks = stage_cost(c, false);
+    const int simd = std::min(km.simd, ks.simd), parts = c->g.microphysics && c->prec == DYN_FP64 ? 2 : 1;
+    double best = 0.0;
+    for (int tj = 2; tj * pitch <= kPackThreads; tj++) {
+        if (!pack && tj != 2 && tj != 4 && tj != 8) continue;
+        const size_t lds = std::max(stage_lds(c, true, tj, pitch), stage_lds(c, false, tj, pitch));
+        if (lds > c->pp.lds_max) continue;
+        const int waves = pack ? (tj * c->g.nz + KP - 1) / KP : tj, per_simd = (waves + 3) / 4;
+        const int fit = std::min(simd / per_simd, (int)(c->pp.lds_max / lds)), nbj = (ny + tj - 1) / tj;
+        for (int tm = 2; tm <= 32; tm++)
+            for (int ts = 2; ts <= 32; ts++) {
+                const int n = nbj * ((nx + tm - 1) / tm + parts * ((nx + ts - 1) / ts)), per_cu = (n + cus - 1) / cus;
+                if (per_cu > fit) continue;
+                const double t = std::max((tm + 1) * std::max(km.lat, km.issue * per_cu * per_simd),
+                                          (ts + 1) * std::max(ks.lat, ks.issue * per_cu * per_simd)) * (1.0 + 0.3 / tj);
+                if (c->auto_one.tj == 0 || t < best) {
+                    best = t;
+                    c->auto_one = StageOne{tj, tm, ts};
+                }
+            }
+    }
+    if (best > (parts == 2 ? 15.0 : 12.0)) c->auto_one = StageOne{};
+}
+
 template <typename T, int TJ, bool PACK, bool TURB>
 int set_lds_limits(const Ctx *c) {
     const int most = (int)c->pp.lds_max;
-    const void *k[] = {(const void *)k_adv_momentum<T, TJ, true, PACK, TURB>, (const void *)k_adv_momentum<T, TJ, false, PACK, TURB>,
+    const void *k[] = {(const void *)k_adv_stage<T, TJ, true, PACK, TURB>, (const void *)k_adv_stage<T, TJ, false, PACK, TURB>,
+                       (const void *)k_adv_momentum<T, TJ, true, PACK, TURB>, (const void *)k_adv_momentum<T, TJ, false, PACK, TURB>,
                        (const void *)k_adv_scalars<T, TJ, true, PACK, TURB>, (const void *)k_adv_scalars<T, TJ, false, PACK, TURB>};
     for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, most));
     return DYN_OK;
@@ -1568,6 +1737,7 @@ int set_lds_limits_all(const Ctx *c) {
 // the stage kernels may use more than 64 KiB of LDS: raise the per-launch limit once, outside any capture
 int fused_prepare(Ctx *c) {
     choose_stage_shapes(c);
+    choose_stage_one(c);
     int rc = c->prec == DYN_FP32 ? set_lds_limits_all<float, false>(c) : set_lds_limits_all<double, false>(c);
     if (!rc) rc = c->prec == DYN_FP32 ? set_lds_limits_all<float, true>(c) : set_lds_limits_all<double, true>(c);
     return rc;
@@ -1621,7 +1791,7 @@ template <typename T, int TJ, bool PACK>
 int ens_scalars_t(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, T step, int ti, int total) {
     const dim3 blk = PACK ? dim3((TJ * c0->geo.NZ + KP - 1) / KP * KP) : dim3(KP, TJ);
     Timed _t(c0, "ens_scalars", 0.0);
-    hipLaunchKernelGGL((k_ens_scalars<T, TJ, false, PACK>), dim3(total), blk, (ScalLds<T, false>::bytes(TJ, PACK ? c0->geo.NZ : KP)),
+    hipLaunchKernelGGL((k_ens_scalars<T, TJ, false, PACK>), dim3(total), blk, (scalar_lds<T, false>(TJ, PACK ? c0->geo.NZ : KP)),
                        c0->stream, d, nmem, ro, step, ti, total);
     DYN_LAUNCH_CHECK();
     return DYN_OK;
@@ -1658,7 +1828,7 @@ int ens_lds_limits() {
     DYN_HIP(hipFuncSetAttribute((const void *)k_ens_momentum<T, TJ, false, PACK>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)MomLds<T>::bytes(TJ, KP)));
     DYN_HIP(hipFuncSetAttribute((const void *)k_ens_scalars<T, TJ, false, PACK>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)ScalLds<T, false>::bytes(TJ, KP)));
+                                (int)scalar_lds<T, false>(TJ, KP)));
     return DYN_OK;
 }
 template <typename T>

@@ -169,6 +169,11 @@ struct StageShape {
     int tj, ti;
     bool pack;
 };
+// both halves of a stage in one launch: rows per block, march lengths of the momentum and the scalar tiles (tj 0: two
+// launches)
+struct StageOne {
+    int tj, ti_mom, ti_scal;
+};
 // the two halves of a fused stage (launch_fused_advect's `parts`)
 constexpr int kStageMomentum = 1, kStageScalars = 2;
 
@@ -244,6 +249,7 @@ struct Ctx {
     // launches of the scalar [0] and the momentum [1] stage kernel while their knobs are unset (tj = 0: the
     // nominal shape), chosen from the grid's size at creation
     StageShape auto_shape[2] = {};
+    StageOne auto_one{};
     // launch-shape knobs (DYN_TUNE_*), 0 = default
     int tune[DYN_TUNE_COUNT] = {0};
     // timing
@@ -304,6 +310,7 @@ int step_with_hook(Ctx *c, StageHook hook, void *arg, bool share_end = false);
 void unshare_roles(Ctx *c);
 bool fused_supported(const Ctx *c);
 int fused_waves(const Ctx *c);
+bool stage_in_one(const Ctx *c);
 // ensembles: batched launches over a device table of members (dyn_fused.hip, dyn_pressure.hip)
 int ens_prepare(bool fp32);
 int launch_ens_stage(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, const int *shape, int tot_mom, int tot_scal);
