@@ -43,6 +43,7 @@ struct Ensemble {
     int tot_mom = 0, tot_scal = 0, tot_post = 0, tot_px = 0, tot_py = 0, tot_cp = 0;
     bool batched_pressure = false;
     size_t lds_x = 0, lds_y = 0;
+    int xform = 0, yform = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     std::vector<EnsGroup> groups;
@@ -186,7 +187,7 @@ int ens_launch_step(Ensemble *e) {
             if (rc) return rc;
             if (e->batched_pressure) {
                 rc = on_stream(c0, gr.stream, [&](Ctx *c) {
-                    return launch_pressure_ens(c, gr.d, nm, ro, steps[s], gr.tot_px, gr.tot_py, e->lds_x, e->lds_y);
+                    return launch_pressure_ens(c, gr.d, nm, ro, steps[s], gr.tot_px, gr.tot_py, e->lds_x, e->lds_y, e->xform, e->yform);
                 });
             } else {
                 // FP64 members: each member's own solve, on the group's stream
@@ -328,6 +329,8 @@ int dyn_ensemble_create(dyn_ctx *const *members, int n, dyn_ensemble **out) {
         if (all_batched && pressure_ens_fill(c, t, lx, ly)) {
             e->lds_x = std::max(e->lds_x, lx);
             e->lds_y = std::max(e->lds_y, ly);
+            e->xform = std::max(e->xform, t.xform);
+            e->yform = std::max(e->yform, t.ydft ? 2 : t.ynarrow ? 0 : 1);
         } else {
             all_batched = false;
         }
@@ -335,9 +338,9 @@ int dyn_ensemble_create(dyn_ctx *const *members, int n, dyn_ensemble **out) {
     e->batched_pressure = all_batched;
     for (int f = 0; f < 7; f++)
         for (int r = 0; r < 3; r++) e->perm[f][r] = (unsigned char)r;
-    if (c0->prec != DYN_FP32) {
-        e->shape[0] = e->shape[2] = 4;
-    }
+    std::vector<std::pair<int, int>> sides;
+    for (const EnsMember &t : e->h) sides.emplace_back(t.g.NX - 6, t.g.NY - 6);
+    choose_ens_shape(c0, sides, e->shape);
     int rc = ens_prepare(c0->prec == DYN_FP32);
     if (!rc && all_batched) rc = pressure_ens_prepare(c0);
     if (!rc && hipMalloc(&e->d, sizeof(EnsMember) * n) != hipSuccess) {

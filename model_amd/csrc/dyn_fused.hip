@@ -1379,20 +1379,20 @@ __device__ __forceinline__ PostArgs ens_post_args(const EnsMember &e, const EnsR
 }
 
 template <typename T, int TJ, bool MOIST, bool PACK>
-__global__ void __launch_bounds__(KP *TJ) k_ens_momentum(const EnsMember *mem, int nmem, EnsRoles ro, T step, int ti, int total) {
+__global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_ens_momentum(const EnsMember *mem, int nmem, EnsRoles ro, T step, int tj, int ti, int total) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int item = blockIdx.x;
     const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::mom0)];
-    const StageArgs a = ens_stage_args(e, ro, TJ, ti, e.nbj_mom);
+    const StageArgs a = ens_stage_args(e, ro, tj, ti, e.nbj_mom);
     adv_momentum_tile<T, TJ, MOIST, PACK>(e.g, e.c, a, step, item - e.mom0, smem_raw);
 }
 
 template <typename T, int TJ, bool MOIST, bool PACK>
-__global__ void __launch_bounds__(KP *TJ) k_ens_scalars(const EnsMember *mem, int nmem, EnsRoles ro, T step, int ti, int total) {
+__global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_ens_scalars(const EnsMember *mem, int nmem, EnsRoles ro, T step, int tj, int ti, int total) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int item = blockIdx.x;
     const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::scal0)];
-    const StageArgs a = ens_stage_args(e, ro, TJ, ti, e.nbj_scal);
+    const StageArgs a = ens_stage_args(e, ro, tj, ti, e.nbj_scal);
     adv_scalars_tile<T, TJ, kTheta, PACK>(e.g, e.c, a, step, item - e.scal0, smem_raw);
 }
 
@@ -1604,11 +1604,10 @@ StageCost stage_cost(const Ctx *c, bool momentum) {
     if (moist) return f32 ? StageCost{2.70, 1.00, 3} : StageCost{1.60, 1.20, 2};
     return f32 ? StageCost{1.00, 0.38, 5} : StageCost{1.40, 0.65, 3};
 }
-double stage_model(const Ctx *c, bool momentum, bool pack, int tj, int ti) {
+double stage_model(const Ctx *c, bool momentum, bool pack, int tj, int ti, long long blocks) {
     const StageCost k = stage_cost(c, momentum);
     const int waves = pack ? (tj * c->g.nz + KP - 1) / KP : tj, per_simd = (waves + 3) / 4, cus = std::max(1, c->pp.cus);
     const int fit = std::max(1, std::min(k.simd / per_simd, (int)(c->pp.lds_max / stage_lds(c, momentum, tj, pack ? c->g.nz : KP))));
-    const long long blocks = (long long)((c->g.ny - 6 + tj - 1) / tj) * ((c->g.nx - 6 + ti - 1) / ti) * (!momentum && c->g.microphysics && c->prec == DYN_FP64 ? 2 : 1);
     const int per_cu = (int)((blocks + cus - 1) / cus);
     auto column = [&](int n) { return n ? std::max(k.lat, k.issue * n * per_simd) : 0.0; };
     return (ti + 1) * (per_cu / fit * column(fit) + column(per_cu % fit)) * (1.0 + 0.3 / tj);
@@ -1647,7 +1646,7 @@ int stage_streams(const Ctx *c) {
 namespace {
 // auto_shape of both kernels; left empty (tj = 0) where the nominal shape is kept
 void choose_stage_shapes(Ctx *c) {
-    const bool pack = stage_packs(c);
+    const bool pack = stage_packs(c), two = c->g.microphysics && c->prec == DYN_FP64;  // scalar_parts
     const int nx = c->g.nx - 6, ny = c->g.ny - 6;
     for (int m = 0; m < 2; m++) {
         const bool momentum = m == 1;
@@ -1662,7 +1661,8 @@ void choose_stage_shapes(Ctx *c) {
             if (!pack && tj != 2 && tj != 4 && tj != 8) continue;
             if (stage_lds(c, momentum, tj, pack ? c->g.nz : KP) > c->pp.lds_max) continue;
             for (int ti = 2; ti <= 48; ti++) {
-                const double t = stage_model(c, momentum, pack, tj, ti);
+                const long long n = (long long)((ny + tj - 1) / tj) * ((nx + ti - 1) / ti) * (!momentum && two ? 2 : 1);
+                const double t = stage_model(c, momentum, pack, tj, ti, n);
                 if (c->auto_shape[m].tj == 0 || t < best) {
                     best = t;
                     c->auto_shape[m] = StageShape{tj, ti, pack};
@@ -1707,40 +1707,73 @@ void choose_stage_one(Ctx *c) {
     if (best > (parts == 2 ? 15.0 : 12.0)) c->auto_one = StageOne{};
 }
 
-template <typename T, int TJ, bool PACK, bool TURB>
+template <typename T, int TJ, bool MOIST, bool PACK, bool TURB>
 int set_lds_limits(const Ctx *c) {
     const int most = (int)c->pp.lds_max;
-    const void *k[] = {(const void *)k_adv_stage<T, TJ, true, PACK, TURB>, (const void *)k_adv_stage<T, TJ, false, PACK, TURB>,
-                       (const void *)k_adv_momentum<T, TJ, true, PACK, TURB>, (const void *)k_adv_momentum<T, TJ, false, PACK, TURB>,
-                       (const void *)k_adv_scalars<T, TJ, true, PACK, TURB>, (const void *)k_adv_scalars<T, TJ, false, PACK, TURB>};
+    const void *k[] = {(const void *)k_adv_stage<T, TJ, MOIST, PACK, TURB>, (const void *)k_adv_momentum<T, TJ, MOIST, PACK, TURB>,
+                       (const void *)k_adv_scalars<T, TJ, MOIST, PACK, TURB>};
     for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, most));
     return DYN_OK;
 }
 
-template <typename T, bool TURB>
+template <typename T, bool MOIST, bool TURB>
 int set_lds_limits_all(const Ctx *c) {
-    int rc = set_lds_limits<T, 2, true, TURB>(c);
-    if (!rc) rc = set_lds_limits<T, 4, true, TURB>(c);
-    if (!rc) rc = set_lds_limits<T, 8, true, TURB>(c);
-    if (!rc) rc = set_lds_limits<T, 2, false, TURB>(c);
-    if (!rc) rc = set_lds_limits<T, 4, false, TURB>(c);
-    if (!rc) rc = set_lds_limits<T, 8, false, TURB>(c);
+    int rc = set_lds_limits<T, 2, MOIST, true, TURB>(c);
+    if (!rc) rc = set_lds_limits<T, 4, MOIST, true, TURB>(c);
+    if (!rc) rc = set_lds_limits<T, 8, MOIST, true, TURB>(c);
+    if (!rc) rc = set_lds_limits<T, 2, MOIST, false, TURB>(c);
+    if (!rc) rc = set_lds_limits<T, 4, MOIST, false, TURB>(c);
+    if (!rc) rc = set_lds_limits<T, 8, MOIST, false, TURB>(c);
     if (rc) return rc;
     const int most = (int)c->pp.lds_max;
-    const void *k[] = {(const void *)k_adv_momentum<T, 16, true, false, TURB>, (const void *)k_adv_momentum<T, 16, false, false, TURB>,
-                       (const void *)k_adv_scalars<T, 12, true, false, TURB>, (const void *)k_adv_scalars<T, 12, false, false, TURB>};
+    const void *k[] = {(const void *)k_adv_momentum<T, 16, MOIST, false, TURB>, (const void *)k_adv_scalars<T, 12, MOIST, false, TURB>};
     for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, most));
     return DYN_OK;
 }
 }  // namespace
 
 // the stage kernels may use more than 64 KiB of LDS: raise the per-launch limit once, outside any capture
+int fused_lds_limits(Ctx *c, bool turbulence) {
+    auto run = [&](auto turb) {
+        constexpr bool TURB = decltype(turb)::value;
+        if (c->prec == DYN_FP32)
+            return c->g.microphysics ? set_lds_limits_all<float, true, TURB>(c) : set_lds_limits_all<float, false, TURB>(c);
+        return c->g.microphysics ? set_lds_limits_all<double, true, TURB>(c) : set_lds_limits_all<double, false, TURB>(c);
+    };
+    return turbulence ? run(std::true_type{}) : run(std::false_type{});
+}
+
+// The model's shape for a batch's blocks; without packed rows the nominal one.  Most batches fill the chip many times
+// over, so what counts is whole groups of four wavefronts and long marches (32 FP32 members of 96 to 192 points a
+// side and 40 levels, in two batches: momentum 265 us a launch in blocks of 8 rows and 16 columns, 200 in the model's;
+// scalars 142 and 130).
+void choose_ens_shape(const Ctx *c0, const std::vector<std::pair<int, int>> &sides, int *shape) {
+    const int nominal = c0->prec == DYN_FP32 ? 8 : 4;
+    for (int m = 0; m < 2; m++) {
+        shape[2 * m] = nominal;
+        shape[2 * m + 1] = 16;
+        if (!stage_packs(c0)) continue;
+        double best = 0.0;
+        for (int tj = 2; tj * c0->g.nz <= kPackThreads; tj++) {
+            if (stage_lds(c0, m == 0, tj, c0->g.nz) > c0->pp.lds_max) continue;
+            for (int ti = 2; ti <= 48; ti++) {
+                long long n = 0;
+                for (const auto &p : sides) n += (long long)((p.second + tj - 1) / tj) * ((p.first + ti - 1) / ti);
+                const double t = stage_model(c0, m == 0, true, tj, ti, n);
+                if (best == 0.0 || t < best) {
+                    best = t;
+                    shape[2 * m] = tj;
+                    shape[2 * m + 1] = ti;
+                }
+            }
+        }
+    }
+}
+
 int fused_prepare(Ctx *c) {
     choose_stage_shapes(c);
     choose_stage_one(c);
-    int rc = c->prec == DYN_FP32 ? set_lds_limits_all<float, false>(c) : set_lds_limits_all<double, false>(c);
-    if (!rc) rc = c->prec == DYN_FP32 ? set_lds_limits_all<float, true>(c) : set_lds_limits_all<double, true>(c);
-    return rc;
+    return fused_lds_limits(c, false);
 }
 
 // advect_uvw_velocity + advect_theta (+ advect_microphysics_cell and the interior zero_moisture)
@@ -1779,33 +1812,33 @@ int launch_zero_moisture_shell(Ctx *c, int il, int ih, int jl, int jh) {
 namespace {
 // packed rows in the ensemble's batches too (every member has the same level count; at most 8 rows of 64)
 template <typename T, int TJ, bool PACK>
-int ens_momentum_t(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, T step, int ti, int total) {
-    const dim3 blk = PACK ? dim3((TJ * c0->geo.NZ + KP - 1) / KP * KP) : dim3(KP, TJ);
+int ens_momentum_t(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, T step, int tj, int ti, int total) {
+    const dim3 blk = PACK ? dim3((tj * c0->geo.NZ + KP - 1) / KP * KP) : dim3(KP, TJ);
     Timed _t(c0, "ens_momentum", 0.0);
-    hipLaunchKernelGGL((k_ens_momentum<T, TJ, false, PACK>), dim3(total), blk, MomLds<T>::bytes(TJ, PACK ? c0->geo.NZ : KP), c0->stream,
-                       d, nmem, ro, step, ti, total);
+    hipLaunchKernelGGL((k_ens_momentum<T, TJ, false, PACK>), dim3(total), blk, MomLds<T>::bytes(tj, PACK ? c0->geo.NZ : KP), c0->stream,
+                       d, nmem, ro, step, tj, ti, total);
     DYN_LAUNCH_CHECK();
     return DYN_OK;
 }
 template <typename T, int TJ, bool PACK>
-int ens_scalars_t(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, T step, int ti, int total) {
-    const dim3 blk = PACK ? dim3((TJ * c0->geo.NZ + KP - 1) / KP * KP) : dim3(KP, TJ);
+int ens_scalars_t(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, T step, int tj, int ti, int total) {
+    const dim3 blk = PACK ? dim3((tj * c0->geo.NZ + KP - 1) / KP * KP) : dim3(KP, TJ);
     Timed _t(c0, "ens_scalars", 0.0);
-    hipLaunchKernelGGL((k_ens_scalars<T, TJ, false, PACK>), dim3(total), blk, (scalar_lds<T, false>(TJ, PACK ? c0->geo.NZ : KP)),
-                       c0->stream, d, nmem, ro, step, ti, total);
+    hipLaunchKernelGGL((k_ens_scalars<T, TJ, false, PACK>), dim3(total), blk, (scalar_lds<T, false>(tj, PACK ? c0->geo.NZ : KP)),
+                       c0->stream, d, nmem, ro, step, tj, ti, total);
     DYN_LAUNCH_CHECK();
     return DYN_OK;
 }
 template <typename T, bool PACK>
 int ens_stage_t(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, const int *shape, int tot_mom, int tot_scal) {
     int rc;
-    if (shape[0] == 2) rc = ens_momentum_t<T, 2, PACK>(c0, d, nmem, ro, T(step), shape[1], tot_mom);
-    else if (shape[0] == 4) rc = ens_momentum_t<T, 4, PACK>(c0, d, nmem, ro, T(step), shape[1], tot_mom);
-    else rc = ens_momentum_t<T, 8, PACK>(c0, d, nmem, ro, T(step), shape[1], tot_mom);
+    if (shape[0] <= 2) rc = ens_momentum_t<T, 2, PACK>(c0, d, nmem, ro, T(step), shape[0], shape[1], tot_mom);
+    else if (shape[0] <= 5) rc = ens_momentum_t<T, 4, PACK>(c0, d, nmem, ro, T(step), shape[0], shape[1], tot_mom);
+    else rc = ens_momentum_t<T, 8, PACK>(c0, d, nmem, ro, T(step), shape[0], shape[1], tot_mom);
     if (rc) return rc;
-    if (shape[2] == 2) return ens_scalars_t<T, 2, PACK>(c0, d, nmem, ro, T(step), shape[3], tot_scal);
-    if (shape[2] == 4) return ens_scalars_t<T, 4, PACK>(c0, d, nmem, ro, T(step), shape[3], tot_scal);
-    return ens_scalars_t<T, 8, PACK>(c0, d, nmem, ro, T(step), shape[3], tot_scal);
+    if (shape[2] <= 2) return ens_scalars_t<T, 2, PACK>(c0, d, nmem, ro, T(step), shape[2], shape[3], tot_scal);
+    if (shape[2] <= 5) return ens_scalars_t<T, 4, PACK>(c0, d, nmem, ro, T(step), shape[2], shape[3], tot_scal);
+    return ens_scalars_t<T, 8, PACK>(c0, d, nmem, ro, T(step), shape[2], shape[3], tot_scal);
 }
 template <typename T>
 int ens_post_t(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, bool pgf, int total) {
@@ -1825,10 +1858,11 @@ int ens_copy_t(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, int to
 }
 template <typename T, int TJ, bool PACK>
 int ens_lds_limits() {
-    DYN_HIP(hipFuncSetAttribute((const void *)k_ens_momentum<T, TJ, false, PACK>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)MomLds<T>::bytes(TJ, KP)));
-    DYN_HIP(hipFuncSetAttribute((const void *)k_ens_scalars<T, TJ, false, PACK>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)scalar_lds<T, false>(TJ, KP)));
+    int dev = 0, most = 0;
+    DYN_HIP(hipGetDevice(&dev));
+    DYN_HIP(hipDeviceGetAttribute(&most, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    const void *k[] = {(const void *)k_ens_momentum<T, TJ, false, PACK>, (const void *)k_ens_scalars<T, TJ, false, PACK>};
+    for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, most));
     return DYN_OK;
 }
 template <typename T>

@@ -6,6 +6,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/dyncore.h"
@@ -138,6 +139,7 @@ struct EnsMember {
     void *spec;
     const double *twx, *twy, *zpiv, *acoef, *ccoef, *dftx, *dfty;
     int ydft, pxn;  // the j pass by matrix products; work items of its i passes
+    int xform, ynarrow;  // form of the i passes (launch_pressure_ens); the j pass fits half-sized blocks
     Radix rx, ry;
     int ni, nj, nk2, kcx;
     // first work item of this member in each batched launch
@@ -311,6 +313,7 @@ void unshare_roles(Ctx *c);
 bool fused_supported(const Ctx *c);
 int fused_waves(const Ctx *c);
 bool stage_in_one(const Ctx *c);
+int fused_lds_limits(Ctx *c, bool turbulence);
 // ensembles: batched launches over a device table of members (dyn_fused.hip, dyn_pressure.hip)
 int ens_prepare(bool fp32);
 int launch_ens_stage(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, const int *shape, int tot_mom, int tot_scal);
@@ -318,8 +321,11 @@ int launch_ens_post(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, d
 int launch_ens_copy(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, int total);
 bool pressure_ens_fill(Ctx *c, EnsMember &e, size_t &lds_x, size_t &lds_y);
 int pressure_ens_prepare(const Ctx *c);
+// xform: the i passes with up to three butterflies a thread (0), four (1), four and members by matrix products (2); yform: the j pass in blocks of 512 threads (0), of 1024 (1), of 1024 with members by matrix products (2)
 int launch_pressure_ens(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, int tot_px, int tot_py, size_t lds_x,
-                        size_t lds_y);
+                        size_t lds_y, int xform, int yform);
+// rows per block and march length {momentum, scalars} for a batch of members of these sides
+void choose_ens_shape(const Ctx *c0, const std::vector<std::pair<int, int>> &sides, int *shape);
 // launch shapes of the stage kernels (DYN_TUNE_*): validity and the value in force
 bool fused_shape_ok(const Ctx *c, int param, int value);
 int fused_shape(const Ctx *c, int param);

@@ -749,7 +749,7 @@ constexpr int half_maxb() { return sizeof(T) == 4 ? 4 : 6; }
 // The periodic column UP(NX-3) is read as UP(3), the value periodic_uvw_boundaries puts there.
 // With src != nullptr the transform reads a ready real field src(i+3, j, k) instead of the divergence
 // (the transposed solve of the adjoint).
-template <typename T>
+template <typename T, int MAXB = kMaxBX>
 __device__ __forceinline__ void div_rfft_x_block(const Geo &g, const Cols &c, const T *__restrict__ UP, const T *__restrict__ VP,
                                                  const T *__restrict__ WP, T *__restrict__ spec, const Radix &rad, const double *tw,
                                                  int nk2, int kc, double step, const T *__restrict__ src, int j, int chunk,
@@ -782,7 +782,6 @@ __device__ __forceinline__ void div_rfft_x_block(const Geo &g, const Cols &c, co
         const DivStep<decltype(arithmetic)> ds(g, step);
         for (int idx0 = (int)threadIdx.x; idx0 < ne; idx0 += kU * nt) {
             T f0[kU], f1[kU], f2[kU], f3[kU], f4[kU], f5[kU];
-            double ru[kU], rw1[kU], rw0[kU], mk[kU];
 #pragma unroll
             for (int u = 0; u < kU; u++) {
                 const int idx = min(idx0 + u * nt, ne - 1), b = idx % kc, i = idx / kc;
@@ -797,10 +796,6 @@ __device__ __forceinline__ void div_rfft_x_block(const Geo &g, const Cols &c, co
                     f3[u] = VP[IX(ia, jj, k)];
                     f4[u] = WP[IX(ia, jj, k + 1)];
                     f5[u] = WP[IX(ia, jj, k)];
-                    ru[u] = colc[4 * b];
-                    rw1[u] = colc[4 * b + 1];
-                    rw0[u] = colc[4 * b + 2];
-                    mk[u] = colc[4 * b + 3];
                 }
             }
 #pragma unroll
@@ -811,7 +806,8 @@ __device__ __forceinline__ void div_rfft_x_block(const Geo &g, const Cols &c, co
                 if (kk < nk2 && kSrc) {
                     d = f0[u];
                 } else if (kk < nk2) {
-                    d = T(ds(ru[u], rw1[u], rw0[u], mk[u], f0[u], f1[u], f2[u], f3[u], f4[u], f5[u]));
+                    const double *cb = colc + 4 * b;
+                    d = T(ds(cb[0], cb[1], cb[2], cb[3], f0[u], f1[u], f2[u], f3[u], f4[u], f5[u]));
                 }
                 if (idx < ne) {
                     if (b & 1) im[i * P + (b >> 1)] = d;
@@ -824,7 +820,7 @@ __device__ __forceinline__ void div_rfft_x_block(const Geo &g, const Cols &c, co
     else if (sizeof(T) == 4 && wide) gather(std::false_type{}, double(0));
     else gather(std::false_type{}, T(0));
     __syncthreads();
-    lds_fft_ip<T, kMaxBX>(re, im, rad, P, P, 1, twl, -1);
+    lds_fft_ip<T, MAXB>(re, im, rad, P, P, 1, twl, -1);
     // split the packed pair: A = (Z[m] + conj Z[-m]) / 2, B = (Z[m] - conj Z[-m]) / 2i
     for (int idx = threadIdx.x; idx < nkx * P; idx += blockDim.x) {
         int pp = idx % P, m = idx / P;
@@ -848,7 +844,7 @@ __device__ __forceinline__ void div_rfft_x_block(const Geo &g, const Cols &c, co
 }
 
 // Q3: backward real DFT along i -> PI (pressure.cpp:878-892) with the ghost levels and periodic halos
-template <typename T>
+template <typename T, int MAXB = kMaxBX>
 __device__ __forceinline__ void irfft_x_out_block(const Geo &g, const T *__restrict__ spec, T *__restrict__ PI, const Radix &rad,
                                                   const double *tw, int nk2, int kc, int j, int chunk, unsigned char *smem,
                                                   int jhalf = 0) {
@@ -926,7 +922,7 @@ __device__ __forceinline__ void irfft_x_out_block(const Geo &g, const T *__restr
         }
     }
     __syncthreads();
-    lds_fft_ip<T, kMaxBX>(re, im, rad, P, P, 1, twl, +1);
+    lds_fft_ip<T, MAXB>(re, im, rad, P, P, 1, twl, +1);
     const int shift = g.NX - 6;
     const bool fixed_b = (blockDim.x % kc) == 0;
     const int di = blockDim.x / kc;
@@ -1238,7 +1234,7 @@ __device__ __forceinline__ void lds_to_slab(T *__restrict__ spec, long long base
 
 // Q2 (fused): forward DFT along j, FP64 tridiagonal solve, backward DFT along j for one kx, with the
 // whole (j, k) slab of that kx resident in LDS
-template <typename T, bool TR, bool POW2 = true>
+template <typename T, bool TR, bool POW2 = true, int MAXB = ypass_maxb<T>()>
 __device__ __forceinline__ void ypass_block(T *__restrict__ spec, int nk2, const Radix &rady, const double *twy, const ThomasArgs &ta,
                                             int pad, int kx, unsigned char *smem) {
     const int nj = rady.n, P2 = nk2 + pad;
@@ -1250,7 +1246,7 @@ __device__ __forceinline__ void ypass_block(T *__restrict__ spec, int nk2, const
     const long long base = (long long)kx * nj * nk2 * 2;
     slab_to_lds(spec, base, nj * nk2, nk2, P2, re, im);
     __syncthreads();
-    lds_fft_ip<T, ypass_maxb<T>(), POW2>(re, im, rady, nk2, P2, 1, twl, -1);
+    lds_fft_ip<T, MAXB, POW2>(re, im, rady, nk2, P2, 1, twl, -1);
     if ((int)threadIdx.x < 2 * nj) {
         // one thread per real sequence: threads [0, nj) take the real parts, [nj, 2 nj) the imaginary parts
         const int part = (int)threadIdx.x >= nj, ky = (int)threadIdx.x - part * nj;
@@ -1260,29 +1256,29 @@ __device__ __forceinline__ void ypass_block(T *__restrict__ spec, int nk2, const
         else thomas_part<T>(ta, co, kx, ky, Z, nj, x, 1, mean + part);
     }
     __syncthreads();
-    lds_fft_ip<T, ypass_maxb<T>(), POW2>(re, im, rady, nk2, P2, 1, twl, +1);
+    lds_fft_ip<T, MAXB, POW2>(re, im, rady, nk2, P2, 1, twl, +1);
     lds_to_slab(spec, base, nj * nk2, nk2, P2, re, im);
 }
 
-template <typename T>
+template <typename T, int MAXB>
 __global__ void __launch_bounds__(kThreadsX) k_div_rfft_x(Geo g, Cols c, const T *__restrict__ UP, const T *__restrict__ VP,
                                                          const T *__restrict__ WP, T *__restrict__ spec, Radix rad, const double *tw,
                                                          int nk2, int kc, double step, const T *__restrict__ src, bool wide) {
     extern __shared__ unsigned char smem[];
-    div_rfft_x_block<T>(g, c, UP, VP, WP, spec, rad, tw, nk2, kc, step, src, blockIdx.x, blockIdx.y, smem, wide);
+    div_rfft_x_block<T, MAXB>(g, c, UP, VP, WP, spec, rad, tw, nk2, kc, step, src, blockIdx.x, blockIdx.y, smem, wide);
 }
 
-template <typename T>
+template <typename T, int MAXB>
 __global__ void __launch_bounds__(kThreadsX) k_irfft_x_out(Geo g, const T *__restrict__ spec, T *__restrict__ PI, Radix rad,
                                                           const double *tw, int nk2, int kc, int half) {
     extern __shared__ unsigned char smem[];
-    irfft_x_out_block<T>(g, spec, PI, rad, tw, nk2, kc, blockIdx.x, blockIdx.y, smem, half);
+    irfft_x_out_block<T, MAXB>(g, spec, PI, rad, tw, nk2, kc, blockIdx.x, blockIdx.y, smem, half);
 }
 
 // The same after the half-slab j pass, one block per row pair (j', jhalf + j') and chunk of kc levels:
 // it reads v0 (row j') and v1 (row jhalf + j') once for both rows (v0 + v1 and v0 - v1), and transforms
 // the two rows as one batch of kc level pairs.  Values as irfft_x_out_block's, bit for bit.
-template <typename T>
+template <typename T, int MAXB = kMaxBX>
 __device__ __forceinline__ void irfft_x_out_pair_block(const Geo &g, const T *__restrict__ spec, T *__restrict__ PI, const Radix &rad,
                                                        const double *tw, int nk2, int kc, int jp, int chunk, unsigned char *smem,
                                                        int jhalf) {
@@ -1335,7 +1331,7 @@ __device__ __forceinline__ void irfft_x_out_pair_block(const Geo &g, const T *__
         }
     }
     __syncthreads();
-    lds_fft_ip<T, kMaxBX>(re, im, rad, B, B, 1, twl, +1);
+    lds_fft_ip<T, MAXB>(re, im, rad, B, B, 1, twl, +1);
     const int shift = g.NX - 6;
     for (int idx = threadIdx.x; idx < 2 * n * kc; idx += blockDim.x) {
         const int r = idx / (n * kc), rem = idx - r * (n * kc);
@@ -1358,11 +1354,11 @@ __device__ __forceinline__ void irfft_x_out_pair_block(const Geo &g, const T *__
     }
 }
 
-template <typename T>
+template <typename T, int MAXB>
 __global__ void __launch_bounds__(kThreadsX) k_irfft_x_out_pair(Geo g, const T *__restrict__ spec, T *__restrict__ PI, Radix rad,
                                                                const double *tw, int nk2, int kc, int jhalf) {
     extern __shared__ unsigned char smem[];
-    irfft_x_out_pair_block<T>(g, spec, PI, rad, tw, nk2, kc, blockIdx.x, blockIdx.y, smem, jhalf);
+    irfft_x_out_pair_block<T, MAXB>(g, spec, PI, rad, tw, nk2, kc, blockIdx.x, blockIdx.y, smem, jhalf);
 }
 
 // Q2 on half slabs (even nj, L = nj/2): the j transform's first radix-2 split (decimation in frequency)
@@ -1628,13 +1624,18 @@ __global__ void __launch_bounds__(64 * kYDftWaves) k_ypass_dft(T *__restrict__ s
 // concatenates the members' (row, level chunk) or (kx) items -------------------------------------------
 
 constexpr int kEnsTiles = 2;  // column tiles per block of a member's matrix products
-template <typename T>
+// Threads of a batch's j pass: 512 where every member's slab leaves room for two blocks on a CU and its butterflies fit
+// (one block's sweeps then run beside the other's transforms: 113 us a launch against 207, 16 FP32 members of 96 to
+// 192 points a side and 40 levels), else 1024, and with matrix products
+constexpr int kEnsYNarrow = 512;
+constexpr int ens_ymaxb(int threads) { return threads == kEnsYNarrow ? 6 : kMaxBY; }
+template <typename T, bool DFT, int MAXB>
 __global__ void __launch_bounds__(kThreadsX) k_ens_div_rfft_x(const EnsMember *mem, int nmem, EnsRoles roles, int total, double step) {
     extern __shared__ __align__(16) unsigned char smem[];
     {
         const int item = blockIdx.x;
         const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::px0)];
-        if (e.dftx) {
+        if (DFT && e.dftx) {
             div_dft_x_block<T, kEnsTiles, false>(e.g, e.c, (const T *)e.buf[DYN_U][roles.r[DYN_U][DYN_ROLE_P]],
                                                  (const T *)e.buf[DYN_V][roles.r[DYN_V][DYN_ROLE_P]],
                                                  (const T *)e.buf[DYN_W][roles.r[DYN_W][DYN_ROLE_P]], (T *)e.spec, e.ni, e.dftx, e.nk2, step,
@@ -1642,40 +1643,42 @@ __global__ void __launch_bounds__(kThreadsX) k_ens_div_rfft_x(const EnsMember *m
             return;
         }
         const int local = item - e.px0, nch = (e.nk2 + e.kcx - 1) / e.kcx;
-        div_rfft_x_block<T>(e.g, e.c, (const T *)e.buf[DYN_U][roles.r[DYN_U][DYN_ROLE_P]], (const T *)e.buf[DYN_V][roles.r[DYN_V][DYN_ROLE_P]],
+        div_rfft_x_block<T, MAXB>(e.g, e.c, (const T *)e.buf[DYN_U][roles.r[DYN_U][DYN_ROLE_P]], (const T *)e.buf[DYN_V][roles.r[DYN_V][DYN_ROLE_P]],
                             (const T *)e.buf[DYN_W][roles.r[DYN_W][DYN_ROLE_P]], (T *)e.spec, e.rx, e.twx, e.nk2, e.kcx, step,
                             (const T *)nullptr, local / nch, local % nch, smem, e.dfty != nullptr);
     }
 }
 
-template <typename T>
+template <typename T, bool DFT, int MAXB>
 __global__ void __launch_bounds__(kThreadsX) k_ens_irfft_x_out(const EnsMember *mem, int nmem, int total) {
     extern __shared__ __align__(16) unsigned char smem[];
     {
         const int item = blockIdx.x;
         const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::px0)];
-        if (e.dftx) {
+        if (DFT && e.dftx) {
             idft_x_out_block<T, kEnsTiles>(e.g, (const T *)e.spec, (T *)e.pi, e.ni, e.dftx, e.nk2, item - e.px0, smem);
             return;
         }
         const int local = item - e.px0, nch = (e.nk2 + e.kcx - 1) / e.kcx;
-        irfft_x_out_block<T>(e.g, (const T *)e.spec, (T *)e.pi, e.rx, e.twx, e.nk2, e.kcx, local / nch, local % nch, smem);
+        irfft_x_out_block<T, MAXB>(e.g, (const T *)e.spec, (T *)e.pi, e.rx, e.twx, e.nk2, e.kcx, local / nch, local % nch, smem);
     }
 }
 
-template <typename T>
-__global__ void __launch_bounds__(1024) k_ens_ypass(const EnsMember *mem, int nmem, int total) {
+template <typename T, int THREADS, bool DFT>
+__global__ void __launch_bounds__(THREADS) k_ens_ypass(const EnsMember *mem, int nmem, int total) {
     extern __shared__ __align__(16) unsigned char smem[];
     {
         const int item = blockIdx.x;
         const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::py0)];
         ThomasArgs ta{e.acoef, e.ccoef, e.zpiv, e.ni, e.nj, e.g.NZ};
-        if (e.ydft) {
-            ypass_dft_block<T, false, kEnsYDftPairs>((T *)e.spec, e.nj, e.dfty, e.nk2, ta, item - e.py0, smem);
-            return;
+        if constexpr (DFT) {
+            if (e.ydft) {
+                ypass_dft_block<T, false, kEnsYDftPairs>((T *)e.spec, e.nj, e.dfty, e.nk2, ta, item - e.py0, smem);
+                return;
+            }
         }
         // the generic transform passes (the straight-line power-of-two ones measured no faster here)
-        ypass_block<T, false, false>((T *)e.spec, e.nk2, e.ry, e.twy, ta, 1, item - e.py0, smem);
+        ypass_block<T, false, false, ens_ymaxb(THREADS)>((T *)e.spec, e.nk2, e.ry, e.twy, ta, 1, item - e.py0, smem);
     }
 }
 
@@ -1750,6 +1753,15 @@ bool factorize(int n, Radix &rad) {
 int level_chunk(int n, size_t elt, int nk2);
 size_t x_pass_lds(int ni, int kc, size_t elt);
 
+int max_butterflies(const Radix &r, int nbatch, int nthr);
+// The i passes hold a thread's butterflies of a radix pass in registers: the instance with no more of them than the
+// grid's pass needs (FP32 86 registers with four, 69 with three and 52 with two, so three and four blocks on a CU instead of two; FP64
+// 148, 120 and 92, so two instead of one).
+template <typename T>
+auto div_rfft_x_kernel(const Radix &rx, int kc) {
+    const int b = max_butterflies(rx, kc / 2, kThreadsX);
+    return b <= 2 ? k_div_rfft_x<T, 2> : b <= 3 ? k_div_rfft_x<T, 3> : k_div_rfft_x<T, kMaxBX>;
+}
 // the inverse i pass into `out`: after the half-slab j pass (half = nj/2) one block per row pair and
 // chunk of an even number of levels, at most kc/2 (same LDS and butterflies per thread as kc levels of
 // one row); otherwise one block per row and chunk of kc levels
@@ -1760,11 +1772,15 @@ void launch_irfft_x_out(Ctx *c, const T *spec, T *out, const Radix &rx, int kc, 
     const size_t shx = x_pass_lds(pp.ni, kc, sizeof(T));
     const int kcp = (kc / 2) & ~1;
     if (half && kcp >= 2) {
-        hipLaunchKernelGGL(k_irfft_x_out_pair<T>, dim3(half, (pp.nk2 + kcp - 1) / kcp), dim3(kThreadsX), shx, c->stream, g, spec, out, rx,
+        const int b = max_butterflies(rx, 2 * (kcp / 2), kThreadsX);
+        auto k = b <= 2 ? k_irfft_x_out_pair<T, 2> : b <= 3 ? k_irfft_x_out_pair<T, 3> : k_irfft_x_out_pair<T, kMaxBX>;
+        hipLaunchKernelGGL(k, dim3(half, (pp.nk2 + kcp - 1) / kcp), dim3(kThreadsX), shx, c->stream, g, spec, out, rx,
                            pp.twx, pp.nk2, kcp, half);
         return;
     }
-    hipLaunchKernelGGL(k_irfft_x_out<T>, dim3(g.NY, (pp.nk2 + kc - 1) / kc), dim3(kThreadsX), shx, c->stream, g, spec, out, rx, pp.twx,
+    const int b = max_butterflies(rx, kc / 2, kThreadsX);
+    auto k = b <= 2 ? k_irfft_x_out<T, 2> : b <= 3 ? k_irfft_x_out<T, 3> : k_irfft_x_out<T, kMaxBX>;
+    hipLaunchKernelGGL(k, dim3(g.NY, (pp.nk2 + kc - 1) / kc), dim3(kThreadsX), shx, c->stream, g, spec, out, rx, pp.twx,
                        pp.nk2, kc, half);
 }
 
@@ -1976,7 +1992,7 @@ int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
             launch_div_dft_x<T>(c, spec, step);
         } else {
             Timed _t(c, "p1_div_rfft_x", pts);
-            hipLaunchKernelGGL(k_div_rfft_x<T>, gx, dim3(kThreadsX), shx, c->stream, g, c->cols, (const T *)c->prog[DYN_U][2],
+            hipLaunchKernelGGL(div_rfft_x_kernel<T>(rx, kc), gx, dim3(kThreadsX), shx, c->stream, g, c->cols, (const T *)c->prog[DYN_U][2],
                                (const T *)c->prog[DYN_V][2], (const T *)c->prog[DYN_W][2], spec, rx, pp.twx, pp.nk2, kc, step,
                                (const T *)nullptr, pp.dfty != nullptr);
         }
@@ -2162,7 +2178,7 @@ int solve_adjoint_t(Ctx *c, double step, T *pihat, T *uh, T *vh, T *wh, T *r1, T
         launch_div_dft_x<T>(c, spec, step, (const T *)r1);
     } else {
         Timed _t(c, "adj_rfft_x", pts);
-        hipLaunchKernelGGL(k_div_rfft_x<T>, gx, dim3(kThreadsX), shx, c->stream, g, c->cols, (const T *)nullptr, (const T *)nullptr,
+        hipLaunchKernelGGL(div_rfft_x_kernel<T>(rx, kc), gx, dim3(kThreadsX), shx, c->stream, g, c->cols, (const T *)nullptr, (const T *)nullptr,
                            (const T *)nullptr, spec, rx, pp.twx, pp.nk2, kc, step, (const T *)r1, false);
     }
     DYN_LAUNCH_CHECK();
@@ -2390,40 +2406,48 @@ bool pressure_ens_fill(Ctx *c, EnsMember &e, size_t &lds_x, size_t &lds_y) {
     e.pxn = pp.dftx ? (pp.nj * pp.nk2 + 16 * kEnsTiles - 1) / (16 * kEnsTiles) : c->g.ny * ((pp.nk2 + e.kcx - 1) / e.kcx);
     lds_x = pp.dftx ? dft_lds(pp.ni, 16 * kEnsTiles) : x_pass_lds(pp.ni, e.kcx, sizeof(float));
     if (pp.dftx && lds_x > pp.lds_max) return false;
+    e.xform = pp.dftx ? 2 : max_butterflies(e.rx, e.kcx / 2, kThreadsX) <= 3 ? 0 : 1;
     if (e.ydft) {
         lds_y = ypass_dft_lds(pp.nj, pp.nk2);
         return true;
     }
     lds_y = y_pass_lds(pp.nj, pp.nk2, sizeof(float));
+    e.ynarrow = 2 * lds_y <= pp.lds_max && 2 * pp.nj <= kEnsYNarrow && max_butterflies(e.ry, pp.nk2, kEnsYNarrow) <= ens_ymaxb(kEnsYNarrow);
     return lds_y <= pp.lds_max && 2 * pp.nj <= 1024 && max_butterflies(e.ry, pp.nk2, 1024) <= kMaxBY;
 }
 
 // the batched passes may take more than 64 KiB of LDS
 int pressure_ens_prepare(const Ctx *c) {
-    const void *k[] = {(const void *)k_ens_div_rfft_x<float>, (const void *)k_ens_irfft_x_out<float>, (const void *)k_ens_ypass<float>};
+    const void *k[] = {(const void *)k_ens_div_rfft_x<float, false, 3>, (const void *)k_ens_irfft_x_out<float, false, 3>,
+                       (const void *)k_ens_div_rfft_x<float, false, kMaxBX>, (const void *)k_ens_irfft_x_out<float, false, kMaxBX>,
+                       (const void *)k_ens_div_rfft_x<float, true, kMaxBX>, (const void *)k_ens_irfft_x_out<float, true, kMaxBX>, (const void *)k_ens_ypass<float, kEnsYNarrow, false>,
+                       (const void *)k_ens_ypass<float, 1024, false>, (const void *)k_ens_ypass<float, 1024, true>};
     for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->pp.lds_max));
     return DYN_OK;
 }
 
 // solve_pressure(step) of every member without the uvw halo copy (as in the fused step): three launches
 int launch_pressure_ens(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, int tot_px, int tot_py, size_t lds_x,
-                        size_t lds_y) {
+                        size_t lds_y, int xform, int yform) {
     {
         const int grid = tot_px;
         Timed _t(c0, "ens_p1_div_rfft_x", 0.0);
-        hipLaunchKernelGGL(k_ens_div_rfft_x<float>, dim3(grid), dim3(kThreadsX), lds_x, c0->stream, d, nmem, ro, tot_px, step);
+        auto k = xform == 0 ? k_ens_div_rfft_x<float, false, 3> : xform == 1 ? k_ens_div_rfft_x<float, false, kMaxBX> : k_ens_div_rfft_x<float, true, kMaxBX>;
+        hipLaunchKernelGGL(k, dim3(grid), dim3(kThreadsX), lds_x, c0->stream, d, nmem, ro, tot_px, step);
         DYN_LAUNCH_CHECK();
     }
     {
         const int grid = tot_py;
         Timed _t(c0, "ens_p2_ypass", 0.0);
-        hipLaunchKernelGGL(k_ens_ypass<float>, dim3(grid), dim3(1024), lds_y, c0->stream, d, nmem, tot_py);
+        auto k = yform == 0 ? k_ens_ypass<float, kEnsYNarrow, false> : yform == 1 ? k_ens_ypass<float, 1024, false> : k_ens_ypass<float, 1024, true>;
+        hipLaunchKernelGGL(k, dim3(grid), dim3(yform == 0 ? kEnsYNarrow : 1024), lds_y, c0->stream, d, nmem, tot_py);
         DYN_LAUNCH_CHECK();
     }
     {
         const int grid = tot_px;
         Timed _t(c0, "ens_p5_irfft_x_out", 0.0);
-        hipLaunchKernelGGL(k_ens_irfft_x_out<float>, dim3(grid), dim3(kThreadsX), lds_x, c0->stream, d, nmem, tot_px);
+        auto k = xform == 0 ? k_ens_irfft_x_out<float, false, 3> : xform == 1 ? k_ens_irfft_x_out<float, false, kMaxBX> : k_ens_irfft_x_out<float, true, kMaxBX>;
+        hipLaunchKernelGGL(k, dim3(grid), dim3(kThreadsX), lds_x, c0->stream, d, nmem, tot_px);
         DYN_LAUNCH_CHECK();
     }
     return DYN_OK;

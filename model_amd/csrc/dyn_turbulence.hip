@@ -510,6 +510,8 @@ int dyn_set_turbulence(dyn_ctx *ctx, int on, const double *landsea, size_t count
         turb_release(c);
         return DYN_OK;
     }
+    if (fused_supported(c))
+        if (int rc = fused_lds_limits(c, true)) return rc;
     Turbulence &t = c->turb;
     if (!t.buf[0]) {
         for (void *&p : t.buf) {
