@@ -204,7 +204,7 @@ __global__ void __launch_bounds__(dft_bound(NT)) k_div_dft_x(Geo g, Cols c, cons
                                                              const double *__restrict__ tab, int nk2, double step,
                                                              const T *__restrict__ src) {
     extern __shared__ __align__(16) unsigned char smem[];
-    div_dft_x_block<T, NT, SRC>(g, c, UP, VP, WP, spec, n, tab, nk2, step, src, blockIdx.x, smem);
+    div_dft_x_block<T, NT, SRC>(g, c, UP, VP, WP, spec, n, tab, nk2, step, src, xcd_tile(blockIdx.x, gridDim.x), smem);
 }
 
 // Backward along i: the half spectrum's rows, weighted for their mirror images (2, and 1 for the
@@ -285,7 +285,7 @@ template <typename T, int NT>
 __global__ void __launch_bounds__(dft_bound(NT)) k_idft_x_out(Geo g, const T *__restrict__ spec, T *__restrict__ PI, int n,
                                                               const double *__restrict__ tab, int nk2, int jhalf) {
     extern __shared__ __align__(16) unsigned char smem[];
-    idft_x_out_block<T, NT>(g, spec, PI, n, tab, nk2, blockIdx.x, smem, jhalf);
+    idft_x_out_block<T, NT>(g, spec, PI, n, tab, nk2, xcd_tile(blockIdx.x, gridDim.x), smem, jhalf);
 }
 
 // value of the neighbouring lane (lane ^ 1) by a DPP quad permutation
@@ -307,9 +307,10 @@ __global__ void __launch_bounds__(dft_bound(NT)) k_dft_y(const TI *in, TO *out, 
     constexpr int NC = 16 * NT;
     const int pitch = dft_pitch(NC), h = dft_rows(n), hk = (h + 3) & ~3, ncol = 2 * nk2;
     double *E = (double *)smem, *D = E + hk * pitch;
-    const TI *x = in + (long long)blockIdx.x * n * ncol;
-    TO *o = out + (long long)blockIdx.x * n * ncol;
-    const int c0 = blockIdx.y * NC, b = threadIdx.x % NC, q = min(c0 + b, ncol - 1);
+    const TileXY tile = xcd_tile_xy();
+    const TI *x = in + (long long)tile.x * n * ncol;
+    TO *o = out + (long long)tile.x * n * ncol;
+    const int c0 = tile.y * NC, b = threadIdx.x % NC, q = min(c0 + b, ncol - 1);
     const int rows = blockDim.x / NC;
     for (int i = threadIdx.x / NC; i < hk; i += 4 * rows) {
         TI a[4], m[4];

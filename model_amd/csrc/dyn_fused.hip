@@ -1381,7 +1381,7 @@ __device__ __forceinline__ PostArgs ens_post_args(const EnsMember &e, const EnsR
 template <typename T, int TJ, bool MOIST, bool PACK>
 __global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_ens_momentum(const EnsMember *mem, int nmem, EnsRoles ro, T step, int tj, int ti, int total) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    const int item = blockIdx.x;
+    const int item = xcd_tile(blockIdx.x, gridDim.x);
     const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::mom0)];
     const StageArgs a = ens_stage_args(e, ro, tj, ti, e.nbj_mom);
     adv_momentum_tile<T, TJ, MOIST, PACK>(e.g, e.c, a, step, item - e.mom0, smem_raw);
@@ -1390,7 +1390,7 @@ __global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_ens_momentum(co
 template <typename T, int TJ, bool MOIST, bool PACK>
 __global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_ens_scalars(const EnsMember *mem, int nmem, EnsRoles ro, T step, int tj, int ti, int total) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    const int item = blockIdx.x;
+    const int item = xcd_tile(blockIdx.x, gridDim.x);
     const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::scal0)];
     const StageArgs a = ens_stage_args(e, ro, tj, ti, e.nbj_scal);
     adv_scalars_tile<T, TJ, kTheta, PACK>(e.g, e.c, a, step, item - e.scal0, smem_raw);
@@ -1398,7 +1398,7 @@ __global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_ens_scalars(con
 
 template <typename T>
 __global__ void __launch_bounds__(256) k_ens_post(const EnsMember *mem, int nmem, EnsRoles ro, T step, bool pgf, bool scalars, int total) {
-    const int item = blockIdx.x;
+    const int item = xcd_tile(blockIdx.x, gridDim.x);
     const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::post0)];
     const PostArgs a = ens_post_args(e, ro);
     const int local = item - e.post0, nb = (e.g.NY + 3) / 4;

@@ -166,6 +166,15 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
     const int q = n / 8, rem = n % 8, x = b % 8;
     return x * q + min(x, rem) + b / 8;
 }
+// ... and of block (x, y) of a 2-D grid, the tiles counted with y fastest: tiles of one x (which share cache lines, and
+// rows with those of x + 1) run on one XCD at about the same time
+struct TileXY {
+    int x, y;
+};
+__device__ __forceinline__ TileXY xcd_tile_xy() {
+    const int ny = gridDim.y, t = xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * ny);
+    return TileXY{t / ny, t % ny};
+}
 // rows per block, march length and lane mapping of a stage kernel's launch (dyn_fused.hip)
 struct StageShape {
     int tj, ti;

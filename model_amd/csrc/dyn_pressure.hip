@@ -690,7 +690,8 @@ __global__ void __launch_bounds__(kFftYThreads) k_fft_y_pow2(T *__restrict__ spe
     const int n = rad.n, P2 = kc + 1;
     T *re = (T *)smem, *im = re + n * P2, *twl = im + n * P2;
     load_twiddles(twl, tw, n);
-    const int kx = blockIdx.x, kk0 = blockIdx.y * kc;
+    const TileXY tile = xcd_tile_xy();
+    const int kx = tile.x, kk0 = tile.y * kc;
     for (int idx = threadIdx.x; idx < n * kc; idx += blockDim.x) {
         const int b = idx % kc, ky = idx / kc, kk = kk0 + b;
         T vr = T(0), vi = T(0);
@@ -1265,14 +1266,16 @@ __global__ void __launch_bounds__(kThreadsX) k_div_rfft_x(Geo g, Cols c, const T
                                                          const T *__restrict__ WP, T *__restrict__ spec, Radix rad, const double *tw,
                                                          int nk2, int kc, double step, const T *__restrict__ src, bool wide) {
     extern __shared__ unsigned char smem[];
-    div_rfft_x_block<T, MAXB>(g, c, UP, VP, WP, spec, rad, tw, nk2, kc, step, src, blockIdx.x, blockIdx.y, smem, wide);
+    const TileXY t = xcd_tile_xy();
+    div_rfft_x_block<T, MAXB>(g, c, UP, VP, WP, spec, rad, tw, nk2, kc, step, src, t.x, t.y, smem, wide);
 }
 
 template <typename T, int MAXB>
 __global__ void __launch_bounds__(kThreadsX) k_irfft_x_out(Geo g, const T *__restrict__ spec, T *__restrict__ PI, Radix rad,
                                                           const double *tw, int nk2, int kc, int half) {
     extern __shared__ unsigned char smem[];
-    irfft_x_out_block<T, MAXB>(g, spec, PI, rad, tw, nk2, kc, blockIdx.x, blockIdx.y, smem, half);
+    const TileXY t = xcd_tile_xy();
+    irfft_x_out_block<T, MAXB>(g, spec, PI, rad, tw, nk2, kc, t.x, t.y, smem, half);
 }
 
 // The same after the half-slab j pass, one block per row pair (j', jhalf + j') and chunk of kc levels:
@@ -1358,7 +1361,8 @@ template <typename T, int MAXB>
 __global__ void __launch_bounds__(kThreadsX) k_irfft_x_out_pair(Geo g, const T *__restrict__ spec, T *__restrict__ PI, Radix rad,
                                                                const double *tw, int nk2, int kc, int jhalf) {
     extern __shared__ unsigned char smem[];
-    irfft_x_out_pair_block<T, MAXB>(g, spec, PI, rad, tw, nk2, kc, blockIdx.x, blockIdx.y, smem, jhalf);
+    const TileXY t = xcd_tile_xy();
+    irfft_x_out_pair_block<T, MAXB>(g, spec, PI, rad, tw, nk2, kc, t.x, t.y, smem, jhalf);
 }
 
 // Q2 on half slabs (even nj, L = nj/2): the j transform's first radix-2 split (decimation in frequency)
@@ -1633,7 +1637,7 @@ template <typename T, bool DFT, int MAXB>
 __global__ void __launch_bounds__(kThreadsX) k_ens_div_rfft_x(const EnsMember *mem, int nmem, EnsRoles roles, int total, double step) {
     extern __shared__ __align__(16) unsigned char smem[];
     {
-        const int item = blockIdx.x;
+        const int item = xcd_tile(blockIdx.x, gridDim.x);
         const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::px0)];
         if (DFT && e.dftx) {
             div_dft_x_block<T, kEnsTiles, false>(e.g, e.c, (const T *)e.buf[DYN_U][roles.r[DYN_U][DYN_ROLE_P]],
@@ -1653,7 +1657,7 @@ template <typename T, bool DFT, int MAXB>
 __global__ void __launch_bounds__(kThreadsX) k_ens_irfft_x_out(const EnsMember *mem, int nmem, int total) {
     extern __shared__ __align__(16) unsigned char smem[];
     {
-        const int item = blockIdx.x;
+        const int item = xcd_tile(blockIdx.x, gridDim.x);
         const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::px0)];
         if (DFT && e.dftx) {
             idft_x_out_block<T, kEnsTiles>(e.g, (const T *)e.spec, (T *)e.pi, e.ni, e.dftx, e.nk2, item - e.px0, smem);
@@ -1668,7 +1672,7 @@ template <typename T, int THREADS, bool DFT>
 __global__ void __launch_bounds__(THREADS) k_ens_ypass(const EnsMember *mem, int nmem, int total) {
     extern __shared__ __align__(16) unsigned char smem[];
     {
-        const int item = blockIdx.x;
+        const int item = xcd_tile(blockIdx.x, gridDim.x);
         const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::py0)];
         ThomasArgs ta{e.acoef, e.ccoef, e.zpiv, e.ni, e.nj, e.g.NZ};
         if constexpr (DFT) {
