@@ -36,9 +36,11 @@ template <typename T>
 __device__ __forceinline__ T i3(T pm1, T p0, T p1, T p2, T sign) { return face_i3(pm1, p0, p1, p2, sign); }
 template <typename T>
 __device__ __forceinline__ T i2(T p0, T p1) { return T(0.5) * (p1 + p0); }
-// thread -> point (i, j, k) of the whole array, k fastest (every lane busy whatever NZ is)
+// thread -> point (i, j, k) of the whole array, k fastest (every lane busy whatever NZ is); an XCD's blocks cover one
+// run of columns, so the stencils' neighbours come from its own L2 (192x192x40 FP64: faces AF0 -> AF1 us, gather
+// AG0 -> AG1)
 __device__ __forceinline__ bool point_of(const Geo &g, int &i, int &j, int &k) {
-    const unsigned q = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned q = (unsigned)xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (q >= (unsigned)g.NX * (unsigned)g.NYNZ) return false;
     i = (int)(q / (unsigned)g.NYNZ);
     const int r = (int)(q - (unsigned)i * (unsigned)g.NYNZ);
@@ -54,7 +56,9 @@ struct AdvAdjArgs {
     const T *UB, *VB, *WB, *THB;  // basic state
     const T *PU, *PV, *PW, *PTH;  // adjoints of the forecast buffers
     T *CU, *CV, *CW, *CTH;        // adjoints of the current buffers (accumulated)
+    T *MU, *MV, *MW, *MTH;        // adjoints of the M buffers (take the forecasts')
     int il, ih, jl, jh;
+    bool dead;                    // the box of the current adjoints is to be read as zero
 };
 
 // Transpose of advect_uvw_velocity + advect_theta over the box at fixed upwind signs, in two passes.
@@ -279,10 +283,21 @@ __global__ void __launch_bounds__(256) k_adj_gather(Geo g, Cols c, AdvAdjArgs<T>
         if (icol && jrow) gth += dt * T(kGrav) * T(0.5) * (aw0 + (k + 1 < NZ ? aw1 : T(0))) / T(tbvk);
     }
     const long long p = IX(i, j, k);
-    a.CU[p] += gu;
-    a.CV[p] += gv;
-    a.CW[p] += gw;
-    a.CTH[p] += gth;
+    // forecast = M + step * tendency on the box: the M adjoint takes the forecast adjoint, which the overwrite then
+    // clears.  Its neighbours still read it here, so it is left as it is and the box counts as zero from now on
+    // (AdjState::dead): the next gather into that buffer stores instead of adding.
+    const bool box = icol && jrow && krow, boxw = box && k >= 2;
+    if (box) {
+        a.MU[p] += a.PU[p];
+        a.MV[p] += a.PV[p];
+        a.MTH[p] += a.PTH[p];
+        if (boxw) a.MW[p] += a.PW[p];
+    }
+    const bool st = a.dead && box, stw = a.dead && boxw;
+    a.CU[p] = st ? gu : a.CU[p] + gu;
+    a.CV[p] = st ? gv : a.CV[p] + gv;
+    a.CW[p] = stw ? gw : a.CW[p] + gw;
+    a.CTH[p] = st ? gth : a.CTH[p] + gth;
 }
 
 // Pass 1 with every load unconditional: indices are pulled into the array (IXC) and only the stores are
@@ -386,44 +401,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
 
 #undef IXC
 
-// forecast = M + step * tendency on the box: the M adjoint takes the forecast adjoint, which the overwrite
-// then clears
+// zero in the box of buffers left dead by k_adj_gather
 template <typename T>
-__global__ void k_adj_advect_finish(Geo g, T *MU, T *MV, T *MW, T *MTH, T *PU, T *PV, T *PW, T *PTH, int il, int jl, int jh) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int j = blockIdx.y * blockDim.y + threadIdx.y + jl;
-    const int i = blockIdx.z + il;
-    if (k > g.NZ - 2 || j >= jh) return;
-    const long long p = IX(i, j, k);
-    MU[p] += PU[p];
-    PU[p] = T(0);
-    MV[p] += PV[p];
-    PV[p] = T(0);
-    MTH[p] += PTH[p];
-    PTH[p] = T(0);
-    if (k >= 2) {
-        MW[p] += PW[p];
-        PW[p] = T(0);
-    }
-}
-
-// transpose of the pressure-gradient force (solver.cpp:123-135) over [1,NX-1) x [1,NY-1): the forecast
-// adjoints pass through, PI's adjoint gathers the gradient stencil
-template <typename T>
-__global__ void k_adj_pgf(Geo g, Cols c, const T *__restrict__ UH, const T *__restrict__ VH, const T *__restrict__ WH,
-                          T *__restrict__ PH, T step) {
+__global__ void k_adj_clear_box(Geo g, T *PU, T *PV, T *PW, T *PTH, int il, int ih, int jl, int jh) {
     int i, j, k;
-    if (!point_of(g, i, j, k)) return;
-    auto inr = [&](int ii, int jj, int kk) { return ii >= 1 && ii < g.NX - 1 && jj >= 1 && jj < g.NY - 1 && kk >= 1 && kk <= g.NZ - 2; };
+    if (!point_of(g, i, j, k) || i < il || i >= ih || j < jl || j >= jh || k < 1 || k > g.NZ - 2) return;
     const long long p = IX(i, j, k);
-    const T sx = step * T(g.dtx), sy = step * T(g.dty);
-    T acc = T(0);
-    if (inr(i, j, k)) acc -= sx * UH[p] + sy * VH[p];
-    if (inr(i + 1, j, k)) acc += sx * UH[p + g.NYNZ];
-    if (inr(i, j + 1, k)) acc += sy * VH[p + g.NZ];
-    if (inr(i, j, k) && k >= 2) acc -= step * (T(g.dtz) * T(c.mw[k])) * WH[p];
-    if (inr(i, j, k + 1) && k + 1 >= 2) acc += step * (T(g.dtz) * T(c.mw[k + 1])) * WH[p + 1];
-    PH[p] += acc;
+    PU[p] = PV[p] = PTH[p] = T(0);
+    if (k >= 2) PW[p] = T(0);
 }
 
 struct AdjList {
@@ -454,15 +439,16 @@ __global__ void k_adj_lid(Geo g, AdjList fl, int nfill) {
     }
 }
 
-// transpose of periodic_boundaries_east_west: halo adjoints return to their source columns
+// transpose of periodic_boundaries_east_west: halo adjoints return to their source columns; a thread per field
+// (and per halo column where no column is a source twice, NX >= 12)
 template <typename T>
 __global__ void k_adj_periodic(Geo g, AdjList fl) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= g.NYNZ) return;
     const long long s = g.NYNZ;
-    for (int f = 0; f < fl.n; f++) {
-        T *A = (T *)fl.f[f];
-        for (int h = 0; h < 3; h++) {
+    {
+        T *A = (T *)fl.f[blockIdx.y];
+        for (int h = blockIdx.z; h < 3; h += gridDim.z) {
             A[q + (long long)(g.NX - 6 + h) * s] += A[q + (long long)h * s];
             A[q + (long long)h * s] = T(0);
             A[q + (long long)(3 + h) * s] += A[q + (long long)(g.NX - 3 + h) * s];
@@ -508,8 +494,12 @@ __global__ void k_adj_rayleigh(Geo g, const double *__restrict__ coef, T *U, T *
     TH[p] -= cu * TH[p];
 }
 
+struct AddClear {
+    void *dst[kAdjFields], *src[kAdjFields];
+};
 template <typename T>
-__global__ void k_add_clear(T *__restrict__ dst, T *__restrict__ src, long long n) {
+__global__ void k_add_clear(AddClear l, long long n) {
+    T *__restrict__ dst = (T *)l.dst[blockIdx.y], *__restrict__ src = (T *)l.src[blockIdx.y];
     const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (p < n) {
         dst[p] += src[p];
@@ -579,7 +569,8 @@ struct AdjState {
     bool adj_pending[2] = {false, false};  // ev_adj[b]: adjoint steps that read rec[b] were queued
     void *spec_a = nullptr, *spec2_a = nullptr;
     void *adj[kAdjFields][3] = {{nullptr}};
-    void *pihat = nullptr, *r1 = nullptr, *r2 = nullptr;
+    int dead = -1;  // role whose buffers' box [3, NX-3) x [3, NY-3) counts as zero (-1: none)
+    void *r1 = nullptr, *r2 = nullptr;
     void *faces[18] = {nullptr};  // per-face adjoint weights of the advection transpose (Aw, G per kind)
     void *face_sgn[9] = {nullptr};  // per-face upwind signs (one byte each)
     double *stage_dbl = nullptr;  // host-transfer staging (double)
@@ -600,7 +591,7 @@ void adj_free(Ctx *c) {
     for (hipEvent_t e : {s->ev_rec[0], s->ev_rec[1], s->ev_adj[0], s->ev_adj[1]})
         if (e) (void)hipEventDestroy(e);
     if (s->astream) (void)hipStreamDestroy(s->astream);
-    void *ptrs[] = {s->pihat, s->r1, s->r2, s->stage_dbl, s->spec_a, s->spec2_a};
+    void *ptrs[] = {s->r1, s->r2, s->stage_dbl, s->spec_a, s->spec2_a};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (void *p : s->faces)
@@ -661,8 +652,8 @@ int bc_adjoint(Ctx *c) {
     hipLaunchKernelGGL(k_adj_lid<T>, dim3((g.NY - 1 + 63) / 64, g.NX - 1), dim3(64), 0, c->stream, g, AdjList{{U, V, TH, W}, 4}, 3);
     DYN_LAUNCH_CHECK();
     const long long n = g.NYNZ;
-    hipLaunchKernelGGL(k_adj_periodic<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, g,
-                       AdjList{{U, V, s->pihat, TH, W}, 5});
+    hipLaunchKernelGGL(k_adj_periodic<T>, dim3((unsigned)((n + 255) / 256), 4, g.NX >= 12 ? 3 : 1), dim3(256), 0, c->stream, g,
+                       AdjList{{U, V, TH, W}, 4});
     DYN_LAUNCH_CHECK();
     const int rows = c->g.sponge_south + c->g.sponge_north;
     if (rows > 0) {
@@ -681,17 +672,12 @@ int stage_adjoint(Ctx *c, int n, int stage, double step) {
     auto P = [&](int f) { return (T *)s->adj[f][DYN_ROLE_P]; };
     int rc = bc_adjoint<T>(c);
     if (rc) return rc;
-    {
-        Timed _t(c, "adj_pgf", (double)c->npts);
-        hipLaunchKernelGGL(k_adj_pgf<T>, point_grid(g), dim3(256), 0, c->stream, g, c->cols,
-                           (const T *)P(0), (const T *)P(1), (const T *)P(2), (T *)s->pihat, T(step));
-        DYN_LAUNCH_CHECK();
-    }
-    rc = launch_pressure_adjoint(c, step, s->pihat, P(0), P(1), P(2), s->r1, s->r2);
+    // the gradient force and the solve
+    rc = launch_pressure_adjoint(c, step, P(0), P(1), P(2), s->r1, s->r2);
     if (rc) return rc;
     {  // periodic_uvw_boundaries of solve_pressure
         const long long nq = g.NYNZ;
-        hipLaunchKernelGGL(k_adj_periodic<T>, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, c->stream, g,
+        hipLaunchKernelGGL(k_adj_periodic<T>, dim3((unsigned)((nq + 255) / 256), 3, g.NX >= 12 ? 3 : 1), dim3(256), 0, c->stream, g,
                            AdjList{{P(0), P(1), P(2)}, 3});
         DYN_LAUNCH_CHECK();
     }
@@ -714,6 +700,11 @@ int stage_adjoint(Ctx *c, int n, int stage, double step) {
     a.CV = (T *)s->adj[1][DYN_ROLE_CUR];
     a.CW = (T *)s->adj[2][DYN_ROLE_CUR];
     a.CTH = (T *)s->adj[3][DYN_ROLE_CUR];
+    a.MU = (T *)s->adj[0][DYN_ROLE_M];
+    a.MV = (T *)s->adj[1][DYN_ROLE_M];
+    a.MW = (T *)s->adj[2][DYN_ROLE_M];
+    a.MTH = (T *)s->adj[3][DYN_ROLE_M];
+    a.dead = s->dead == DYN_ROLE_CUR;
     a.il = 3;
     a.ih = NX - 3;
     a.jl = 3;
@@ -728,16 +719,14 @@ int stage_adjoint(Ctx *c, int n, int stage, double step) {
         DYN_LAUNCH_CHECK();
         hipLaunchKernelGGL(k_adj_gather<T>, point_grid(g), dim3(256), 0, c->stream, g, c->cols, a, fa, T(step));
         DYN_LAUNCH_CHECK();
-        auto M = [&](int f) { return (T *)s->adj[f][DYN_ROLE_M]; };
-        hipLaunchKernelGGL(k_adj_advect_finish<T>, dim3((g.NZ - 2 + 63) / 64, (a.jh - a.jl + 3) / 4, a.ih - a.il), dim3(64, 4), 0, c->stream, g,
-                           M(0), M(1), M(2), M(3), P(0), P(1), P(2), P(3), a.il, a.jl, a.jh);
-        DYN_LAUNCH_CHECK();
+        s->dead = DYN_ROLE_P;
     }
     return DYN_OK;
 }
 
 void swap_cur_p(AdjState *s) {
     for (int f = 0; f < kAdjFields; f++) std::swap(s->adj[f][DYN_ROLE_CUR], s->adj[f][DYN_ROLE_P]);
+    if (s->dead >= 0) s->dead = s->dead == DYN_ROLE_P ? DYN_ROLE_CUR : DYN_ROLE_P;
 }
 
 // reverse of one forward step n (records of the step's stages in place)
@@ -749,10 +738,13 @@ int step_adjoint(Ctx *c, int n) {
     const dim3 blocks((unsigned)((npts + 255) / 256));
     // advance_outer: memcpy(M <- P) then swap(current, forecast)
     swap_cur_p(s);
+    AddClear ac;
     for (int f = 0; f < kAdjFields; f++) {
-        hipLaunchKernelGGL(k_add_clear<T>, blocks, dim3(256), 0, c->stream, (T *)s->adj[f][DYN_ROLE_P], (T *)s->adj[f][DYN_ROLE_M], npts);
-        DYN_LAUNCH_CHECK();
+        ac.dst[f] = s->adj[f][DYN_ROLE_P];
+        ac.src[f] = s->adj[f][DYN_ROLE_M];
     }
+    hipLaunchKernelGGL(k_add_clear<T>, dim3(blocks.x, kAdjFields), dim3(256), 0, c->stream, ac, npts);
+    DYN_LAUNCH_CHECK();
     if (c->g.rayleigh_level < c->g.nz) {
         const int lev = c->g.rayleigh_level;
         hipLaunchKernelGGL(k_adj_rayleigh<T>, dim3((g.NZ - lev + 63) / 64, (g.NY - 2 + 3) / 4, g.NX - 2), dim3(64, 4), 0, c->stream, g,
@@ -776,7 +768,7 @@ int step_adjoint(Ctx *c, int n) {
 int ensure_pipeline(Ctx *c) {
     AdjState *s = c->adj;
     if (s->astream) return DYN_OK;
-    const size_t spec_bytes = sizeof(double) * 2 * (size_t)c->pp.ni * c->pp.nj * c->pp.nk2;
+    const size_t spec_bytes = pressure_spec_bytes(c->pp);
     if (alloc_fields(s, s->rec[1], (size_t)s->every * 12, s->field_bytes) != DYN_OK) {
         set_error("");
         return DYN_E_HIP;
@@ -802,8 +794,7 @@ int backward_t(Ctx *c, const double *const *seed, double *const *grad) {
             hipLaunchKernelGGL(k_zero<T>, blocks, dim3(256), 0, c->stream, (T *)s->adj[f][r], npts);
             DYN_LAUNCH_CHECK();
         }
-    hipLaunchKernelGGL(k_zero<T>, blocks, dim3(256), 0, c->stream, (T *)s->pihat, npts);
-    DYN_LAUNCH_CHECK();
+    s->dead = -1;
     // seed: the adjoint of the final current buffers
     for (int f = 0; f < kAdjFields; f++) {
         if (!seed[f]) continue;
@@ -894,6 +885,13 @@ int backward_t(Ctx *c, const double *const *seed, double *const *grad) {
         }
         DYN_HIP(hipStreamWaitEvent(c->stream, s->ev_adj[b], 0));  // the gradients follow the last adjoint step
     }
+    if (s->dead >= 0) {
+        const Geo &g = c->geo;
+        hipLaunchKernelGGL(k_adj_clear_box<T>, point_grid(g), dim3(256), 0, c->stream, g, (T *)s->adj[0][s->dead], (T *)s->adj[1][s->dead],
+                           (T *)s->adj[2][s->dead], (T *)s->adj[3][s->dead], 3, g.NX - 3, 3, g.NY - 3);
+        DYN_LAUNCH_CHECK();
+        s->dead = -1;
+    }
     // the initial fields are set into all three buffers: their gradient is the sum of the three adjoints
     for (int f = 0; f < kAdjFields; f++) {
         if (!grad[f]) continue;
@@ -971,7 +969,6 @@ int dyn_adjoint_record(dyn_ctx *ctx, int nsteps, int every) {
     }
     for (auto &f : s->adj)
         for (auto &p : f) DYN_HIP(hipMalloc(&p, s->field_bytes));
-    DYN_HIP(hipMalloc(&s->pihat, s->field_bytes));
     DYN_HIP(hipMalloc(&s->r1, s->field_bytes));
     DYN_HIP(hipMalloc(&s->r2, s->field_bytes));
     for (auto &p : s->faces) DYN_HIP(hipMalloc(&p, s->field_bytes));

@@ -310,7 +310,7 @@ int pressure_free(Ctx *c);
 // queued; a nonzero return ends the solve with that code
 using PressureHook = int (*)(Ctx *c, void *arg);
 int launch_solve_pressure(Ctx *c, double step, bool halos = true, PressureHook after_i = nullptr, void *arg = nullptr);
-int launch_pressure_adjoint(Ctx *c, double step, void *pihat, void *uh, void *vh, void *wh, void *r1, void *r2);
+int launch_pressure_adjoint(Ctx *c, double step, void *uh, void *vh, void *wh, void *r1, void *r2);
 int launch_convert(Ctx *c, void *dst, const double *src, size_t n, bool to_device_type);
 void adjoint_release(Ctx *c);
 // a whole RK3 step with a callback at the start of each stage (stage 0, 1, 2); a non-zero return aborts
@@ -328,6 +328,7 @@ int ens_prepare(bool fp32);
 int launch_ens_stage(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, const int *shape, int tot_mom, int tot_scal);
 int launch_ens_post(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, bool pgf, int total);
 int launch_ens_copy(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, int total);
+size_t pressure_spec_bytes(const PressurePlan &pp);
 bool pressure_ens_fill(Ctx *c, EnsMember &e, size_t &lds_x, size_t &lds_y);
 int pressure_ens_prepare(const Ctx *c);
 // xform: the i passes with up to three butterflies a thread (0), four (1), four and members by matrix products (2); yform: the j pass in blocks of 512 threads (0), of 1024 (1), of 1024 with members by matrix products (2)

@@ -2088,22 +2088,37 @@ int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
 
 
 // ---- adjoint of the solve (transposed projection for the hand-written adjoint) -----------------------
-// Transpose of P5's output stage: the value v(i, j, kk) was written to PI at (i+3, j, kk+1), at the ghost
-// level 0 (kk = 0) or NZ-1 (kk = nk2-1), and at the periodic halo copies; its adjoint is the sum of the
-// adjoints of every location it was written to.
+// Transpose of the pressure-gradient force (solver.cpp:123-135) over [1,NX-1) x [1,NY-1), which gathers PI's adjoint
+// at a point from the forecast velocities' (they pass through), and of P5's output stage: the value v(i, j, kk)
+// was written to PI at (i+3, j, kk+1), at the ghost level 0 (kk = 0) or NZ-1 (kk = nk2-1), and at the periodic halo
+// copies; its adjoint is the sum of the adjoints of every location it was written to.
 template <typename T>
-__global__ void k_adj_pi_fold(Geo g, const T *__restrict__ PH, T *__restrict__ R, int nk2) {
-    const int kk = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y, ia = blockIdx.z + 3;
-    if (kk >= nk2) return;
+__global__ void k_adj_pi_fold(Geo g, Cols c, const T *__restrict__ UH, const T *__restrict__ VH, const T *__restrict__ WH,
+                              T *__restrict__ R, int nk2, T step) {
+    // levels, rows and columns one after another over the lanes
+    const unsigned q = (unsigned)xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x, row = q / (unsigned)nk2;
+    const int kk = (int)(q - row * (unsigned)nk2), j = (int)(row % (unsigned)g.NY), ia = (int)(row / (unsigned)g.NY) + 3;
+    if (ia >= g.NX - 3) return;
+    auto inr = [&](int ii, int jj, int kz) { return ii >= 1 && ii < g.NX - 1 && jj >= 1 && jj < g.NY - 1 && kz >= 1 && kz <= g.NZ - 2; };
+    const T sx = step * T(g.dtx), sy = step * T(g.dty);
+    auto pgf = [&](int i, int k) -> T {
+        const long long p = IX(i, j, k);
+        T acc = T(0);
+        if (inr(i, j, k)) acc -= sx * UH[p] + sy * VH[p];
+        if (inr(i + 1, j, k)) acc += sx * UH[p + g.NYNZ];
+        if (inr(i, j + 1, k)) acc += sy * VH[p + g.NZ];
+        if (inr(i, j, k) && k >= 2) acc -= step * (T(g.dtz) * T(c.mw[k])) * WH[p];
+        if (inr(i, j, k + 1) && k + 1 >= 2) acc += step * (T(g.dtz) * T(c.mw[k + 1])) * WH[p + 1];
+        return acc;
+    };
     const int shift = g.NX - 6, k = kk + 1;
     const int ks[3] = {k, kk == 0 ? 0 : -1, kk == nk2 - 1 ? g.NZ - 1 : -1};
     T v = T(0);
     for (int t = 0; t < 3; t++) {
         if (ks[t] < 0) continue;
-        v += PH[IX(ia, j, ks[t])];
-        if (ia >= shift && ia < shift + 3) v += PH[IX(ia - shift, j, ks[t])];
-        if (ia >= 3 && ia < 6) v += PH[IX(ia + shift, j, ks[t])];
+        v += pgf(ia, ks[t]);
+        if (ia >= shift && ia < shift + 3) v += pgf(ia - shift, ks[t]);
+        if (ia >= 3 && ia < 6) v += pgf(ia + shift, ks[t]);
     }
     R[IX(ia, j, k)] = v;
 }
@@ -2114,7 +2129,7 @@ __global__ void k_adj_pi_fold(Geo g, const T *__restrict__ PH, T *__restrict__ R
 template <typename T>
 __global__ void k_adj_div(Geo g, Cols c, const T *__restrict__ R, T *__restrict__ UH, T *__restrict__ VH, T *__restrict__ WH,
                           double step) {
-    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long q = (long long)xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (q >= (long long)g.NX * g.NYNZ) return;
     const int x = (int)(q / g.NYNZ), r = (int)(q - (long long)x * g.NYNZ), y = r / g.NZ, k = r - y * g.NZ;
     const T sdt = T(step * g.dt);
@@ -2145,13 +2160,7 @@ __global__ void k_adj_div(Geo g, Cols c, const T *__restrict__ R, T *__restrict_
 }
 
 template <typename T>
-__global__ void k_zero_field(T *__restrict__ A, long long n) {
-    long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < n) A[p] = T(0);
-}
-
-template <typename T>
-int solve_adjoint_t(Ctx *c, double step, T *pihat, T *uh, T *vh, T *wh, T *r1, T *r2) {
+int solve_adjoint_t(Ctx *c, double step, T *uh, T *vh, T *wh, T *r1, T *r2) {
     PressurePlan &pp = c->pp;
     const Geo &g = c->geo;
     if (pp.ni % 2 != 0 || !pp.smooth_x) {
@@ -2165,10 +2174,8 @@ int solve_adjoint_t(Ctx *c, double step, T *pihat, T *uh, T *vh, T *wh, T *r1, T
     const double pts = (double)pp.ni * pp.nj * pp.nk2;
     {
         Timed _t(c, "adj_pi_fold", pts);
-        hipLaunchKernelGGL(k_adj_pi_fold<T>, dim3((pp.nk2 + 63) / 64, g.NY, pp.ni), dim3(64), 0, c->stream, g, (const T *)pihat, r1, pp.nk2);
-        DYN_LAUNCH_CHECK();
-        long long n = (long long)c->npts;
-        hipLaunchKernelGGL(k_zero_field<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, pihat, n);
+        hipLaunchKernelGGL(k_adj_pi_fold<T>, dim3((unsigned)(((long long)pp.ni * g.NY * pp.nk2 + 255) / 256)), dim3(256), 0, c->stream, g,
+                           c->cols, (const T *)uh, (const T *)vh, (const T *)wh, r1, pp.nk2, T(step));
         DYN_LAUNCH_CHECK();
     }
     T *spec = (T *)pp.spec;
@@ -2236,6 +2243,13 @@ int y_lds_limits(int most) {
 
 }  // namespace
 
+// Bytes of a spectrum buffer: the full complex spectrum in 64 bits, or the two half spectra of an FP32 context's products
+// (more than that on the narrowest grids)
+size_t pressure_spec_bytes(const PressurePlan &pp) {
+    const size_t col = (size_t)pp.nj * pp.nk2 * 2 * sizeof(double);
+    return std::max(col * pp.ni, wide_spec_at(pp) + col * (pp.ni / 2 + 1));
+}
+
 int pressure_init(Ctx *c) {
     PressurePlan &pp = c->pp;
     const int NZ = c->g.nz;
@@ -2261,9 +2275,7 @@ int pressure_init(Ctx *c) {
         set_error("pressure solver: twiddle upload failed");
         return DYN_E_HIP;
     }
-    // (on the narrowest grids the two half spectra of an FP32 context take more than the full one in 64 bits)
-    DYN_HIP(hipMalloc(&pp.spec, std::max(sizeof(double) * 2 * (size_t)pp.ni * pp.nj * pp.nk2,
-                                         wide_spec_at(pp) + sizeof(double) * 2 * (size_t)(pp.ni / 2 + 1) * pp.nj * pp.nk2)));
+    DYN_HIP(hipMalloc(&pp.spec, pressure_spec_bytes(pp)));
     int dev = 0, lds = 0;
     DYN_HIP(hipGetDevice(&dev));
     DYN_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
@@ -2457,13 +2469,13 @@ int launch_pressure_ens(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &r
     return DYN_OK;
 }
 
-// adjoint of solve_pressure(step) minus its periodic_uvw_boundaries: consumes (and zeroes) the adjoint of
-// PI and adds the adjoint of the divergence input to the forecast-velocity adjoints; r1, r2 are scratch
-// fields of the context's element type
-int launch_pressure_adjoint(Ctx *c, double step, void *pihat, void *uh, void *vh, void *wh, void *r1, void *r2) {
+// adjoint of the gradient force and of solve_pressure(step) minus its periodic_uvw_boundaries: PI's adjoint from the
+// forecast-velocity adjoints, to which the adjoint of the divergence input is added; r1, r2 are scratch fields of
+// the context's element type
+int launch_pressure_adjoint(Ctx *c, double step, void *uh, void *vh, void *wh, void *r1, void *r2) {
     if (c->prec == DYN_FP32)
-        return solve_adjoint_t<float>(c, step, (float *)pihat, (float *)uh, (float *)vh, (float *)wh, (float *)r1, (float *)r2);
-    return solve_adjoint_t<double>(c, step, (double *)pihat, (double *)uh, (double *)vh, (double *)wh, (double *)r1, (double *)r2);
+        return solve_adjoint_t<float>(c, step, (float *)uh, (float *)vh, (float *)wh, (float *)r1, (float *)r2);
+    return solve_adjoint_t<double>(c, step, (double *)uh, (double *)vh, (double *)wh, (double *)r1, (double *)r2);
 }
 
 }  // namespace dyn
