@@ -2289,19 +2289,26 @@ int pressure_init(Ctx *c) {
     const int nthr = f32 ? ypass_threads<float>() : ypass_threads<double>();
     const int maxb = f32 ? ypass_maxb<float>() : ypass_maxb<double>();
     pp.fused_y = pp.smooth_y && need <= pp.lds_max && 2 * pp.nj <= nthr && max_butterflies(ry, pp.nk2, nthr) <= maxb;
-    // Which sides go by matrix products: lengths with a prime factor above 5, and short smooth ones.  FP32 grids
-    // whose sides are both smooth (and even along i) take them on both sides or on neither: what a factored FP32
-    // transform loses on one side the products' 64 bits on the other don't give back (pi of 160x128x40, 6 steps,
-    // is 2 to 6e-6 off either way, 313 us a step against 314), while both together lose an order less.  Dry ones
-    // that an ensemble can hold, past 64 points a side, keep the factored passes: a member's bits are those of
-    // its run alone, and the batch, which fills the chip without them, is no faster with products (32 members
-    // of 96 to 192 points a side: 4.87 ms a step against 4.82).
+    // Which sides go by matrix products: lengths with a prime factor above 5, and short smooth ones.
+    // FP32 is choosier.  The longest waves' columns are nearly singular systems, the more so the wider the domain is
+    // for its depth, and what a factored FP32 transform rounds away on one side the products' 64 bits on the
+    // other don't give back (pi of 160x128x40, 6 steps, is 2 to 6e-6 off a 64-bit run either way, at 313 and
+    // 314 us a step).  So smooth sides (even along i) take products on both or on neither, and only in domains up
+    // to twice as many points wide as deep, where the change of rounding stays at 1e-5 of pi and below (2e-4 at
+    // 190x190x12 after two steps).  Dry domains wider than that keep the former passes whatever their factors, and
+    // with smooth sides past 64 points at every width that an ensemble can hold: its members' bits are those
+    // of runs alone, and a batch fills the chip without products (32 members of 96 to 192 points: 4.87 ms a
+    // step with them, 4.82 without).
+    const int widest = std::max(pp.ni, pp.nj);
+    const bool shallow = widest > 2 * c->g.nz, dry = !c->g.microphysics;
     bool prod_x = pp.ni <= (!pp.smooth_x ? kDftMax : f32 ? dft_x_smooth<float>() : dft_x_smooth<double>());
     bool prod_y = pp.nj <= (!pp.smooth_y ? kDftMax : kDftYSmooth);
     if (f32 && pp.smooth_x && pp.smooth_y && pp.ni % 2 == 0) {
         const bool y_taken = prod_y && (pp.nj <= kDftYThree || !pp.fused_y);
-        const bool batched = !c->g.microphysics && fused_waves(c) == 1 && std::max(pp.ni, pp.nj) > 64;
-        prod_x = prod_y = prod_x && y_taken && !batched;
+        const bool batched = dry && fused_waves(c) == 1 && widest > 64;
+        prod_x = prod_y = prod_x && y_taken && !shallow && !batched;
+    } else if (f32 && dry && shallow) {
+        prod_x = prod_y = false;
     }
     auto matrices = [](int n, double **out) -> int {
         const std::vector<double> h = dft_matrices(n);
