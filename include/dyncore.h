@@ -165,7 +165,8 @@ void *dyn_stream(dyn_ctx *ctx);
  * returns DYN_E_ARG.  Setting a knob drops the captured step graph.  dyn_tune_get returns a knob's value or
  * its nominal default.  While the knobs of a stage kernel are unset, grids whose nominal blocks would leave
  * compute units idle, and level counts far from a wavefront's 64 lanes, are launched in a shape chosen from
- * the grid's size instead, and DYN_TUNE_STAGE_STREAMS likewise; the values computed never depend on it. */
+ * the grid's size instead, and DYN_TUNE_STAGE_STREAMS likewise (small grids run both halves of a stage in one
+ * launch on one stream while all five are unset); the values computed never depend on it. */
 enum {
     DYN_TUNE_MOMENTUM_TJ = 0, /* j-rows per block of the momentum stage kernel: 2, 4, 8 or 16 (16, like 8,
                                  only with one wavefront per column) */

@@ -37,8 +37,8 @@ __device__ __forceinline__ T i3(T pm1, T p0, T p1, T p2, T sign) { return face_i
 template <typename T>
 __device__ __forceinline__ T i2(T p0, T p1) { return T(0.5) * (p1 + p0); }
 // thread -> point (i, j, k) of the whole array, k fastest (every lane busy whatever NZ is); an XCD's blocks cover one
-// run of columns, so the stencils' neighbours come from its own L2 (192x192x40 FP64: faces AF0 -> AF1 us, gather
-// AG0 -> AG1)
+// run of columns (no change for the two face passes, which their own loads and stores bound: 170 and 175 us, 123 and
+// 125 at 192x192x40 FP64)
 __device__ __forceinline__ bool point_of(const Geo &g, int &i, int &j, int &k) {
     const unsigned q = (unsigned)xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (q >= (unsigned)g.NX * (unsigned)g.NYNZ) return false;

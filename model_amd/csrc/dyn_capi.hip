@@ -963,8 +963,8 @@ static int fused_step(dyn_ctx *ctx, StageHook hook = nullptr, void *arg = nullpt
     return DYN_OK;
 }
 
-// the sequence dyn_step records: the fused stages when NZ fits one wavefront, else the per-operator
-// kernels
+// the sequence dyn_step records two of where it keeps one graph: the fused stages (with the turbulence closure), else
+// the per-operator kernels (NZ the fused kernels do not take)
 static int graph_step(dyn_ctx *ctx) {
     Ctx *c = as_ctx(ctx);
     if (fused_supported(c)) return fused_step(ctx);
@@ -1074,8 +1074,9 @@ static int replay_steps(Ctx *c, int steps, int times) {
 
 // Steps replayed from hipGraphs.  Fused steps: the first step ends with M and current sharing a buffer,
 // the steps between run from graphs of three such steps, the last step separates the roles again with
-// the M <- P copy.  Per-operator steps (NZ the fused kernels do not take) permute the current/forecast
-// buffers with period 2, so their graph records two steps and an odd trailing step runs eagerly.
+// the M <- P copy.  Per-operator steps (NZ the fused kernels do not take) and steps with the turbulence closure permute
+// the current/forecast buffers with period 2, so their graph records two steps and an odd trailing step runs
+// eagerly.
 int dyn_step(dyn_ctx *ctx, int nsteps) {
     Ctx *c = as_ctx(ctx);
     CHECK_CTX(c);

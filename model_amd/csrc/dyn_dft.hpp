@@ -13,7 +13,7 @@
 //
 // Measured, us of the i transforms (forward with the divergence, then inverse): against direct sums over the
 // prime factors, 194x100x40 FP32 194 + 185 -> 14.5 + 12.6, 251x251x94 FP64 2214 + 2166 -> 73 + 51; against the
-// radix passes of smooth lengths, FP64 64x64x40 20.6 + 18.7 -> 7.3 + 8.3, 192x192x40 42.2 + 33.4 -> 26.5 + 18.8,
+// radix passes of smooth lengths, FP64 64x64x40 20.6 + 18.7 -> 7.3 + 8.3, 192x192x40 42.2 + 33.4 -> 19.4 + 17.1,
 // 384x384x80 238 + 171 -> 211 + 141; FP32 64x64x40 14.9 + 14.2 -> 7.5 + 7.9, 192x192x40 27.3 + 23.7 -> 22.5 +
 // 18.1, but 256x256x64 33.1 + 28.3 -> 52.7 + 38.2: the work grows with n where the passes' grows with log n,
 // and FP32 passes move half the bytes, so FP32 changes over below 256.
@@ -27,7 +27,7 @@
 namespace dyn {
 namespace {
 
-// smooth lengths that take the matrix products: measured faster up to these
+// smooth lengths that take the matrix products: measured faster up to these (FP32 within the limits of pressure_init)
 template <typename T>
 constexpr int dft_x_smooth() { return sizeof(T) == 4 ? 192 : 384; }
 constexpr int kDftYSmooth = 192, kDftYThree = 112;

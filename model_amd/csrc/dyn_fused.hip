@@ -1379,7 +1379,8 @@ __device__ __forceinline__ PostArgs ens_post_args(const EnsMember &e, const EnsR
 }
 
 template <typename T, int TJ, bool MOIST, bool PACK>
-__global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_ens_momentum(const EnsMember *mem, int nmem, EnsRoles ro, T step, int tj, int ti, int total) {
+__global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_ens_momentum(const EnsMember *mem, int nmem, EnsRoles ro, T step,
+                                                                                   int tj, int ti, int total) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int item = xcd_tile(blockIdx.x, gridDim.x);
     const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::mom0)];
@@ -1388,7 +1389,8 @@ __global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_ens_momentum(co
 }
 
 template <typename T, int TJ, bool MOIST, bool PACK>
-__global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_ens_scalars(const EnsMember *mem, int nmem, EnsRoles ro, T step, int tj, int ti, int total) {
+__global__ void __launch_bounds__((stage_threads<TJ, PACK>())) k_ens_scalars(const EnsMember *mem, int nmem, EnsRoles ro, T step,
+                                                                                   int tj, int ti, int total) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int item = xcd_tile(blockIdx.x, gridDim.x);
     const EnsMember &e = mem[ens_member(mem, nmem, item, &EnsMember::scal0)];

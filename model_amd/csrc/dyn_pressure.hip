@@ -1136,7 +1136,8 @@ __device__ __forceinline__ void thomas_t_back_chunk(const ThomasCoef &co, const 
 // b_k = z_k (q_k - a_{k+1} b_{k+1}), result b / S.  The singular last pivot of (0,0) is never used.
 // The table entries come in chunks through two register sets that take turns, as in thomas_part.
 template <typename R, int kTC = kThomasChunk, typename T>
-__device__ __forceinline__ void thomas_part_t(const ThomasArgs &ta, const ThomasCoef &co, int kx, int ky, const double *Z, long long fs, T *x, int xs) {
+__device__ __forceinline__ void thomas_part_t(const ThomasArgs &ta, const ThomasCoef &co, int kx, int ky, const double *Z, long long fs,
+                                              T *x, int xs) {
     const int N = ta.nk - 2;
     const double size2d = (double)(ta.ni * ta.nj), rsize = 1.0 / size2d;
     const bool m0 = (kx == 0 && ky == 0);
@@ -1759,8 +1760,9 @@ size_t x_pass_lds(int ni, int kc, size_t elt);
 
 int max_butterflies(const Radix &r, int nbatch, int nthr);
 // The i passes hold a thread's butterflies of a radix pass in registers: the instance with no more of them than the
-// grid's pass needs (FP32 86 registers with four, 69 with three and 52 with two, so three and four blocks on a CU instead of two; FP64
-// 148, 120 and 92, so two instead of one).
+// grid's pass needs (FP32 86 registers with four, 69 with three and 52 with two, so two, three and four blocks on a
+// CU; FP64 148, 120 and 92, so one, two and two).  192x192x40 FP32 dry 390 -> 345 us a step, 512x256x40 FP64 1867 ->
+// 1745.
 template <typename T>
 auto div_rfft_x_kernel(const Radix &rx, int kc) {
     const int b = max_butterflies(rx, kc / 2, kThreadsX);
@@ -2443,7 +2445,8 @@ bool pressure_ens_fill(Ctx *c, EnsMember &e, size_t &lds_x, size_t &lds_y) {
 int pressure_ens_prepare(const Ctx *c) {
     const void *k[] = {(const void *)k_ens_div_rfft_x<float, false, 3>, (const void *)k_ens_irfft_x_out<float, false, 3>,
                        (const void *)k_ens_div_rfft_x<float, false, kMaxBX>, (const void *)k_ens_irfft_x_out<float, false, kMaxBX>,
-                       (const void *)k_ens_div_rfft_x<float, true, kMaxBX>, (const void *)k_ens_irfft_x_out<float, true, kMaxBX>, (const void *)k_ens_ypass<float, kEnsYNarrow, false>,
+                       (const void *)k_ens_div_rfft_x<float, true, kMaxBX>, (const void *)k_ens_irfft_x_out<float, true, kMaxBX>,
+                       (const void *)k_ens_ypass<float, kEnsYNarrow, false>,
                        (const void *)k_ens_ypass<float, 1024, false>, (const void *)k_ens_ypass<float, 1024, true>};
     for (const void *f : k) DYN_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->pp.lds_max));
     return DYN_OK;
@@ -2455,7 +2458,9 @@ int launch_pressure_ens(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &r
     {
         const int grid = tot_px;
         Timed _t(c0, "ens_p1_div_rfft_x", 0.0);
-        auto k = xform == 0 ? k_ens_div_rfft_x<float, false, 3> : xform == 1 ? k_ens_div_rfft_x<float, false, kMaxBX> : k_ens_div_rfft_x<float, true, kMaxBX>;
+        auto k = xform == 0   ? k_ens_div_rfft_x<float, false, 3>
+                 : xform == 1 ? k_ens_div_rfft_x<float, false, kMaxBX>
+                              : k_ens_div_rfft_x<float, true, kMaxBX>;
         hipLaunchKernelGGL(k, dim3(grid), dim3(kThreadsX), lds_x, c0->stream, d, nmem, ro, tot_px, step);
         DYN_LAUNCH_CHECK();
     }
@@ -2469,7 +2474,9 @@ int launch_pressure_ens(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &r
     {
         const int grid = tot_px;
         Timed _t(c0, "ens_p5_irfft_x_out", 0.0);
-        auto k = xform == 0 ? k_ens_irfft_x_out<float, false, 3> : xform == 1 ? k_ens_irfft_x_out<float, false, kMaxBX> : k_ens_irfft_x_out<float, true, kMaxBX>;
+        auto k = xform == 0   ? k_ens_irfft_x_out<float, false, 3>
+                 : xform == 1 ? k_ens_irfft_x_out<float, false, kMaxBX>
+                              : k_ens_irfft_x_out<float, true, kMaxBX>;
         hipLaunchKernelGGL(k, dim3(grid), dim3(kThreadsX), lds_x, c0->stream, d, nmem, tot_px);
         DYN_LAUNCH_CHECK();
     }
