@@ -76,14 +76,10 @@ int launch_zero_moisture_shell(Ctx *c, int il, int ih, int jl, int jh);
 int launch_post_stage(Ctx *c, double step, bool pgf, bool scalars, bool clip, bool uvw, int ray_level = -1,
                       bool interior_done = false);
 
-// the captured step graph bakes in launch shapes and the kernel sequence: drop it when a knob or the
+// the captured step graphs bake in launch shapes and the kernel sequence: drop them when a knob or the
 // turbulence switch changes
 void drop_graph(Ctx *c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
-    if (c->graph) (void)hipGraphDestroy(c->graph);
-    c->graph_exec = nullptr;
-    c->graph = nullptr;
     for (auto &sg : c->graphs) {
         (void)hipGraphExecDestroy(sg.exec);
         (void)hipGraphDestroy(sg.graph);
@@ -963,11 +959,10 @@ static int fused_step(dyn_ctx *ctx, StageHook hook = nullptr, void *arg = nullpt
     return DYN_OK;
 }
 
-// the sequence dyn_step records two of where it keeps one graph: the fused stages (with the turbulence closure), else
-// the per-operator kernels (NZ the fused kernels do not take)
-static int graph_step(dyn_ctx *ctx) {
-    Ctx *c = as_ctx(ctx);
-    if (fused_supported(c)) return fused_step(ctx);
+// one step of dyn_step: the fused stages (share_end as in fused_step), else the per-operator kernels (NZ the fused
+// kernels do not take)
+static int graph_step(dyn_ctx *ctx, bool share_end = false) {
+    if (fused_supported(as_ctx(ctx))) return fused_step(ctx, nullptr, nullptr, share_end);
     return reference_step(ctx);
 }
 
@@ -1034,7 +1029,7 @@ static int capture_step_graph(Ctx *c, int steps) {
     c->capturing = true;
     int rc = DYN_OK;
     const bool share = steps > 2 && !(steps % 2 == 0 && stage_in_one(c));
-    for (int n = 0; n < steps && !rc; n++) rc = fused_step(ctx, nullptr, nullptr, share && n < steps - 1);
+    for (int n = 0; n < steps && !rc; n++) rc = graph_step(ctx, share && n < steps - 1);
     c->capturing = false;
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(c->stream, &graph);
@@ -1074,9 +1069,9 @@ static int replay_steps(Ctx *c, int steps, int times) {
 
 // Steps replayed from hipGraphs.  Fused steps: the first step ends with M and current sharing a buffer,
 // the steps between run from graphs of three such steps, the last step separates the roles again with
-// the M <- P copy.  Per-operator steps (NZ the fused kernels do not take) and steps with the turbulence closure permute
-// the current/forecast buffers with period 2, so their graph records two steps and an odd trailing step runs
-// eagerly.
+// the M <- P copy.  Per-operator steps (NZ the fused kernels do not take) and steps with the turbulence closure run
+// from a graph of two steps, an odd trailing step eagerly.  Each of them exchanges the current and the forecast
+// buffer, so a call after an odd one meets the other assignment, which has a graph of its own.
 int dyn_step(dyn_ctx *ctx, int nsteps) {
     Ctx *c = as_ctx(ctx);
     CHECK_CTX(c);
@@ -1104,35 +1099,12 @@ int dyn_step(dyn_ctx *ctx, int nsteps) {
         if (!rc) rc = replay_steps(c, 2, n2);
         return rc;
     }
-    int pairs = nsteps / 2;
+    const int pairs = nsteps / 2;
     if (pairs > 0) {
-        if (!c->graph_exec) {
-            void *saved[7][3];
-            memcpy(saved, c->prog, sizeof(saved));
-            DYN_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-            c->capturing = true;
-            int rc = graph_step(ctx);
-            if (!rc) rc = graph_step(ctx);
-            c->capturing = false;
-            hipGraph_t graph = nullptr;
-            hipError_t e = hipStreamEndCapture(c->stream, &graph);
-            if (rc || e != hipSuccess) {
-                if (graph) (void)hipGraphDestroy(graph);
-                memcpy(c->prog, saved, sizeof(saved));
-                if (!rc) set_error(std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
-                return rc ? rc : DYN_E_HIP;
-            }
-            // two steps restore the buffer assignment
-            if (memcmp(saved, c->prog, sizeof(saved)) != 0) {
-                (void)hipGraphDestroy(graph);
-                memcpy(c->prog, saved, sizeof(saved));
-                set_error("internal: two steps did not restore the buffer assignment");
-                return DYN_E_STATE;
-            }
-            DYN_HIP(hipGraphInstantiate(&c->graph_exec, graph, nullptr, nullptr, 0));
-            c->graph = graph;
-        }
-        for (int p = 0; p < pairs; p++) DYN_HIP(hipGraphLaunch(c->graph_exec, c->stream));
+        if (!find_step_graph(c, 2))
+            if (int rc = capture_step_graph(c, 2)) return rc;
+        const hipGraphExec_t exec = find_step_graph(c, 2)->exec;
+        for (int p = 0; p < pairs; p++) DYN_HIP(hipGraphLaunch(exec, c->stream));
     }
     if (nsteps % 2) {
         int rc = graph_step(ctx);

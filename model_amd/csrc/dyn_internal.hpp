@@ -241,15 +241,12 @@ struct Ctx {
     int *dflag = nullptr;                             // device error flag (Kessler guard)
     int *fflag = nullptr;                             // device bit mask of fields holding a NaN or Inf
     PressurePlan pp;
-    // graph for dyn_step (per-operator steps: two steps restore the buffer assignment)
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t graph_exec = nullptr;
     // Between the fused steps of one dyn_step / dyn_step_fused call the M and current roles of the
     // stepped prognostics share a buffer (both hold the state at the start of the step); spare[f] is
     // then the field's third buffer, nullptr otherwise.  Calls end with M and current apart again.
     void *spare[7] = {nullptr};
-    // graphs of 6, 3 or 2 fused steps that restore the buffer assignment they start from, keyed by
-    // that assignment
+    // graphs of 6, 3 or 2 steps that restore the buffer assignment they start from, keyed by that
+    // assignment
     struct StepGraph {
         int steps;
         void *key[7][3];
