@@ -44,8 +44,13 @@ struct Ensemble {
     bool batched_pressure = false;
     size_t lds_x = 0, lds_y = 0;
     int xform = 0, yform = 0;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
+    // graphs of two steps, each for the roles it was recorded with (a step exchanges two of them)
+    struct StepGraph {
+        unsigned char key[7][3];
+        hipGraph_t graph;
+        hipGraphExec_t exec;
+    };
+    std::vector<StepGraph> graphs;
     std::vector<EnsGroup> groups;
     hipEvent_t fork = nullptr;
     Ctx *c0() const { return mem[0]; }
@@ -145,10 +150,16 @@ int make_groups(Ensemble *e, int n) {
 }
 
 void drop_graph(Ensemble *e) {
-    if (e->exec) (void)hipGraphExecDestroy(e->exec);
-    if (e->graph) (void)hipGraphDestroy(e->graph);
-    e->exec = nullptr;
-    e->graph = nullptr;
+    for (auto &sg : e->graphs) {
+        (void)hipGraphExecDestroy(sg.exec);
+        (void)hipGraphDestroy(sg.graph);
+    }
+    e->graphs.clear();
+}
+hipGraphExec_t find_graph(const Ensemble *e) {
+    for (auto &sg : e->graphs)
+        if (!memcmp(sg.key, e->perm, sizeof(sg.key))) return sg.exec;
+    return nullptr;
 }
 
 // swap the current and forecast roles of u, v, w, theta in the ensemble and in every member context
@@ -416,9 +427,9 @@ int dyn_ensemble_step(dyn_ensemble *ens, int nsteps) {
     Ctx *c0 = e->c0();
     const int pairs = nsteps / 2;
     if (pairs > 0) {
-        if (!e->exec) {
-            unsigned char saved[7][3];
-            memcpy(saved, e->perm, sizeof(saved));
+        if (!find_graph(e)) {
+            Ensemble::StepGraph ng{};
+            memcpy(ng.key, e->perm, sizeof(ng.key));
             std::vector<std::vector<void *>> saved_prog;
             for (Ctx *c : e->mem) saved_prog.emplace_back(&c->prog[0][0], &c->prog[0][0] + 21);
             DYN_HIP(hipStreamBeginCapture(c0->stream, hipStreamCaptureModeThreadLocal));
@@ -426,20 +437,20 @@ int dyn_ensemble_step(dyn_ensemble *ens, int nsteps) {
             int rc = ens_step(e);
             if (!rc) rc = ens_step(e);
             for (Ctx *c : e->mem) c->capturing = false;
-            hipGraph_t graph = nullptr;
-            hipError_t err = hipStreamEndCapture(c0->stream, &graph);
-            if (rc || err != hipSuccess || memcmp(saved, e->perm, sizeof(saved)) != 0) {
-                if (graph) (void)hipGraphDestroy(graph);
-                memcpy(e->perm, saved, sizeof(saved));
+            hipError_t err = hipStreamEndCapture(c0->stream, &ng.graph);
+            if (rc || err != hipSuccess || memcmp(ng.key, e->perm, sizeof(ng.key)) != 0) {
+                if (ng.graph) (void)hipGraphDestroy(ng.graph);
+                memcpy(e->perm, ng.key, sizeof(ng.key));
                 for (size_t m = 0; m < e->mem.size(); m++) memcpy(&e->mem[m]->prog[0][0], saved_prog[m].data(), sizeof(void *) * 21);
                 if (!rc) set_error(err != hipSuccess ? std::string("hipStreamEndCapture: ") + hipGetErrorString(err)
                                                      : std::string("internal: two ensemble steps did not restore the roles"));
                 return rc ? rc : DYN_E_HIP;
             }
-            DYN_HIP(hipGraphInstantiate(&e->exec, graph, nullptr, nullptr, 0));
-            e->graph = graph;
+            DYN_HIP(hipGraphInstantiate(&ng.exec, ng.graph, nullptr, nullptr, 0));
+            e->graphs.push_back(ng);
         }
-        for (int p = 0; p < pairs; p++) DYN_HIP(hipGraphLaunch(e->exec, c0->stream));
+        const hipGraphExec_t exec = find_graph(e);
+        for (int p = 0; p < pairs; p++) DYN_HIP(hipGraphLaunch(exec, c0->stream));
     }
     if (nsteps % 2) return ens_step(e);
     return DYN_OK;
