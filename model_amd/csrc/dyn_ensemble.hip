@@ -462,6 +462,8 @@ int dyn_ensemble_step(dyn_ensemble *ens, int nsteps) {
 int dyn_ensemble_autotune(dyn_ensemble *ens, int *shape_out) {
     Ensemble *e = reinterpret_cast<Ensemble *>(ens);
     if (!e) return DYN_E_ARG;
+    // steps still queued read the member tables, which every shape rewrites
+    DYN_HIP(hipStreamSynchronize(e->c0()->stream));
     drop_graph(e);
     const int tjs[3] = {2, 4, 8}, tis[4] = {8, 16, 32, 64};
     for (int kern = 0; kern < 2; kern++) {
