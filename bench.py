@@ -266,7 +266,8 @@ def ensemble_bench(steps, warmup):
     members = [DynCore(c, precision=DYN_FP32) for c in cases]
     pts = sum(c.interior_points for c in cases)
     ens = Ensemble(members)
-    shape = ens.autotune()
+    ens.autotune()
+    shape = ens.shape
     groups = ens.groups
     ens.step(warmup)
     ens.sync()

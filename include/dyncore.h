@@ -267,10 +267,14 @@ int dyn_ensemble_destroy(dyn_ensemble *ens);
 int dyn_ensemble_synchronize(dyn_ensemble *ens);
 int dyn_ensemble_step(dyn_ensemble *ens, int nsteps);
 int dyn_ensemble_step_eager(dyn_ensemble *ens, int nsteps);
-/* launch shape {momentum rows per block, momentum march length, scalar rows, scalar march length} */
+/* launch shape {momentum rows per block, momentum march length, scalar rows, scalar march length}: rows 2, 4 or 8, or
+ * with NZ <= 56 any number from 2 whose levels fit 512 threads and the LDS; march lengths 2 .. 512.
+ * dyn_ensemble_shape writes the shape in force to shape[4]; dyn_ensemble_create chooses one from the members' sizes. */
 int dyn_ensemble_set_shape(dyn_ensemble *ens, const int *shape);
-/* times every shape of the two stage kernels on the members' grids and keeps the fastest (written to
- * shape_out[4] when not NULL); the model state is unchanged */
+int dyn_ensemble_shape(dyn_ensemble *ens, int *shape);
+/* times the two stage kernels on the members' grids, with 2, 4 and 8 rows and marches of 8 to 64 columns; the fastest
+ * (written to shape_out[4] when not NULL) is taken for each kernel where it beats the shape in force, which stays
+ * otherwise; the model state is unchanged */
 int dyn_ensemble_autotune(dyn_ensemble *ens, int *shape_out);
 /* splits the members into ngroups groups of about equal point counts, each advanced by the same batched
  * launches on a stream of its own (forked from and joined back into the first member's stream, one

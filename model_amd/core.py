@@ -31,7 +31,7 @@ EXPORTS = [
     "dyn_stream", "dyn_tune_set", "dyn_tune_get", "dyn_adjoint_record", "dyn_adjoint_backward", "dyn_adjoint_release",
     "dyn_adjoint_interval",
     "dyn_ensemble_create", "dyn_ensemble_destroy", "dyn_ensemble_synchronize", "dyn_ensemble_step", "dyn_ensemble_step_eager",
-    "dyn_ensemble_set_shape", "dyn_ensemble_autotune", "dyn_ensemble_set_groups", "dyn_ensemble_groups",
+    "dyn_ensemble_set_shape", "dyn_ensemble_shape", "dyn_ensemble_autotune", "dyn_ensemble_set_groups", "dyn_ensemble_groups",
     "dyn_get_field_noalloc", "dyn_check_finite", "dyn_output_stage", "dyn_output_ready", "dyn_output_get", "dyn_netcdf_create", "dyn_netcdf_init",
     "dyn_netcdf_write_staged", "dyn_netcdf_put", "dyn_netcdf_read", "dyn_netcdf_records", "dyn_netcdf_set_status",
     "dyn_netcdf_get_status", "dyn_set_turbulence", "dyn_calculate_diff_tend", "dyn_apply_velocity_diffusion",
@@ -110,6 +110,7 @@ def load():
     for fn in ("dyn_ensemble_step", "dyn_ensemble_step_eager"):
         getattr(L, fn).argtypes = [ctypes.c_void_p, ctypes.c_int]
     L.dyn_ensemble_set_shape.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int)]
+    L.dyn_ensemble_shape.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int)]
     L.dyn_ensemble_autotune.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int)]
     L.dyn_ensemble_set_groups.argtypes = [ctypes.c_void_p, ctypes.c_int]
     L.dyn_ensemble_groups.argtypes = [ctypes.c_void_p]
@@ -267,7 +268,15 @@ class Ensemble:
         arr = (ctypes.c_int * 4)(*shape)
         _check(self.L.dyn_ensemble_set_shape(self.h, arr))
 
+    @property
+    def shape(self):
+        """Rows per block and march length in force: momentum, then scalars."""
+        arr = (ctypes.c_int * 4)()
+        _check(self.L.dyn_ensemble_shape(self.h, arr))
+        return tuple(arr)
+
     def autotune(self):
+        """The fastest of the timed shapes; `shape` is what it left in force."""
         arr = (ctypes.c_int * 4)()
         _check(self.L.dyn_ensemble_autotune(self.h, arr))
         return tuple(arr)

@@ -1745,6 +1745,12 @@ int fused_lds_limits(Ctx *c, bool turbulence) {
     return turbulence ? run(std::true_type{}) : run(std::false_type{});
 }
 
+// rows per block that a batch's stage kernels take: any number of packed rows that fit, else the instances' own
+bool ens_rows_ok(const Ctx *c0, bool momentum, int tj) {
+    if (!stage_packs(c0)) return tj == 2 || tj == 4 || tj == 8;
+    return tj >= 2 && tj <= kPackThreads / c0->g.nz && stage_lds(c0, momentum, tj, c0->g.nz) <= c0->pp.lds_max;
+}
+
 // The model's shape for a batch's blocks; without packed rows the nominal one.  Most batches fill the chip many times
 // over, so what counts is whole groups of four wavefronts and long marches (32 FP32 members of 96 to 192 points a
 // side and 40 levels, in two batches: momentum 265 us a launch in blocks of 8 rows and 16 columns, 200 in the model's;
@@ -1757,7 +1763,7 @@ void choose_ens_shape(const Ctx *c0, const std::vector<std::pair<int, int>> &sid
         if (!stage_packs(c0)) continue;
         double best = 0.0;
         for (int tj = 2; tj * c0->g.nz <= kPackThreads; tj++) {
-            if (stage_lds(c0, m == 0, tj, c0->g.nz) > c0->pp.lds_max) continue;
+            if (!ens_rows_ok(c0, m == 0, tj)) continue;
             for (int ti = 2; ti <= 48; ti++) {
                 long long n = 0;
                 for (const auto &p : sides) n += (long long)((p.second + tj - 1) / tj) * ((p.first + ti - 1) / ti);

@@ -332,7 +332,8 @@ int pressure_ens_prepare(const Ctx *c);
 // xform: the i passes with up to three butterflies a thread (0), four (1), four and members by matrix products (2); yform: the j pass in blocks of 512 threads (0), of 1024 (1), of 1024 with members by matrix products (2)
 int launch_pressure_ens(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &ro, double step, int tot_px, int tot_py, size_t lds_x,
                         size_t lds_y, int xform, int yform);
-// rows per block and march length {momentum, scalars} for a batch of members of these sides
+// rows per block and march length {momentum, scalars} for a batch of members of these sides, and the rows a batch takes
+bool ens_rows_ok(const Ctx *c0, bool momentum, int tj);
 void choose_ens_shape(const Ctx *c0, const std::vector<std::pair<int, int>> &sides, int *shape);
 // launch shapes of the stage kernels (DYN_TUNE_*): validity and the value in force
 bool fused_shape_ok(const Ctx *c, int param, int value);
