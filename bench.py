@@ -120,21 +120,20 @@ def time_form(case, precision, steps, warmup, stage_streams):
                                             "wall_ms_per_step": [round(x, 4) for x in wall_ms]}
 
 
-def kernel_profile(g, steps, fused, shape=None):
+def kernel_profile(g, steps, fused, shape=None, stage_streams=0):
     """Per-kernel HIP-event timings of the same step sequence the graph replays, launched eagerly, with
     the whole stage on one stream: the scalar half, which the step runs beside the pressure solve, would
     otherwise share the GPU with the kernels it overlaps and its duration would not be its own.  On one
     stream the stage kernels take the library's one-stream launch shapes; `shape` (a dict), when given,
-    receives them."""
+    receives them.  stage_streams is the knob's value afterwards."""
     from model_amd.core import DYN_TUNE_STAGE_STREAMS
-    before = g.tune_get(DYN_TUNE_STAGE_STREAMS)
     g.tune_set(DYN_TUNE_STAGE_STREAMS, 1)
     if shape is not None:
         shape.update(launch_shape(g))
     g.timing(1)
     (g.step_fused if fused else g.step_reference)(steps)
     g.sync()
-    g.tune_set(DYN_TUNE_STAGE_STREAMS, before)
+    g.tune_set(DYN_TUNE_STAGE_STREAMS, stage_streams)
     import ctypes
     buf = ctypes.create_string_buffer(1 << 16)
     g.timing_report(buf, len(buf))
@@ -149,8 +148,8 @@ def kernel_profile(g, steps, fused, shape=None):
 def launch_shape(g):
     """Rows per block and march length of the two stage kernels as the context launches them now."""
     from model_amd.core import DYN_TUNE_MOMENTUM_TI, DYN_TUNE_MOMENTUM_TJ, DYN_TUNE_SCALAR_TI, DYN_TUNE_SCALAR_TJ
-    return {"momentum_rows": g.tune_get(DYN_TUNE_MOMENTUM_TJ), "momentum_march": g.tune_get(DYN_TUNE_MOMENTUM_TI),
-            "scalar_rows": g.tune_get(DYN_TUNE_SCALAR_TJ), "scalar_march": g.tune_get(DYN_TUNE_SCALAR_TI)}
+    return {"momentum_rows": g.tune_in_force(DYN_TUNE_MOMENTUM_TJ), "momentum_march": g.tune_in_force(DYN_TUNE_MOMENTUM_TI),
+            "scalar_rows": g.tune_in_force(DYN_TUNE_SCALAR_TJ), "scalar_march": g.tune_in_force(DYN_TUNE_SCALAR_TI)}
 
 
 def roofline(rows, elt, moist):
@@ -431,14 +430,14 @@ def main():
     for name, prec in ([] if args.profile_only else forms):
         g, ms, reps = time_form(case, prec, args.steps, args.warmup, args.stage_streams)
         res[name] = {"ms_per_step": round(ms, 4), "value": round(npts / (ms * 1e-3), 1),
-                     "stage_streams": g.tune_get(DYN_TUNE_STAGE_STREAMS), **reps}
+                     "stage_streams": g.tune_in_force(DYN_TUNE_STAGE_STREAMS), **reps}
         handles[name] = g
         log(f"bench: {name} {ms:.3f} ms/step (median of {REPEATS} x {args.steps} steps), "
             f"{res[name]['value']:.4g} gridpoint-steps/s")
     main_form = forms[0][0]
     g = handles[main_form]
     step_shape, profile_shape = launch_shape(g), {}
-    rows = kernel_profile(g, args.profile_steps, fused=True, shape=profile_shape)
+    rows = kernel_profile(g, args.profile_steps, fused=True, shape=profile_shape, stage_streams=args.stage_streams)
     for r in sorted(rows, key=lambda r: -r[2]):
         log(f"bench: kernel {r[0]:16s} launches {r[1]:5d} total {r[2]:9.3f} ms avg {r[2] / r[1] * 1e3:8.1f} us")
     roof = roofline(rows, 4 if main_form == "fp32" else 8, case.microphysics)

@@ -161,12 +161,14 @@ void *dyn_stream(dyn_ctx *ctx);
 
 /* ---- launch-shape parameters ------------------------------------------------------------- */
 /* Knobs of the fused kernels (no counterpart in the reference: they set how the work maps onto the
- * GPU, never what is computed).  0 restores the built-in default; a value the kernels do not support
- * returns DYN_E_ARG.  Setting a knob drops the captured step graph.  dyn_tune_get returns a knob's value or
- * its nominal default.  While the knobs of a stage kernel are unset, grids whose nominal blocks would leave
- * compute units idle, and level counts far from a wavefront's 64 lanes, are launched in a shape chosen from
- * the grid's size instead, and DYN_TUNE_STAGE_STREAMS likewise (small grids run both halves of a stage in one
- * launch on one stream while all five are unset); the values computed never depend on it. */
+ * GPU).  0 restores the built-in default; a value the kernels do not support returns DYN_E_ARG.  Setting a knob
+ * drops the captured step graphs.  While the knobs of a stage kernel are unset, grids whose nominal blocks would
+ * leave compute units idle, and level counts far from a wavefront's 64 lanes, are launched in a shape chosen
+ * from the grid's size, and DYN_TUNE_STAGE_STREAMS likewise (small grids run both halves of a stage in one launch
+ * on one stream while the five of them are unset).  dyn_tune_get returns the value set, or for an unset knob its
+ * nominal default (the ones below); dyn_tune_in_force what the next step is launched with.  Of the knobs only
+ * DYN_TUNE_PRESSURE_JPASS reaches the values computed, by rounding: the forms order the sums of the j
+ * transforms in their own ways, matrix products and radix passes among them. */
 enum {
     DYN_TUNE_MOMENTUM_TJ = 0, /* j-rows per block of the momentum stage kernel: 2, 4, 8 or 16 (16, like 8,
                                  only with one wavefront per column) */
@@ -178,7 +180,8 @@ enum {
     DYN_TUNE_SCALAR_TI = 3,   /* columns one scalar block marches along i: 2 .. 512.  With 12 rows the
                                  default fills the device with one wave of blocks (at least 16) */
     DYN_TUNE_PRESSURE_JPASS = 4, /* pressure j pass: 1 one LDS-resident kernel per kx (when the slab fits), 2 three
-                                    kernels, 3 two LDS-resident kernels per kx on half slabs (even NY, when they fit) */
+                                    kernels, 3 two LDS-resident kernels per kx on half slabs (even NY, when they fit).
+                                    Lengths by matrix products take 1 where a slab has few tiles, else 2 */
     DYN_TUNE_STAGE_STREAMS = 5,  /* fused step: 1 runs the whole stage on the context's stream; 2 runs a
                                     stage's scalar half on a second stream beside the pressure solve, forked
                                     after the momentum kernel; 3 the same, forked after the solve's first
@@ -189,6 +192,7 @@ enum {
 };
 int dyn_tune_set(dyn_ctx *ctx, int param, int value);
 int dyn_tune_get(dyn_ctx *ctx, int param);
+int dyn_tune_in_force(dyn_ctx *ctx, int param);
 
 /* ---- output: asynchronous staging and the reference's NetCDF file ------------------------------- */
 /* The reference writes u, v, w, pi, theta (and qv, qc, qr, rainfall when moist) every outfilefreq steps

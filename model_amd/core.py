@@ -28,7 +28,7 @@ EXPORTS = [
     "dyn_solve_pressure", "dyn_pgf", "dyn_apply_bc", "dyn_apply_bc_micro", "dyn_kessler", "dyn_rayleigh",
     "dyn_advance_inner", "dyn_advance_outer", "dyn_micro_advance_inner", "dyn_micro_advance_outer",
     "dyn_step_reference", "dyn_step", "dyn_step_fused", "dyn_algorithmic_bytes_per_point", "dyn_timing", "dyn_timing_report",
-    "dyn_stream", "dyn_tune_set", "dyn_tune_get", "dyn_adjoint_record", "dyn_adjoint_backward", "dyn_adjoint_release",
+    "dyn_stream", "dyn_tune_set", "dyn_tune_get", "dyn_tune_in_force", "dyn_adjoint_record", "dyn_adjoint_backward", "dyn_adjoint_release",
     "dyn_adjoint_interval",
     "dyn_ensemble_create", "dyn_ensemble_destroy", "dyn_ensemble_synchronize", "dyn_ensemble_step", "dyn_ensemble_step_eager",
     "dyn_ensemble_set_shape", "dyn_ensemble_shape", "dyn_ensemble_autotune", "dyn_ensemble_set_groups", "dyn_ensemble_groups",
@@ -100,6 +100,7 @@ def load():
     L.dyn_stream.argtypes = [ctypes.c_void_p]
     L.dyn_tune_set.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int]
     L.dyn_tune_get.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    L.dyn_tune_in_force.argtypes = [ctypes.c_void_p, ctypes.c_int]
     L.dyn_adjoint_record.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int]
     L.dyn_adjoint_backward.argtypes = [ctypes.c_void_p] + [_dp] * 8
     L.dyn_adjoint_release.argtypes = [ctypes.c_void_p]
@@ -232,6 +233,11 @@ class DynCore:
 
     def tune_get(self, param: int) -> int:
         v = self.L.dyn_tune_get(self.h, param)
+        _check(min(v, 0))
+        return v
+
+    def tune_in_force(self, param: int) -> int:
+        v = self.L.dyn_tune_in_force(self.h, param)
         _check(min(v, 0))
         return v
 

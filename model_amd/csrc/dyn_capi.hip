@@ -1204,6 +1204,12 @@ int dyn_tune_get(dyn_ctx *ctx, int param) {
     return fused_shape(c, param);
 }
 
+int dyn_tune_in_force(dyn_ctx *ctx, int param) {
+    Ctx *c = as_ctx(ctx);
+    if (!c || param < 0 || param >= DYN_TUNE_COUNT) return DYN_E_ARG;
+    return tune_in_force(c, param);
+}
+
 }  // extern "C"
 
 namespace dyn {

@@ -1645,6 +1645,19 @@ int stage_streams(const Ctx *c) {
     return nominal == 2 && c->g.microphysics && c->npts >= 3000000u ? nominal : 4;
 }
 
+int tune_in_force(const Ctx *c, int param) {
+    const bool one = stage_in_one(c);
+    switch (param) {
+    case DYN_TUNE_MOMENTUM_TJ: return one ? c->auto_one.tj : stage_shape(c, true).tj;
+    case DYN_TUNE_MOMENTUM_TI: return one ? c->auto_one.ti_mom : stage_shape(c, true).ti;
+    case DYN_TUNE_SCALAR_TJ: return one ? c->auto_one.tj : stage_shape(c, false).tj;
+    case DYN_TUNE_SCALAR_TI: return one ? c->auto_one.ti_scal : stage_shape(c, false).ti;
+    case DYN_TUNE_PRESSURE_JPASS: return pressure_jpass(c);
+    case DYN_TUNE_STAGE_STREAMS: return one ? 1 : stage_streams(c);
+    default: return DYN_E_ARG;
+    }
+}
+
 namespace {
 // auto_shape of both kernels; left empty (tj = 0) where the nominal shape is kept
 void choose_stage_shapes(Ctx *c) {

@@ -335,10 +335,12 @@ int launch_pressure_ens(Ctx *c0, const EnsMember *d, int nmem, const EnsRoles &r
 // rows per block and march length {momentum, scalars} for a batch of members of these sides, and the rows a batch takes
 bool ens_rows_ok(const Ctx *c0, bool momentum, int tj);
 void choose_ens_shape(const Ctx *c0, const std::vector<std::pair<int, int>> &sides, int *shape);
-// launch shapes of the stage kernels (DYN_TUNE_*): validity and the value in force
+// launch shapes of the stage kernels (DYN_TUNE_*): validity, the set or nominal value, and what is in force
 bool fused_shape_ok(const Ctx *c, int param, int value);
 int fused_shape(const Ctx *c, int param);
 StageShape stage_shape(const Ctx *c, bool momentum);
 int stage_streams(const Ctx *c);
+int pressure_jpass(const Ctx *c);
+int tune_in_force(const Ctx *c, int param);  // ... as the next step launches it
 
 }  // namespace dyn

@@ -2400,6 +2400,9 @@ int pressure_free(Ctx *c) {
     return DYN_OK;
 }
 
+// the form of the j pass in force (the full complex spectrum has the one with three kernels)
+int pressure_jpass(const Ctx *c) { return c->pp.smooth_x || c->pp.dftx ? jpass_in_use(c) : 2; }
+
 int launch_solve_pressure(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
     return c->prec == DYN_FP32 ? solve_t<float>(c, step, halos, after_i, arg) : solve_t<double>(c, step, halos, after_i, arg);
 }
