@@ -2011,7 +2011,7 @@ int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
         const int jpass = jpass_in_use(c);
         int half = 0;
         if (jpass == 1) {
-            Timed _t(c, "p2_ypass", pts);
+            Timed _t(c, pp.ydft ? "p2_ypass_dft" : "p2_ypass", pts);
             launch_ypass<T, false>(c, spec, nkx, ry);
             DYN_LAUNCH_CHECK();
         } else if (jpass == 3) {
@@ -2024,7 +2024,7 @@ int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
             DYN_LAUNCH_CHECK();
         } else {
             {
-                Timed _t(c, "p2_fft_y", pts);
+                Timed _t(c, pp.dfty ? "p2_dft_y" : "p2_fft_y", pts);
                 launch_fft_y<T>(c, spec, nkx, ry, -1);
             }
             DYN_LAUNCH_CHECK();
@@ -2034,7 +2034,7 @@ int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
             }
             DYN_LAUNCH_CHECK();
             {
-                Timed _t(c, "p4_ifft_y", pts);
+                Timed _t(c, pp.dfty ? "p4_idft_y" : "p4_ifft_y", pts);
                 launch_fft_y<T>(c, spec, nkx, ry, +1);
             }
             DYN_LAUNCH_CHECK();
@@ -2199,7 +2199,7 @@ int solve_adjoint_t(Ctx *c, double step, T *uh, T *vh, T *wh, T *r1, T *r2) {
     const int jpass = jpass_in_use(c);
     int half = 0;
     if (jpass == 1) {
-        Timed _t(c, "adj_ypass", pts);
+        Timed _t(c, pp.ydft ? "adj_ypass_dft" : "adj_ypass", pts);
         launch_ypass<T, true>(c, spec, nkx, ry);
         DYN_LAUNCH_CHECK();
     } else if (jpass == 3) {
@@ -2211,7 +2211,7 @@ int solve_adjoint_t(Ctx *c, double step, T *uh, T *vh, T *wh, T *r1, T *r2) {
                            c->stream, (const T *)spec, (T *)pp.spec2, pp.nk2, rh, pp.twy, ta, pad);
         DYN_LAUNCH_CHECK();
     } else {
-        Timed _t(c, "adj_ypass", pts);
+        Timed _t(c, pp.dfty ? "adj_dft_y" : "adj_ypass", pts);
         launch_fft_y<T>(c, spec, nkx, ry, -1);
         DYN_LAUNCH_CHECK();
         launch_thomas<T, true>(c, spec, nkx);
