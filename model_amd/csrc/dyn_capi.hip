@@ -860,11 +860,9 @@ static int fused_step(dyn_ctx *ctx, StageHook hook = nullptr, void *arg = nullpt
     // The scalar half of a stage reads the current buffers only and writes buffers nothing else in the
     // stage reads, so it runs on the second stream beside the pressure solve, which needs only the u,
     // v, w forecasts of the momentum half.  Forked after the momentum kernel (the head of the stage's
-    // critical path), its blocks fill the CUs the latency-bound transforms leave idle.  Where the j pass
-    // runs on half slabs, whose blocks each take most of a CU's LDS, it is forked after the solve's
-    // first pass instead (2.08 -> 1.99 ms per FP64 step at 256x256x64; elsewhere neutral or slower).
-    // Value 4 keeps the fork after the momentum kernel but queues (and captures) the scalar launches
-    // after the solve's first pass, which measured faster for FP64 on the other grids.
+    // critical path; value 2), its blocks fill the CUs the latency-bound transforms leave idle.  Value 3 forks
+    // it after the solve's first pass; value 4 keeps the fork after the momentum kernel but queues (and
+    // captures) the scalar launches after the solve's first pass.  stage_streams says which grids take which.
     const bool one = stage_in_one(c);
     const int streams = one ? 1 : stage_streams(c);
     const bool two = streams >= 2, late = streams >= 3;

@@ -1,5 +1,6 @@
 // Transforms as products with the matrices of their cosines and sines on the FP64 matrix units: lengths with
-// a prime factor above 5 (up to kDftMax), and the smooth lengths up to dft_x_smooth() (along i) and kDftYSmooth (along j).
+// a prime factor above 5 up to kDftMax, and smooth lengths up to dft_x_smooth() (along i) and kDftYSmooth (along j),
+// on the grids that pressure_init gives them to (all of these in FP64, fewer in FP32).
 //
 // A length-n transform needs only rows 0 .. n/2 of the cosine matrix C and the sine matrix S once its input
 // is folded into sums and differences of mirrored elements, E(i) = x(i) + x(n-i), D(i) = x(i) - x(n-i):
@@ -12,11 +13,11 @@
 // Sums run in FP64 in both forms.
 //
 // Measured, us of the i transforms (forward with the divergence, then inverse): against direct sums over the
-// prime factors, 194x100x40 FP32 194 + 185 -> 14.5 + 12.6, 251x251x94 FP64 2214 + 2166 -> 73 + 51; against the
-// radix passes of smooth lengths, FP64 64x64x40 20.6 + 18.7 -> 7.3 + 8.3, 192x192x40 42.2 + 33.4 -> 19.4 + 17.1,
-// 384x384x80 238 + 171 -> 211 + 141; FP32 64x64x40 14.9 + 14.2 -> 7.5 + 7.9, 192x192x40 27.3 + 23.7 -> 22.5 +
-// 18.1, but 256x256x64 33.1 + 28.3 -> 52.7 + 38.2: the work grows with n where the passes' grows with log n,
-// and FP32 passes move half the bytes, so FP32 changes over below 256.
+// prime factors, 194x100x40 FP32 moist 194 + 185 -> 14.5 + 12.6, 251x251x94 FP64 2214 + 2166 -> 73 + 51; against
+// the radix passes of smooth lengths, FP64 64x64x40 20.6 + 18.7 -> 7.3 + 8.3, 192x192x40 42.2 + 33.4 -> 19.4 +
+// 17.1, 384x384x80 238 + 171 -> 211 + 141; FP32 64x64x40 14.9 + 14.2 -> 7.5 + 7.9.  The work grows with n where the
+// passes' grows with log n, and FP32 passes move half the bytes, so FP32 changes over between 192 points (27.3 + 23.7
+// against 22.5 + 18.1 by products, 40 levels) and 256 (33.1 + 28.3 against 52.7 + 38.2, 64 levels).
 #pragma once
 
 #include <cmath>
@@ -27,7 +28,7 @@
 namespace dyn {
 namespace {
 
-// smooth lengths that take the matrix products: measured faster up to these (FP32 within the limits of pressure_init)
+// smooth lengths that may take the matrix products: measured faster up to these
 template <typename T>
 constexpr int dft_x_smooth() { return sizeof(T) == 4 ? 192 : 384; }
 constexpr int kDftYSmooth = 192, kDftYThree = 112;

@@ -1561,6 +1561,7 @@ int fused_shape(const Ctx *c, int param) {
         if (param == DYN_TUNE_SCALAR_TJ && scalar_one_round(c)) return 12;
         return tj;
     case DYN_TUNE_MOMENTUM_TI: return fused_waves(c) == 2 ? 32 : 16;  // 512x512x80: 32 measured 3 % faster
+    // (Nominal values; while the knobs are unset stage_streams and stage_shape decide.)
     // The scalar kernel beside the pressure solve (fork after the momentum kernel): 24 columns, about 2 %
     // faster per step than 16 (FP32 at 256x256x64 moist and 192x192x40 dry, FP64 at 192x192x40 dry).
     // Its 352 blocks at 256x256 leave most CUs one block, beside which a j-pass block still fits; alone
@@ -1638,7 +1639,9 @@ bool stage_in_one(const Ctx *c) {
 // With short marches the scalar kernel no longer delays the divergence pass it is queued behind, so the late
 // queueing (4) is the faster form nearly everywhere (us per step, nominal form against 4: FP32 moist 344 and
 // 319 at 128x128x64, 679 and 655 at 256x256x40; FP64 579 and 522 moist at 128x128x64, 1314 and 1239 dry at
-// 256x256x64); the largest moist FP32 grids keep the nominal form (256x256x64: 833 against 874).
+// 256x256x64); the largest moist FP32 grids keep the nominal form (256x256x64: 833 against 874).  FP64 moist on
+// half slabs at 256x256x64, us per step by form and scalar march: 2 1742 (16 columns) and 1785 (24), 3 1820 and 1804,
+// 4 1805 and 1737; 16 columns is the march in force.
 int stage_streams(const Ctx *c) {
     const int nominal = fused_shape(c, DYN_TUNE_STAGE_STREAMS);
     if (c->tune[DYN_TUNE_STAGE_STREAMS]) return nominal;

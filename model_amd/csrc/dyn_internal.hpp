@@ -104,7 +104,7 @@ struct PressurePlan {
     void *spec = nullptr;              // spectral work array [kx][ky][kk] complex (T)
     double *zpiv = nullptr;            // Thomas pivot reciprocals [kx][kk][ky] (FP64)
     // transform lengths whose factors are all 2, 3 and 5 (the in-place LDS transforms' butterflies); a
-    // length with a larger prime factor takes the matrix products, or above their largest length the
+    // length with a larger prime factor takes the matrix products, or where pressure_init gives it none the
     // out-of-place transforms, whose passes sum any radix
     bool smooth_x = true, smooth_y = true;
     // cosine and sine matrices of the lengths that are transformed by matrix products (dyn_dft.hpp)

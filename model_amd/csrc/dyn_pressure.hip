@@ -7,9 +7,9 @@
 //   P3  1/(ni*nj) scaling + tridiagonal solve in k, FP64      spec -> spec (in place)
 //   P4  backward DFT along j                                 spec -> spec
 //   P5  backward DFT along i + real part -> PI with the k=0/NZ-1 copies and periodic halos fused
-// The DFTs of lengths with factors 2, 3 and 5 are Stockham auto-sort passes over an LDS tile [n][kc] (radix
-// 4/2/3/5), batched over a chunk of kc consecutive levels so every global access is a contiguous kc-run of a
-// k column; other lengths are products with their matrices (dyn_dft.hpp).
+// The DFTs are Stockham auto-sort passes over an LDS tile [n][kc] (radix 4/2/3/5, direct sums for larger primes),
+// batched over a chunk of kc consecutive levels so every global access is a contiguous kc-run of a k column, or
+// products with their matrices (dyn_dft.hpp); pressure_init says which lengths take which.
 #include <cmath>
 #include <cstdlib>
 #include <type_traits>
@@ -1481,7 +1481,7 @@ __global__ void __launch_bounds__(ypass_threads<T>()) k_ypass(T *__restrict__ sp
 // One launch serves slabs of few tiles (a pair of products per wavefront, PT = 1: 48x48x40 FP32 a step of 138 us
 // against 143 with three launches, and the radix passes, a chain of two barriers per radix, take 19 us
 // instead of 14); with more, the matrix units of nkx CUs are outrun by three launches spread over all of them
-// (96x96x40 206 against 181 us), except in an ensemble's batch.
+// (a step at 96x96x40 FP32, forced to products, 206 against 181 us), except in an ensemble's batch.
 inline int dft_y_tiles(int nk2) { return (2 * nk2 + 15) / 16; }
 inline int dft_y_pairs(int n, int nk2) { return dft_pad(n) / 16 * dft_y_tiles(nk2); }  // (row tile, column tile)
 // doubles per row: 14 or 18 modulo 32, so that the two rows a half-wavefront of the products reads overlap in
@@ -1847,9 +1847,8 @@ void launch_dft_y(Ctx *c, const T *in, TO *out, int nrows, int sign) {
 inline size_t wide_spec_at(const PressurePlan &pp) { return ((size_t)(pp.ni / 2 + 1) * pp.nj * pp.nk2 * 8 + 15) & ~(size_t)15; }
 inline double *wide_spec(const PressurePlan &pp) { return (double *)((char *)pp.spec + wide_spec_at(pp)); }
 
-// one j transform of the three-kernel j pass over nrows kx rows: the matrix products for lengths with a
-// prime factor above 5, the power-of-two kernel when nj is a power of two and its plan fits, else the
-// mixed-radix one
+// one j transform of the three-kernel j pass over nrows kx rows: the matrix products where the plan has them, the
+// power-of-two kernel when nj is a power of two and its plan fits, else the mixed-radix one
 template <typename T>
 void launch_fft_y(Ctx *c, T *spec, int nrows, const Radix &ry, int sign) {
     const PressurePlan &pp = c->pp;
@@ -1924,9 +1923,9 @@ int x_level_chunk(const PressurePlan &pp, const Geo &g, const Radix &rx, size_t 
 }
 
 // The j pass of a solve while no form is asked for: the one-slab form by matrix products where a slab has few
-// tiles, three launches with them up to kDftYThree (96x96x40 FP32: 181 us per step against 189 with the radix
-// passes' slab, FP64 210 against 235), the nominal forms beyond (128x128x64 FP32: the slab takes 26 us, three
-// launches 38).
+// tiles, three launches with them up to kDftYThree (96x96x40 FP64: 210 us per step against 235 with the radix
+// passes' slab; 96x96x48 FP32: 42 us a solve with products on both sides against 53), the nominal forms beyond
+// (128x128x64 FP32: the slab takes 26 us, three launches 38).
 int jpass_in_use(const Ctx *c) {
     if (c->tune[DYN_TUNE_PRESSURE_JPASS]) return fused_shape(c, DYN_TUNE_PRESSURE_JPASS);
     if (c->pp.ydft) return 1;
@@ -1986,8 +1985,8 @@ int solve_t(Ctx *c, double step, bool halos, PressureHook after_i, void *arg) {
     T *spec = (T *)pp.spec;
     const double pts = (double)pp.ni * pp.nj * pp.nk2;
     const ThomasArgs ta = thomas_args(pp, c->g.nz);
-    // half-spectrum transforms, except for lengths with a prime factor above 5 that are too long for the
-    // matrix products: those take the full complex spectrum
+    // half-spectrum transforms, except along i for lengths with a prime factor above 5 that have no matrix
+    // products: those take the full complex spectrum
     if (pp.smooth_x || pp.dftx) {
         const int nkx = pp.ni / 2 + 1;
         const int kc = x_level_chunk(pp, g, rx, sizeof(T));
@@ -2297,10 +2296,18 @@ int pressure_init(Ctx *c) {
     // other don't give back (pi of 160x128x40, 6 steps, is 2 to 6e-6 off a 64-bit run either way, at 313 and
     // 314 us a step).  So smooth sides (even along i) take products on both or on neither, and only in domains up
     // to twice as many points wide as deep, where the change of rounding stays at 1e-5 of pi and below (2e-4 at
-    // 190x190x12 after two steps).  Dry domains wider than that keep the former passes whatever their factors, and
-    // with smooth sides past 64 points at every width that an ensemble can hold: its members' bits are those
-    // of runs alone, and a batch fills the chip without products (32 members of 96 to 192 points: 4.87 ms a
-    // step with them, 4.82 without).
+    // 190x190x12 after two steps).  Dry domains wider than that keep the passes without products whatever their
+    // factors.  Neither time nor the accuracy of a solve speaks for that: with the same winds, a dry context and a
+    // moist one (which takes the products) give, us a solve and pi's rms distance from a 64-bit solve, 303 and 2.3e-7
+    // against 95 and 5.7e-8 at 184x150x57, 449 and 2.1e-7 against 57 and 7.6e-8 at 194x100x40, 589 and 6.1e-7 against
+    // 36 and 6.9e-8 at 97x97x40, 39 and 1.7e-6 against 32 and 1.1e-6 at 45x75x30.  It keeps the results of dry
+    // runs: their pi is 2e-5 to 8e-4 off a 64-bit run after two steps by the winds' own rounding, whatever the
+    // transforms, and a change of transform moves it by as much.
+    // Dry grids with smooth sides past 64 points keep those passes at every width that an ensemble can hold: its
+    // members' bits are those of runs alone, and a batch of 32 members of 96 to 192 points takes 4.82 ms a step
+    // without products and 4.87 with them.  Single runs pay for it (us a solve without and with products, 46 and 36
+    // at 72x72x40, 44 and 37 at 80x80x40, 53 and 42 at 96x96x48); batches of members of 65 to 95 points were not
+    // measured.
     const int widest = std::max(pp.ni, pp.nj);
     const bool shallow = widest > 2 * c->g.nz, dry = !c->g.microphysics;
     bool prod_x = pp.ni <= (!pp.smooth_x ? kDftMax : f32 ? dft_x_smooth<float>() : dft_x_smooth<double>());
@@ -2410,7 +2417,7 @@ int launch_solve_pressure(Ctx *c, double step, bool halos, PressureHook after_i,
 
 
 // the pressure part of an ensemble member's table entry; false when the member cannot join the batched
-// solve (odd ni, or a (j, k) slab too large for the LDS-resident j pass)
+// solve (FP64, the full complex spectrum, or a (j, k) slab too large for the LDS-resident j pass)
 bool pressure_ens_fill(Ctx *c, EnsMember &e, size_t &lds_x, size_t &lds_y) {
     PressurePlan &pp = c->pp;
     const int jpass = jpass_in_use(c);
