@@ -263,8 +263,9 @@ int dyn_adjoint_release(dyn_ctx *ctx);
  * An ensemble advances existing contexts of possibly different NX, NY (same precision and NZ, dry,
  * NZ <= 64) together: every pass of the step is one launch over all members' work, and
  * dyn_ensemble_step replays a captured hipGraph.  Members must outlive the ensemble; call
- * dyn_ensemble_synchronize before reading or writing a member's fields.  Per member the results are
- * bit for bit those of dyn_step on that member alone. */
+ * dyn_ensemble_synchronize before reading or writing a member's fields or stepping it on its own (and
+ * dyn_synchronize on the member after that).  Per member the results are bit for bit those of dyn_step on
+ * that member alone. */
 typedef struct dyn_ensemble dyn_ensemble;
 int dyn_ensemble_create(dyn_ctx *const *members, int n, dyn_ensemble **out);
 int dyn_ensemble_destroy(dyn_ensemble *ens);

@@ -162,6 +162,24 @@ hipGraphExec_t find_graph(const Ensemble *e) {
     return nullptr;
 }
 
+// A member that was stepped on its own has exchanged its buffers since: take every member's roles as they are now
+// (between calls; the tables and graphs of the former roles go)
+int follow_members(Ensemble *e) {
+    bool same = true;
+    for (int m = 0; m < e->nmem; m++)
+        for (int f = 0; f < 7; f++)
+            for (int r = 0; r < 3; r++) same = same && e->h[m].buf[f][e->perm[f][r]] == e->mem[m]->prog[f][r];
+    if (same) return DYN_OK;
+    DYN_HIP(hipStreamSynchronize(e->c0()->stream));
+    drop_graph(e);
+    for (int f = 0; f < 7; f++)
+        for (int r = 0; r < 3; r++) {
+            e->perm[f][r] = (unsigned char)r;
+            for (int m = 0; m < e->nmem; m++) e->h[m].buf[f][r] = e->mem[m]->prog[f][r];
+        }
+    return layout(e);
+}
+
 // swap the current and forecast roles of u, v, w, theta in the ensemble and in every member context
 void advance_roles(Ensemble *e) {
     const int fs[4] = {DYN_U, DYN_V, DYN_W, DYN_TH};
@@ -413,6 +431,7 @@ int dyn_ensemble_synchronize(dyn_ensemble *ens) {
 int dyn_ensemble_step_eager(dyn_ensemble *ens, int nsteps) {
     Ensemble *e = reinterpret_cast<Ensemble *>(ens);
     if (!e) return DYN_E_ARG;
+    if (int rc = follow_members(e)) return rc;
     for (int n = 0; n < nsteps; n++) {
         int rc = ens_step(e);
         if (rc) return rc;
@@ -424,6 +443,7 @@ int dyn_ensemble_step(dyn_ensemble *ens, int nsteps) {
     Ensemble *e = reinterpret_cast<Ensemble *>(ens);
     if (!e) return DYN_E_ARG;
     if (nsteps <= 0) return DYN_OK;
+    if (int rc = follow_members(e)) return rc;
     Ctx *c0 = e->c0();
     const int pairs = nsteps / 2;
     if (pairs > 0) {
@@ -465,6 +485,7 @@ int dyn_ensemble_autotune(dyn_ensemble *ens, int *shape_out) {
     Ensemble *e = reinterpret_cast<Ensemble *>(ens);
     if (!e) return DYN_E_ARG;
     // steps still queued read the member tables, which every shape rewrites
+    if (int rc = follow_members(e)) return rc;
     DYN_HIP(hipStreamSynchronize(e->c0()->stream));
     drop_graph(e);
     const int tjs[3] = {2, 4, 8}, tis[4] = {8, 16, 32, 64};
